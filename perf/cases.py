@@ -105,6 +105,18 @@ def _activation(g, rows, cols, dtype):
     return x.to(dtype)
 
 
+def _tensors(case, seed):
+    """Weight, bias, input and output gradient of a layer."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    train = case["kind"] == "train"
+    weight = (0.02 * torch.randn(case["outf"], case["inf"], generator=g, device="cuda")).to(
+        TYPES[case["master"]] if train else torch.bfloat16)
+    bias = torch.randn(case["outf"], generator=g, device="cuda").bfloat16() if train or case["bias"] else None
+    x = _activation(g, case["tokens"], case["inf"], torch.bfloat16)
+    grad = (0.001 * torch.randn(case["tokens"], case["outf"], generator=g, device="cuda")).bfloat16() if train else None
+    return weight, bias, x, grad
+
+
 def prepare(case, seed):
     g = torch.Generator(device="cuda").manual_seed(seed)
     if case["kind"] == "quantize":
@@ -120,17 +132,14 @@ def prepare(case, seed):
     train = case["kind"] == "train"
     layer = nn.Linear(case["inf"], case["outf"], bias=train or case["bias"], device="cuda",
                       dtype=TYPES[case["master"]] if train else torch.bfloat16)
+    weight, bias, x, grad = _tensors(case, seed)
     with torch.no_grad():
-        layer.weight.copy_(0.02 * torch.randn(case["outf"], case["inf"], generator=g, device="cuda"))
+        layer.weight.copy_(weight)
         if layer.bias is not None:
-            layer.bias.copy_(torch.randn(case["outf"], generator=g, device="cuda"))
-            if train:
-                layer.bias = nn.Parameter(layer.bias.to(torch.bfloat16))
+            layer.bias = nn.Parameter(bias, requires_grad=train)
     model = nn.Sequential(layer)
-    x = _activation(g, case["tokens"], case["inf"], torch.bfloat16)
     if train:
         fos.quantize_model(model, fos.ModelQuantizationConfig(keep_master_weights=True, weight_scale_2d=True))
-        grad = (0.001 * torch.randn(case["tokens"], case["outf"], generator=g, device="cuda")).bfloat16()
         return {"case": case, "model": model, "x": x.requires_grad_(), "grad": grad, "seed": seed}
     if case["format"] == "mxfp4":  # (one rule, 1 x 32 blocks)
         config = fos.ModelQuantizationConfig(dtype="mxfp4", scale_rule="static_6")
@@ -178,3 +187,82 @@ def tolerance(case):
     # (one step of bf16 is up to 2^-7 of the value).  Against the fp64 product of the same operands rounded to bf16:
     # up to 1.2e-5 for NVFP4 and MXFP4 and 6.3e-5 for IF4, 7.8e-3 at most for one value
     return {"rel": 2.5e-4, "max": 0.032}
+
+
+def _e2m1(v):
+    # round to nearest, ties to even, on 0, 0.5, 1, 1.5, 2, 3, 4, 6
+    a = v.abs()
+    r = torch.where(a < 2, (a + a).round() / 2, torch.where(a < 4, a.round(), 2 * (a / 2).round()))
+    return r * v.sign()
+
+
+def _decoded(x, fmt, block2d):
+    """x quantized (the adaptive rule by squared error where the format has one) and read back, in plain torch.
+
+    Scales, codes and decisions follow the formats' fp32 arithmetic; what the codes stand for comes back in 64 bits.
+    """
+    rows, cols = x.shape
+    step = 32 if fmt == "mxfp4" else 16
+    tall = 16 if block2d else 1
+    x = nn.functional.pad(x.float(), (0, -cols % step, 0, -rows % tall))
+    amax = x.abs().max()
+    # (tensors: torch divides by a plain number on the GPU as a product with its reciprocal)
+    six, seven_sixths = (torch.tensor(v, device=x.device) for v in (6.0, 7 / 6))
+    out = torch.empty(x.shape, dtype=torch.float64, device=x.device)
+    for top in range(0, x.shape[0], 2048):
+        part = x[top : top + 2048]
+        blocks = part.reshape(-1, tall, part.shape[1] // step, step)
+        bmax = blocks.abs().amax((1, 3), keepdim=True)
+        if fmt == "mxfp4":  # smallest power of two that takes the block's maximum to at most 6
+            mantissa, exponent = torch.frexp(bmax / six)
+            exponent = torch.where(mantissa == 0.5, exponent - 1, exponent)
+            scale = torch.where(bmax > 0, torch.ldexp(torch.ones_like(bmax), exponent), 0)
+            read = _e2m1(torch.where(scale > 0, blocks / scale, 0)).double() * scale.double()
+        else:
+            whole = six * (448.0 if fmt == "if4" else 256.0)
+            enc, dec = whole / amax, amax / whole
+
+            def scaled(expand):
+                s = ((bmax / six) * enc * expand).to(torch.float8_e4m3fn).float()
+                return s, torch.where(s > 0, blocks * (1 / (dec * s)), 0)
+
+            def error(q, s, factor):
+                e = ((q * s * amax) * factor / whole - blocks) ** 2
+                # (added as the sum of a contiguous run is on the CPU: even and odd rows, halves, eight columns)
+                even, odd = e[:, 0], e[:, 1] if tall > 1 else None
+                for row in range(2, tall, 2):
+                    even, odd = even + e[:, row], odd + e[:, row + 1]
+                lanes = even[..., :8] + even[..., 8:]
+                if tall > 1:
+                    lanes = lanes + odd[..., :8] + odd[..., 8:]
+                total = lanes[..., 0]
+                for lane in range(1, 8):
+                    total = total + lanes[..., lane]
+                return total[:, None, :, None]
+
+            s6, v6 = scaled(1.0)
+            q6 = _e2m1(v6)
+            if fmt == "if4":  # the other candidate: whole numbers to 7 on the same scale, in sevenths of 6
+                qi = (v6 * seven_sixths).clamp(-7, 7).round()
+                integer = error(qi, s6, 6 / 7) < error(q6, s6, 1.0)
+                # (an integer block's values are defined as products in fp16)
+                read = torch.where(integer, (qi * (6 / 7)).half() * s6.half(), q6.half() * s6.half())
+            else:  # the other candidate: maximum at 4
+                s4, v4 = scaled(1.5)
+                q4 = _e2m1(v4)
+                read = torch.where(error(q4, s4, 1.0) < error(q6, s6, 1.0), q4 * s4, q6 * s6)
+            read = read.double() * amax.double() / whole.double()
+        out[top : top + 2048] = read.reshape(part.shape)
+    return out[:rows, :cols]
+
+
+def exact(case, seed):
+    if case["kind"] == "quantize":
+        return None  # (whole numbers and bytes)
+    weight, bias, x, grad = _tensors(case, seed)
+    fmt = case.get("format", "nvfp4")
+    out = _decoded(x, fmt, False) @ _decoded(weight, fmt, fmt != "mxfp4").T
+    if bias is not None:
+        out += bias.double()
+    # (the gradients of input and weight are products of randomly rounded operands)
+    return (out, None, None, grad.double().sum(0)) if case["kind"] == "train" else out
