@@ -444,6 +444,30 @@ def test_gemm_records_the_output_maximum(m, n, k, out_dtype):
     assert float(amax) == float(out.float().abs().max())
 
 
+@pytest.mark.parametrize(("m", "n", "k", "env"), [
+    (1, 128, 4096, {"FOS_GEMM_SPLITK": "2"}),    # 32 quads for the reduction's one workgroup
+    (33, 384, 2048, {"FOS_GEMM_SPLITK": "3"}),   # four workgroups, the last one partly idle
+    (128, 4096, 4096, {"FOS_GEMM_SPLITK": "2"}),
+    (128, 256, 512, {"FOS_GEMM_TILE": "32"}),    # four A tiles per wavefront, unsplit
+    (128, 256, 512, {"FOS_GEMM_TILE": "129"}),   # 128 x 256 tile
+    (256, 512, 320, {"FOS_GEMM_TILE": "256"}),
+    (256, 384, 320, {"FOS_GEMM_TILE": "128"}),
+])
+def test_recorded_maximum_over_whole_workgroups(monkeypatch, m, n, k, env):
+    """The maximum is folded once per workgroup: it may sit in any wavefront of any workgroup."""
+    from fouroversix_amd.quantize import known_amax
+
+    for name, value in env.items():
+        monkeypatch.setenv(name, value)
+    a, b = make_input("randn", (m, k), 71), make_input("randn", (n, k), 72)
+    qb = fos.quantize(b.cuda())
+    for row in (0, m // 2, m - 1):
+        boosted = a.clone()
+        boosted[row] *= 8
+        out = fos.quantized_matmul(fos.quantize(boosted.cuda()), qb, emit_amax=True)
+        assert float(known_amax(out)) == float(out.abs().max())
+
+
 def test_known_amax_follows_the_tensor():
     """quantize() uses a recorded maximum exactly as long as the tensor is the one that was
     measured: same result as measuring again; an in-place write or a new tensor drops it."""
