@@ -202,10 +202,8 @@ struct Staged {
 // Output tile of workgroup `bid`: workgroups with equal bid % 8 share an XCD; give each
 // XCD a contiguous run of tiles, ordered in column bands of 8 tile rows.
 FOS_DEVICE void tile_of(int bid, int tiles_m, int tiles_n, int &tm, int &tn) {
-    const int total = tiles_m * tiles_n;
-    const int per_xcd = (total + 7) / 8;
-    int t = (bid & 7) * per_xcd + (bid >> 3);
-    if (t >= total || (total & 7) != 0) t = bid;  // ragged counts: plain order
+    const int per_xcd = tiles_m * tiles_n / 8;
+    const int t = bid < 8 * per_xcd ? (bid & 7) * per_xcd + (bid >> 3) : bid;  // (the remainder in plain order)
     constexpr int kBand = 8;
     const int band = t / (kBand * tiles_n), in_band = t - band * kBand * tiles_n;
     const int rows = (tiles_m - band * kBand) < kBand ? (tiles_m - band * kBand) : kBand;
@@ -245,10 +243,13 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
     // (QUARTER: ld_half counts quarter rows, 0..3)
     const int ld_row = QUARTER ? tid >> 2 : tid >> 1, ld_half = QUARTER ? tid & 3 : tid & 1;
     const bool stager = __builtin_amdgcn_readfirstlane(tid) < 2 * BM;  // wavefront-uniform
-    const BufferRsrc ra = make_rsrc(p.A + m0 * kbytes, (uint32_t)(BM * kbytes));
-    const BufferRsrc rb = make_rsrc(p.B + n0 * kbytes, (uint32_t)(BN * kbytes));
-    const BufferRsrc rsa = make_rsrc(p.sfA + (m0 >> 7) * sf_groups * 512, (uint32_t)((BM >> 7) * sf_groups * 512));
-    const BufferRsrc rsb = make_rsrc(p.sfB + (n0 >> 7) * sf_groups * 512, (uint32_t)((BN >> 7) * sf_groups * 512));
+    // (M and N are multiples of 128: a 256-wide tile may hang over the last 128 rows or columns.  The descriptors end
+    // there, what lies beyond reads as zero codes with zero scales)
+    const uint32_t rows_a = (uint32_t)(p.M - m0 < BM ? p.M - m0 : BM), rows_b = (uint32_t)(p.N - n0 < BN ? p.N - n0 : BN);
+    const BufferRsrc ra = make_rsrc(p.A + m0 * kbytes, (uint32_t)(rows_a * kbytes));
+    const BufferRsrc rb = make_rsrc(p.B + n0 * kbytes, (uint32_t)(rows_b * kbytes));
+    const BufferRsrc rsa = make_rsrc(p.sfA + (m0 >> 7) * sf_groups * 512, (uint32_t)((rows_a >> 7) * sf_groups * 512));
+    const BufferRsrc rsb = make_rsrc(p.sfB + (n0 >> 7) * sf_groups * 512, (uint32_t)((rows_b >> 7) * sf_groups * 512));
     const uint32_t q_off = (uint32_t)(ld_row * kbytes + ld_half * (QUARTER ? 8 : 16));
     const uint32_t s_off = (uint32_t)((ld_row >> 7) * sf_groups * 512 + (ld_row & 31) * 16 + ((ld_row & 127) >> 5) * 4);
     // this lane's B rows: row (lane & 31) of tile j of the wavefront's columns, K half lane >> 5
@@ -422,10 +423,14 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
 
     // epilogue: acc[i][j][4*g + e] is D[m][n] with m = wm*WM*32 + i*32 + (lane & 31),
     // n = wn*WN*32 + j*32 + 8*g + 4*(lane >> 5) + e
+    // (32-row tiles and 32-column strips lie wholly inside or outside the output)
+    const bool strip_inside = (uint32_t)(wn * WN * 32) < rows_b;
+    static_assert(WN == 1 || BN == 128, "a wavefront's strip does not cross a multiple of 128 columns");
     if (OUT == kOutPartial) {
         float *P = p.partials + (int64_t)blockIdx.y * p.M * p.N;
 #pragma unroll
         for (int i = 0; i < WM; ++i) {
+            if (!strip_inside || (uint32_t)(wm * WM * 32 + i * 32) >= rows_a) break;
             const int64_t m = m0 + wm * WM * 32 + i * 32 + (lane & 31);
 #pragma unroll
             for (int j = 0; j < WN; ++j)
@@ -453,6 +458,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
     uint32_t umax = 0u;
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
+        if (!strip_inside || (uint32_t)(wm * WM * 32 + i * 32) >= rows_a) break;  // (uniform over the wavefront)
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
 #pragma unroll
@@ -1040,8 +1046,8 @@ static int launch_gemm(GemmParams &p, int out_type, hipStream_t s) {
     constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
     constexpr int kThreadsG = 64 * WAVES_M * WAVES_N;
     constexpr size_t lds_bytes = 2 * (size_t)BM * kPitch * sizeof(_Float16);  // two buffers of A
-    p.tiles_m = (int)(p.M / BM);
-    p.tiles_n = (int)(p.N / BN);
+    p.tiles_m = (int)((p.M + BM - 1) / BM);
+    p.tiles_n = (int)((p.N + BN - 1) / BN);
     dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.splits);
     auto kbf = gemm_nvfp4_kernel<WAVES_M, WAVES_N, WM, WN, kOutBF16, QUARTER>;
     auto kh = gemm_nvfp4_kernel<WAVES_M, WAVES_N, WM, WN, kOutF16, QUARTER>;
@@ -1094,6 +1100,37 @@ struct GemmPlan {
     int wide;    // M > 32: workgroups of 64 rows of B and 64 rows of A, four wavefronts with two by two tiles each
 };
 constexpr int kTargetWorkgroups = 256;
+
+// Time of `tiles` output tiles: whole generations (as many tiles as run at a time) at `generation` each, then the
+// last, partial one, whose time depends on how full the chip is (fewer compute units clock higher): `tail`, by
+// eighths of a generation.
+static float tiles_cost(int64_t tiles, int64_t per_generation, float generation, const float (&tail)[8]) {
+    const int64_t whole = tiles / per_generation, rest = tiles % per_generation;
+    if (rest == 0) return whole == 1 ? tail[7] : (float)whole * generation;
+    return (float)whole * generation + tail[(rest * 8 - 1) / per_generation];
+}
+
+// Tile size: the cheapest of the three by what their generations take (us at K = 4096; all scale with K).  256
+// workgroups of the 256 x 256 and 128 x 256 tiles run at a time, 512 of the 128 x 128 tile.  Measured with the
+// tile forced (72 shapes, 256 ... 6144 rows, N = 1024 ... 14336, K = 2048 ... 14336); where the choice differs from
+// "256 x 256 from 256 tiles on, 128 x 256 for 128 to 256 tiles, else 128 x 128":
+//   1024 x 14336 x 4096 (224 tiles of 256 x 256) 116 -> 94 us, 3072 x 4096 x 4096 (192) 93 -> 86,
+//   2560 x 4096 x 14336 (160) 275 -> 253, 6144 x 2560 x 2048 (240) 65 -> 55,
+//   1280 x 14336 x 4096 (280: a second generation nearly empty) 168 -> 141, 2560 x 8192 x 8192 (320) 322 -> 292.
+// A 256-wide tile over the edge of the output counts as a whole one.
+static int pick_tile(int64_t M, int64_t N, int forced) {
+    const int64_t m128 = M / 128, n128 = N / 128, m256 = (m128 + 1) / 2, n256 = (n128 + 1) / 2;
+    if (forced == 128 || M < 128) return kPlanSmall;
+    if (forced == 129) return kPlanWide;
+    if (forced == 256) return kPlanBig;
+    static const float big[8] = {69, 69, 70, 75, 79, 86, 94, 104}, wide[8] = {42, 43, 43, 44, 46, 49.5f, 54, 59},
+                       small[8] = {24, 34, 36.5f, 38.5f, 53, 56, 60, 64.5f};
+    const float cost_big = tiles_cost(m256 * n256, 256, 92, big), cost_wide = tiles_cost(m128 * n256, 256, 56, wide),
+                cost_small = tiles_cost(m128 * n128, 512, 59, small);
+    if (cost_big <= cost_wide && cost_big <= cost_small) return kPlanBig;
+    return cost_wide < cost_small ? kPlanWide : kPlanSmall;
+}
+
 static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K) {
     GemmPlan g;
     g.narrow = g.wide = 0;
@@ -1118,28 +1155,15 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K) {
             g.wide = 1;
             tiles = (N / 64) * (M > 64 ? 2 : 1);
         }
-    } else if ((M % 256 == 0) && (N % 256 == 0) && ((M / 256) * (N / 256) >= 256 || tile == 256) && tile != 128) {
-        // 256 x 256 tiles once they give each of the 256 compute units a workgroup
-        g.kind = kPlanBig;
-        g.splits = 1;
-        g.ksteps_per_split = (int)(K / BK);
-        return g;
-    } else if (tile != 128 && M % 128 == 0 && N % 256 == 0 && M >= 128 &&
-               (tile == 129 || ((M / 128) * (N / 256) > 128 && (M / 128) * (N / 256) <= 256))) {
-        // 128 x 256 tiles (eight wavefronts of 128 x 32; every thread stages a quarter row of A) where they give
-        // every compute unit at most one workgroup and more than half of them one: A is converted
-        // once per 256 columns instead of once per 128.  Against the 128 x 128 tile, alternating
-        // runs: 2048 x 4096 x 4096 71.9 -> 69.3 us, 2048 x 4096 x 14336 242.5 -> 228 us,
-        // 1792 x 4096 x 4096 67.0 -> 64.6 us; with 1.5 workgroups per compute unit
-        // (3072 x 4096 x 4096) 109 -> 123 us, with half a one (1024 x 4096 x 4096) 41.7 -> 51.8 us.
-        g.kind = kPlanWide;
-        g.splits = 1;
-        g.ksteps_per_split = (int)(K / BK);
-        return g;
     } else {
-        g.kind = kPlanSmall;
+        g.kind = pick_tile(M, N, tile);
+        if (g.kind != kPlanSmall) {
+            g.splits = 1;
+            g.ksteps_per_split = (int)(K / BK);
+            return g;
+        }
         steps = K / BK;
-        tiles = ((M + 127) / 128) * (N / 128);
+        tiles = (M / 128) * (N / 128);
     }
     // split so that about kTargetWorkgroups workgroups run, each with a useful share of K
     // (at M <= 32 a split must leave two steps per wavefront: 16 x 4096 x 4096 takes 6.4 us

@@ -468,6 +468,25 @@ def test_recorded_maximum_over_whole_workgroups(monkeypatch, m, n, k, env):
         assert float(known_amax(out)) == float(out.abs().max())
 
 
+@pytest.mark.parametrize("tile", ["129", "256"])
+@pytest.mark.parametrize(("m", "n", "k"), [(128, 128, 64), (384, 640, 320), (256, 384, 192), (640, 256, 1088)])
+def test_tiles_over_the_edge_of_the_output(monkeypatch, m, n, k, tile):
+    """A 256-wide tile that hangs over the last 128 rows or columns: the same bits as 128 x 128 tiles, bias and
+    recorded maximum included (the bias is larger than the product, so that a maximum over rows that do not
+    exist would show)."""
+    from fouroversix_amd.quantize import known_amax
+
+    qa, qb = fos.quantize(make_input("randn", (m, k), 73).cuda()), fos.quantize(make_input("weight", (n, k), 74).cuda())
+    bias = torch.linspace(-2, 40, n, device="cuda").bfloat16()
+    monkeypatch.setenv("FOS_GEMM_TILE", "128")
+    monkeypatch.setenv("FOS_GEMM_SPLITK", "1")
+    expect = fos.quantized_matmul(qa, qb, emit_amax=True, bias=bias)
+    monkeypatch.setenv("FOS_GEMM_TILE", tile)
+    out = fos.quantized_matmul(qa, qb, emit_amax=True, bias=bias)
+    assert torch.equal(out, expect)
+    assert float(known_amax(out)) == float(expect.abs().max())
+
+
 def test_known_amax_follows_the_tensor():
     """quantize() uses a recorded maximum exactly as long as the tensor is the one that was
     measured: same result as measuring again; an in-place write or a new tensor drops it."""
