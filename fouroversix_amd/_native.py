@@ -40,6 +40,8 @@ EXPORTS = (
     "fos_gemm_nvfp4_amax",
     "fos_gemm_nvfp4_amax_out",
     "fos_gemm_nvfp4_linear",
+    "fos_gemm_if4",
+    "fos_gemm_if4_workspace_bytes",
     "fos_gemm_mxfp4",
     "fos_gemm_alpha",
     "fos_padded_cols_for",
@@ -106,6 +108,10 @@ def lib() -> ctypes.CDLL:
     L.fos_gemm_nvfp4_amax_out.restype = i32
     L.fos_gemm_nvfp4_linear.argtypes = [vp, vp, vp, vp, vp, vp, dbl, i64, i64, i64, vp, i32, i64, vp, vp, vp, ctypes.c_size_t, vp]
     L.fos_gemm_nvfp4_linear.restype = i32
+    L.fos_gemm_if4.argtypes = [vp, vp, vp, vp, vp, vp, dbl, i64, i64, i64, vp, i32, i64, vp, vp, vp, ctypes.c_size_t, vp]
+    L.fos_gemm_if4.restype = i32
+    L.fos_gemm_if4_workspace_bytes.argtypes = [i64, i64, i64]
+    L.fos_gemm_if4_workspace_bytes.restype = ctypes.c_size_t
     L.fos_gemm_alpha.argtypes = [vp, vp, dbl, vp, vp]
     L.fos_gemm_alpha.restype = i32
     L.fos_gemm_mxfp4.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, vp, i32, i64, vp]

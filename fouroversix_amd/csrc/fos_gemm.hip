@@ -55,6 +55,7 @@ struct GemmParams {
     const float *alpha;        // output scale on the device, or null: (amax_a * amax_b) * inv_den
     const float *amax_a, *amax_b;
     float inv_den;
+    int tiny_scale;            // an output scale below the normal range is applied in two factors (load_alpha)
     void *D;
     const void *bias;          // optional: N values of the output type, added to the rounded product and rounded again
     float *d_amax;             // optional: max|D| as stored is folded into d_amax[0] (unsigned atomic max on the bits)
@@ -68,8 +69,17 @@ struct GemmParams {
 
 // Output scale: read from the device, or formed from the two tensor maxima with the
 // arithmetic of gemm_alpha_kernel (product, then times the fp32 reciprocal of the divisor).
-FOS_DEVICE float load_alpha(const GemmParams &p) {
-    return p.alpha ? *p.alpha : (*p.amax_a * *p.amax_b) * p.inv_den;
+// `post`: with tiny_scale, what is left to multiply alpha * acc with (1 otherwise): maxima whose product, divided by
+// the denominator, would be a sub-normal number with a few bits are multiplied 2^64 times too large.
+FOS_DEVICE float load_alpha(const GemmParams &p, float &post) {
+    post = 1.0f;
+    if (p.alpha) return *p.alpha;
+    const float a = *p.amax_a, b = *p.amax_b;
+    if (p.tiny_scale && a * b < 0x1p-90f) {
+        post = 0x1p-64f;
+        return ((fminf(a, b) * 0x1p64f) * fmaxf(a, b)) * p.inv_den;
+    }
+    return (a * b) * p.inv_den;
 }
 
 // One value of the result as stored: alpha * acc rounded to the output type (16 bits returned).
@@ -178,6 +188,47 @@ FOS_DEVICE half8_t dequant8(uint32_t word, half2_t s) {
     return r;
 }
 
+// 8 packed IF4 codes times their block scale -> 8 fp16 in k order.  A block holds E2M1 codes or (`integer`) two's
+// complement integers q with the value RN16(6/7 q), and the product with the scale is rounded to fp16: the
+// numbers the dequantization of the format is defined by (src/fouroversix/quantize/backend.py:89-160).
+// Blocks differ from lane to lane, so both decodings are formed and one is selected: 34 instructions a word
+// against 8 for E2M1 alone, and what bounds the product (2048 x 4096 x 4096 99 us, NVFP4 61;
+// two dequantize kernels, a library fp32 product and the conversion of its result took 570).  Integers: q + 8 = nibble ^ 8 is a byte 0 .. 15, which E4M3 reads as (q + 8) / 512 (the
+// sub-normals run on into the first normal binade); 6/7 q is then formed from a two-part constant, equal to the rounded
+// product for all 16 integers.
+FOS_DEVICE half8_t dequant8_if4(uint32_t word, half2_t s, bool integer) {
+    const uint32_t u = word ^ 0x88888888u, even = u & 0x0f0f0f0fu, odd = (u >> 4) & 0x0f0f0f0fu;
+    const uint32_t pairs[2] = {__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u)};
+    constexpr _Float16 hi = (_Float16)(6.0 / 7.0), lo = (_Float16)(6.0 / 7.0 - (double)hi);
+    const half2_t k512 = {(_Float16)512.0f, (_Float16)512.0f}, m8 = {(_Float16)-8.0f, (_Float16)-8.0f}, hi2 = {hi, hi}, lo2 = {lo, lo};
+    auto sevenths = [&](half2_t x) {
+        const half2_t q = __builtin_elementwise_fma(x, k512, m8);
+        return __builtin_elementwise_fma(q, hi2, q * lo2);
+    };
+    auto pick = [&](half2_t i, half2_t f) {
+        return __builtin_bit_cast(half2_t, integer ? __builtin_bit_cast(uint32_t, i) : __builtin_bit_cast(uint32_t, f)) * s;
+    };
+    const half2_t p0 = pick(sevenths(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pairs[0], 1.0f, false)),
+                            __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 0));
+    const half2_t p1 = pick(sevenths(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pairs[0], 1.0f, true)),
+                            __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 1));
+    const half2_t p2 = pick(sevenths(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pairs[1], 1.0f, false)),
+                            __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 2));
+    const half2_t p3 = pick(sevenths(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pairs[1], 1.0f, true)),
+                            __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 3));
+    half8_t r = {p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
+    return r;
+}
+
+// One word of block `blk` (0, 1) of the two whose scale bytes are the low 16 bits of `two`.
+template <bool IF4>
+FOS_DEVICE half8_t dequant_word(uint32_t word, uint32_t two, int blk) {
+    const half2_t s2 = e4m3x2_to_half2(IF4 ? two & 0x7f7fu : two);
+    const half2_t s = blk ? __builtin_shufflevector(s2, s2, 1, 1) : __builtin_shufflevector(s2, s2, 0, 0);
+    if constexpr (IF4) return dequant8_if4(word, s, (two & (blk ? 0x8000u : 0x80u)) != 0);
+    else return dequant8(word, s);
+}
+
 constexpr int BK = 64;
 constexpr int kPitch = BK + 8;  // halfs per LDS row (144 bytes: conflict-free 128-bit accesses)
 
@@ -219,7 +270,9 @@ enum { kOutF16 = 0, kOutBF16 = 1, kOutPartial = 2 };
 
 // QUARTER (4 * BM == threads): every thread stages a quarter row of A (16 codes) instead of the first 2 * BM threads
 // half a row each, so that all wavefronts carry the same conversion work.
-template <int WAVES_M, int WAVES_N, int WM, int WN, int OUT, bool QUARTER = false>
+// IF4: operands in the IF4 format, whose scale bytes lie row-major (K / 16 a row) with bit 7 marking integer blocks,
+// instead of NVFP4 with its 128 x 4 tiles; only the scales' addresses and the conversion differ.
+template <int WAVES_M, int WAVES_N, int WM, int WN, int OUT, bool QUARTER = false, bool IF4 = false>
 __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const GemmParams p) {
     constexpr bool OUT_BF16 = OUT == kOutBF16;
     constexpr int kThreadsG = 64 * WAVES_M * WAVES_N;
@@ -248,10 +301,15 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
     const uint32_t rows_a = (uint32_t)(p.M - m0 < BM ? p.M - m0 : BM), rows_b = (uint32_t)(p.N - n0 < BN ? p.N - n0 : BN);
     const BufferRsrc ra = make_rsrc(p.A + m0 * kbytes, (uint32_t)(rows_a * kbytes));
     const BufferRsrc rb = make_rsrc(p.B + n0 * kbytes, (uint32_t)(rows_b * kbytes));
-    const BufferRsrc rsa = make_rsrc(p.sfA + (m0 >> 7) * sf_groups * 512, (uint32_t)((rows_a >> 7) * sf_groups * 512));
-    const BufferRsrc rsb = make_rsrc(p.sfB + (n0 >> 7) * sf_groups * 512, (uint32_t)((rows_b >> 7) * sf_groups * 512));
+    // (either layout takes sf_groups * 4 bytes a row)
+    const BufferRsrc rsa = make_rsrc(p.sfA + m0 * sf_groups * 4, (uint32_t)(rows_a * sf_groups * 4));
+    const BufferRsrc rsb = make_rsrc(p.sfB + n0 * sf_groups * 4, (uint32_t)(rows_b * sf_groups * 4));
+    auto scale_offset = [&](int row) {
+        return (uint32_t)(IF4 ? row * sf_groups * 4 : (row >> 7) * sf_groups * 512 + (row & 31) * 16 + ((row & 127) >> 5) * 4);
+    };
+    constexpr uint32_t kScaleStep = IF4 ? 4u : 512u;
     const uint32_t q_off = (uint32_t)(ld_row * kbytes + ld_half * (QUARTER ? 8 : 16));
-    const uint32_t s_off = (uint32_t)((ld_row >> 7) * sf_groups * 512 + (ld_row & 31) * 16 + ((ld_row & 127) >> 5) * 4);
+    const uint32_t s_off = scale_offset(ld_row);
     // this lane's B rows: row (lane & 31) of tile j of the wavefront's columns, K half lane >> 5
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
     const int lh = lane >> 5;
@@ -260,7 +318,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
     for (int j = 0; j < WN; ++j) {
         const int row = wn * WN * 32 + j * 32 + (lane & 31);
         qb_off[j] = (uint32_t)(row * kbytes + lh * 16);
-        sb_off[j] = (uint32_t)((row >> 7) * sf_groups * 512 + (row & 31) * 16 + ((row & 127) >> 5) * 4);
+        sb_off[j] = scale_offset(row);
     }
     // this workgroup's share of the K steps (all of them unless the launch splits K)
     const int64_t ks0 = OUT == kOutPartial ? (int64_t)blockIdx.y * p.ksteps_per_split : 0;
@@ -270,7 +328,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
 
     typedef Staged<WN> StagedT;
     auto fetch = [&](int64_t ks, StagedT &s) {
-        const uint32_t kq = (uint32_t)(ks0 + ks) * 32u, ksf = (uint32_t)(ks0 + ks) * 512u;
+        const uint32_t kq = (uint32_t)(ks0 + ks) * 32u, ksf = (uint32_t)(ks0 + ks) * kScaleStep;
         if constexpr (QUARTER) {
             const uint2 w = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(ra, (int)q_off, (int)kq, 0));
             s.qa.x = w.x;
@@ -292,19 +350,15 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
             // the thread's 16 codes are one block: its two words go out in the first and the third slice of a step
             if (q & 1) return;
             const uint32_t wq = q == 0 ? s.qa.x : s.qa.y;
-            const half2_t s2 = e4m3x2_to_half2(s.sa >> (8 * ld_half));
-            const half2_t sq = __builtin_shufflevector(s2, s2, 0, 0);
             half8_t *dq = reinterpret_cast<half8_t *>(lds_a[buf] + ld_row * kPitch + ld_half * 16);
-            dq[q >> 1] = dequant8(wq, sq);
+            dq[q >> 1] = dequant_word<IF4>(wq, s.sa >> (8 * ld_half), 0);
             return;
         }
         if (!kAllStage && !stager) return;
         const uint32_t wa = q == 0 ? s.qa.x : q == 1 ? s.qa.y : q == 2 ? s.qa.z : s.qa.w;
         // this thread's two block scales: bytes 2*ld_half, 2*ld_half + 1
-        const half2_t sa2 = e4m3x2_to_half2(s.sa >> (16 * ld_half));
-        const half2_t sa = (q >> 1) ? __builtin_shufflevector(sa2, sa2, 1, 1) : __builtin_shufflevector(sa2, sa2, 0, 0);
         half8_t *da = reinterpret_cast<half8_t *>(lds_a[buf] + ld_row * kPitch + ld_half * 32);
-        da[q] = dequant8(wa, sa);
+        da[q] = dequant_word<IF4>(wa, s.sa >> (16 * ld_half), q >> 1);
     };
     // MFMA operands of slice kk from this lane's packed B rows: word kk of its 16 bytes, blocks
     // 2 h + (kk >> 1) of the step
@@ -312,9 +366,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
             const uint32_t wb = kk == 0 ? s.qb[j].x : kk == 1 ? s.qb[j].y : kk == 2 ? s.qb[j].z : s.qb[j].w;
-            const half2_t sb2 = e4m3x2_to_half2(s.sb[j] >> (16 * lh));
-            const half2_t sb = (kk >> 1) ? __builtin_shufflevector(sb2, sb2, 1, 1) : __builtin_shufflevector(sb2, sb2, 0, 0);
-            fb[j] = dequant8(wb, sb);
+            fb[j] = dequant_word<IF4>(wb, s.sb[j] >> (16 * lh), kk >> 1);
         }
     };
 
@@ -443,7 +495,8 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
         }
         return;
     }
-    const float alpha = load_alpha(p);
+    float post;
+    const float alpha = load_alpha(p, post);
     uint16_t *D = reinterpret_cast<uint16_t *>(p.D);
     // A lane holds 4 consecutive n of row m = lane & 31: written as they are, a store
     // instruction touches 32 rows with 16 bytes each, and the counters showed 2.2 bytes
@@ -463,8 +516,12 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
         for (int j = 0; j < WN; ++j) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const float v[4] = {alpha * acc[i][j][4 * g], alpha * acc[i][j][4 * g + 1], alpha * acc[i][j][4 * g + 2],
-                                    alpha * acc[i][j][4 * g + 3]};
+                float v[4] = {alpha * acc[i][j][4 * g], alpha * acc[i][j][4 * g + 1], alpha * acc[i][j][4 * g + 2],
+                              alpha * acc[i][j][4 * g + 3]};
+                if (IF4) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] *= post;
+                }
                 const int nl = j * 32 + 8 * g + 4 * (lane >> 5);  // column inside the wavefront's strip
                 *reinterpret_cast<uint2 *>(epi + (lane & 31) * kEpiPitch + nl * 2) =
                     pack_outputs<OUT_BF16>(v, p.bias, n0 + wn * WN * 32 + nl, umax);
@@ -719,7 +776,8 @@ __global__ __launch_bounds__(64 * skinny_waves(WN), (WN == 2 && MT == 2) ? 2 : 1
     };
 
     // read now, used in the epilogue: short launches would otherwise end on this latency
-    const float alpha = OUT == kOutPartial ? 0.0f : load_alpha(p);
+    float post;  // (1: NVFP4)
+    const float alpha = OUT == kOutPartial ? 0.0f : load_alpha(p, post);
 
     SkinnyRegs<MT, WN> st[2];
     int64_t step = wave;  // counts this workgroup's steps, see phys()
@@ -937,7 +995,8 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams
     };
 
     // read now, used in the epilogue: short launches would otherwise end on this latency
-    const float alpha = OUT == kOutPartial ? 0.0f : load_alpha(p);
+    float post;  // (1: NVFP4)
+    const float alpha = OUT == kOutPartial ? 0.0f : load_alpha(p, post);
 
     DecodeRegs<NB> st[kDepth];
     int64_t step = wave;  // counts this workgroup's steps, see phys()
@@ -1025,8 +1084,9 @@ __global__ __launch_bounds__(kReduceThreads) void gemm_reduce_kernel(const GemmP
         const float4 v = P[y * stride];
         s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
-    const float alpha = load_alpha(p);
-    const float v[4] = {alpha * s.x, alpha * s.y, alpha * s.z, alpha * s.w};
+    float post;
+    const float alpha = load_alpha(p, post);
+    const float v[4] = {(alpha * s.x) * post, (alpha * s.y) * post, (alpha * s.z) * post, (alpha * s.w) * post};
     uint32_t um = 0u;
     const uint2 o = pack_outputs<OUT_BF16>(v, p.bias, n, um);
     if (mine) *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.D) + m * p.ldd + n) = o;
@@ -1041,7 +1101,7 @@ static int launch_reduce(const GemmParams &p, int out_type, hipStream_t s) {
     return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;
 }
 
-template <int WAVES_M, int WAVES_N, int WM, int WN, bool QUARTER = false>
+template <int WAVES_M, int WAVES_N, int WM, int WN, bool QUARTER = false, bool IF4 = false>
 static int launch_gemm(GemmParams &p, int out_type, hipStream_t s) {
     constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
     constexpr int kThreadsG = 64 * WAVES_M * WAVES_N;
@@ -1049,9 +1109,9 @@ static int launch_gemm(GemmParams &p, int out_type, hipStream_t s) {
     p.tiles_m = (int)((p.M + BM - 1) / BM);
     p.tiles_n = (int)((p.N + BN - 1) / BN);
     dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.splits);
-    auto kbf = gemm_nvfp4_kernel<WAVES_M, WAVES_N, WM, WN, kOutBF16, QUARTER>;
-    auto kh = gemm_nvfp4_kernel<WAVES_M, WAVES_N, WM, WN, kOutF16, QUARTER>;
-    auto kp = gemm_nvfp4_kernel<WAVES_M, WAVES_N, WM, WN, kOutPartial, QUARTER>;
+    auto kbf = gemm_nvfp4_kernel<WAVES_M, WAVES_N, WM, WN, kOutBF16, QUARTER, IF4>;
+    auto kh = gemm_nvfp4_kernel<WAVES_M, WAVES_N, WM, WN, kOutF16, QUARTER, IF4>;
+    auto kp = gemm_nvfp4_kernel<WAVES_M, WAVES_N, WM, WN, kOutPartial, QUARTER, IF4>;
     auto kernel = p.splits > 1 ? kp : out_type == FOS_T_BF16 ? kbf : kh;
     if (lds_bytes > 64 * 1024) {
         // more than the default dynamic LDS limit: opt in (idempotent, no device state besides the function attribute)
@@ -1131,12 +1191,12 @@ static int pick_tile(int64_t M, int64_t N, int forced) {
     return cost_wide < cost_small ? kPlanWide : kPlanSmall;
 }
 
-static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K) {
+static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool if4) {
     GemmPlan g;
     g.narrow = g.wide = 0;
     const int tile = tuning().gemm_tile;  // tuning / tests: 128 = small tile, 129 = 128 x 256 tile and 256 = 256 x 256 tile wherever M and N allow, 1 = no weight-streaming kernel
     int64_t steps, tiles;
-    if (M <= 128 && K % 256 == 0 && (tile == 0 || tile == 16 || tile == 32 || tile == 64)) {
+    if (!if4 && M <= 128 && K % 256 == 0 && (tile == 0 || tile == 16 || tile == 32 || tile == 64)) {
         // one 128-row band: weight streaming, steps of 256 along K shared by 8 wavefronts
         g.kind = kPlanSkinny;
         steps = K / 256;
@@ -1207,14 +1267,14 @@ extern "C" int fos_gemm_alpha(const float *amax_a, const float *amax_b, double d
 extern "C" size_t fos_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || (M > 128 && M % 128 != 0) || (M < 128 && K % 256 != 0) || N % 128 != 0 || K % 64 != 0)
         return 0;
-    const GemmPlan g = plan_gemm(M, N, K);
+    const GemmPlan g = plan_gemm(M, N, K, false);
     return g.splits > 1 ? (size_t)g.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
 static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
                            const float *alpha, const float *amax_a, const float *amax_b, double denominator,
                            int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
-                           void *workspace, size_t workspace_bytes, fos_stream_t stream) {
+                           void *workspace, size_t workspace_bytes, fos_stream_t stream, bool if4 = false) {
     if (!A || !B || !sfA || !sfB || !D) return FOS_E_NULL_POINTER;
     if (((uintptr_t)d_amax & 3) || ((uintptr_t)bias & 7)) return FOS_E_BAD_ALIGNMENT;
     if (!alpha && (!amax_a || !amax_b)) return FOS_E_NULL_POINTER;
@@ -1229,9 +1289,10 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     GemmParams p;
     p.A = A; p.B = B; p.sfA = sfA; p.sfB = sfB; p.alpha = alpha; p.D = D; p.bias = bias; p.d_amax = d_amax;
     p.amax_a = amax_a; p.amax_b = amax_b; p.inv_den = alpha ? 0.0f : (float)(1.0 / denominator);
+    p.tiny_scale = if4;
     p.M = M; p.N = N; p.K = K; p.ldd = ldd;
     hipStream_t s = (hipStream_t)stream;
-    GemmPlan g = plan_gemm(M, N, K);
+    GemmPlan g = plan_gemm(M, N, K, if4);
     if (M < 128 && g.kind != kPlanSkinny) return FOS_E_BAD_SHAPE;
     // the tile kernels store whole rows of their output tiles, 16 bytes per lane
     if (g.kind != kPlanSkinny && (((uintptr_t)D & 15) || (ldd % 8 != 0))) return FOS_E_BAD_ALIGNMENT;  // partial bands only through the weight-streaming kernel
@@ -1244,6 +1305,11 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     p.partials = g.splits > 1 ? static_cast<float *>(workspace) : nullptr;
     p.splits = g.splits;
     p.ksteps_per_split = g.ksteps_per_split;
+    if (if4) {
+        if (g.kind == kPlanBig) return launch_gemm<1, 8, 8, 1, false, true>(p, out_type, s);
+        if (g.kind == kPlanWide) return launch_gemm<1, 8, 4, 1, true, true>(p, out_type, s);
+        return launch_gemm<1, 4, 4, 1, false, true>(p, out_type, s);
+    }
     switch (g.kind) {
         case kPlanBig: return launch_gemm<1, 8, 8, 1>(p, out_type, s);
         // (quarter rows of A per thread: with half rows the first four wavefronts carried all of A's conversion; alternating
@@ -1302,4 +1368,20 @@ extern "C" int fos_gemm_nvfp4_linear(const uint8_t *A, const uint8_t *B, const u
     if (!(denominator > 0.0)) return FOS_E_BAD_SHAPE;
     return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, workspace,
                            workspace_bytes, stream);
+}
+
+extern "C" size_t fos_gemm_if4_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || M % 128 != 0 || N % 128 != 0 || K % 64 != 0) return 0;
+    const GemmPlan g = plan_gemm(M, N, K, true);
+    return g.splits > 1 ? (size_t)g.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+
+extern "C" int fos_gemm_if4(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
+                            const float *amax_a, const float *amax_b, double denominator,
+                            int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
+                            float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream) {
+    if (!amax_a || !amax_b) return FOS_E_NULL_POINTER;
+    if (!(denominator > 0.0) || M % 128 != 0) return FOS_E_BAD_SHAPE;
+    return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, workspace,
+                           workspace_bytes, stream, true);
 }

@@ -304,6 +304,35 @@ Tensor gemm_nvfp4_amax(const Tensor &a, const Tensor &b, const Tensor &a_sf, con
                        bias.has_value() ? &*bias : nullptr);
 }
 
+// IF4 x IF4 (row-major E4M3 scales), output scale from the two maxima, optional bias and recorded maximum as above.
+Tensor gemm_if4(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tensor &b_sf, const Tensor &amax_a, const Tensor &amax_b,
+                double denominator, at::ScalarType out_dtype, const c10::optional<Tensor> &d_amax, const c10::optional<Tensor> &bias) {
+    const Tensor *scales[2] = {&amax_a, &amax_b};
+    const char *names[2] = {"amax_a", "amax_b"};
+    check_gemm_operands(a, b, a_sf, b_sf, scales, 2, names);
+    TORCH_CHECK(amax_a.scalar_type() == at::kFloat && amax_b.scalar_type() == at::kFloat, "gemm: the maxima must be float32");
+    const int64_t m = a.size(0), n = b.size(0), k = a.size(1) * 2;
+    const int out_type = type_id(out_dtype, "gemm: out_dtype");
+    if (d_amax.has_value()) require_gpu(*d_amax, "d_amax");
+    if (bias.has_value()) {
+        require_gpu(*bias, "bias");
+        TORCH_CHECK(bias->scalar_type() == out_dtype && bias->dim() == 1 && bias->size(0) == n && bias->is_contiguous(),
+                    "gemm: bias must be a contiguous [N] tensor of the output type");
+    }
+    Tensor out = at::empty({m, n}, a.options().dtype(out_dtype));
+    const size_t ws_bytes = fos_gemm_if4_workspace_bytes(m, n, k);
+    const DeviceGuard guard(a.device());
+    Tensor ws;
+    if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
+    check(fos_gemm_if4(a.data_ptr<uint8_t>(), b.data_ptr<uint8_t>(), static_cast<const uint8_t *>(a_sf.data_ptr()),
+                       static_cast<const uint8_t *>(b_sf.data_ptr()), amax_a.data_ptr<float>(), amax_b.data_ptr<float>(), denominator, m,
+                       n, k, out.data_ptr(), out_type, n, bias.has_value() ? bias->data_ptr() : nullptr,
+                       d_amax.has_value() ? d_amax->data_ptr<float>() : nullptr, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes,
+                       current_stream(a)),
+          "fouroversix::gemm_if4");
+    return out;
+}
+
 // alpha[0] = (amax_a * amax_b) * f32(1 / denominator) on the device
 void gemm_alpha(const Tensor &amax_a, const Tensor &amax_b, double denominator, Tensor alpha) {
     const DeviceGuard guard(alpha.device());
@@ -400,6 +429,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("transform_quantize", &transform_quantize);
     m.def("gemm_nvfp4", &gemm_nvfp4);
     m.def("gemm_nvfp4_amax", &gemm_nvfp4_amax);
+    m.def("gemm_if4", &gemm_if4);
     m.def("gemm_alpha", &gemm_alpha);
     m.def("gemm_mxfp4", &gemm_mxfp4_typed);
     m.def("dequantize", &dequantize);

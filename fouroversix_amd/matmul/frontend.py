@@ -111,6 +111,50 @@ def _gemm_record(q: QuantizedTensor) -> tuple:
     return rec
 
 
+def _if4_gemm_applies(input: QuantizedTensor, other: QuantizedTensor, out_dtype: DataType) -> bool:
+    """Two IF4 tensors as ``quantize`` lays them out (row-major scales), on one GPU, for the IF4 GEMM."""
+
+    def fits(q: QuantizedTensor) -> bool:
+        return (
+            q.dtype == DataType.if4
+            and not q.scale_factors_are_in_blackwell_layout
+            and type(q.values) is torch.Tensor
+            and q.values.is_cuda
+            and q.amax is not None
+            and q.amax.dtype == torch.float32
+            and q.amax.numel() == 1
+            and q.amax.device == q.values.device
+            and q.padded_shape[0] % 128 == 0
+            and q.padded_shape[1] % 64 == 0
+            and q.values.shape[0] == q.padded_shape[0]
+            and _members_fit(q, q.values)
+            and q.values.data_ptr() % 16 == 0
+            and q.scale_factors.data_ptr() % 16 == 0
+        )
+
+    return (
+        out_dtype in (DataType.bfloat16, DataType.float16)
+        and fits(input)
+        and fits(other)
+        and input.values.device == other.values.device
+        and input.padded_shape[1] == other.padded_shape[1]
+        and not torch.compiler.is_compiling()
+    )
+
+
+def _fusable_bias(bias: torch.Tensor | None, dtype: torch.dtype, columns: int, device: torch.device) -> bool:
+    """Whether the GEMM's epilogue can add ``bias`` (``columns``: the weight's rows with their padding)."""
+    return (
+        bias is not None
+        and bias.dtype == dtype
+        and bias.dim() == 1
+        and bias.shape[0] == columns  # (no row padding of the weight between the bias and the product)
+        and bias.device == device
+        and bias.is_contiguous()
+        and bias.data_ptr() % 8 == 0
+    )
+
+
 _UNIT_ALPHA: dict = {}
 
 
@@ -197,15 +241,7 @@ def quantized_matmul(
         and not torch.compiler.is_compiling()
     ):
         torch_dtype = torch.bfloat16 if out_dtype is DataType.bfloat16 else torch.float16
-        fused_bias = (
-            bias is not None
-            and bias.dtype == torch_dtype
-            and bias.dim() == 1
-            and bias.shape[0] == rb[0].shape[0]  # (no row padding of the weight between the bias and the product)
-            and bias.device == ra[6]
-            and bias.is_contiguous()
-            and bias.data_ptr() % 8 == 0
-        )
+        fused_bias = _fusable_bias(bias, torch_dtype, rb[0].shape[0], ra[6])
         d_amax = _fresh_amax_word(ra[6]) if emit_amax and (bias is None or fused_bias) else None
         out = ops.gemm_nvfp4_from_amax(
             ra[4], rb[0], ra[1], rb[1], ra[2], rb[2], ra[5] * rb[5], torch_dtype, d_amax, True,
@@ -221,8 +257,24 @@ def quantized_matmul(
         return out
 
     if not is_supported(input, other, out_dtype=out_dtype):
+        if _if4_gemm_applies(input, other, out_dtype):
+            # the dequantized operands' product (src/fouroversix/matmul/pytorch.py:33-52) without forming them: fp16
+            # values as the dequantization defines them, the tensor maxima in the output scale
+            device = input.values.device
+            fused_bias = _fusable_bias(bias, out_dtype.torch_dtype, other.values.shape[0], device)
+            d_amax = _fresh_amax_word(device) if emit_amax and (bias is None or fused_bias) else None
+            out = ops.gemm_if4(
+                input.values, other.values, input.scale_factors, other.scale_factors, input.amax, other.amax,
+                dequantize_divisor(input) * dequantize_divisor(other), out_dtype.torch_dtype, d_amax,
+                bias.detach() if fused_bias else None,
+            )
+            out_shape = (input.original_shape[0], other.original_shape[0])
+            out = out if tuple(out.shape) == out_shape else out[: out_shape[0], : out_shape[1]]
+            if d_amax is not None:
+                attach_known_amax(out, d_amax)
+            return out if bias is None or fused_bias else out + bias
         if _dequantize_form_applies(input, other, out_dtype):
-            # formats without a native GEMM (IF4; mixed formats): the reference's PyTorch backend,
+            # formats and result types without a native GEMM (mixed formats, fp32 results): the reference's PyTorch backend,
             # ``matmul(dequantize(a, f32), dequantize(b, f32).T)`` rounded to the output type
             # (src/fouroversix/matmul/pytorch.py:33-52) -- the dequantize kernel plus a library GEMM
             out = torch.matmul(

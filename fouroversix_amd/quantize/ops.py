@@ -119,6 +119,11 @@ def gemm_nvfp4_from_amax(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtyp
     return _C.gemm_nvfp4_amax(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, checked, bias)
 
 
+def gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax=None, bias=None):
+    """IF4 x IF4 product with the output scale of ``gemm_nvfp4_from_amax``; ``d_amax`` and ``bias`` as there."""
+    return _C.gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, bias)
+
+
 def gemm_alpha_into(amax_a, amax_b, denominator, alpha):
     """alpha[0] = (amax_a * amax_b) * f32(1 / denominator) on the device, torch's GPU arithmetic for
     ``(amax_a * amax_b) / denominator``."""

@@ -254,7 +254,7 @@ int fos_gemm_nvfp4_amax(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, 
 
 /*
  * fos_gemm_nvfp4_amax that also folds max|D| -- of the values as stored, in the output type --
- * into d_amax[0] (device f32[1]): every wavefront does an unsigned atomic max on the value's
+ * into d_amax[0] (device f32[1]): every workgroup does an unsigned atomic max on the value's
  * bits, so the caller sets d_amax[0] to 0 before the call (or leaves an earlier maximum there to
  * extend it).  A NaN among the outputs is recorded as NaN (its bits lie above every number's), as the
  * reference's `x.abs().max()` would report it.  The next layer's activation quantization can then take d_amax as its
@@ -279,6 +279,18 @@ int fos_gemm_nvfp4_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA
                           const float *amax_a, const float *amax_b, double denominator,
                           int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
                           float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream);
+
+/*
+ * IF4 x IF4 product: as fos_gemm_nvfp4_linear for operands in the IF4 format (row-major scale bytes, bit 7 = integer
+ * block; values and block scales meet in fp16 as in fos_dequantize with intermediate_type FOS_T_F16).  M, N multiples
+ * of 128, K of 64 (the padded extents of quantized tensors).  The reference has no native product for this format: it
+ * multiplies dequantized fp32 matrices (src/fouroversix/matmul/pytorch.py:33-52).
+ */
+int fos_gemm_if4(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
+                 const float *amax_a, const float *amax_b, double denominator,
+                 int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
+                 float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream);
+size_t fos_gemm_if4_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
  * alpha[0] = (amax_a[0] * amax_b[0]) * f32(1 / denominator), in fp32 on the device: the

@@ -309,6 +309,44 @@ def test_formats_without_a_native_gemm_take_the_dequantize_form(oracle):
     assert float((out32.cpu() - torch.from_numpy(ref32)).abs().max()) <= 1e-3 * float(np.abs(ref32).max())
 
 
+@pytest.mark.parametrize(("m", "n", "k", "tile", "amaxes"), [
+    (128, 128, 64, "0", (1.0, 1.0)),
+    (1, 300, 1024, "0", (3.0, 0.5)),          # one row of a padded band, K split
+    (200, 384, 320, "129", (2.0, 1.0)),       # 128 x 256 tile over the edge
+    (384, 640, 192, "256", (1.0, 1.0)),       # 256 x 256 tile over both edges
+    (384, 640, 1088, "128", (1.0, 7.5)),
+    (256, 256, 128, "0", (2.0 ** -100, 2.0 ** -20)),  # the output scale alone is a sub-normal number
+    (256, 256, 128, "0", (2.0 ** 100, 2.0 ** -100)),
+])
+def test_if4_gemm_over_all_codes_and_scales(monkeypatch, m, n, k, tile, amaxes):
+    """Every code (the integer -8, which the quantizer does not write, among them) under every finite scale byte of
+    both kinds of blocks: the IF4 product against the fp64 product of the dequantized operands.  Error bound: fp32
+    accumulation over K (K 2^-24 of the sum of magnitudes, doubled for the output scale and its rounding) plus half a
+    unit of bf16 (8 significant bits: 2^-8 relative; 2^-134 absolute below its normal range)."""
+    monkeypatch.setenv("FOS_GEMM_TILE", tile)
+    g = torch.Generator("cpu").manual_seed(m + n + k)
+
+    def operand(rows, amax):
+        rows_p, cols_p = -(-rows // 128) * 128, -(-k // 64) * 64
+        codes = torch.randint(0, 256, (rows_p, cols_p // 2), generator=g, dtype=torch.uint8)
+        scales = torch.randint(0, 127, (rows_p * cols_p // 16,), generator=g, dtype=torch.uint8)
+        scales |= torch.randint(0, 2, scales.shape, generator=g, dtype=torch.uint8) << 7
+        return fos.QuantizedTensor(codes.cuda(), scales.cuda().view(torch.float8_e4m3fn), torch.tensor(amax, device="cuda"),
+                                   fos.DataType.if4, (rows, k), fos.ScaleRule.mse, fos.RoundStyle.nearest, padded_shape=(rows_p, cols_p),
+                                   scale_factors_are_in_blackwell_layout=False)
+
+    qa, qb = operand(m, amaxes[0]), operand(n, amaxes[1])
+    a, b = (fos.dequantize(q, dtype=torch.float32).double().cpu() for q in (qa, qb))
+    exact, size = a @ b.T, a.abs() @ b.abs().T
+    out = fos.quantized_matmul(qa, qb)
+    assert out.shape == (m, n)
+    err = (out.double().cpu() - exact).abs()
+    assert bool((err <= 2.0 ** -8 * exact.abs() + 2 * k * 2.0 ** -24 * size + 2.0 ** -134).all())
+    bias = torch.linspace(-1, 1, n, device="cuda").bfloat16()
+    with_bias = fos.quantized_matmul(qa, qb, bias=bias, emit_amax=True)
+    assert torch.equal(with_bias, out + bias)
+
+
 def test_linear_forward_replays_in_a_hip_graph():
     """A decode-sized forward (quantize -> alpha -> weight-streaming GEMM, twice) captured in
     a HIP graph: every replay, interleaved with eager work and synchronisations, equals
