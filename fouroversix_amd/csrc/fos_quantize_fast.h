@@ -670,6 +670,32 @@ __device__ __attribute__((noinline)) BlockOut generic_block_if4(Block16 blk, Qua
     return BlockOut{codes[0], codes[1], sbyte};
 }
 
+// Exact selection of a 1x16 block from its two candidates' codes: the reference's error terms and order in
+// registers (no call, no scratch memory, no IEEE division; see exact_pick_b_1d).  Needs q * s * amax exact, i.e. a
+// maximum of at most 8 significant bits, and the divisor 2688 with normal quotients.
+// It is reached often: in a block with one element far above the others (activations with outlier channels) both
+// candidates keep that element and round the rest to zero, so the two errors differ by roundings at most.  With one
+// channel in a hundred 50 times the others, 2048 x 4096 bf16: pass 2 55 us with the operation-by-operation form here,
+// 14 with this one.
+FOS_DEVICE bool exact_pick_integer_1d(const float *x, uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, const FastLutEntry &A,
+                                      float g) {
+    constexpr float kDiv = 2688.0f, kRec = 1.0f / 2688.0f;
+    float eA[16], eB[16];
+    static_for<0, 8>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const float2_t fa = unpack_fp4<(j & 3)>(j < 4 ? a0 : a1);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float dA = candidate_residual(fa[h], A, x[2 * j + h]);
+            const int q = ((int)((j < 4 ? b0 : b1) << (28 - 8 * (j & 3) - 4 * h))) >> 28;  // the nibble, sign-extended
+            const float dB = div_const(((float)q * g) * 0.8571428571f, kDiv, kRec) - x[2 * j + h];
+            eA[2 * j + h] = dA * dA;
+            eB[2 * j + h] = dB * dB;
+        }
+    });
+    return sum16(eB) < sum16(eA);
+}
+
 template <bool TWO_D>
 FOS_DEVICE BlockOut quantize_block_if4_mse(const Block16 &blk, const QuantConsts &k, float enc, float rq,
                                            bool in_range, const FastLutEntry *lut) {
@@ -720,6 +746,12 @@ FOS_DEVICE BlockOut quantize_block_if4_mse(const Block16 &blk, const QuantConsts
             if (cmp > 0) return BlockOut{b0, b1, s | 0x80u};
             if (cmp < 0) return BlockOut{a0, a1, s};
             // undecided (uniform over the 16 lanes of a tile when TWO_D: both sums are tile sums)
+            if constexpr (!TWO_D) {
+                if (k.shortcut_ok && k.errdiv == 2688.0f && (f2u(k.amax) & 0xffffu) == 0) {
+                    const bool pickB = exact_pick_integer_1d(x, a0, a1, b0, b1, A, e4m3_decode(s) * k.amax);
+                    return BlockOut{pickB ? b0 : a0, pickB ? b1 : a1, pickB ? s | 0x80u : s};
+                }
+            }
         } else if (bmax == 0.0f) {
             return BlockOut{0, 0, 0};
         }

@@ -420,6 +420,19 @@ def test_caller_supplied_amax(oracle):
             assert_same_quantization(q, ref, f"{kind} {cfg}")
 
 
+@pytest.mark.parametrize("shape", [(128, 256), (100, 272), (1, 16)])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -38, 2.0 ** 50])
+def test_if4_blocks_whose_candidates_nearly_tie(oracle, shape, scale):
+    """One large element a block: both candidates keep it and round the rest to zero, and the choice hangs on the
+    last bits of two error sums.  The larger elements run through every bf16 mantissa."""
+    x = make_input("randn", shape, 91).float() * 0.02
+    big = torch.arange(x.shape[0] * (x.shape[1] // 16)).reshape(x.shape[0], -1)
+    x[:, 5 :: 16] = (1 + (big % 128) / 128) * 2.0 ** (big // 128 % 6) * (1 - 2 * (big % 2))
+    x = (x * scale).bfloat16()
+    q = hip_quantize(x, dtype="if4", scale_rule="mse")
+    assert_same_quantization(q, oracle.quantize(x, dtype="if4", scale_rule="mse"), f"{shape} scale {scale}")
+
+
 @pytest.mark.parametrize(("rows", "cols", "ld"), [
     (2051, 4096, 4096),     # window order (cols % 2048 == 0, >= 16 MiB), rows not a multiple of anything
     (4096, 2048, 2048 + 64),  # the same scan over a strided view
