@@ -437,10 +437,6 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
     p.ldo = ldo;
     p.x = (const uint16_t *)x;
     p.x_type = x_type;
-    {
-        const int64_t esize = x_type == FOS_T_F32 ? 4 : 2;
-        p.x_vec = x_type != FOS_T_BF16 && ((uintptr_t)x & 15) == 0 && (ld * esize) % 16 == 0 && cols % 16 == 0;
-    }
     p.rows = rows; p.cols = cols; p.ld = ld;
     p.rows_p = rows_p; p.cols_p = cols_p;
     p.codes = codes; p.sf = sf;

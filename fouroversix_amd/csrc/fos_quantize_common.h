@@ -19,7 +19,6 @@ constexpr int kMaxPartials = 1024;  // pairs of 32-bit words in the workspace
 struct QuantParams {
     const uint16_t *x;           // bf16 / fp16 elements, or (x_type == FOS_T_F32) really const float *
     int x_type = FOS_T_BF16;     // fp16 and fp32 inputs go through the element-wise kernel only
-    int x_vec = 0;               // ... with 128-bit loads when base, row pitch and width allow (16-byte aligned rows, cols % 16 == 0)
     int64_t rows, cols, ld;      // logical input
     int64_t rows_p, cols_p;      // padded output extents
     uint8_t *codes;              // [rows_p, cols_p / 2]
@@ -429,20 +428,29 @@ FOS_DEVICE void quantize_block(const uint32_t *w, const QuantConsts &k, uint64_t
     quantize_block_f32<DT, RULE, ROUND, TWO_D>(x, k, seed, offset, blk, codes, sbyte);
 }
 
-// The 16 elements of block column cb of row r as fp32, 128-bit loads (QuantParams::x_vec).
+// Sixteen 16-bit elements as packed words, and N fp32 values, from any address the element type allows: the types say
+// that 2 (4) bytes is all the alignment there is, and the compiler takes wide loads where the hardware takes them so.
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+FOS_DEVICE void load_words8(const uint16_t *src, uint32_t *w) {
+    const u32x4_a2 lo = *reinterpret_cast<const u32x4_a2 *>(src), hi = *reinterpret_cast<const u32x4_a2 *>(src + 8);
+    w[0] = lo.x, w[1] = lo.y, w[2] = lo.z, w[3] = lo.w;
+    w[4] = hi.x, w[5] = hi.y, w[6] = hi.z, w[7] = hi.w;
+}
+
+// The 16 elements of row r from column c0 on (all inside the row) as fp32.
 FOS_DEVICE void load_block16(const QuantParams &p, int64_t r, int64_t c0, float *x) {
     if (p.x_type == FOS_T_F32) {
-        const float4 *src = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(p.x) + r * p.ld + c0);
+        const float *src = reinterpret_cast<const float *>(p.x) + r * p.ld + c0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float4 v = src[i];
+            const f32x4_a4 v = *reinterpret_cast<const f32x4_a4 *>(src + 4 * i);
             x[4 * i] = v.x, x[4 * i + 1] = v.y, x[4 * i + 2] = v.z, x[4 * i + 3] = v.w;
         }
         return;
     }
-    const uint4 *src = reinterpret_cast<const uint4 *>(p.x + r * p.ld + c0);
-    const uint4 lo = src[0], hi = src[1];
-    const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    uint32_t w[8];
+    load_words8(p.x + r * p.ld + c0, w);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         if (p.x_type == FOS_T_F16) {

@@ -654,6 +654,81 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_fast(const Block16 &blk, const QuantCon
 }
 
 // ---------------------------------------------------------------------------------------
+// The same for a block given as fp32 values (fp32 inputs; fp16 ones off the streaming kernels), round to nearest
+// ---------------------------------------------------------------------------------------
+//
+// What the element type changes:
+//  * the block maximum has up to 24 significant bits, for which the 3-operation division by 6 or 4 is not proven:
+//    one IEEE division a block;
+//  * so has the tensor maximum, and the reference's fq * s * amax rounds: one more unit u = 2^-24, 6u on a scaled
+//    residual, and 2u on the weight h.  The bounds of shortcut_compare grow from 40u to 46u an element, inside its
+//    threefold margins (2.6-fold with these);
+//  * there is no exact evaluation from the codes for the same reason: undecided blocks (7 in 10^4 of N(0,1) data)
+//    take the operation-by-operation form, out of line.
+// Abs-max blocks tie too often for a shortcut to pay (3 % of N(0,1) blocks): they are left to that form altogether.
+struct Block16F {
+    float x[16];
+};
+template <int RULE, bool TWO_D>
+__device__ __attribute__((noinline)) BlockOut generic_block_f32(Block16F blk, QuantConsts k) {
+    uint32_t codes[2], sbyte;
+    quantize_block_f32<FOS_DTYPE_NVFP4, RULE, FOS_ROUND_NEAREST, TWO_D>(blk.x, k, 0, 0, 0, codes, sbyte);
+    return BlockOut{codes[0], codes[1], sbyte};
+}
+
+template <int RULE, bool TWO_D>
+FOS_DEVICE BlockOut quantize_block_nvfp4_f32(const Block16F &blk, const QuantConsts &k, float enc, bool in_range, const FastLutEntry *lut) {
+    constexpr bool STATIC = RULE == FOS_RULE_STATIC_6 || RULE == FOS_RULE_STATIC_4;
+    if (in_range) {
+        const float *x = blk.x;
+        float bmax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) bmax = fmaxf(fmaxf(fabsf(x[i]), fabsf(x[i + 1])), bmax);
+        if (TWO_D) bmax = row16_max(bmax);
+        const float s_hp6 = (bmax / k.qdiv) * enc, s_hp4 = s_hp6 * 1.5f;
+        const uint32_t pk = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(s_hp6, s_hp4, 0, false);
+        const uint32_t s6 = pk & 0xffu, s4 = (pk >> 8) & 0xffu;
+        const FastLutEntry A = lut[s6];
+        // (the exclusions of quantize_block_nvfp4_fast; a given maximum may be below the tensor's own: beyond 7 as well)
+        if (s6 != 0u && bmax * A.inv < 7.0f) {
+            const FastLutEntry B = STATIC ? A : lut[s4];
+            uint32_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;
+            float SA = 0.0f, SB = 0.0f;
+            static_for<0, 8>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                const float xa0 = scaled(x[2 * j], A.inv), xa1 = scaled(x[2 * j + 1], A.inv);
+                uint32_t &a = j < 4 ? a0 : a1;
+                a = pack_fp4<(j & 3)>(a, xa0, xa1);
+                if constexpr (!STATIC) {
+                    const float xb0 = scaled(x[2 * j], B.inv), xb1 = scaled(x[2 * j + 1], B.inv);
+                    uint32_t &b = j < 4 ? b0 : b1;
+                    b = pack_fp4<(j & 3)>(b, xb0, xb1);
+                    const float2_t fa = unpack_fp4<(j & 3)>(a), fb = unpack_fp4<(j & 3)>(b);
+                    accumulate_scaled<RULE>(fa.x - xa0, fa.y - xa1, SA);
+                    accumulate_scaled<RULE>(fb.x - xb0, fb.y - xb1, SB);
+                }
+            });
+            if (STATIC) return BlockOut{a0, a1, s6};
+            if (TWO_D) {
+                SA = row16_sum_lane0(SA);
+                SB = row16_sum_lane0(SB);
+            }
+            int cmp = k.shortcut_ok ? shortcut_compare<RULE, TWO_D>(SA, shortcut_weight<RULE>(A), SB, shortcut_weight<RULE>(B)) : 0;
+            if (cmp == 0) {
+                // (codes that stand for the same numbers: an exact tie, the first candidate wins)
+                bool tie = e4m3_decode(s4) == 1.5f * e4m3_decode(s6) && (tie_violations(a0, b0) | tie_violations(a1, b1)) == 0;
+                if (TWO_D) tie = row16_max(tie ? 0.0f : 1.0f) == 0.0f;
+                if (tie) cmp = -1;
+            }
+            if (cmp != 0) return BlockOut{cmp > 0 ? b0 : a0, cmp > 0 ? b1 : a1, cmp > 0 ? s4 : s6};
+        } else if (bmax == 0.0f) {
+            return BlockOut{0, 0, 0};
+        }
+    }
+    return generic_block_f32<RULE, TWO_D>(blk, k);
+}
+
+// ---------------------------------------------------------------------------------------
 // IF4 (one scale; E2M1 candidate against INT4 candidate), 4/6-style MSE selection
 // ---------------------------------------------------------------------------------------
 //

@@ -433,6 +433,42 @@ def test_if4_blocks_whose_candidates_nearly_tie(oracle, shape, scale):
     assert_same_quantization(q, oracle.quantize(x, dtype="if4", scale_rule="mse"), f"{shape} scale {scale}")
 
 
+@pytest.mark.parametrize("rule", ["mse", "mae", "static_6", "static_4"])
+@pytest.mark.parametrize("two_d", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_element_wise_fast_form_bit_exact(oracle, dtype, two_d, rule):
+    """fp32 and fp16 inputs of the element-wise kernel: odd widths and heights (rows that start at any element),
+    24-bit maxima, blocks far below the tensor maximum (sub-normal and zero scales), ties, ranges outside the
+    shortcut's, and a given maximum below the tensor's own."""
+    cfg = dict(scale_rule=rule, block_scale_2d=two_d)
+    g = torch.Generator("cpu").manual_seed(5)
+    for rows, cols in ((1, 1), (17, 33), (130, 257), (100, 1000), (256, 512)):
+        x = torch.randn(rows, cols, generator=g)
+        x[::3] *= torch.exp(-torch.rand(x[::3].shape[0], 1, generator=g) * 12)
+        for y in (x, torch.round(x * 2) / 2):
+            y = y.to(dtype)
+            assert_same_quantization(hip_quantize(y, **cfg), oracle.quantize(y, **cfg), f"{rows}x{cols}")
+    for scale in (2.0 ** -70, 2.0 ** -39, 2.0 ** 59, 2.0 ** 70) if dtype == torch.float32 else (2.0 ** -12, 2.0 ** 12):
+        y = (torch.randn(33, 100, generator=g) * scale).to(dtype)
+        assert_same_quantization(hip_quantize(y, **cfg), oracle.quantize(y, **cfg), f"scale {scale}")
+    y = torch.randn(48, 96, generator=g).to(dtype)
+    # (the largest block scale, 448 / 0.98 = 457, still rounds to E4M3's 448; from 464 on, half way to the next
+    # binade step, it is NaN, whose blocks' codes mean nothing)
+    given = float(y.abs().max()) * 0.98
+    q = hip_quantize(y, **cfg, kwargs={"amax": torch.tensor(given, device="cuda")})
+    assert_same_quantization(q, oracle.quantize(y, **cfg, amax=float(np.float32(given))), "given maximum")
+
+
+@pytest.mark.parametrize("shape", [(3, 17), (129, 301), (64, 1025)])
+def test_unaligned_bf16_rows(oracle, shape):
+    for offset in (0, 1, 3):  # rows that start at any element of the buffer
+        flat = make_input("randn", (1, shape[0] * shape[1] + offset), 17)[0]
+        x = flat[offset:].view(*shape)
+        for cfg in (dict(scale_rule="mse"), dict(scale_rule="mse", block_scale_2d=True), dict(dtype="if4", scale_rule="mse")):
+            q = fos.quantize(flat.cuda()[offset:].view(*shape), fos.QuantizationConfig(**cfg))
+            assert_same_quantization(q, oracle.quantize(x.contiguous(), **cfg), f"{shape} + {offset}")
+
+
 @pytest.mark.parametrize(("rows", "cols", "ld"), [
     (2051, 4096, 4096),     # window order (cols % 2048 == 0, >= 16 MiB), rows not a multiple of anything
     (4096, 2048, 2048 + 64),  # the same scan over a strided view
