@@ -42,7 +42,9 @@ struct RowsTile {
 // IF4: the IF4 format with its MSE rule (E2M1 candidate against INT4 candidate on one scale,
 // quantize_block_if4_mse) instead of NVFP4.
 // F16: fp16 elements instead of bf16 (NVFP4, round to nearest, codes out).
-template <int RULE, bool FULL, bool PSEUDO, bool SR, bool IF4 = false, bool F16 = false>
+// SPLIT: a workgroup covers 32 rows (one q) of a tile instead of 128, and one tile only: tensors with few tiles
+// otherwise run one workgroup a compute unit at most, eight steps one after the other (see launch_rows).
+template <int RULE, bool FULL, bool PSEUDO, bool SR, bool IF4 = false, bool F16 = false, bool SPLIT = false>
 // (the stochastic instantiations hold two sets of scaled values and the Philox state: with 128
 // registers they spilled -- 30 MB of scratch traffic per launch at 8192 x 8192 -- and the launch
 // grid of three workgroups per compute unit leaves 168; the IF4 instantiation spilled as well)
@@ -64,6 +66,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
     const bool tiled = !PSEUDO && p.sf_layout == FOS_SF_TILED_128X4;
     const int64_t code_pitch = p.cols_p >> 1;
     const uint32_t n_tiles = (uint32_t)(p.rows_p >> 7) * (uint32_t)p.tiles_x;
+    static_assert(!(SPLIT && PSEUDO), "split tiles: codes and scales out");
+    const uint32_t sub = SPLIT ? blockIdx.x / n_tiles : 0u;  // (the four parts of a tile on one die where n_tiles % 8 == 0)
     // byte offsets inside a tile (the host checked that a tile spans less than 2^31 bytes);
     // step g starts 32 (g >> 1) + 4 (g & 1) rows below step 0
     const uint32_t x_lane = (uint32_t)(rl * p.ld + lb * 16) * 2u, x_row = (uint32_t)p.ld * 2u;
@@ -79,7 +83,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
         const TileYX yx = map_tile(tile, n_tiles, (uint32_t)p.tiles_x, p.tile_map);
         t.tile_y = yx.y;
         t.tile_x = yx.x;
-        t.row_base = (int64_t)t.tile_y * 128;
+        t.row_base = (int64_t)t.tile_y * 128 + 32 * sub;
         const int64_t col_base = (int64_t)t.tile_x * 256;
         t.cb = (int64_t)t.tile_x * 16 + lb;
         // input: everything from the tile's first element to the end of the tensor's last row
@@ -119,12 +123,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
         for (int u = 0; u < kMaxPartials / kThreads; ++u)
             if ((int)threadIdx.x + u * kThreads < p.n_partials) pm[u] = p.partials[2 * (threadIdx.x + u * kThreads)];
     }
-    uint32_t tile = blockIdx.x;
+    uint32_t tile = SPLIT ? blockIdx.x - sub * n_tiles : blockIdx.x;
     RowsTile cur = open_tile(tile, tile < n_tiles);
     Block16 ring[4];
     load(cur, 0, ring[0]);
     load(cur, 1, ring[1]);
-    load(cur, 2, ring[2]);
+    if (!SPLIT) load(cur, 2, ring[2]);
 
     // setup: tensor maximum, constants, per-scale table
     uint32_t amax_bits;
@@ -236,10 +240,23 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
         const u32x2 c01 = {o.c0, o.c1};
         const BufferRsrc rcodes = make_rsrc(reinterpret_cast<const void *>(uniform64(t.codes_base)), 0xffffffffu);
         __builtin_amdgcn_raw_buffer_store_b64(c01, rcodes, c_lane, step_row(g) * c_row, kStreamStore);
-        if (tiled) stage[(g & 1) * 64 + (g >> 1) * 4] = (uint8_t)o.s;
+        if (SPLIT && tiled) {
+            // the four scales of a row in one scale tile: word `sub` of the row's 16-byte unit
+            uint32_t word = o.s & 0xffu;
+            word |= (uint32_t)__builtin_amdgcn_mov_dpp((int)o.s, 0x55, 0xf, 0xf, true) << 8;
+            word |= (uint32_t)__builtin_amdgcn_mov_dpp((int)o.s, 0xaa, 0xf, 0xf, true) << 16;
+            word |= (uint32_t)__builtin_amdgcn_mov_dpp((int)o.s, 0xff, 0xf, 0xf, true) << 24;
+            if ((lb & 3) == 0)
+                *reinterpret_cast<uint32_t *>(p.sf + ((int64_t)t.tile_y * (sf_cols >> 2) + (t.cb >> 2)) * 512 + (rl + step_row(g)) * 16 + sub * 4) = word;
+        } else if (tiled) stage[(g & 1) * 64 + (g >> 1) * 4] = (uint8_t)o.s;
         else p.sf[row * sf_cols + t.cb] = (uint8_t)o.s;
     };
 
+    if constexpr (SPLIT) {
+        process(cur, 0, ring[0]);
+        process(cur, 1, ring[1]);
+        return;
+    }
     __builtin_amdgcn_s_setprio(3);
     while (tile < n_tiles) {
         const uint32_t next = tile + gridDim.x;
@@ -287,6 +304,39 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
 template <int RULE, bool PSEUDO, bool SR>
 void launch_quantize_nvfp4_tiles(QuantParams &p, hipStream_t s);
 
+// Launch of the streaming kernel.
+// Three workgroups per compute unit (256 CUs), each walking several tiles: measured at
+// 8192 x 8192 with the 4/6-MSE rule, 768 workgroups take 31.6 us where 1024 take 33.2 and the
+// 1280 that fit (<= 102 VGPRs) 35.5 -- the setup is paid fewer times and the wavefronts stay
+// in their streaming loop longer.  FOS_QUANT_GRID overrides for tuning runs.
+// Few tiles: in four parts each, so that a compute unit holds several wavefronts a SIMD and each does two steps instead
+// of eight.  Pass 2 of bf16, whole / in four (us): 128 x 4096 (16 tiles) 8.2 / 4.1, 1024 x 4096 (128) 8.6 / 5.3,
+// 2048 x 4096 (256) 9.2 / 6.6, 3072 x 4096 (384) 10.0 / 8.1, 4096 x 4096 (512) 10.4 / 10.2 (IF4 12.1 / 13.2),
+// 6144 x 4096 (768) 13.9 / 16.4.
+constexpr int64_t kSplitTiles = 384;
+template <int RULE, bool PSEUDO, bool SR, bool IF4, bool F16>
+static void launch_rows(QuantParams &p, hipStream_t s) {
+    p.tiles_x = (int)((p.cols_p + 255) / 256);
+    const int64_t n = (p.rows_p / 128) * p.tiles_x;
+    p.tile_map = kMapRowMajor;
+    if (const int forced = tuning().quant_map) p.tile_map = forced - 1;
+    const bool full = p.rows % 128 == 0 && p.cols % 256 == 0;
+    if constexpr (!PSEUDO) {
+        const int split = tuning().quant_split;  // tuning / tests: 1 = never, 2 = always
+        if (split == 2 ? 4 * n <= 0x7fffffff : (split == 0 && n <= kSplitTiles)) {
+            const dim3 grid((unsigned)(4 * n));
+            if (full) hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, true, false, SR, IF4, F16, true>), grid, dim3(kThreads), 0, s, p);
+            else hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, false, false, SR, IF4, F16, true>), grid, dim3(kThreads), 0, s, p);
+            return;
+        }
+    }
+    int64_t grid = 768;
+    if (const int forced = tuning().quant_grid) grid = forced > 0 ? forced : grid;
+    if (grid > n) grid = n;
+    if (full) hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, true, PSEUDO, SR, IF4, F16>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+    else hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, false, PSEUDO, SR, IF4, F16>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+}
+
 template <int RULE, bool PSEUDO, bool SR>
 static void by_dim(QuantParams &p, bool two_d, bool aligned, hipStream_t s) {
     if (!aligned) {
@@ -296,32 +346,10 @@ static void by_dim(QuantParams &p, bool two_d, bool aligned, hipStream_t s) {
         return;
     }
     if (!two_d) {
-        p.tiles_x = (int)((p.cols_p + 255) / 256);
-        const int64_t n = (p.rows_p / 128) * p.tiles_x;
-        // three workgroups per compute unit (256 CUs), each walking several tiles: measured at
-        // 8192 x 8192 with the 4/6-MSE rule, 768 workgroups take 31.6 us where 1024 take 33.2 and the
-        // 1280 that fit (<= 102 VGPRs) 35.5 -- the setup is paid fewer times and the wavefronts stay
-        // in their streaming loop longer.  FOS_QUANT_GRID overrides for tuning runs.
-        int64_t grid = 768;
-        if (const int forced = tuning().quant_grid) grid = forced > 0 ? forced : grid;
-        if (grid > n) grid = n;
-        p.tile_map = kMapRowMajor;
-        if (const int forced = tuning().quant_map) p.tile_map = forced - 1;
-        const bool full = p.rows % 128 == 0 && p.cols % 256 == 0;
         if constexpr (!SR) {
-            if (p.x_type == FOS_T_F16) {
-                if (full)
-                    hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, true, PSEUDO, false, false, true>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-                else
-                    hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, false, PSEUDO, false, false, true>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-                return;
-            }
+            if (p.x_type == FOS_T_F16) return launch_rows<RULE, PSEUDO, false, false, true>(p, s);
         }
-        if (full)
-            hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, true, PSEUDO, SR>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-        else
-            hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, false, PSEUDO, SR>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-        return;
+        return launch_rows<RULE, PSEUDO, SR, false, false>(p, s);
     }
     launch_quantize_nvfp4_tiles<RULE, PSEUDO, SR>(p, s);
 }
@@ -342,22 +370,8 @@ static void by_rule(QuantParams &p, int rule, bool two_d, bool aligned, hipStrea
 
 // IF4 with the MSE rule, round to nearest, 1x16 blocks, aligned input: the streaming kernel.
 void launch_quantize_if4_mse_rows(QuantParams &p, hipStream_t s) {
-    p.tiles_x = (int)((p.cols_p + 255) / 256);
-    const int64_t n = (p.rows_p / 128) * p.tiles_x;
-    int64_t grid = 768;
-    if (const int forced = tuning().quant_grid) grid = forced > 0 ? forced : grid;
-    if (grid > n) grid = n;
-    p.tile_map = kMapRowMajor;
-    if (const int forced = tuning().quant_map) p.tile_map = forced - 1;
-    const bool full = p.rows % 128 == 0 && p.cols % 256 == 0;
-    if (p.pseudo_out) {
-        if (full) hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<FOS_RULE_MSE, true, true, false, true>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-        else hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<FOS_RULE_MSE, false, true, false, true>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-    } else if (full) {
-        hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<FOS_RULE_MSE, true, false, false, true>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-    } else {
-        hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<FOS_RULE_MSE, false, false, false, true>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-    }
+    if (p.pseudo_out) launch_rows<FOS_RULE_MSE, true, false, true, false>(p, s);
+    else launch_rows<FOS_RULE_MSE, false, false, true, false>(p, s);
 }
 
 // `sr`: a stochastic style on an aligned input.  The fast exact evaluation is tied to the

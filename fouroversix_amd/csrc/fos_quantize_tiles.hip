@@ -165,7 +165,8 @@ FOS_DEVICE uint32_t quad_bytes(uint32_t l0, uint32_t l1, uint32_t l2, uint32_t l
 // bit 7 of the scale byte) instead of NVFP4.
 // SR: a stochastic rounding style (NVFP4); its two sets of scaled values and the Philox state take the
 // registers of three wavefronts per SIMD.
-template <int RULE, bool FULL, bool PSEUDO, bool IF4 = false, bool SR = false>
+// SPLIT: a workgroup covers one group (q) of a tile, one tile only (tensors with few tiles; launch_tiles).
+template <int RULE, bool FULL, bool PSEUDO, bool IF4 = false, bool SR = false, bool SPLIT = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3 : 4, SR ? 3 : 8))) void quantize_nvfp4_tiles_kernel(
     const QuantParams p) {
     static_assert(!(SR && IF4), "stochastic styles: NVFP4");
@@ -183,6 +184,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
     const bool tiled = !PSEUDO && p.sf_layout == FOS_SF_TILED_128X4;
     const int64_t code_pitch = p.cols_p >> 1;
     const uint32_t n_tiles = (uint32_t)(p.rows_p >> 7) * (uint32_t)p.tiles_x;
+    static_assert(!(SPLIT && PSEUDO), "split tiles: codes and scales out");
+    const uint32_t sub = SPLIT ? blockIdx.x / n_tiles : 0u;
     // byte offsets inside the wavefront's share (the host checked that a tile spans less than
     // 2^31 bytes); step s of group q starts 32 q + 4 s rows below the first
     const uint32_t x_lane = (uint32_t)(li * p.ld + lb * 16) * 2u, x_row = (uint32_t)p.ld * 2u;
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
         TilesPos t;
         const TileYX yx = map_tile(tile, n_tiles, (uint32_t)p.tiles_x, p.tile_map);
         const uint32_t tile_y = yx.y, tile_x = yx.x;
-        t.row0 = (int32_t)(tile_y * 128u) + 16 * par;
+        t.row0 = (int32_t)(tile_y * 128u) + 16 * par + 32 * (int32_t)sub;
         // The two 256-column windows of a workgroup lie eight windows apart inside each complete run
         // of sixteen (kMapSplitHalves; side by side otherwise and in what is left of a row): with
         // row-major units an XCD then reads every eighth 512-byte window of a row, the pattern of the
@@ -243,7 +246,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
         for (int u = 0; u < kMaxPartials / kThreads; ++u)
             if ((int)threadIdx.x + u * kThreads < p.n_partials) pm[u] = p.partials[2 * (threadIdx.x + u * kThreads)];
     }
-    uint32_t tile = blockIdx.x;
+    uint32_t tile = SPLIT ? blockIdx.x - sub * n_tiles : blockIdx.x;
     TilesPos cur = open_tile(tile, tile < n_tiles);
     // One register set holds a group; each block's registers are refilled with the next group's as
     // soon as the block has been consumed.  (More loads in flight do not help: with a second set,
@@ -581,6 +584,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
         return os;
     };
 
+    if constexpr (SPLIT) {
+        const TilesPos none = open_tile(tile, false);  // (loads of nothing)
+        const uint32_t sw = process(cur, 0, none, 0);
+        if (tiled) {
+            // the quad's four bytes: word `sub` of the 16-byte unit
+            const uint32_t l0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)sw, 0x00, 0xf, 0xf, true);
+            const uint32_t l1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)sw, 0x55, 0xf, 0xf, true);
+            const uint32_t l2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)sw, 0xaa, 0xf, 0xf, true);
+            const uint32_t l3 = (uint32_t)__builtin_amdgcn_mov_dpp((int)sw, 0xff, 0xf, 0xf, true);
+            if (FULL || cur.cb < (int32_t)sf_cols)
+                *reinterpret_cast<uint32_t *>(p.sf + cur.unit_base + (lb >> 2) * 512 + (4 * (lb & 3) + li) * 16 + sub * 4) = quad_bytes<0>(l0, l1, l2, l3);
+        }
+        return;
+    }
     while (tile < n_tiles) {
         const uint32_t next = tile + gridDim.x;
         const bool has_next = next < n_tiles;
@@ -609,39 +626,40 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
 
 }  // namespace
 
-template <int RULE, bool PSEUDO, bool SR>
-void launch_quantize_nvfp4_tiles(QuantParams &p, hipStream_t s) {
+// Three workgroups per compute unit (256 CUs; four would fit), walking the tiles between them:
+// measured best at 8192 x 8192 (43.9 us against 45.9 with 1024).  FOS_QUANT_GRID overrides for
+// tuning runs.  Few tiles: in four parts each, as the 1x16 kernel's.  Pass 2 of bf16, 4/6-MSE,
+// whole / in four (us): 128 x 4096 (8 tiles) 11.9 / 5.9, 2048 x 4096 (128) 12.2 / 7.9, 4096 x 4096 (256) 13.3 / 11.0,
+// 2048 x 14336 (448) 19.9 / 16.7.
+template <int RULE, bool PSEUDO, bool IF4, bool SR>
+static void launch_tiles(QuantParams &p, hipStream_t s) {
+    constexpr int64_t kSplitTiles = 448;
     p.tiles_x = (int)((p.cols_p + 511) / 512);
     const int64_t n = (p.rows_p / 128) * p.tiles_x;
-    // three workgroups per compute unit (256 CUs; four would fit), walking the tiles between them:
-    // measured best at 8192 x 8192 (43.9 us against 45.9 with 1024).  FOS_QUANT_GRID overrides for
-    // tuning runs.
-    int64_t grid = 768;
-    if (const int forced = tuning().quant_grid) grid = forced > 0 ? forced : grid;
-    if (grid > n) grid = n;
     p.tile_map = kMapSplitHalves;
     if (const int forced = tuning().quant_map) p.tile_map = forced - 1;
     const bool full = p.rows % 128 == 0 && p.cols % 512 == 0;
-    if (full)
-        hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, true, PSEUDO, false, SR>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-    else
-        hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, false, PSEUDO, false, SR>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-}
-
-// IF4 with the MSE rule, round to nearest, 16x16 tiles, aligned input.
-void launch_quantize_if4_mse_tiles(QuantParams &p, hipStream_t s) {
-    p.tiles_x = (int)((p.cols_p + 511) / 512);
-    const int64_t n = (p.rows_p / 128) * p.tiles_x;
+    if constexpr (!PSEUDO) {
+        const int split = tuning().quant_split;  // tuning / tests: 1 = never, 2 = always
+        if (split == 2 ? 4 * n <= 0x7fffffff : (split == 0 && n <= kSplitTiles)) {
+            const dim3 grid((unsigned)(4 * n));
+            if (full) hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, true, false, IF4, SR, true>), grid, dim3(kThreads), 0, s, p);
+            else hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, false, false, IF4, SR, true>), grid, dim3(kThreads), 0, s, p);
+            return;
+        }
+    }
     int64_t grid = 768;
     if (const int forced = tuning().quant_grid) grid = forced > 0 ? forced : grid;
     if (grid > n) grid = n;
-    p.tile_map = kMapSplitHalves;
-    if (const int forced = tuning().quant_map) p.tile_map = forced - 1;
-    if (p.rows % 128 == 0 && p.cols % 512 == 0)
-        hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<FOS_RULE_MSE, true, false, true>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-    else
-        hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<FOS_RULE_MSE, false, false, true>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+    if (full) hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, true, PSEUDO, IF4, SR>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+    else hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, false, PSEUDO, IF4, SR>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
 }
+
+template <int RULE, bool PSEUDO, bool SR>
+void launch_quantize_nvfp4_tiles(QuantParams &p, hipStream_t s) { launch_tiles<RULE, PSEUDO, false, SR>(p, s); }
+
+// IF4 with the MSE rule, round to nearest, 16x16 tiles, aligned input.
+void launch_quantize_if4_mse_tiles(QuantParams &p, hipStream_t s) { launch_tiles<FOS_RULE_MSE, false, true, false>(p, s); }
 
 template void launch_quantize_nvfp4_tiles<FOS_RULE_STATIC_6, false, false>(QuantParams &, hipStream_t);
 template void launch_quantize_nvfp4_tiles<FOS_RULE_STATIC_6, true, false>(QuantParams &, hipStream_t);

@@ -433,6 +433,26 @@ def test_if4_blocks_whose_candidates_nearly_tie(oracle, shape, scale):
     assert_same_quantization(q, oracle.quantize(x, dtype="if4", scale_rule="mse"), f"{shape} scale {scale}")
 
 
+@pytest.mark.parametrize("cfg", [dict(), dict(block_scale_2d=True), dict(dtype="if4"), dict(dtype="if4", block_scale_2d=True),
+                                 dict(round_style="stochastic", kwargs={"seed": 3}),
+                                 dict(round_style="stochastic", block_scale_2d=True, kwargs={"seed": 3}),
+                                 dict(scale_rule="static_6"), dict(scale_rule="abs_max", block_scale_2d=True)], ids=str)
+@pytest.mark.parametrize("shape", [(1, 16), (33, 272), (128, 256), (129, 512), (300, 4112), (256, 8192)])
+def test_tiles_in_four_parts_equal_whole_tiles(monkeypatch, oracle, shape, cfg):
+    """Rows that end in each of a tile's four parts, widths that end in each of its windows: the bytes of the kernels
+    that walk whole tiles, padding included, and the oracle's."""
+    x = make_input("outlier", shape, 57)
+    xs = [x] + ([x.half()] if "dtype" not in cfg and "round_style" not in cfg else [])
+    for y in xs:
+        parts = []
+        for split in ("1", "2"):
+            monkeypatch.setenv("FOS_QUANT_SPLIT", split)
+            parts.append(hip_quantize(y, **cfg))
+        assert torch.equal(parts[0].values, parts[1].values)
+        assert torch.equal(parts[0].scale_factors.view(torch.uint8), parts[1].scale_factors.view(torch.uint8))
+        assert_same_quantization(parts[1], oracle.quantize(y, **{k: v for k, v in cfg.items() if k != "kwargs"}, **cfg.get("kwargs", {})), f"{shape}")
+
+
 @pytest.mark.parametrize("rule", ["mse", "mae", "static_6", "static_4"])
 @pytest.mark.parametrize("two_d", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
