@@ -386,7 +386,8 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
                          uint64_t seed, uint64_t offset, int sf_layout,
                          uint8_t *codes, uint8_t *sf, float *amax, int amax_is_input,
                          void *workspace, size_t workspace_bytes, fos_stream_t stream,
-                         uint16_t *pseudo_out, int64_t ldo, const uint64_t *key = nullptr, int ready_partials = 0) {
+                         uint16_t *pseudo_out, int64_t ldo, const uint64_t *key = nullptr, int ready_partials = 0,
+                         float *zero_out = nullptr) {
     if (!x || !amax || (!pseudo_out && (!codes || !sf))) return FOS_E_NULL_POINTER;
     if ((uintptr_t)key & 7) return FOS_E_BAD_ALIGNMENT;
     if (dtype == FOS_DTYPE_MXFP4) {
@@ -442,6 +443,7 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
     p.codes = codes; p.sf = sf;
     p.seed = seed; p.offset = offset;
     p.key = key;
+    p.zero_out = zero_out;
     p.sf_layout = sf_layout;
 
     if (ready_partials > 0) {
@@ -505,6 +507,56 @@ extern "C" int fos_quantize(const void *x, int x_type, int64_t rows, int64_t col
                             void *workspace, size_t workspace_bytes, fos_stream_t stream) {
     return quantize_impl(x, x_type, rows, cols, ld, dtype, rule, round_style, block2d, seed, offset, sf_layout, codes, sf,
                          amax, amax_is_input, workspace, workspace_bytes, stream, nullptr, 0);
+}
+
+// Scratch of fos_linear_nvfp4: codes, scales, tensor maximum, pass-1 partials and split-K partials, each from a
+// 256-byte boundary on.
+namespace {
+struct LinearScratch {
+    size_t codes = 0, sf, amax, partials, gemm, total;
+    LinearScratch(int64_t rows, int64_t cols, int64_t N) {
+        auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+        const size_t elems = (size_t)fos_padded_rows(rows) * (size_t)fos_padded_cols(cols);
+        sf = up(elems / 2);
+        amax = sf + up(elems / 16);
+        partials = amax + 256;
+        gemm = partials + up(fos_quantize_workspace_bytes(rows, cols));
+        total = gemm + fos_gemm_workspace_bytes(gemm_rows(rows, cols), N, fos_padded_cols(cols));
+    }
+    // rows the product is made for: a small batch's own where the weight-streaming kernels take it
+    static int64_t gemm_rows(int64_t rows, int64_t cols) {
+        return rows < 128 && fos_padded_cols(cols) % 256 == 0 ? rows : fos_padded_rows(rows);
+    }
+};
+}  // namespace
+
+extern "C" size_t fos_linear_nvfp4_scratch_bytes(int64_t rows, int64_t cols, int64_t N) {
+    if (rows <= 0 || cols <= 0 || N <= 0) return 0;
+    return LinearScratch(rows, cols, N).total;
+}
+
+extern "C" int64_t fos_linear_nvfp4_rows(int64_t rows, int64_t cols) {
+    return rows <= 0 || cols <= 0 ? 0 : LinearScratch::gemm_rows(rows, cols);
+}
+
+extern "C" int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int rule, const float *x_amax,
+                                const uint8_t *W, const uint8_t *sfW, const float *w_amax, double denominator, int64_t N,
+                                void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
+                                void *scratch, size_t scratch_bytes, fos_stream_t stream) {
+    if (!scratch) return FOS_E_NULL_POINTER;
+    if (rows <= 0 || cols <= 0 || N <= 0) return FOS_E_BAD_SHAPE;
+    if (((uintptr_t)scratch & 255) || ((uintptr_t)d_amax & 3)) return FOS_E_BAD_ALIGNMENT;
+    const LinearScratch at(rows, cols, N);
+    if (scratch_bytes < at.total) return FOS_E_WORKSPACE;
+    uint8_t *base = static_cast<uint8_t *>(scratch);
+    float *amax = x_amax ? const_cast<float *>(x_amax) : reinterpret_cast<float *>(base + at.amax);
+    const int rc = quantize_impl(x, x_type, rows, cols, ld, FOS_DTYPE_NVFP4, rule, FOS_ROUND_NEAREST, 0, 0, 0, FOS_SF_TILED_128X4,
+                                 base + at.codes, base + at.sf, amax, x_amax != nullptr, base + at.partials, at.gemm - at.partials, stream,
+                                 nullptr, 0, nullptr, 0, d_amax);
+    if (rc != FOS_OK) return rc;
+    return fos_gemm_nvfp4_linear(base + at.codes, W, base + at.sf, sfW, amax, w_amax, denominator, LinearScratch::gemm_rows(rows, cols), N,
+                                 fos_padded_cols(cols), D, out_type, ldd, bias, d_amax, at.total > at.gemm ? base + at.gemm : nullptr,
+                                 at.total - at.gemm, stream);
 }
 
 extern "C" int fos_quantize_devkey(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld,

@@ -27,6 +27,7 @@ struct QuantParams {
     int n_partials;              // number of pairs; 0 = `partials` points at a caller-supplied f32 amax;
                                  // -1 = no pass 1 ran: pass 2 scans the (small, contiguous, aligned) input itself
     float *amax_out;             // written by workgroup 0 when not null
+    float *zero_out = nullptr;   // set to 0 by workgroup 0 when not null (a word that the next kernel folds a maximum into)
     uint64_t seed, offset;       // dither key of the stochastic styles ...
     const uint64_t *key = nullptr;  // ... or, when not null, where the kernels read {seed, offset} from (device memory)
     int sf_layout;

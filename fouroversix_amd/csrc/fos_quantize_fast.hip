@@ -145,6 +145,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
     k.exact_ok = k.errdiv == 1536.0f && (amax_bits & (F16 ? 0x1fffu : 0xffffu)) == 0;
     k.shortcut_ok = shortcut_range(k.amax);
     if (blockIdx.x == 0 && threadIdx.x == 0 && p.amax_out) *p.amax_out = k.amax;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && p.zero_out) *p.zero_out = 0.0f;
     // dither key: launch arguments, or read from device memory (a captured launch whose key the caller advances)
     uint64_t key_seed = p.seed, key_offset = p.offset;
     if (SR && p.key) {

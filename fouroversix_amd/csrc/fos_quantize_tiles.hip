@@ -269,6 +269,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
     k.qdiv = p.qdiv;
     k.errdiv = p.errdiv;
     if (blockIdx.x == 0 && threadIdx.x == 0 && p.amax_out) *p.amax_out = k.amax;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && p.zero_out) *p.zero_out = 0.0f;
     const bool in_range = k.amax >= 0x1p-100f && k.amax <= 0x1p100f;
     const float enc_fast = in_range ? k.enc : 0.0f;
     const float rq = sgpr(1.0f / k.qdiv), rc = sgpr(1.0f / p.c);

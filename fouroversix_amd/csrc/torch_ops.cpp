@@ -304,6 +304,63 @@ Tensor gemm_nvfp4_amax(const Tensor &a, const Tensor &b, const Tensor &a_sf, con
                        bias.has_value() ? &*bias : nullptr);
 }
 
+// A word for a recorded maximum: one of a block of 4096 per (device, stream), each handed out once, so that the block is
+// not given back, and the word not overwritten, while a reader on another stream may still be at work on a result whose
+// lifetime was extended without this word's.  Inside a capture a tensor of its own (the graph's private pool).
+Tensor amax_word(const Tensor &like, fos_stream_t stream) {
+    const auto opts = like.options().dtype(at::kFloat);
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return at::empty({1}, opts);
+    constexpr int64_t kWords = 4096;
+    struct Block {
+        Tensor words;
+        int64_t used = kWords;
+    };
+    static std::mutex mutex;
+    static std::unordered_map<uint64_t, Block> blocks;
+    std::lock_guard<std::mutex> lock(mutex);
+    Block &b = blocks[((uint64_t)(uintptr_t)stream << 8) ^ (uint64_t)like.get_device()];
+    if (b.used == kWords) {
+        b.words = at::empty({kWords}, opts);
+        b.used = 0;
+    }
+    return b.words.narrow(0, b.used++, 1);
+}
+
+// A linear layer in one call: x quantized to NVFP4 (1x16 blocks, round to nearest), times the quantized weight.  What the
+// frontends do in two calls with a QuantizedTensor between them (decode-sized layers cost the host more than
+// the GPU).  The weight's members have been looked at by the frontend; the result has the padded extents, or
+// x's own rows where the kernel skips the padding of a small batch.
+// Returns {result, recorded maximum or None}.
+std::tuple<Tensor, c10::optional<Tensor>> linear_nvfp4(const Tensor &x, int64_t rule, const c10::optional<Tensor> &x_amax, const Tensor &w,
+                                                       const Tensor &w_sf, const Tensor &w_amax, double denominator,
+                                                       at::ScalarType out_dtype, bool emit_amax, const c10::optional<Tensor> &bias) {
+    TORCH_CHECK(x.dim() == 2 && x.size(0) > 0 && x.size(1) > 0 && x.stride(-1) == 1 && x.is_cuda() && x.device() == w.device(),
+                "linear: a non-empty 2-D input with contiguous rows on the weight's GPU");
+    const int64_t rows = x.size(0), cols = x.size(1), n = w.size(0);
+    TORCH_CHECK(fos_padded_cols(cols) == w.size(1) * 2, "Inner dims mismatch: ", fos_padded_cols(cols), " vs ", w.size(1) * 2);
+    const int out_type = type_id(out_dtype, "linear: out_dtype");
+    if (bias.has_value())
+        TORCH_CHECK(bias->scalar_type() == out_dtype && bias->dim() == 1 && bias->size(0) == n && bias->is_contiguous() && bias->device() == x.device(),
+                    "linear: bias must be a contiguous [N] tensor of the output type");
+    Tensor known;
+    if (x_amax.has_value()) known = amax_buffer(x_amax, x);
+    Tensor out = at::empty({fos_linear_nvfp4_rows(rows, cols), n}, x.options().dtype(out_dtype));
+    const DeviceGuard guard(x.device());
+    const fos_stream_t stream = current_stream(x);
+    c10::optional<Tensor> d_amax;
+    if (emit_amax) d_amax = amax_word(x, stream);
+    // (one block for the quantized input and the workspaces, from the caching allocator on the current stream)
+    const size_t bytes = fos_linear_nvfp4_scratch_bytes(rows, cols, n);
+    const Tensor scratch = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+    check(fos_linear_nvfp4(x.data_ptr(), type_id(x.scalar_type(), "linear: x"), rows, cols, x.stride(0), (int)rule,
+                           x_amax.has_value() ? known.data_ptr<float>() : nullptr, w.data_ptr<uint8_t>(),
+                           static_cast<const uint8_t *>(w_sf.data_ptr()), w_amax.data_ptr<float>(), denominator, n, out.data_ptr(), out_type,
+                           n, bias.has_value() ? bias->data_ptr() : nullptr, emit_amax ? d_amax->data_ptr<float>() : nullptr,
+                           scratch.data_ptr(), bytes, stream),
+          "fouroversix::linear_nvfp4");
+    return {out, d_amax};
+}
+
 // IF4 x IF4 (row-major E4M3 scales), output scale from the two maxima, optional bias and recorded maximum as above.
 Tensor gemm_if4(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tensor &b_sf, const Tensor &amax_a, const Tensor &amax_b,
                 double denominator, at::ScalarType out_dtype, const c10::optional<Tensor> &d_amax, const c10::optional<Tensor> &bias) {
@@ -429,6 +486,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("transform_quantize", &transform_quantize);
     m.def("gemm_nvfp4", &gemm_nvfp4);
     m.def("gemm_nvfp4_amax", &gemm_nvfp4_amax);
+    m.def("linear_nvfp4", &linear_nvfp4);
     m.def("gemm_if4", &gemm_if4);
     m.def("gemm_alpha", &gemm_alpha);
     m.def("gemm_mxfp4", &gemm_mxfp4_typed);

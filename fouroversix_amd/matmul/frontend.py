@@ -17,8 +17,14 @@ import torch
 from fouroversix_amd import _native as nat
 from fouroversix_amd.quantize import QuantizationConfig, QuantizedTensor, quantize
 from fouroversix_amd.quantize import ops
-from fouroversix_amd.quantize.frontend import attach_known_amax, dequantize, dequantize_divisor
-from fouroversix_amd.utils import NATIVE_FORMAT_IDS, DataType, MatmulBackend
+from fouroversix_amd.quantize.frontend import (
+    attach_known_amax,
+    dequantize,
+    dequantize_divisor,
+    format_divisor,
+    known_amax,
+)
+from fouroversix_amd.utils import NATIVE_FORMAT_IDS, DataType, MatmulBackend, RoundStyle, ScaleRule
 
 
 def is_supported(input: QuantizedTensor, other: QuantizedTensor, *, out_dtype: DataType) -> bool:
@@ -199,6 +205,51 @@ def gemm_alpha(input: QuantizedTensor, other: QuantizedTensor) -> torch.Tensor:
         ops.gemm_alpha_into(a, b, den, alpha)
         return alpha
     return ((a * b) / den).to(torch.float32).reshape(1)
+
+
+_NVFP4_RULES = frozenset(DataType.nvfp4.supported_scale_rules)
+
+
+def nvfp4_linear(
+    x: torch.Tensor,
+    weight: QuantizedTensor,
+    scale_rule: ScaleRule,
+    out_dtype: DataType,
+    bias: torch.Tensor | None,
+    *,
+    emit_amax: bool,
+) -> torch.Tensor | None:
+    """``quantize`` of ``x`` ([tokens, in], NVFP4, 1x16 blocks, round to nearest) and ``quantized_matmul`` with
+    ``weight`` as one call into the library, with the same result; None where the two calls have to be made (other
+    layouts, devices or types, an input they refuse)."""
+    rec = _gemm_record(weight)
+    if not (
+        rec[3]
+        and type(x) is torch.Tensor
+        and x.dim() == 2
+        and x.device == rec[6]
+        and x.shape[0] > 0
+        and x.shape[1] == rec[7] > 0
+        and x.stride(1) == 1
+        and x.dtype in nat.TORCH_TO_T
+        and scale_rule in _NVFP4_RULES
+        and rec[0].shape[0] % 128 == 0
+        and (out_dtype is DataType.bfloat16 or out_dtype is DataType.float16)
+    ):
+        return None
+    torch_dtype = torch.bfloat16 if out_dtype is DataType.bfloat16 else torch.float16
+    fused_bias = bias is not None and _fusable_bias(bias, torch_dtype, rec[0].shape[0], rec[6])
+    out, d_amax = ops.linear_nvfp4(
+        x, scale_rule.cuda_id, known_amax(x), rec[0], rec[1], rec[2],
+        format_divisor(DataType.nvfp4, scale_rule, RoundStyle.nearest) * rec[5], torch_dtype,
+        emit_amax and (bias is None or fused_bias), bias.detach() if fused_bias else None,
+    )
+    m, n = x.shape[0], weight.original_shape[0]
+    if out.shape[0] != m or out.shape[1] != n:
+        out = out[:m, :n]  # (the padding is zeros: same maximum)
+    if d_amax is not None:
+        attach_known_amax(out, d_amax)
+    return out if bias is None or fused_bias else out + bias
 
 
 def quantized_matmul(

@@ -20,9 +20,10 @@ import torch
 import torch.nn as nn
 
 from fouroversix_amd.matmul import quantized_matmul
+from fouroversix_amd.matmul.frontend import nvfp4_linear
 from fouroversix_amd.quantize import QuantizedTensor, dequantize, quantize
 from fouroversix_amd.quantize.frontend import attach_known_amax, known_amax
-from fouroversix_amd.utils import DataType
+from fouroversix_amd.utils import DataType, RoundStyle
 
 from .config import ModuleQuantizationConfig
 from .quantize import QuantizedModule
@@ -52,15 +53,24 @@ def fp4_linear(
                 attach_known_amax(flat, amax_in)
             # (the bias goes into the GEMM's epilogue with the two roundings of `out + bias`; the recorded
             # maximum is then that of the sum)
-            out2d = quantized_matmul(
-                flat,
-                weight,
-                backend=config.matmul_backend,
-                input_config=config.get_activation_config(),
-                out_dtype=config.output_dtype,
-                emit_amax=config.emit_output_amax,
-                bias=bias,
-            )
+            out2d = None
+            if (
+                config.activation_dtype is DataType.nvfp4
+                and config.activation_round_style is RoundStyle.nearest
+                and not torch.compiler.is_compiling()
+            ):
+                out2d = nvfp4_linear(flat, weight, config.activation_scale_rule, config.output_dtype, bias,
+                                     emit_amax=config.emit_output_amax)
+            if out2d is None:
+                out2d = quantized_matmul(
+                    flat,
+                    weight,
+                    backend=config.matmul_backend,
+                    input_config=config.get_activation_config(),
+                    out_dtype=config.output_dtype,
+                    emit_amax=config.emit_output_amax,
+                    bias=bias,
+                )
             out = out2d.reshape(*input.shape[:-1], weight.original_shape[0])
             amax_out = known_amax(out2d)
             if amax_out is not None and out is not out2d:
@@ -127,6 +137,17 @@ class FourOverSixLinearFunction(torch.autograd.Function):
 
         grad_bias = g.sum(0) if bias is not None and ctx.needs_input_grad[3] else None
         return None, grad_input, grad_weight, grad_bias
+
+
+def _seen_by_autograd_functions() -> bool:
+    """Whether something other than backward mode looks at autograd functions: a trace, a functorch transform or
+    forward-mode differentiation (which stays on under ``torch.no_grad()``)."""
+    return (
+        torch.compiler.is_compiling()
+        or torch._C._get_tracing_state() is not None
+        or torch._C._are_functorch_transforms_active()
+        or torch.autograd.forward_ad._current_level >= 0
+    )
 
 
 @QuantizedModule.register(nn.Linear)
@@ -221,4 +242,6 @@ class FourOverSixLinear(nn.Linear):
         return self._quantized_weight
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
+        if not torch.is_grad_enabled() and not _seen_by_autograd_functions():
+            return fp4_linear(self.config, input, self.quantized_weight(), self.bias)
         return FourOverSixLinearFunction.apply(self.config, input, self.quantized_weight(), self.bias)

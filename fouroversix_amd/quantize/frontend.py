@@ -248,7 +248,8 @@ def quantize(
 
 
 @functools.lru_cache(maxsize=None)
-def _divisor(dtype: DataType, scale_rule, round_style) -> float:
+def format_divisor(dtype: DataType, scale_rule, round_style) -> float:
+    """qmax * smax * adjustment of a format under a scale rule and rounding style."""
     return (
         dtype.quantized_value_type.get_maximum_value(scale_rule)
         * dtype.scale_type.get_maximum_value(scale_rule)
@@ -258,7 +259,7 @@ def _divisor(dtype: DataType, scale_rule, round_style) -> float:
 
 def dequantize_divisor(tensor: QuantizedTensor) -> float:
     """qmax * smax * adjustment of the tensor's scale rule and rounding style."""
-    return _divisor(tensor.dtype, tensor.scale_rule, tensor.round_style)
+    return format_divisor(tensor.dtype, tensor.scale_rule, tensor.round_style)
 
 
 def dequantize(

@@ -119,6 +119,12 @@ def gemm_nvfp4_from_amax(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtyp
     return _C.gemm_nvfp4_amax(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, checked, bias)
 
 
+def linear_nvfp4(x, selection_rule, x_amax, w, w_sf, w_amax, denominator, out_dtype, emit_amax=False, bias=None):
+    """``quantize_ex`` of ``x`` to NVFP4 (1x16 blocks, round to nearest) and ``gemm_nvfp4_from_amax`` with the
+    quantized weight's members, in one call: ``(out, max|out| or None)``."""
+    return _C.linear_nvfp4(x, selection_rule, x_amax, w, w_sf, w_amax, denominator, out_dtype, emit_amax, bias)
+
+
 def gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax=None, bias=None):
     """IF4 x IF4 product with the output scale of ``gemm_nvfp4_from_amax``; ``d_amax`` and ``bias`` as there."""
     return _C.gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, bias)

@@ -281,6 +281,21 @@ int fos_gemm_nvfp4_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA
                           float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream);
 
 /*
+ * A linear layer in one call: x ([rows, cols], bf16 / fp16 / fp32) quantized to NVFP4 (1x16 blocks, round to nearest, scale
+ * rule `rule`; maximum x_amax[0] if given, found otherwise), times the quantized weight W [N, padded cols], as
+ * fos_quantize followed by fos_gemm_nvfp4_linear gives it.  D has fos_linear_nvfp4_rows(rows, cols) rows (the padded
+ * ones, or `rows` where the product skips the padding of a small batch).  d_amax, when given, is set to max|D| (unlike
+ * there it needs no initial value: the quantize kernel clears it).  `scratch`: fos_linear_nvfp4_scratch_bytes bytes,
+ * 256-byte aligned, in use until the product is done.
+ */
+size_t fos_linear_nvfp4_scratch_bytes(int64_t rows, int64_t cols, int64_t N);
+int64_t fos_linear_nvfp4_rows(int64_t rows, int64_t cols);
+int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int rule, const float *x_amax,
+                     const uint8_t *W, const uint8_t *sfW, const float *w_amax, double denominator, int64_t N,
+                     void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
+                     void *scratch, size_t scratch_bytes, fos_stream_t stream);
+
+/*
  * IF4 x IF4 product: as fos_gemm_nvfp4_linear for operands in the IF4 format (row-major scale bytes, bit 7 = integer
  * block; values and block scales meet in fp16 as in fos_dequantize with intermediate_type FOS_T_F16).  M, N multiples
  * of 128, K of 64 (the padded extents of quantized tensors).  The reference has no native product for this format: it

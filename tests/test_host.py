@@ -171,3 +171,24 @@ def test_reference_import_name_and_rht_matrix(oracle):
     assert torch.equal(m.float() @ m.float().T, torch.eye(16))
     plain = get_rht_matrix(with_random_sign_mask=False, device="cpu")
     assert torch.equal(plain[0].float(), torch.full((16,), 0.25)) and torch.equal(plain.float(), plain.float().T)
+
+
+def test_layers_without_gradients_keep_the_autograd_function_where_it_is_seen():
+    """The direct forward pass is for plain calls: a functorch transform and forward-mode differentiation (on under
+    no_grad as well) still meet the autograd function."""
+    from fouroversix_amd.model.linear import _seen_by_autograd_functions
+
+    seen = []
+
+    def note(x):
+        seen.append(_seen_by_autograd_functions())
+        return x
+
+    x = torch.ones(2, 3)
+    with torch.no_grad():
+        note(x)
+        torch.func.vmap(note)(x)
+        with torch.autograd.forward_ad.dual_level():
+            note(x)
+    torch.jit.trace(note, (x,), check_trace=False)
+    assert seen == [False, True, True, True]

@@ -233,6 +233,35 @@ def test_linear_layer_forward(oracle):
     assert torch.equal(keep(x.cuda()), y)
 
 
+@pytest.mark.parametrize(("tokens", "inf", "outf"), [(1, 256, 128), (16, 4096, 256), (100, 1024, 300), (129, 80, 144), (0, 256, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "fp16", "fp32"])
+def test_layer_in_one_call_equals_quantize_and_matmul(tokens, inf, outf, dtype):
+    """The forward pass without gradients (one call into the library) against the two calls it stands for: strides,
+    sizes that get padding, biases that are fused and that are not, a recorded maximum on the input."""
+    from fouroversix_amd.quantize import attach_known_amax, known_amax
+
+    for bias_dtype in (None, torch.bfloat16, torch.float32):
+        layer = nn.Linear(inf, outf, bias=bias_dtype is not None, device="cuda", dtype=torch.bfloat16)
+        if bias_dtype is not None:
+            layer.bias = nn.Parameter(torch.randn(outf, device="cuda").to(bias_dtype))
+        model = nn.Sequential(layer)
+        fos.quantize_model(model, fos.ModelQuantizationConfig(weight_scale_2d=True))
+        model[0].quantize_weight_()
+        wide = make_input("outlier", (max(tokens, 1), 2 * inf), 81).to(dtype).cuda()
+        for x in (wide[:tokens, :inf].contiguous(), wide[:tokens, :inf], wide[:tokens, ::2]):
+            if tokens == 0:
+                continue
+            with torch.no_grad():
+                out = model(x)
+                expect = fos.quantized_matmul(x, model[0].quantized_weight(), emit_amax=True, bias=model[0].bias)
+                assert torch.equal(out, expect) and out.shape == (tokens, outf)
+                a, b = known_amax(out), known_amax(expect)
+                assert (a is None) == (b is None) and (a is None or float(a) == float(b))
+                known = x.clone()
+                attach_known_amax(known, x.abs().max().float().reshape(1))
+                assert torch.equal(model(known[None])[0], expect)
+
+
 def test_quantized_checkpoint_round_trip():
     """A quantized layer's state_dict -- the four `quantized_weight_*` buffers of the reference
     (src/fouroversix/model/modules/linear.py:326-361,379-443) plus the bias -- saved, read back with
