@@ -39,6 +39,7 @@
 #include <type_traits>
 
 #include "fos_device.h"
+#include "fos_gemm_tiles.h"
 #include "fos_tuning.h"
 #include "fouroversix_hip.h"
 
@@ -249,18 +250,6 @@ struct Staged {
     uint4 qb[WN];  // B row of tile j: codes 32 h ... 32 h + 31 of the step (h = lane >> 5)
     uint32_t sb[WN];
 };
-
-// Output tile of workgroup `bid`: workgroups with equal bid % 8 share an XCD; give each
-// XCD a contiguous run of tiles, ordered in column bands of 8 tile rows.
-FOS_DEVICE void tile_of(int bid, int tiles_m, int tiles_n, int &tm, int &tn) {
-    const int per_xcd = tiles_m * tiles_n / 8;
-    const int t = bid < 8 * per_xcd ? (bid & 7) * per_xcd + (bid >> 3) : bid;  // (the remainder in plain order)
-    constexpr int kBand = 8;
-    const int band = t / (kBand * tiles_n), in_band = t - band * kBand * tiles_n;
-    const int rows = (tiles_m - band * kBand) < kBand ? (tiles_m - band * kBand) : kBand;
-    tm = band * kBand + in_band % rows;
-    tn = in_band / rows;
-}
 
 // WAVES_M x WAVES_N wavefronts, each WM x WN MFMA tiles of 32 x 32.  The MFMA "A" operand
 // is fed from the B matrix (rows n) and the "B" operand from the A matrix (rows m), so
@@ -1160,15 +1149,6 @@ struct GemmPlan {
     int wide;    // M > 32: workgroups of 64 rows of B and 64 rows of A, four wavefronts with two by two tiles each
 };
 constexpr int kTargetWorkgroups = 256;
-
-// Time of `tiles` output tiles: whole generations (as many tiles as run at a time) at `generation` each, then the
-// last, partial one, whose time depends on how full the chip is (fewer compute units clock higher): `tail`, by
-// eighths of a generation.
-static float tiles_cost(int64_t tiles, int64_t per_generation, float generation, const float (&tail)[8]) {
-    const int64_t whole = tiles / per_generation, rest = tiles % per_generation;
-    if (rest == 0) return whole == 1 ? tail[7] : (float)whole * generation;
-    return (float)whole * generation + tail[(rest * 8 - 1) / per_generation];
-}
 
 // Tile size: the cheapest of the three by what their generations take (us at K = 4096; all scale with K).  256
 // workgroups of the 256 x 256 and 128 x 256 tiles run at a time, 512 of the 128 x 128 tile.  Measured with the

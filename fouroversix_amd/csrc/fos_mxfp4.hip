@@ -20,6 +20,7 @@
 #include <cstdlib>
 
 #include "fos_buffer.h"
+#include "fos_gemm_tiles.h"
 #include "fos_quantize_fast.h"
 #include "fos_tuning.h"
 #include "fouroversix_hip.h"
@@ -520,17 +521,8 @@ int launch_dequantize_mxfp4(const uint8_t *codes, const uint8_t *sf, int sf_layo
 // C[8 g + 4 (l >> 5) + e][l & 31] with rows taken from the first operand.  B (rows n) is
 // fed as the first operand so that a lane's consecutive registers are consecutive n.
 //
-// Tile 256 x 256 x 128 (BK = 128 codes = 64 bytes per row = one scale chunk), 8 wavefronts
-// of 128 x 64, LDS pitch 80 bytes (conflict-free 128-bit accesses), two stages; the
-// pipeline is the one of the NVFP4 kernel minus the dequantisation: registers hold step
-// k+2 in flight, step k+1 goes to LDS in halves while step k is multiplied.  Scales bypass
-// LDS: the 128x4 tiled layout holds the four scale bytes of a 128-wide K chunk of rows r,
-// r+32, r+64, r+96 next to each other, so a wavefront's lanes fetch one 32-bit word per
-// row tile and chunk straight from global memory.
-
 typedef int mx_v8i __attribute__((ext_vector_type(8)));
 typedef float mx_v16f __attribute__((ext_vector_type(16)));
-typedef __amdgpu_buffer_rsrc_t MxRsrc;
 
 struct MxGemmParams {
     const uint8_t *A, *B, *sfA, *sfB;
@@ -541,44 +533,10 @@ struct MxGemmParams {
 };
 
 constexpr int kMxBK = 128;    // codes per K step
-constexpr int kMxPitch = 80;  // LDS bytes per row (64 + 16)
-
-FOS_DEVICE MxRsrc mx_rsrc(const void *base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
-}
-
-// N consecutive 32-bit words (N = 1, 2, 4) with one buffer load.
-template <int N>
-FOS_DEVICE void mx_load_words(uint32_t (&dst)[N], MxRsrc r, int voffset, int soffset) {
-    static_assert(N == 1 || N == 2 || N == 4, "one load instruction");
-    if constexpr (N == 1) {
-        dst[0] = __builtin_amdgcn_raw_buffer_load_b32(r, voffset, soffset, 0);
-    } else if constexpr (N == 2) {
-        const auto v = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, voffset, soffset, 0));
-        dst[0] = v.x, dst[1] = v.y;
-    } else {
-        const auto v = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voffset, soffset, 0));
-        dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
-    }
-}
 
 FOS_DEVICE mx_v8i frag_of(const uint4 &q) {
     mx_v8i v = {(int)q.x, (int)q.y, (int)q.z, (int)q.w, 0, 0, 0, 0};  // FP4 operands use the first four registers
     return v;
-}
-
-FOS_DEVICE void mx_tile_of(int bid, int tiles_m, int tiles_n, int &tm, int &tn) {
-    // workgroups with equal bid % 8 share an XCD: give each XCD a compact run of tiles,
-    // ordered in column bands of 8 tile rows
-    const int total = tiles_m * tiles_n;
-    const int per_xcd = (total + 7) / 8;
-    int t = (bid & 7) * per_xcd + (bid >> 3);
-    if (t >= total || (total & 7) != 0) t = bid;
-    constexpr int kBand = 8;
-    const int band = t / (kBand * tiles_n), in_band = t - band * kBand * tiles_n;
-    const int rows = (tiles_m - band * kBand) < kBand ? (tiles_m - band * kBand) : kBand;
-    tm = band * kBand + in_band % rows;
-    tn = in_band / rows;
 }
 
 // Epilogue of the tile kernels.  acc[i][j][4 g + e] is D[m][n] with m = 32 i + r and
@@ -586,16 +544,18 @@ FOS_DEVICE void mx_tile_of(int bid, int tiles_m, int tiles_n, int &tm, int &tn) 
 // the registers, an instruction would touch 32 rows with 16 bytes each (1.6 bytes written to
 // memory per byte of output).  Each wavefront turns a 32-row tile round in its own piece of
 // the operand staging, which is idle by now (the caller has waited for every wavefront), and
-// stores whole rows of its block, 16 bytes per lane.
+// stores whole rows of its block, 16 bytes per lane: the first `rows` of them, or none if the block's columns
+// lie beyond the output.
 template <int WM, int WN, bool OUT_BF16>
 FOS_DEVICE void mx_store_rows(const mx_v16f (&acc)[WM][WN], uint8_t *lds, int wave, int lane, float alpha, uint16_t *D,
-                              int64_t ldd, int64_t m_base, int64_t n_base) {
+                              int64_t ldd, int64_t m_base, int64_t n_base, int rows, bool columns_inside) {
     constexpr int kRowBytes = WN * 64, kEpiPitch = kRowBytes + 16;
     constexpr int kLanesPerRow = kRowBytes / 16, kRowsPerPass = 64 / kLanesPerRow;
     const int r = lane & 31, h = lane >> 5;
     uint8_t *epi = lds + wave * 32 * kEpiPitch;
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
+        if (!columns_inside || 32 * i >= rows) break;  // (beyond the output; uniform over the wavefront)
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
 #pragma unroll
@@ -629,186 +589,14 @@ FOS_DEVICE void mx_store_rows(const mx_v16f (&acc)[WM][WN], uint8_t *lds, int wa
     }
 }
 
-template <int WAVES_M, int WAVES_N, int WM, int WN, bool OUT_BF16>
-__global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_mxfp4_kernel(const MxGemmParams p) {
-    constexpr int kThreadsG = 64 * WAVES_M * WAVES_N;
-    constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
-    constexpr int kRowsPerPass = kThreadsG / 4;  // 4 lanes cover the 64 bytes of a row
-    constexpr int PA = BM / kRowsPerPass, PB = BN / kRowsPerPass;
-    static_assert(PA % 2 == 0 && PB % 2 == 0 && WM * 32 <= 128 && WN * 32 <= 128, "tile shape: staged in two halves");
-    extern __shared__ __attribute__((aligned(16))) uint8_t mx_lds[];
-    uint8_t *lds_a[2] = {mx_lds, mx_lds + (BM + BN) * kMxPitch};
-    uint8_t *lds_b[2] = {mx_lds + BM * kMxPitch, mx_lds + (BM + BN) * kMxPitch + BM * kMxPitch};
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 31, h = lane >> 5;
-    int tile_m, tile_n;
-    mx_tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-    const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
-    const int64_t kbytes = p.K >> 1;
-    const int64_t ksteps = p.K / kMxBK;  // = 128-wide K chunks = scale groups per band
-
-    const MxRsrc ra = mx_rsrc(p.A + m0 * kbytes, (uint32_t)(BM * kbytes));
-    const MxRsrc rb = mx_rsrc(p.B + n0 * kbytes, (uint32_t)(BN * kbytes));
-    const int ld_row = tid >> 2, ld_col = (tid & 3) * 16;
-    const uint32_t q_off = (uint32_t)(ld_row * kbytes + ld_col);
-    const uint32_t lds_off = (uint32_t)(ld_row * kMxPitch + ld_col);
-
-    // scales of this wavefront's rows, straight from global memory
-    const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-    const int64_t a_row0 = m0 + wm * WM * 32, b_row0 = n0 + wn * WN * 32;
-    const MxRsrc rsa = mx_rsrc(p.sfA + (a_row0 >> 7) * ksteps * 512, (uint32_t)(ksteps * 512));
-    const MxRsrc rsb = mx_rsrc(p.sfB + (b_row0 >> 7) * ksteps * 512, (uint32_t)(ksteps * 512));
-    const uint32_t sa_off = (uint32_t)(r * 16 + ((a_row0 & 127) >> 5) * 4);
-    const uint32_t sb_off = (uint32_t)(r * 16 + ((b_row0 & 127) >> 5) * 4);
-
-    struct Staged {
-        uint4 a[PA], b[PB];
-    };
-    struct Scales {
-        uint32_t a[WM], b[WN];  // scale bytes of the step's four K blocks, per row tile
-    };
-    auto fetch = [&](int64_t ks, Staged &s) {
-        // per-pass and per-step displacements ride in the scalar offset: one address register
-        const int kq = (int)(ks * (kMxBK / 2));
-#pragma unroll
-        for (int i = 0; i < PA; ++i)
-            s.a[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)q_off, kq + (int)(i * kRowsPerPass * kbytes), 0));
-#pragma unroll
-        for (int i = 0; i < PB; ++i)
-            s.b[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)q_off, kq + (int)(i * kRowsPerPass * kbytes), 0));
-    };
-    // raw scale words of step ks (bytes = the four K blocks of the chunk)
-    // (the words of a wavefront's row tiles are adjacent in the 16-byte unit of row r: one
-    // load per operand instead of one per row tile)
-    auto fetch_scales = [&](int64_t ks, Scales &s) {
-        const int ksf = (int)(ks * 512);
-        mx_load_words<WM>(s.a, rsa, (int)sa_off, ksf);
-        mx_load_words<WN>(s.b, rsb, (int)sb_off, ksf);
-    };
-    // half q of the staged registers -> LDS stage `buf`
-    auto stage_part = [&](const Staged &s, int buf, int q) {
-#pragma unroll
-        for (int i = q * (PA / 2); i < (q + 1) * (PA / 2); ++i)
-            *reinterpret_cast<uint4 *>(lds_a[buf] + lds_off + i * kRowsPerPass * kMxPitch) = s.a[i];
-#pragma unroll
-        for (int i = q * (PB / 2); i < (q + 1) * (PB / 2); ++i)
-            *reinterpret_cast<uint4 *>(lds_b[buf] + lds_off + i * kRowsPerPass * kMxPitch) = s.b[i];
-    };
-
-    mx_v16f acc[WM][WN];
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-    auto read_frags = [&](int buf, int kk, uint4 *fa, uint4 *fb) {
-        const int kofs = kk * 32 + h * 16;
-#pragma unroll
-        for (int i = 0; i < WM; ++i) fa[i] = *reinterpret_cast<const uint4 *>(lds_a[buf] + (wm * WM * 32 + i * 32 + r) * kMxPitch + kofs);
-#pragma unroll
-        for (int j = 0; j < WN; ++j) fb[j] = *reinterpret_cast<const uint4 *>(lds_b[buf] + (wn * WN * 32 + j * 32 + r) * kMxPitch + kofs);
-    };
-
-    Staged st[2];
-    Scales sc[2];
-    uint4 fa[2][WM], fb[2][WN];
-    fetch(0, st[0]);
-    fetch_scales(0, sc[0]);
-    stage_part(st[0], 0, 0);
-    stage_part(st[0], 0, 1);
-    if (ksteps > 1) fetch(1, st[1]);
-    __syncthreads();
-    read_frags(0, 0, fa[0], fb[0]);
-
-    // One K step: multiply out of stage `buf` (fragments of slice 0 are in registers) while
-    // step ks+1 (`nxt`) goes to the other stage; the barrier sits between the last staging
-    // write and the last slice's MFMAs, and the next step's first fragments are read right
-    // after it.  Branch-free; the last step is its own instantiation.
-    auto kstep = [&](auto have_next_c, int64_t ks, int buf, Staged &cur_regs, Staged &nxt, const Scales &s_cur, Scales &s_nxt) {
-        constexpr bool have_next = decltype(have_next_c)::value;
-        // lanes of the upper half use the next byte: after the shift, byte 0 / byte 2 of every
-        // lane's register are the scales of the K blocks it feeds in slice 0 / slice 1.  Done
-        // here, a step after the load was issued, so that nothing waits on a fresh load.
-        Scales sh;
-#pragma unroll
-        for (int i = 0; i < WM; ++i) sh.a[i] = s_cur.a[i] >> (8 * h);
-#pragma unroll
-        for (int j = 0; j < WN; ++j) sh.b[j] = s_cur.b[j] >> (8 * h);
-        if (have_next) {
-            fetch_scales(ks + 1, s_nxt);
-            fetch(ks + 2 < ksteps ? ks + 2 : ksteps - 1, cur_regs);
-        }
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            if (kk == 0) read_frags(buf, 1, fa[1], fb[1]);
-            if (have_next) {
-                stage_part(nxt, buf ^ 1, kk);
-                if (kk == 1) {
-                    __syncthreads();
-                    read_frags(buf ^ 1, 0, fa[0], fb[0]);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j) {
-                    if (kk == 1)
-                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                            frag_of(fb[1][j]), frag_of(fa[1][i]), acc[i][j], 4, 4, 2, (int)sh.b[j], 2, (int)sh.a[i]);
-                    else
-                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                            frag_of(fb[0][j]), frag_of(fa[0][i]), acc[i][j], 4, 4, 0, (int)sh.b[j], 0, (int)sh.a[i]);
-                }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-
-    using yes = std::integral_constant<bool, true>;
-    using no = std::integral_constant<bool, false>;
-    int64_t ks = 0;
-    for (; ks + 2 < ksteps; ks += 2) {
-        kstep(yes{}, ks, 0, st[0], st[1], sc[0], sc[1]);
-        kstep(yes{}, ks + 1, 1, st[1], st[0], sc[1], sc[0]);
-    }
-    if (ks + 2 == ksteps) {
-        kstep(yes{}, ks, 0, st[0], st[1], sc[0], sc[1]);
-        kstep(no{}, ks + 1, 1, st[1], st[0], sc[1], sc[0]);
-    } else {
-        kstep(no{}, ks, 0, st[0], st[1], sc[0], sc[1]);
-    }
-
-    static_assert(2 * (BM + BN) * kMxPitch >= WAVES_M * WAVES_N * 32 * (WN * 64 + 16), "epilogue staging fits the operand buffers");
-    __syncthreads();  // every wavefront is done reading the operand buffers
-    mx_store_rows<WM, WN, OUT_BF16>(acc, mx_lds, wave, lane, *p.alpha, reinterpret_cast<uint16_t *>(p.D), p.ldd, a_row0, b_row0);
-}
-
-template <int WAVES_M, int WAVES_N, int WM, int WN>
-static int launch_gemm_mxfp4(MxGemmParams &p, int out_type, hipStream_t s) {
-    constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
-    constexpr size_t lds_bytes = 2 * (size_t)(BM + BN) * kMxPitch;
-    p.tiles_m = (int)(p.M / BM);
-    p.tiles_n = (int)(p.N / BN);
-    auto kernel = out_type == FOS_T_BF16 ? gemm_mxfp4_kernel<WAVES_M, WAVES_N, WM, WN, true>
-                                         : gemm_mxfp4_kernel<WAVES_M, WAVES_N, WM, WN, false>;
-    if (lds_bytes > 64 * 1024 &&
-        hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
-        return FOS_E_LAUNCH;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(64 * WAVES_M * WAVES_N), lds_bytes, s, p);
-    return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;
-}
-
 // ---------------------------------------------------------------------------------------
-// The same 256 x 256 x 128 tile with the operands loaded from global memory straight into
-// LDS (buffer_load ... lds: lane i of a wavefront fills the i-th 16-byte unit of a 1 KiB
-// run), so no registers stage them and four LDS stages keep three K steps in flight -- the
-// register-staged kernel above has one step of latency cover, and a step then lasts as long
-// as a load takes whatever the matrix pipe could do.
+// Tiles of 256 x 256, 128 x 256 or 128 x 128 outputs and K steps of 128 codes (64 bytes a row, one scale chunk).  The
+// operands go from global memory straight into LDS (buffer_load ... lds: lane i of a wavefront fills the i-th 16-byte unit
+// of a 1 KiB run), so no registers stage them and four LDS stages keep three K steps in flight.  (A form that
+// staged through registers had one step of latency cover, and a step lasted as long as a load takes: 2048 x 4096 x 14336
+// 82.7 us on its 128 x 128 tile against 69.2 here on 128 x 256.)
 //
-// A stage holds 256 rows x 64 bytes of each operand without padding and the four 512-byte
+// A stage holds the rows of both operands, 64 bytes each without padding, and the 512-byte
 // scale tiles of the step (fetched the same way, 4 bytes per lane); the 16-byte unit c of
 // row rho sits at unit c ^ ((rho >> 2) & 3).  A 128-bit LDS read serves 16 lanes per cycle
 // from 64 banks, i.e. the 16 rows a quarter-wave reads must differ in address bits 7:4:
@@ -817,13 +605,27 @@ static int launch_gemm_mxfp4(MxGemmParams &p, int out_type, hipStream_t s) {
 // long.)  The load of lane i therefore fetches unit (i & 3) ^ ((i >> 4) & 3) of row i >> 2 of
 // its 16-row run.
 constexpr int kDmaStages = 4;
-constexpr int kDmaOperandBytes = 256 * 64;
-constexpr int kDmaStageBytes = 2 * kDmaOperandBytes + 2048;  // + the step's scales: A tiles 0, 1, B tiles 0, 1
+
+// N consecutive 32-bit words (N = 1, 2, 4) with one LDS read.
+template <int N>
+FOS_DEVICE void lds_words(uint32_t (&dst)[N], const uint8_t *src) {
+    static_assert(N == 1 || N == 2 || N == 4, "one read instruction");
+    if constexpr (N == 1) {
+        dst[0] = *reinterpret_cast<const uint32_t *>(src);
+    } else if constexpr (N == 2) {
+        const uint2 v = *reinterpret_cast<const uint2 *>(src);
+        dst[0] = v.x, dst[1] = v.y;
+    } else {
+        const uint4 v = *reinterpret_cast<const uint4 *>(src);
+        dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
+    }
+}
+constexpr int dma_stage_bytes(int BM, int BN) { return (BM + BN) * 64 + 2048; }  // + the step's scales: 512 bytes per 128 rows of A, then of B
 typedef __attribute__((address_space(3))) void *MxLdsPtr;
 typedef int mx_v4i __attribute__((ext_vector_type(4)));
 
 // Buffer descriptor as four plain words (for inline assembly): base, stride 0, size in
-// bytes, raw 32-bit offsets with range checking -- the words mx_rsrc() makes.
+// bytes, raw 32-bit offsets with range checking.
 FOS_DEVICE mx_v4i mx_raw_rsrc(const void *base, uint32_t bytes) {
     const uint64_t a = (uint64_t)(uintptr_t)base;
     mx_v4i v = {(int)(uint32_t)a, (int)(uint32_t)((a >> 32) & 0xffffu), (int)bytes, 0x00020000};
@@ -833,15 +635,18 @@ FOS_DEVICE mx_v4i mx_raw_rsrc(const void *base, uint32_t bytes) {
 // s_waitcnt vmcnt(n) alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14, the other counters at their maxima)
 #define MX_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
 
-template <bool OUT_BF16>
+// BM, BN = 128 or 256: eight wavefronts, two rows of four, each BM / 2 x BN / 4.
+template <int BM, int BN, bool OUT_BF16>
 __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams p) {
-    constexpr int WAVES_N = 4, WM = 4, WN = 2, BM = 256, BN = 256;
+    constexpr int WAVES_N = 4, WM = BM / 64, WN = BN / 128;
+    constexpr int PA = BM / 128, PB = BN / 128;  // load instructions per wavefront and step: 16 rows each
+    constexpr int kABytes = BM * 64, kOperandBytes = (BM + BN) * 64, kStageBytes = dma_stage_bytes(BM, BN);
     extern __shared__ __attribute__((aligned(16))) uint8_t mx_lds[];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, h = lane >> 5;
     int tile_m, tile_n;
-    mx_tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
     const int64_t kbytes = p.K >> 1;
     const int64_t ksteps = p.K / kMxBK;
@@ -851,42 +656,53 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
     // undo the pipelining.  Every global load of the loop is of this kind (the scales too), so
     // the compiler places no vector-memory waits of its own there and the one wait per step
     // is placed by hand in kstep().
-    const mx_v4i ra = mx_raw_rsrc(p.A + m0 * kbytes, (uint32_t)(BM * kbytes));
-    const mx_v4i rb = mx_raw_rsrc(p.B + n0 * kbytes, (uint32_t)(BN * kbytes));
-    // wavefront w loads rows 32 w ... 32 w + 31 of both operands, 16 rows per instruction
-    const int ld_row = lane >> 2;
-    const uint32_t ld_off = (uint32_t)((wave * 32 + ld_row) * kbytes + (((lane & 3) ^ ((ld_row >> 2) & 3)) * 16));
+    // (M and N are multiples of 128: a 256-wide tile may hang over the last 128 rows or columns.  The descriptors end
+    // there; whatever LDS holds in the place of the rows beyond goes into outputs beyond the edge only, which are not stored)
+    const int rows_a = (int)(p.M - m0 < BM ? p.M - m0 : BM), rows_b = (int)(p.N - n0 < BN ? p.N - n0 : BN);
+    const mx_v4i ra = mx_raw_rsrc(p.A + m0 * kbytes, (uint32_t)(rows_a * kbytes));
+    const mx_v4i rb = mx_raw_rsrc(p.B + n0 * kbytes, (uint32_t)(rows_b * kbytes));
+    // wavefront w loads rows BM / 8 w ... of A and BN / 8 w ... of B, 16 rows per instruction
+    const int ld_row = lane >> 2, ld_unit = ((lane & 3) ^ ((ld_row >> 2) & 3)) * 16;
+    const uint32_t lda_off = (uint32_t)((wave * (BM / 8) + ld_row) * kbytes + ld_unit);
+    const uint32_t ldb_off = (uint32_t)((wave * (BN / 8) + ld_row) * kbytes + ld_unit);
     const int ld_half = (int)(16 * kbytes);
-    // ... and 256 of the step's 2 KiB of scales (a 512-byte tile per 128 rows and K step):
-    // waves 0-3 those of A (row tile w >> 1, half w & 1), waves 4-7 those of B
-    const uint8_t *sf_src = (wave < 4 ? p.sfA + (m0 >> 7) * ksteps * 512 : p.sfB + (n0 >> 7) * ksteps * 512) + ((wave >> 1) & 1) * ksteps * 512;
+    // ... and 256 bytes of the step's scales (a 512-byte tile per 128 rows and K step): half w & 1 of tile w >> 1,
+    // A's tiles first.  With fewer tiles than four the last wavefronts load the last one once more, into bytes that
+    // nobody reads: every wavefront has the same number of loads in flight.
+    const int sf_tile = (wave >> 1) < PA + PB ? wave >> 1 : PA + PB - 1;
+    const int sf_rows = 128 * (sf_tile < PA ? sf_tile : sf_tile - PA);  // first row of the scale tile, inside the operand's tile
+    const bool sf_inside = sf_rows < (sf_tile < PA ? rows_a : rows_b);
+    const uint8_t *sf_src = sf_tile < PA ? p.sfA + ((m0 + (sf_inside ? sf_rows : 0)) >> 7) * ksteps * 512
+                                         : p.sfB + ((n0 + (sf_inside ? sf_rows : 0)) >> 7) * ksteps * 512;
     const mx_v4i rs = mx_raw_rsrc(sf_src, (uint32_t)(ksteps * 512));
     const uint32_t sf_off = (uint32_t)((wave & 1) * 256 + lane * 4);
     const uint32_t lds_base = (uint32_t)(uintptr_t)(MxLdsPtr)mx_lds;
     auto issue = [&](int64_t ks, int stage) {
         const int kq = (int)(ks * (kMxBK / 2)), ksf = (int)(ks * 512);
-        const uint32_t base = lds_base + (uint32_t)(stage * kDmaStageBytes);
-        const uint32_t run = base + (uint32_t)(wave * 2048), sf_run = base + (uint32_t)(2 * kDmaOperandBytes + wave * 256);
+        const uint32_t base = lds_base + (uint32_t)(stage * kStageBytes);
+        const uint32_t run_a = base + (uint32_t)(wave * (BM / 8) * 64), run_b = base + (uint32_t)(kABytes + wave * (BN / 8) * 64);
+        const uint32_t sf_run = base + (uint32_t)(kOperandBytes + wave * 256);
         // m0 = LDS address of the run a wavefront fills (lane i: unit i); one wait state
         // between a write of m0 and its use.  (m0 is reserved: the compiler never keeps a
         // value in it across other code, it writes it right before each use of its own.)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        for (int t = 0; t < PA; ++t)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                          :
-                         : "s"(run + t * 1024), "v"(ld_off), "s"(ra), "s"(kq + t * ld_half)
+                         : "s"(run_a + t * 1024), "v"(lda_off), "s"(ra), "s"(kq + t * ld_half)
                          : "memory");
+#pragma unroll
+        for (int t = 0; t < PB; ++t)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                          :
-                         : "s"(run + kDmaOperandBytes + t * 1024), "v"(ld_off), "s"(rb), "s"(kq + t * ld_half)
+                         : "s"(run_b + t * 1024), "v"(ldb_off), "s"(rb), "s"(kq + t * ld_half)
                          : "memory");
-        }
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
                      :
                      : "s"(sf_run), "v"(sf_off), "s"(rs), "s"(ksf)
                      : "memory");
     };
-    constexpr int kLoadsPerStep = 5;
+    constexpr int kLoadsPerStep = PA + PB + 1;
 
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
     mx_v16f acc[WM][WN];
@@ -897,19 +713,20 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-    const uint32_t fa_off = (uint32_t)((wm * WM * 32 + r) * 64), fb_off = (uint32_t)(kDmaOperandBytes + (wn * WN * 32 + r) * 64);
+    const uint32_t fa_off = (uint32_t)((wm * WM * 32 + r) * 64), fb_off = (uint32_t)(kABytes + (wn * WN * 32 + r) * 64);
     const int swz = (r >> 2) & 3;
     auto read_frags = [&](int stage, int kk, uint4 *fa, uint4 *fb) {
-        const uint8_t *base = mx_lds + stage * kDmaStageBytes + (((kk * 2 + h) ^ swz) * 16);
+        const uint8_t *base = mx_lds + stage * kStageBytes + (((kk * 2 + h) ^ swz) * 16);
 #pragma unroll
         for (int i = 0; i < WM; ++i) fa[i] = *reinterpret_cast<const uint4 *>(base + fa_off + i * 32 * 64);
 #pragma unroll
         for (int j = 0; j < WN; ++j) fb[j] = *reinterpret_cast<const uint4 *>(base + fb_off + j * 32 * 64);
     };
     // scale words of this wavefront's row tiles: the 16-byte unit of row r holds those of rows
-    // r, r + 32, r + 64, r + 96 of a 128-row tile (A: all four; B: two of them)
-    const uint32_t sa_off = (uint32_t)(2 * kDmaOperandBytes + wm * 512 + r * 16);
-    const uint32_t sb_off = (uint32_t)(2 * kDmaOperandBytes + 1024 + (wn >> 1) * 512 + r * 16 + (wn & 1) * 8);
+    // r, r + 32, r + 64, r + 96 of a 128-row tile, of which a wavefront uses WM (WN) in a row
+    auto unit_of = [&](int row) { return (row >> 7) * 512 + r * 16 + ((row & 127) >> 5) * 4; };
+    const uint32_t sa_off = (uint32_t)(kOperandBytes + unit_of(wm * WM * 32));
+    const uint32_t sb_off = (uint32_t)(kOperandBytes + PA * 512 + unit_of(wn * WN * 32));
 
     // steps 0 .. 2 in flight (past the end: the last step once more, into stages nobody reads)
 #pragma unroll
@@ -927,13 +744,16 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
         MX_WAIT_VMCNT(2 * kLoadsPerStep);
         __syncthreads();
         issue(ks + 3 < ksteps ? ks + 3 : ksteps - 1, (stage + 3) & (kDmaStages - 1));
-        const uint8_t *st = mx_lds + stage * kDmaStageBytes;
-        const uint4 wa = *reinterpret_cast<const uint4 *>(st + sa_off);
-        const uint2 wb = *reinterpret_cast<const uint2 *>(st + sb_off);
+        const uint8_t *st = mx_lds + stage * kStageBytes;
+        uint32_t sha[WM], shb[WN];
+        lds_words<WM>(sha, st + sa_off);
+        lds_words<WN>(shb, st + sb_off);
         // lanes of the upper half use the next byte: after the shift, byte 0 / byte 2 of every
         // lane's register are the scales of the K blocks it feeds in slice 0 / slice 1
-        const uint32_t sha[WM] = {wa.x >> (8 * h), wa.y >> (8 * h), wa.z >> (8 * h), wa.w >> (8 * h)};
-        const uint32_t shb[WN] = {wb.x >> (8 * h), wb.y >> (8 * h)};
+#pragma unroll
+        for (int i = 0; i < WM; ++i) sha[i] >>= 8 * h;
+#pragma unroll
+        for (int j = 0; j < WN; ++j) shb[j] >>= 8 * h;
         uint4 fa[2][WM], fb[2][WN];
         read_frags(stage, 0, fa[0], fb[0]);
         read_frags(stage, 1, fa[1], fb[1]);
@@ -951,31 +771,50 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
                             frag_of(fb[0][j]), frag_of(fa[0][i]), acc[i][j], 4, 4, 0, (int)shb[j], 0, (int)sha[i]);
                 }
         }
-        // issue order: the scale words and the first slice's fragments, then the second slice's six
-        // fragment reads one at a time between the first MFMAs -- with all twelve reads ahead
-        // of the first MFMA a step began with a longer wait (8192^3: 271 -> 263 us,
+        // issue order: the scale words and the first slice's fragments, then the second slice's
+        // fragment reads one at a time between the first MFMAs -- with all reads ahead
+        // of the first MFMA a step began with a longer wait (256 x 256 tile, 8192^3: 271 -> 263 us,
         // 2048 x 14336 x 4096: 70.8 -> 68.0 us in alternating series)
-        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+        constexpr int kReads = WM + WN, kMfmas = 2 * WM * WN;
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 + kReads, 0);
 #pragma unroll
-        for (int i = 0; i < 6; ++i) {
+        for (int i = 0; i < kReads; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 10, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, kMfmas - kReads, 0);
     }
     // loads still in flight write LDS: drain them before the stages are used again
     MX_WAIT_VMCNT(0);
     __syncthreads();  // ... those of every wavefront, and all fragment reads are done
 
     mx_store_rows<WM, WN, OUT_BF16>(acc, mx_lds, wave, lane, *p.alpha, reinterpret_cast<uint16_t *>(p.D), p.ldd,
-                                     m0 + wm * WM * 32, n0 + wn * WN * 32);
+                                     m0 + wm * WM * 32, n0 + wn * WN * 32, rows_a - wm * WM * 32, wn * WN * 32 < rows_b);
 }
 
+// Tile size: the cheapest by what its generations take (us at K = 4096; all scale with K).  136 and 102 KB of LDS:
+// 256 workgroups of the 256 x 256 and 128 x 256 tiles at a time; 70 KB: 512 of the 128 x 128 tile.  Measured with the
+// tile forced on 60 shapes, 128 ... 8192 rows; against "256 x 256 from 256 tiles on, else 128 x 128 through registers":
+// 2048 x 4096 x 14336 (128 / 256 / 512 tiles) 82.7 -> 69.2 us on 128 x 256, 2560 x 4096 x 4096 35.7 -> 30.9 and
+// 1024 x 14336 x 4096 45.2 -> 35.3 on 256 x 256, 128 x 4096 x 14336 46.8 -> 39.1 on 128 x 128.
+static int mx_pick_tile(int64_t M, int64_t N) {
+    const int forced = tuning().mx_tile;  // tuning / tests: 128, 129 (128 x 256) or 256
+    if (forced == 128 || forced == 129 || forced == 256) return forced;
+    const int64_t m128 = M / 128, n128 = N / 128, m256 = (m128 + 1) / 2, n256 = (n128 + 1) / 2;
+    static const float big[8] = {25, 25, 27, 30, 31, 33, 35.5f, 39}, wide[8] = {16.4f, 16.8f, 17.5f, 18.3f, 19.3f, 20.4f, 22, 24.5f},
+                       small[8] = {13, 13.7f, 14.7f, 15.7f, 22.6f, 23, 25.2f, 27};
+    const float cost_big = tiles_cost(m256 * n256, 256, 37, big), cost_wide = tiles_cost(m128 * n256, 256, 22.3f, wide),
+                cost_small = tiles_cost(m128 * n128, 512, 25, small);
+    if (cost_big <= cost_wide && cost_big <= cost_small) return 256;
+    return cost_wide < cost_small ? 129 : 128;
+}
+
+template <int BM, int BN>
 static int launch_gemm_mxfp4_dma(MxGemmParams &p, int out_type, hipStream_t s) {
-    constexpr size_t lds_bytes = (size_t)kDmaStages * kDmaStageBytes;
-    p.tiles_m = (int)(p.M / 256);
-    p.tiles_n = (int)(p.N / 256);
-    auto kernel = out_type == FOS_T_BF16 ? gemm_mxfp4_dma_kernel<true> : gemm_mxfp4_dma_kernel<false>;
+    constexpr size_t lds_bytes = (size_t)kDmaStages * dma_stage_bytes(BM, BN);
+    p.tiles_m = (int)((p.M + BM - 1) / BM);
+    p.tiles_n = (int)((p.N + BN - 1) / BN);
+    auto kernel = out_type == FOS_T_BF16 ? gemm_mxfp4_dma_kernel<BM, BN, true> : gemm_mxfp4_dma_kernel<BM, BN, false>;
     if (hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
         return FOS_E_LAUNCH;
     hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(512), lds_bytes, s, p);
@@ -1000,11 +839,9 @@ extern "C" int fos_gemm_mxfp4(const uint8_t *A, const uint8_t *B, const uint8_t 
     p.A = A; p.B = B; p.sfA = sfA; p.sfB = sfB; p.alpha = alpha; p.D = D;
     p.M = M; p.N = N; p.K = K; p.ldd = ldd;
     hipStream_t s = (hipStream_t)stream;
-    bool big = (M % 256 == 0) && (N % 256 == 0) && (M / 256) * (N / 256) >= 256;
-    int forced = 0;
-    forced = fos::tuning().mx_tile;  // tuning / tests: 128 small tile, 256 register-staged big tile
-    big = big && forced != 128;
-    if (big && forced != 256) return launch_gemm_mxfp4_dma(p, out_type, s);
-    if (big) return launch_gemm_mxfp4<2, 4, 4, 2>(p, out_type, s);
-    return launch_gemm_mxfp4<2, 2, 2, 2>(p, out_type, s);
+    switch (mx_pick_tile(M, N)) {
+        case 256: return launch_gemm_mxfp4_dma<256, 256>(p, out_type, s);
+        case 129: return launch_gemm_mxfp4_dma<128, 256>(p, out_type, s);
+        default: return launch_gemm_mxfp4_dma<128, 128>(p, out_type, s);
+    }
 }

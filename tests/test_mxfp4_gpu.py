@@ -197,3 +197,21 @@ def test_mxfp4_gemm_kernels_agree_bitwise(monkeypatch, k):
         torch.cuda.synchronize()
     assert not torch.isnan(outs[0].float()).any()
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize(("m", "n", "k"), [(128, 128, 128), (384, 384, 256), (256, 640, 1152), (640, 256, 640)])
+def test_mxfp4_tiles_over_the_edge_of_the_output(monkeypatch, m, n, k):
+    """256-wide tiles that hang over the last 128 rows or columns, and K ranges shorter than the stages in flight: the
+    same bits as 128 x 128 tiles, and the fp64 product of the dequantized operands to half a unit of bf16 (2^-8; the
+    sums of products of powers of two times 4-bit values are exact in fp32 at these K)."""
+    cfg = fos.QuantizationConfig(dtype="mxfp4", scale_rule="static_6")
+    g = torch.Generator("cpu").manual_seed(m + n)
+    qa, qb = (fos.quantize(torch.randn(rows, k, generator=g).bfloat16().cuda(), cfg) for rows in (m, n))
+    a, b = (fos.dequantize(q, dtype=torch.float32).double() for q in (qa, qb))
+    exact, size = a @ b.T, a.abs() @ b.abs().T
+    outs = []
+    for tile in ("128", "129", "256"):
+        monkeypatch.setenv("FOS_MX_TILE", tile)
+        outs.append(fos.quantized_matmul(qa, qb))
+        assert bool(((outs[-1].double() - exact).abs() <= 2.0 ** -8 * exact.abs() + k * 2.0 ** -24 * size).all())
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
