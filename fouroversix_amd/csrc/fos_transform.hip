@@ -233,8 +233,8 @@ __global__ __launch_bounds__(kThreads) void transpose_kernel(const TransformPara
 // fp32 input (the reference converts with `.float()` and multiplies by the fp32 matrix: a library matmul whose
 // summation order is not part of any interface, so the target is the product itself, to fp32 rounding).  One
 // thread per output group of 16: the butterfly in fp32 (four levels of additions: within 4 units in the last
-// place of the largest partial sum), fp32 out.  With transposition a wavefront's lanes take consecutive output
-// rows, i.e. consecutive columns of x, so that each of its 16 loads reads a contiguous run of one row of x.
+// place of the largest partial sum), fp32 out.  Transposition (with or without RHT) goes through LDS,
+// transpose_f32_kernel below.
 struct TransformParamsF32 {
     const float *x;
     int64_t rows, cols, ld;
@@ -242,40 +242,40 @@ struct TransformParamsF32 {
     int64_t ldy;
     uint32_t *partials;
     int64_t out_rows, groups;  // output rows, groups of 16 per output row
+    int64_t n_tiles;           // transposed: 64 x 64 tiles of x
+    int tiles_x;
+    int vec;                   // x is 16-byte aligned with ld % 4 == 0
 };
 
-template <bool TRANSPOSE, bool RHT>
-__global__ __launch_bounds__(kThreads) void transform_f32_kernel(const TransformParamsF32 p) {
+// One group of 16 in registers: signs, butterfly, scale.
+FOS_DEVICE void rht16_f32(float *v) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = ((kRhtNegMask >> i) & 1u) ? -v[i] : v[i];
+#pragma unroll
+    for (int len = 1; len < 16; len <<= 1) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            if ((i & len) == 0) {
+                const float a = v[i], b = v[i + len];
+                v[i] = a + b;
+                v[i + len] = a - b;
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = v[i] * 0.25f + 0.0f;
+}
+
+__global__ __launch_bounds__(kThreads) void rht_rows_f32_kernel(const TransformParamsF32 p) {
     __shared__ uint32_t smem[4];
     uint32_t m = 0;
     const int64_t n_units = p.out_rows * p.groups;
     for (int64_t u = (int64_t)blockIdx.x * kThreads + threadIdx.x; u < n_units; u += (int64_t)gridDim.x * kThreads) {
-        // transposed: consecutive units walk down the output rows (a column of groups at a time)
-        const int64_t r = TRANSPOSE ? u % p.out_rows : u / p.groups, g = TRANSPOSE ? u / p.out_rows : u % p.groups;
+        const int64_t r = u / p.groups, g = u % p.groups;
         float v[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int64_t c = g * 16 + i;  // column of y = (transposed) row of x
-            float e = 0.0f;
-            if (TRANSPOSE) { if (c < p.rows) e = p.x[c * p.ld + r]; }
-            else if (c < p.cols) e = p.x[r * p.ld + c];
-            v[i] = RHT && ((kRhtNegMask >> i) & 1u) ? -e : e;
-        }
-        if (RHT) {
-#pragma unroll
-            for (int len = 1; len < 16; len <<= 1) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    if ((i & len) == 0) {
-                        const float a = v[i], b = v[i + len];
-                        v[i] = a + b;
-                        v[i + len] = a - b;
-                    }
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = v[i] * 0.25f + 0.0f;
-        }
+        for (int i = 0; i < 16; ++i) v[i] = g * 16 + i < p.cols ? p.x[r * p.ld + g * 16 + i] : 0.0f;
+        rht16_f32(v);
         float4 *dst = reinterpret_cast<float4 *>(p.y + r * p.ldy + g * 16);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -286,6 +286,75 @@ __global__ __launch_bounds__(kThreads) void transform_f32_kernel(const Transform
                 m = mag > m ? mag : m;
             }
         }
+    }
+    m = block_max_u32(m, smem);
+    if (threadIdx.x == 0) {
+        p.partials[2 * blockIdx.x] = m;
+        p.partials[2 * blockIdx.x + 1] = 0u;
+    }
+}
+
+// y = x^T (and RHT) for fp32 through an LDS tile of 64 x 64: rows of x come in, and rows of y leave, as runs of 256 bytes,
+// 16 bytes a lane; in between a thread takes one column of 16 rows (consecutive lanes, consecutive words).  Bound by
+// memory: 4096 x 4096 30.8 us.  (One group of 16 per thread straight from and to global memory, 64 output rows per store
+// instruction and two 64-bit divisions a group: 57.8 us.)
+template <bool RHT>
+__global__ __launch_bounds__(kThreads) void transpose_f32_kernel(const TransformParamsF32 p) {
+    constexpr int kT = 64, kPitchIn = kT + 1, kPitchOut = kT + 4;
+    __shared__ uint32_t smem[4];
+    __shared__ float in[kT * kPitchIn];
+    __shared__ __attribute__((aligned(16))) float out[kT * kPitchOut];
+    const int t = threadIdx.x, q4 = (t & 15) * 4, r16 = t >> 4, c = t & 63, g = t >> 6;
+    uint32_t m = 0;
+    auto fetch = [&](int64_t u, float4 (&w)[4]) {
+        const int64_t ty = u / p.tiles_x, tx = u - ty * p.tiles_x;
+        const int64_t col = tx * kT + q4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t row = ty * kT + r16 + 16 * i;
+            const float *src = p.x + row * p.ld + col;
+            if (row < p.rows && p.vec && col + 4 <= p.cols) {
+                w[i] = *reinterpret_cast<const float4 *>(src);
+            } else {
+                w[i].x = row < p.rows && col < p.cols ? src[0] : 0.0f;
+                w[i].y = row < p.rows && col + 1 < p.cols ? src[1] : 0.0f;
+                w[i].z = row < p.rows && col + 2 < p.cols ? src[2] : 0.0f;
+                w[i].w = row < p.rows && col + 3 < p.cols ? src[3] : 0.0f;
+            }
+        }
+    };
+    float4 next[4];
+    if ((int64_t)blockIdx.x < p.n_tiles) fetch(blockIdx.x, next);
+    for (int64_t u = blockIdx.x; u < p.n_tiles; u += gridDim.x) {
+        const int64_t ty = u / p.tiles_x, tx = u - ty * p.tiles_x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float *d = in + (r16 + 16 * i) * kPitchIn + q4;
+            d[0] = next[i].x, d[1] = next[i].y, d[2] = next[i].z, d[3] = next[i].w;
+        }
+        __syncthreads();
+        // the next tile's loads are in flight while this one is turned round and written
+        if (u + gridDim.x < p.n_tiles) fetch(u + gridDim.x, next);
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = in[(g * 16 + i) * kPitchIn + c];
+        if (RHT) rht16_f32(v);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const uint32_t mag = f2u(v[i]) & 0x7fffffffu;  // (columns and rows beyond x are zeros)
+            m = mag > m ? mag : m;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float4 *>(out + c * kPitchOut + g * 16 + 4 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t row = tx * kT + r16 + 16 * i, col = ty * kT + q4;  // of y
+            if (row < p.out_rows && col < p.groups * 16)
+                *reinterpret_cast<float4 *>(p.y + row * p.ldy + col) = *reinterpret_cast<const float4 *>(out + (r16 + 16 * i) * kPitchOut + q4);
+        }
+        // (the next round writes `in`, which every thread has read before the barrier above, and `out` after its own)
     }
     m = block_max_u32(m, smem);
     if (threadIdx.x == 0) {
@@ -336,11 +405,14 @@ int fos::transform_impl(const void *x, int x_type, int64_t rows, int64_t cols, i
         q.out_rows = transpose ? cols : rows;
         q.groups = (out_cols + 15) / 16;
         hipStream_t s32 = (hipStream_t)stream;
-        int64_t grid32 = (q.out_rows * q.groups + kThreads - 1) / kThreads;
+        q.tiles_x = (int)((cols + 63) / 64);
+        q.n_tiles = (rows + 63) / 64 * q.tiles_x;
+        q.vec = ((uintptr_t)x & 15) == 0 && ld % 4 == 0;
+        int64_t grid32 = transpose ? q.n_tiles : (q.out_rows * q.groups + kThreads - 1) / kThreads;
         if (grid32 > 1024) grid32 = 1024;  // pairs the workspace holds
-        if (transpose && rht) hipLaunchKernelGGL((transform_f32_kernel<true, true>), dim3((unsigned)grid32), dim3(kThreads), 0, s32, q);
-        else if (transpose) hipLaunchKernelGGL((transform_f32_kernel<true, false>), dim3((unsigned)grid32), dim3(kThreads), 0, s32, q);
-        else hipLaunchKernelGGL((transform_f32_kernel<false, true>), dim3((unsigned)grid32), dim3(kThreads), 0, s32, q);
+        if (transpose && rht) hipLaunchKernelGGL(transpose_f32_kernel<true>, dim3((unsigned)grid32), dim3(kThreads), 0, s32, q);
+        else if (transpose) hipLaunchKernelGGL(transpose_f32_kernel<false>, dim3((unsigned)grid32), dim3(kThreads), 0, s32, q);
+        else hipLaunchKernelGGL(rht_rows_f32_kernel, dim3((unsigned)grid32), dim3(kThreads), 0, s32, q);
         if (n_partials) *n_partials = (int)grid32;
         if (amax) hipLaunchKernelGGL(transform_amax_kernel, dim3(1), dim3(kThreads), 0, s32, q.partials, (int)grid32, amax);
         return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;

@@ -433,6 +433,33 @@ def test_if4_blocks_whose_candidates_nearly_tie(oracle, shape, scale):
     assert_same_quantization(q, oracle.quantize(x, dtype="if4", scale_rule="mse"), f"{shape} scale {scale}")
 
 
+@pytest.mark.parametrize("shape", [(1, 1), (16, 64), (64, 64), (65, 130), (200, 300), (1024, 4100)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_fp32_transpose_at_the_edges_of_its_tiles(shape, offset):
+    """x^T exactly, groups completed with zeros, rows of x at any alignment; with the random Hadamard transform the
+    butterfly's four rounded additions on the fp64 result (2^-21 of the group's sum of magnitudes, a quarter of it)."""
+    from fouroversix_amd.quantize import ops
+
+    rows, cols = shape
+    flat = torch.randn(rows * cols + offset, generator=torch.Generator("cpu").manual_seed(rows)).cuda()
+    x = flat[offset:].view(rows, cols)
+    y, amax = ops.transform(x, True, False)
+    assert torch.equal(y, x.T) and float(amax) == float(x.abs().max())
+    z, zmax = ops.transform(x, True, True)
+    full = torch.zeros(cols, -(-rows // 16) * 16, dtype=torch.float64, device="cuda")
+    full[:, :rows] = x.T.double()
+    h = torch.ones(1, 1, dtype=torch.float64)
+    for _ in range(4):
+        h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)
+    negated = (3, 5, 6, 7, 8, 9, 10, 12, 14, 15)
+    sign = torch.tensor([-1.0 if i in negated else 1.0 for i in range(16)], dtype=torch.float64)
+    matrix = (sign[:, None] * h / 4).cuda()
+    blocks = full.view(cols, -1, 16)
+    exact = (blocks.reshape(-1, 16) @ matrix).view(cols, -1)
+    bound = (2.0 ** -21 * blocks.abs().sum(-1, keepdim=True) / 4).expand_as(blocks).reshape(cols, -1)
+    assert bool(((z.double() - exact).abs() <= bound).all()) and float(zmax) == float(z.abs().max())
+
+
 @pytest.mark.parametrize("cfg", [dict(), dict(block_scale_2d=True), dict(dtype="if4"), dict(dtype="if4", block_scale_2d=True),
                                  dict(round_style="stochastic", kwargs={"seed": 3}),
                                  dict(round_style="stochastic", block_scale_2d=True, kwargs={"seed": 3}),
