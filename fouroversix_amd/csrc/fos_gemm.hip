@@ -26,10 +26,9 @@
 // 8192^3 811 -> 790 us, 4096^3 107.5 -> 105.0 us in alternating series on one box, and
 // 3072 x 4096 x 4096 131 -> 105 us, 1152 x 4096 x 4096 71 -> 56 us on the 128 x 128 tile (a
 // 256 x 128 tile of 8 wavefronts of 128 x 32 in two rows lost to it wherever 256 x 256 tiles
-// are too few to fill the chip), with bit-identical outputs.  The 128 x 128 tile serves
-// shapes that are not multiples of 256 or too small to fill the chip otherwise, and a 128 x 256
-// tile (the template with BM = 128 and eight wavefronts: every thread stages a quarter row of A) those
-// that it covers with one workgroup per compute unit.
+// are too few to fill the chip), with bit-identical outputs.  The 128 x 128 tile and a 128 x 256
+// tile (the template with BM = 128 and eight wavefronts: every thread stages a quarter row of A) serve the shapes on
+// which their generations are cheaper (pick_tile); 256-wide tiles may hang over the edge of the output.
 // Workgroups are numbered so that the tiles resident on one XCD (blockIdx % 8) form a
 // compact block of the output, which keeps their A/B panels in that XCD's L2.
 #include <hip/hip_runtime.h>
@@ -1203,7 +1202,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool if4) {
             return g;
         }
         steps = K / BK;
-        tiles = (M / 128) * (N / 128);
+        tiles = ((M + 127) / 128) * (N / 128);  // (fewer than 128 rows: refused later)
     }
     // split so that about kTargetWorkgroups workgroups run, each with a useful share of K
     // (at M <= 32 a split must leave two steps per wavefront: 16 x 4096 x 4096 takes 6.4 us

@@ -101,3 +101,14 @@ def test_argument_checks_need_no_device(native):
     assert d(dtype=3) == -3
     assert d(out=9) == -3
     assert d(inter=0) == -3  # value x scale meets in fp16 or fp32 only
+
+
+@pytest.mark.parametrize("tile", ["1", "128", "129", "256"])
+def test_workspace_query_of_a_small_batch_on_forced_tiles(native, monkeypatch, tile):
+    """Fewer rows than a tile has, with the weight-streaming kernels switched off: the query answers (the product itself
+    is refused)."""
+    monkeypatch.setenv("FOS_GEMM_TILE", tile)
+    L = native.lib()
+    for m in (1, 16, 127, 128):
+        assert L.fos_gemm_workspace_bytes(m, 256, 512) >= 0
+        assert L.fos_linear_nvfp4_scratch_bytes(m, 512, 256) > 0
