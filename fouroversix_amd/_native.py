@@ -45,6 +45,7 @@ EXPORTS = (
     "fos_linear_nvfp4_scratch_bytes",
     "fos_gemm_if4",
     "fos_gemm_if4_workspace_bytes",
+    "fos_gemm_linear_rows",
     "fos_gemm_mxfp4",
     "fos_gemm_alpha",
     "fos_padded_cols_for",
@@ -119,6 +120,8 @@ def lib() -> ctypes.CDLL:
     L.fos_linear_nvfp4_scratch_bytes.restype = ctypes.c_size_t
     L.fos_gemm_if4.argtypes = [vp, vp, vp, vp, vp, vp, dbl, i64, i64, i64, vp, i32, i64, vp, vp, vp, ctypes.c_size_t, vp]
     L.fos_gemm_if4.restype = i32
+    L.fos_gemm_linear_rows.argtypes = [i32, vp, vp, vp, vp, vp, vp, dbl, i64, i64, i64, i64, vp, i32, i64, vp, vp, vp, ctypes.c_size_t, vp]
+    L.fos_gemm_linear_rows.restype = i32
     L.fos_gemm_if4_workspace_bytes.argtypes = [i64, i64, i64]
     L.fos_gemm_if4_workspace_bytes.restype = ctypes.c_size_t
     L.fos_gemm_alpha.argtypes = [vp, vp, dbl, vp, vp]

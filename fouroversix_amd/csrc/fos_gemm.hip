@@ -60,6 +60,7 @@ struct GemmParams {
     const void *bias;          // optional: N values of the output type, added to the rounded product and rounded again
     float *d_amax;             // optional: max|D| as stored is folded into d_amax[0] (unsigned atomic max on the bits)
     int64_t M, N, K, ldd;
+    int64_t rows;              // rows 0 ... rows - 1 of D count for d_amax: padding rows hold the bias, not zeros
     int tiles_m, tiles_n;
     // split-K: workgroup (tile, blockIdx.y) contracts K steps [y * ksteps_per_split, ...) and
     // writes its FP32 partial tile to partials[y][M][N]; splits == 1 writes D directly
@@ -500,6 +501,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
         if (!strip_inside || (uint32_t)(wm * WM * 32 + i * 32) >= rows_a) break;  // (uniform over the wavefront)
+        uint32_t um = 0u;
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
 #pragma unroll
@@ -512,9 +514,10 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
                 }
                 const int nl = j * 32 + 8 * g + 4 * (lane >> 5);  // column inside the wavefront's strip
                 *reinterpret_cast<uint2 *>(epi + (lane & 31) * kEpiPitch + nl * 2) =
-                    pack_outputs<OUT_BF16>(v, p.bias, n0 + wn * WN * 32 + nl, umax);
+                    pack_outputs<OUT_BF16>(v, p.bias, n0 + wn * WN * 32 + nl, um);
             }
         }
+        if (um > umax && m0 + wm * WM * 32 + i * 32 + (lane & 31) < p.rows) umax = um;
         // (LDS operations of one wavefront complete in order: its own writes are visible to its reads)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -853,6 +856,7 @@ __global__ __launch_bounds__(64 * skinny_waves(WN), (WN == 2 && MT == 2) ? 2 : 1
     uint32_t umax = 0u;
 #pragma unroll
     for (int c = 0; c < kGroups; ++c) {
+        uint32_t um = 0u;
         const int c4 = R == 2 ? (wave >> 1) : wave * (R / 4) + c;  // group of four columns: c4 = (i WN + t) 4 + g
         const int g = c4 & 3, t = (c4 >> 2) % WN, i = (c4 >> 2) / WN;
         const int m = m_base + 32 * i + r;
@@ -863,16 +867,17 @@ __global__ __launch_bounds__(64 * skinny_waves(WN), (WN == 2 && MT == 2) ? 2 : 1
                 *reinterpret_cast<float2 *>(P + (int64_t)m * p.N + n) = make_float2(mine[0], mine[1]);
             } else {
                 *reinterpret_cast<uint32_t *>(D + (int64_t)m * p.ldd + n) =
-                    pack_outputs2<OUT == kOutBF16>(alpha * mine[0], alpha * mine[1], p.bias, n, umax);
+                    pack_outputs2<OUT == kOutBF16>(alpha * mine[0], alpha * mine[1], p.bias, n, um);
             }
         } else {
             if (OUT == kOutPartial) {
                 *reinterpret_cast<float4 *>(P + (int64_t)m * p.N + n) = make_float4(mine[4 * c], mine[4 * c + 1], mine[4 * c + 2], mine[4 * c + 3]);
             } else {
                 const float v[4] = {alpha * mine[4 * c], alpha * mine[4 * c + 1], alpha * mine[4 * c + 2], alpha * mine[4 * c + 3]};
-                *reinterpret_cast<uint2 *>(D + (int64_t)m * p.ldd + n) = pack_outputs<OUT == kOutBF16>(v, p.bias, n, umax);
+                *reinterpret_cast<uint2 *>(D + (int64_t)m * p.ldd + n) = pack_outputs<OUT == kOutBF16>(v, p.bias, n, um);
             }
         }
+        if (um > umax && m < p.rows) umax = um;
     }
     if (OUT != kOutPartial && p.d_amax) {
         __syncthreads();  // every wavefront has summed its share of the slots
@@ -1047,7 +1052,7 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams
         uint32_t um = 0u;
         const uint2 o = pack_outputs<OUT == kOutBF16>(v, p.bias, n_out + 32 * b, um);
         if (row_ok) {
-            umax = um > umax ? um : umax;
+            if (um > umax && c < p.rows) umax = um;
             *reinterpret_cast<uint2 *>(D + (int64_t)c * p.ldd + n_out + 32 * b) = o;
         }
     }
@@ -1078,7 +1083,7 @@ __global__ __launch_bounds__(kReduceThreads) void gemm_reduce_kernel(const GemmP
     uint32_t um = 0u;
     const uint2 o = pack_outputs<OUT_BF16>(v, p.bias, n, um);
     if (mine) *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.D) + m * p.ldd + n) = o;
-    if (p.d_amax) fold_amax<OUT_BF16, kReduceThreads / 64>(p.d_amax, mine ? um : 0u, words);
+    if (p.d_amax) fold_amax<OUT_BF16, kReduceThreads / 64>(p.d_amax, mine && m < p.rows ? um : 0u, words);
 }
 
 static int launch_reduce(const GemmParams &p, int out_type, hipStream_t s) {
@@ -1253,7 +1258,7 @@ extern "C" size_t fos_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
                            const float *alpha, const float *amax_a, const float *amax_b, double denominator,
                            int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
-                           void *workspace, size_t workspace_bytes, fos_stream_t stream, bool if4 = false) {
+                           void *workspace, size_t workspace_bytes, fos_stream_t stream, bool if4 = false, int64_t rows = -1) {
     if (!A || !B || !sfA || !sfB || !D) return FOS_E_NULL_POINTER;
     if (((uintptr_t)d_amax & 3) || ((uintptr_t)bias & 7)) return FOS_E_BAD_ALIGNMENT;
     if (!alpha && (!amax_a || !amax_b)) return FOS_E_NULL_POINTER;
@@ -1270,6 +1275,7 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     p.amax_a = amax_a; p.amax_b = amax_b; p.inv_den = alpha ? 0.0f : (float)(1.0 / denominator);
     p.tiny_scale = if4;
     p.M = M; p.N = N; p.K = K; p.ldd = ldd;
+    p.rows = rows < 0 ? M : rows;
     hipStream_t s = (hipStream_t)stream;
     GemmPlan g = plan_gemm(M, N, K, if4);
     if (M < 128 && g.kind != kPlanSkinny) return FOS_E_BAD_SHAPE;
@@ -1363,4 +1369,16 @@ extern "C" int fos_gemm_if4(const uint8_t *A, const uint8_t *B, const uint8_t *s
     if (!(denominator > 0.0) || M % 128 != 0) return FOS_E_BAD_SHAPE;
     return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, workspace,
                            workspace_bytes, stream, true);
+}
+
+extern "C" int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
+                                    const float *amax_a, const float *amax_b, double denominator,
+                                    int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
+                                    float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream) {
+    if (!amax_a || !amax_b) return FOS_E_NULL_POINTER;
+    if (dtype != FOS_DTYPE_NVFP4 && dtype != FOS_DTYPE_IF4) return FOS_E_UNSUPPORTED;
+    const bool if4 = dtype == FOS_DTYPE_IF4;
+    if (!(denominator > 0.0) || rows < 0 || rows > M || (if4 && M % 128 != 0)) return FOS_E_BAD_SHAPE;
+    return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, workspace,
+                           workspace_bytes, stream, if4, rows);
 }

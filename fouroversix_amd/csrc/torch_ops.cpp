@@ -237,9 +237,11 @@ void check_gemm_operands(const Tensor &a, const Tensor &b, const Tensor &a_sf, c
 }
 
 // One GEMM launch.  alpha, or (amax_a, amax_b, denominator) for the output scale formed in the kernel;
-// with the latter, d_amax (device f32[1], zero or an earlier maximum) receives max|out|.
+// with the latter, d_amax (device f32[1], zero or an earlier maximum) receives max|out| over the first `rows` rows
+// (negative: all).
 Tensor gemm_launch(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tensor &b_sf, const Tensor *alpha, const Tensor *amax_a,
-                   const Tensor *amax_b, double denominator, at::ScalarType out_dtype, const Tensor *d_amax, const Tensor *bias = nullptr) {
+                   const Tensor *amax_b, double denominator, at::ScalarType out_dtype, const Tensor *d_amax, const Tensor *bias = nullptr,
+                   int64_t rows = -1) {
     const int64_t m = a.size(0), n = b.size(0), k = a.size(1) * 2;
     Tensor out = at::empty({m, n}, a.options().dtype(out_dtype));
     const size_t ws_bytes = fos_gemm_workspace_bytes(m, n, k);
@@ -262,9 +264,9 @@ Tensor gemm_launch(const Tensor &a, const Tensor &b, const Tensor &a_sf, const T
             TORCH_CHECK(bias->scalar_type() == out_dtype && bias->dim() == 1 && bias->size(0) == n && bias->is_contiguous(),
                         "gemm: bias must be a contiguous [N] tensor of the output type");
         }
-        rc = fos_gemm_nvfp4_linear(A, B, sA, sB, amax_a->data_ptr<float>(), amax_b->data_ptr<float>(), denominator, m, n, k,
-                                   out.data_ptr(), out_type, n, bias ? bias->data_ptr() : nullptr,
-                                   d_amax ? d_amax->data_ptr<float>() : nullptr, wsp, ws_bytes, stream);
+        rc = fos_gemm_linear_rows(FOS_DTYPE_NVFP4, A, B, sA, sB, amax_a->data_ptr<float>(), amax_b->data_ptr<float>(), denominator, m,
+                                  rows < 0 || rows > m ? m : rows, n, k, out.data_ptr(), out_type, n, bias ? bias->data_ptr() : nullptr,
+                                  d_amax ? d_amax->data_ptr<float>() : nullptr, wsp, ws_bytes, stream);
     } else {
         rc = fos_gemm_nvfp4_amax(A, B, sA, sB, amax_a->data_ptr<float>(), amax_b->data_ptr<float>(), denominator, m, n, k,
                                  out.data_ptr(), out_type, n, wsp, ws_bytes, stream);
@@ -290,9 +292,10 @@ Tensor gemm_nvfp4_fp16(const Tensor &a, const Tensor &b, const Tensor &a_sf, con
 // less than alpha + GEMM, same result.  `checked`: the operands are the members of two QuantizedTensors on
 // one GPU (the frontend has looked): only the shapes are compared.
 // `bias` ([N], output type): added to the rounded product and rounded again, as `out + bias` would.
+// `rows`: rows of `a` that are not padding, the ones that d_amax covers (negative: all).
 Tensor gemm_nvfp4_amax(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tensor &b_sf, const Tensor &amax_a, const Tensor &amax_b,
                        double denominator, at::ScalarType out_dtype, const c10::optional<Tensor> &d_amax, bool checked,
-                       const c10::optional<Tensor> &bias) {
+                       const c10::optional<Tensor> &bias, int64_t rows) {
     if (checked) {
         TORCH_CHECK(a.size(1) == b.size(1), "Inner dims mismatch: ", a.size(1) * 2, " vs ", b.size(1) * 2);
     } else {
@@ -301,7 +304,7 @@ Tensor gemm_nvfp4_amax(const Tensor &a, const Tensor &b, const Tensor &a_sf, con
         check_gemm_operands(a, b, a_sf, b_sf, scales, 2, names);
     }
     return gemm_launch(a, b, a_sf, b_sf, nullptr, &amax_a, &amax_b, denominator, out_dtype, d_amax.has_value() ? &*d_amax : nullptr,
-                       bias.has_value() ? &*bias : nullptr);
+                       bias.has_value() ? &*bias : nullptr, rows);
 }
 
 // A word for a recorded maximum: one of a block of 4096 per (device, stream), each handed out once, so that the block is
@@ -361,9 +364,11 @@ std::tuple<Tensor, c10::optional<Tensor>> linear_nvfp4(const Tensor &x, int64_t 
     return {out, d_amax};
 }
 
-// IF4 x IF4 (row-major E4M3 scales), output scale from the two maxima, optional bias and recorded maximum as above.
+// IF4 x IF4 (row-major E4M3 scales), output scale from the two maxima, optional bias and recorded maximum (of the first
+// `rows` rows) as above.
 Tensor gemm_if4(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tensor &b_sf, const Tensor &amax_a, const Tensor &amax_b,
-                double denominator, at::ScalarType out_dtype, const c10::optional<Tensor> &d_amax, const c10::optional<Tensor> &bias) {
+                double denominator, at::ScalarType out_dtype, const c10::optional<Tensor> &d_amax, const c10::optional<Tensor> &bias,
+                int64_t rows) {
     const Tensor *scales[2] = {&amax_a, &amax_b};
     const char *names[2] = {"amax_a", "amax_b"};
     check_gemm_operands(a, b, a_sf, b_sf, scales, 2, names);
@@ -381,11 +386,11 @@ Tensor gemm_if4(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tens
     const DeviceGuard guard(a.device());
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
-    check(fos_gemm_if4(a.data_ptr<uint8_t>(), b.data_ptr<uint8_t>(), static_cast<const uint8_t *>(a_sf.data_ptr()),
-                       static_cast<const uint8_t *>(b_sf.data_ptr()), amax_a.data_ptr<float>(), amax_b.data_ptr<float>(), denominator, m,
-                       n, k, out.data_ptr(), out_type, n, bias.has_value() ? bias->data_ptr() : nullptr,
-                       d_amax.has_value() ? d_amax->data_ptr<float>() : nullptr, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes,
-                       current_stream(a)),
+    check(fos_gemm_linear_rows(FOS_DTYPE_IF4, a.data_ptr<uint8_t>(), b.data_ptr<uint8_t>(), static_cast<const uint8_t *>(a_sf.data_ptr()),
+                               static_cast<const uint8_t *>(b_sf.data_ptr()), amax_a.data_ptr<float>(), amax_b.data_ptr<float>(),
+                               denominator, m, rows < 0 || rows > m ? m : rows, n, k, out.data_ptr(), out_type, n,
+                               bias.has_value() ? bias->data_ptr() : nullptr, d_amax.has_value() ? d_amax->data_ptr<float>() : nullptr,
+                               ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, current_stream(a)),
           "fouroversix::gemm_if4");
     return out;
 }
@@ -458,7 +463,7 @@ TORCH_LIBRARY(fouroversix, m) {
     m.def("gemm_mxfp4mxfp4_accum_fp32_out_bf16_tnt(Tensor A, Tensor B, Tensor A_sf, Tensor B_sf, Tensor alpha) -> Tensor");
     m.def(
         "gemm_nvfp4_amax(Tensor A, Tensor B, Tensor A_sf, Tensor B_sf, Tensor amax_a, Tensor amax_b, float denominator, "
-        "ScalarType out_dtype, Tensor(a!)? d_amax, bool checked=False, Tensor? bias=None) -> Tensor");
+        "ScalarType out_dtype, Tensor(a!)? d_amax, bool checked=False, Tensor? bias=None, int rows=-1) -> Tensor");
     m.def(
         "dequantize(Tensor values, Tensor scale_factors, Tensor amax, int dtype, int sf_layout, float divisor, "
         "int rows, int cols, ScalarType out_dtype, bool f32_intermediate=False) -> Tensor");

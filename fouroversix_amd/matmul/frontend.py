@@ -246,7 +246,7 @@ def nvfp4_linear(
     )
     m, n = x.shape[0], weight.original_shape[0]
     if out.shape[0] != m or out.shape[1] != n:
-        out = out[:m, :n]  # (the padding is zeros: same maximum)
+        out = out[:m, :n]  # (padding rows are not in the maximum; padding columns, which have no bias, are zeros)
     if d_amax is not None:
         attach_known_amax(out, d_amax)
     return out if bias is None or fused_bias else out + bias
@@ -294,13 +294,13 @@ def quantized_matmul(
         torch_dtype = torch.bfloat16 if out_dtype is DataType.bfloat16 else torch.float16
         fused_bias = _fusable_bias(bias, torch_dtype, rb[0].shape[0], ra[6])
         d_amax = _fresh_amax_word(ra[6]) if emit_amax and (bias is None or fused_bias) else None
+        m, n = input.original_shape[0], other.original_shape[0]
         out = ops.gemm_nvfp4_from_amax(
             ra[4], rb[0], ra[1], rb[1], ra[2], rb[2], ra[5] * rb[5], torch_dtype, d_amax, True,
-            bias.detach() if fused_bias else None,
+            bias.detach() if fused_bias else None, m,
         )
-        m, n = input.original_shape[0], other.original_shape[0]
         if out.shape[0] != m or out.shape[1] != n:
-            out = out[:m, :n]  # (the padding is zeros: same maximum)
+            out = out[:m, :n]  # (padding rows are not in the maximum; padding columns, which have no bias, are zeros)
         if d_amax is not None:
             attach_known_amax(out, d_amax)
         if bias is not None and not fused_bias:
@@ -317,7 +317,7 @@ def quantized_matmul(
             out = ops.gemm_if4(
                 input.values, other.values, input.scale_factors, other.scale_factors, input.amax, other.amax,
                 dequantize_divisor(input) * dequantize_divisor(other), out_dtype.torch_dtype, d_amax,
-                bias.detach() if fused_bias else None,
+                bias.detach() if fused_bias else None, input.original_shape[0],
             )
             out_shape = (input.original_shape[0], other.original_shape[0])
             out = out if tuple(out.shape) == out_shape else out[: out_shape[0], : out_shape[1]]

@@ -110,13 +110,14 @@ def gemm_nvfp4nvfp4_accum_fp32_out_fp16_tnt(a, b, a_sf, b_sf, alpha):
     return torch.ops.fouroversix.gemm_nvfp4nvfp4_accum_fp32_out_fp16_tnt.default(a, b, a_sf, b_sf, alpha)
 
 
-def gemm_nvfp4_from_amax(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax=None, checked=False, bias=None):
+def gemm_nvfp4_from_amax(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax=None, checked=False, bias=None, rows=-1):
     """The NVFP4 GEMM with the output scale ``(amax_a * amax_b) * f32(1 / denominator)`` formed
     in the kernel (``fos_gemm_nvfp4_amax``): one launch less than alpha + GEMM, same result.
-    ``d_amax`` (device f32[1] holding 0) additionally receives max|out|.  ``checked``: the operands are
+    ``d_amax`` (device f32[1] holding 0) additionally receives max|out|, over the first ``rows`` rows where the rest
+    are padding (negative: all rows).  ``checked``: the operands are
     the members of two QuantizedTensors on one GPU (the frontend has looked): only the shapes are compared.
     ``bias`` ([N], output type) is added to the rounded product and the sum rounded again, as ``out + bias``."""
-    return _C.gemm_nvfp4_amax(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, checked, bias)
+    return _C.gemm_nvfp4_amax(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, checked, bias, rows)
 
 
 def linear_nvfp4(x, selection_rule, x_amax, w, w_sf, w_amax, denominator, out_dtype, emit_amax=False, bias=None):
@@ -125,9 +126,9 @@ def linear_nvfp4(x, selection_rule, x_amax, w, w_sf, w_amax, denominator, out_dt
     return _C.linear_nvfp4(x, selection_rule, x_amax, w, w_sf, w_amax, denominator, out_dtype, emit_amax, bias)
 
 
-def gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax=None, bias=None):
-    """IF4 x IF4 product with the output scale of ``gemm_nvfp4_from_amax``; ``d_amax`` and ``bias`` as there."""
-    return _C.gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, bias)
+def gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax=None, bias=None, rows=-1):
+    """IF4 x IF4 product with the output scale of ``gemm_nvfp4_from_amax``; ``d_amax``, ``bias`` and ``rows`` as there."""
+    return _C.gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, bias, rows)
 
 
 def gemm_alpha_into(amax_a, amax_b, denominator, alpha):
@@ -211,5 +212,5 @@ def _(x, transpose, rht, dtype, selection_rule, round_style, is_2d, seed, offset
 
 
 @torch.library.register_fake("fouroversix::gemm_nvfp4_amax")
-def _(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, checked=False, bias=None):
+def _(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, checked=False, bias=None, rows=-1):
     return torch.empty(a.shape[0], b.shape[0], dtype=out_dtype, device=a.device)

@@ -285,7 +285,7 @@ int fos_gemm_nvfp4_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA
  * rule `rule`; maximum x_amax[0] if given, found otherwise), times the quantized weight W [N, padded cols], as
  * fos_quantize followed by fos_gemm_nvfp4_linear gives it.  D has fos_linear_nvfp4_rows(rows, cols) rows (the padded
  * ones, or `rows` where the product skips the padding of a small batch).  d_amax, when given, is set to max|D| (unlike
- * there it needs no initial value: the quantize kernel clears it).  `scratch`: fos_linear_nvfp4_scratch_bytes bytes,
+ * there it needs no initial value: the quantize kernel clears it), over the first `rows` rows.  `scratch`: fos_linear_nvfp4_scratch_bytes bytes,
  * 256-byte aligned, in use until the product is done.
  */
 size_t fos_linear_nvfp4_scratch_bytes(int64_t rows, int64_t cols, int64_t N);
@@ -306,6 +306,16 @@ int fos_gemm_if4(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const u
                  int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
                  float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream);
 size_t fos_gemm_if4_workspace_bytes(int64_t M, int64_t N, int64_t K);
+
+/*
+ * fos_gemm_nvfp4_linear (dtype FOS_DTYPE_NVFP4) or fos_gemm_if4 (FOS_DTYPE_IF4) for an A whose rows from `rows` on are
+ * padding: all M rows of D are written, and d_amax receives the maximum over the first `rows` alone (with a bias the
+ * padding rows of D are not zeros but hold the bias).
+ */
+int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
+                         const float *amax_a, const float *amax_b, double denominator,
+                         int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
+                         float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream);
 
 /*
  * alpha[0] = (amax_a[0] * amax_b[0]) * f32(1 / denominator), in fp32 on the device: the

@@ -256,7 +256,7 @@ def test_layer_in_one_call_equals_quantize_and_matmul(tokens, inf, outf, dtype):
                 expect = fos.quantized_matmul(x, model[0].quantized_weight(), emit_amax=True, bias=model[0].bias)
                 assert torch.equal(out, expect) and out.shape == (tokens, outf)
                 a, b = known_amax(out), known_amax(expect)
-                assert (a is None) == (b is None) and (a is None or float(a) == float(b))
+                assert (a is None) == (b is None) and (a is None or float(a) == float(b) == float(out.abs().max()))
                 known = x.clone()
                 attach_known_amax(known, x.abs().max().float().reshape(1))
                 assert torch.equal(model(known[None])[0], expect)
@@ -533,6 +533,37 @@ def test_recorded_maximum_over_whole_workgroups(monkeypatch, m, n, k, env):
         boosted[row] *= 8
         out = fos.quantized_matmul(fos.quantize(boosted.cuda()), qb, emit_amax=True)
         assert float(known_amax(out)) == float(out.abs().max())
+
+
+@pytest.mark.parametrize("env", [{}, {"FOS_GEMM_TILE": "128"}, {"FOS_GEMM_TILE": "129"}, {"FOS_GEMM_TILE": "256"},
+                                 {"FOS_GEMM_SPLITK": "2", "FOS_GEMM_TILE": "128"}, {"FOS_GEMM_SPLITK": "1"}], ids=str)
+@pytest.mark.parametrize("dtype", ["nvfp4", "if4"])
+@pytest.mark.parametrize("tokens", [1, 100, 129, 1000])
+def test_recorded_maximum_leaves_out_the_padding_rows(monkeypatch, tokens, dtype, env):
+    """Products of positive numbers and a bias of -64: every output is smaller than the bias in magnitude, which is what
+    the rows that complete a band of 128 hold.  Layer and product, K with and without the weight-streaming kernels."""
+    from fouroversix_amd.quantize import known_amax
+
+    if "FOS_GEMM_TILE" in env and tokens < 128:
+        env = {"FOS_GEMM_SPLITK": env.get("FOS_GEMM_SPLITK", "1")}  # (small batches: the kernel that the shape takes)
+    for name, value in env.items():
+        monkeypatch.setenv(name, value)
+    g = torch.Generator("cpu").manual_seed(tokens)
+    for inf in (320, 1024):
+        layer = nn.Linear(inf, 384, device="cuda", dtype=torch.bfloat16)
+        with torch.no_grad():
+            layer.weight.copy_(torch.rand(384, inf, generator=g) * 0.04)
+            layer.bias.fill_(-64.0)
+        model = nn.Sequential(layer)
+        fos.quantize_model(model, fos.ModelQuantizationConfig(dtype=dtype))
+        model[0].quantize_weight_()
+        x = torch.rand(tokens, inf, generator=g).bfloat16().cuda()
+        with torch.no_grad():
+            qx = fos.quantize(x, fos.QuantizationConfig(dtype=dtype))
+            for out in (model(x), fos.quantized_matmul(qx, model[0].quantized_weight(), emit_amax=True, bias=model[0].bias)):
+                assert 0 < float(out.abs().max()) < 64
+                assert float(known_amax(out)) == float(out.abs().max())
+                assert torch.equal(fos.quantize(out).values, fos.quantize(out.clone()).values)
 
 
 @pytest.mark.parametrize("tile", ["129", "256"])
