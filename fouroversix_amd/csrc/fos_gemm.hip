@@ -55,7 +55,7 @@ struct GemmParams {
     const float *alpha;        // output scale on the device, or null: (amax_a * amax_b) * inv_den
     const float *amax_a, *amax_b;
     float inv_den;
-    int tiny_scale;            // an output scale below the normal range is applied in two factors (load_alpha)
+    int two_factors;           // an output scale outside fp32's normal range is applied in two factors (load_alpha)
     void *D;
     const void *bias;          // optional: N values of the output type, added to the rounded product and rounded again
     float *d_amax;             // optional: max|D| as stored is folded into d_amax[0] (unsigned atomic max on the bits)
@@ -70,15 +70,23 @@ struct GemmParams {
 
 // Output scale: read from the device, or formed from the two tensor maxima with the
 // arithmetic of gemm_alpha_kernel (product, then times the fp32 reciprocal of the divisor).
-// `post`: with tiny_scale, what is left to multiply alpha * acc with (1 otherwise): maxima whose product, divided by
-// the denominator, would be a sub-normal number with a few bits are multiplied 2^64 times too large.
+// `post`: with two_factors, what is left to multiply alpha * acc with (1 otherwise).  Maxima whose product, divided by
+// the denominator, would be a sub-normal number with a few bits are multiplied 2^64 times too large; finite maxima
+// whose product overflows, 2^64 times too small (with an infinite scale a sum of zero would become NaN and a small
+// one infinite).  What still overflows then is a scale of 2^192 or more: any sum but zero, 2^-20 at least, is infinite
+// with the largest number in its place too.
 FOS_DEVICE float load_alpha(const GemmParams &p, float &post) {
+    constexpr float kMax = 0x1.fffffep127f;
     post = 1.0f;
     if (p.alpha) return *p.alpha;
     const float a = *p.amax_a, b = *p.amax_b;
-    if (p.tiny_scale && a * b < 0x1p-90f) {
+    if (p.two_factors && a * b < 0x1p-90f) {
         post = 0x1p-64f;
         return ((fminf(a, b) * 0x1p64f) * fmaxf(a, b)) * p.inv_den;
+    }
+    if (p.two_factors && a * b > kMax && a <= kMax && b <= kMax) {
+        post = 0x1p64f;
+        return fminf(((fmaxf(a, b) * 0x1p-64f) * fminf(a, b)) * p.inv_den, kMax);
     }
     return (a * b) * p.inv_den;
 }
@@ -1273,7 +1281,7 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     GemmParams p;
     p.A = A; p.B = B; p.sfA = sfA; p.sfB = sfB; p.alpha = alpha; p.D = D; p.bias = bias; p.d_amax = d_amax;
     p.amax_a = amax_a; p.amax_b = amax_b; p.inv_den = alpha ? 0.0f : (float)(1.0 / denominator);
-    p.tiny_scale = if4;
+    p.two_factors = if4;
     p.M = M; p.N = N; p.K = K; p.ldd = ldd;
     p.rows = rows < 0 ? M : rows;
     hipStream_t s = (hipStream_t)stream;

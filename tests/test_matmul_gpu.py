@@ -3,6 +3,7 @@ and the reference's matmul vectors.  Budget, as the reference holds its own back
 (tests/test_matmul.py:15,81-88): at most 1e-3 of the bf16 outputs differ at all; and
 max |diff| <= 1e-2 of the output range."""
 
+import copy
 import os
 
 import numpy as np
@@ -374,6 +375,49 @@ def test_if4_gemm_over_all_codes_and_scales(monkeypatch, m, n, k, tile, amaxes):
     bias = torch.linspace(-1, 1, n, device="cuda").bfloat16()
     with_bias = fos.quantized_matmul(qa, qb, bias=bias, emit_amax=True)
     assert torch.equal(with_bias, out + bias)
+
+
+@pytest.mark.parametrize("tile", ["128", "129", "256", "split"])
+@pytest.mark.parametrize("amaxes", [(2.0 ** 70, 2.0 ** 60), (2.0 ** 64, 2.0 ** 64), (2.0 ** 100, 2.0 ** 100),
+                                    (3.0 * 2.0 ** 126, 3.0 * 2.0 ** 126), (2.0 ** 127, 2.0 ** -20)])
+def test_if4_product_of_large_maxima(monkeypatch, amaxes, tile):
+    """The product of the two maxima leaves fp32's range: results inside the range stay finite, rows and columns of
+    zeros stay zero, the rest is infinite.  Bounds as above; an infinity has to lie within the bound of bf16's overflow."""
+    if tile == "split":
+        monkeypatch.setenv("FOS_GEMM_SPLITK", "2")
+    monkeypatch.setenv("FOS_GEMM_TILE", "128" if tile == "split" else tile)
+    from fouroversix_amd.quantize import known_amax
+
+    m, n, k = 130, 256, 128
+    g = torch.Generator("cpu").manual_seed(7)
+
+    def operand(rows, amax, zero):
+        rows_p = -(-rows // 128) * 128
+        codes = torch.randint(0, 256, (rows_p, k // 2), generator=g, dtype=torch.uint8)
+        codes[zero] = 0
+        codes[rows:] = 0
+        scales = torch.randint(0, 57, (rows_p * k // 16,), generator=g, dtype=torch.uint8)  # at most 1
+        scales |= torch.randint(0, 2, scales.shape, generator=g, dtype=torch.uint8) << 7
+        return fos.QuantizedTensor(codes.cuda(), scales.cuda().view(torch.float8_e4m3fn), torch.tensor(amax, device="cuda"),
+                                   fos.DataType.if4, (rows, k), fos.ScaleRule.mse, fos.RoundStyle.nearest, padded_shape=(rows_p, k),
+                                   scale_factors_are_in_blackwell_layout=False)
+
+    qa, qb = operand(m, amaxes[0], [3, 129]), operand(n, amaxes[1], [5])
+    units = copy.copy(qa), copy.copy(qb)
+    for unit in units:
+        unit.amax = torch.ones_like(unit.amax)
+    # (dequantized with a maximum of 1: `value * maximum` overflows for the largest ones)
+    a, b = (fos.dequantize(unit, dtype=torch.float32).double().cpu() * amax for unit, amax in zip(units, amaxes))
+    exact, size = a @ b.T, a.abs() @ b.abs().T
+    bound = 2.0 ** -8 * exact.abs() + 2 * k * 2.0 ** -24 * size
+    out = fos.quantized_matmul(qa, qb, emit_amax=True)
+    assert float(known_amax(out)) == float(out.abs().max())
+    out = out.double().cpu()
+    assert not bool(out.isnan().any())
+    assert bool((out[[3, 129]] == 0).all()) and bool((out[:, 5] == 0).all())
+    inside = out.isfinite()
+    assert bool(((out - exact).abs() <= bound)[inside].all())
+    assert bool((exact * out.sign() + bound >= (2 - 2.0 ** -8) * 2.0 ** 127)[~inside].all())
 
 
 def test_linear_forward_replays_in_a_hip_graph():
