@@ -24,7 +24,14 @@ from fouroversix_amd.quantize.frontend import (
     format_divisor,
     known_amax,
 )
-from fouroversix_amd.utils import NATIVE_FORMAT_IDS, DataType, MatmulBackend, RoundStyle, ScaleRule
+from fouroversix_amd.utils import (
+    NATIVE_FORMAT_IDS,
+    DataType,
+    MatmulBackend,
+    RoundStyle,
+    ScaleRule,
+    seen_by_autograd_functions,
+)
 
 
 def is_supported(input: QuantizedTensor, other: QuantizedTensor, *, out_dtype: DataType) -> bool:
@@ -149,9 +156,13 @@ def _if4_gemm_applies(input: QuantizedTensor, other: QuantizedTensor, out_dtype:
 
 
 def _fusable_bias(bias: torch.Tensor | None, dtype: torch.dtype, columns: int, device: torch.device) -> bool:
-    """Whether the GEMM's epilogue can add ``bias`` (``columns``: the weight's rows with their padding)."""
+    """Whether the GEMM's epilogue can add ``bias`` (``columns``: the weight's rows with their padding).  It reads the
+    memory of ``bias``: a sum that something differentiates or transforms stays a sum of torch's."""
     return (
         bias is not None
+        and (type(bias) is torch.Tensor or type(bias) is torch.nn.Parameter)
+        and not (bias.requires_grad and torch.is_grad_enabled())
+        and not seen_by_autograd_functions()
         and bias.dtype == dtype
         and bias.dim() == 1
         and bias.shape[0] == columns  # (no row padding of the weight between the bias and the product)

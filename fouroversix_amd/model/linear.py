@@ -24,6 +24,7 @@ from fouroversix_amd.matmul.frontend import nvfp4_linear
 from fouroversix_amd.quantize import QuantizedTensor, dequantize, quantize
 from fouroversix_amd.quantize.frontend import attach_known_amax, known_amax
 from fouroversix_amd.utils import DataType, RoundStyle
+from fouroversix_amd.utils import seen_by_autograd_functions as _seen_by_autograd_functions
 
 from .config import ModuleQuantizationConfig
 from .quantize import QuantizedModule
@@ -137,17 +138,6 @@ class FourOverSixLinearFunction(torch.autograd.Function):
 
         grad_bias = g.sum(0) if bias is not None and ctx.needs_input_grad[3] else None
         return None, grad_input, grad_weight, grad_bias
-
-
-def _seen_by_autograd_functions() -> bool:
-    """Whether something other than backward mode looks at autograd functions: a trace, a functorch transform or
-    forward-mode differentiation (which stays on under ``torch.no_grad()``)."""
-    return (
-        torch.compiler.is_compiling()
-        or torch._C._get_tracing_state() is not None
-        or torch._C._are_functorch_transforms_active()
-        or torch.autograd.forward_ad._current_level >= 0
-    )
 
 
 @QuantizedModule.register(nn.Linear)

@@ -255,3 +255,14 @@ DataType.torch_dtype = property(_torch_dtype)
 
 # Formats that have a gfx950 kernel, with their id at the native boundary.
 NATIVE_FORMAT_IDS = {"nvfp4": 0, "if4": 1, "mxfp4": 2}
+
+
+def seen_by_autograd_functions() -> bool:
+    """Whether something other than backward mode looks at autograd functions and operators: a trace, a functorch
+    transform or forward-mode differentiation (which stays on under ``torch.no_grad()``)."""
+    return (
+        torch.compiler.is_compiling()
+        or torch._C._get_tracing_state() is not None
+        or torch._C._are_functorch_transforms_active()
+        or torch.autograd.forward_ad._current_level >= 0
+    )

@@ -420,6 +420,30 @@ def test_if4_product_of_large_maxima(monkeypatch, amaxes, tile):
     assert bool((exact * out.sign() + bound >= (2 - 2.0 ** -8) * 2.0 ** 127)[~inside].all())
 
 
+@pytest.mark.parametrize("dtype", ["nvfp4", "if4"])
+def test_product_with_a_bias_that_is_differentiated(dtype):
+    """``bias=`` is ``out + bias`` to autograd, forward-mode differentiation and vmap too; without them the sum is formed
+    in the GEMM, with the same bits."""
+    import torch.autograd.forward_ad as fwd
+
+    cfg = fos.QuantizationConfig(dtype=dtype)
+    qa, qb = (fos.quantize(make_input("randn", (rows, 256), rows).cuda(), cfg) for rows in (32, 128))
+    bias = torch.randn(128, generator=torch.Generator("cpu").manual_seed(1)).bfloat16().cuda()
+    expect = fos.quantized_matmul(qa, qb) + bias
+    assert torch.equal(fos.quantized_matmul(qa, qb, bias=bias), expect)
+    leaf = nn.Parameter(bias.clone())
+    out = fos.quantized_matmul(qa, qb, bias=leaf)
+    assert torch.equal(out.detach(), expect)
+    assert torch.equal(torch.autograd.grad(out.sum(), leaf)[0], torch.full_like(bias, 32))
+    with torch.no_grad():
+        assert torch.equal(fos.quantized_matmul(qa, qb, bias=leaf), expect)
+    with fwd.dual_level():
+        dual = fwd.unpack_dual(fos.quantized_matmul(qa, qb, bias=fwd.make_dual(bias, torch.ones_like(bias))))
+        assert torch.equal(dual.primal, expect) and torch.equal(dual.tangent, torch.ones_like(expect))
+    both = torch.func.vmap(lambda b: fos.quantized_matmul(qa, qb, bias=b))(torch.stack([bias, 2 * bias]))
+    assert torch.equal(both, torch.stack([expect, fos.quantized_matmul(qa, qb) + 2 * bias]))
+
+
 def test_linear_forward_replays_in_a_hip_graph():
     """A decode-sized forward (quantize -> alpha -> weight-streaming GEMM, twice) captured in
     a HIP graph: every replay, interleaved with eager work and synchronisations, equals
