@@ -60,6 +60,7 @@ struct GemmParams {
     const void *bias;          // optional: N values of the output type, added to the rounded product and rounded again
     float *d_amax;             // optional: max|D| as stored is folded into d_amax[0] (unsigned atomic max on the bits)
     int64_t M, N, K, ldd;
+    uint32_t k_tail;           // IF4: mask on the scale bytes of the last 64 codes of a row, 0 for blocks that are padding
     int64_t rows;              // rows 0 ... rows - 1 of D count for d_amax: padding rows hold the bias, not zeros
     int tiles_m, tiles_n;
     // split-K: workgroup (tile, blockIdx.y) contracts K steps [y * ksteps_per_split, ...) and
@@ -323,6 +324,19 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
     const int64_t ksteps =
         OUT == kOutPartial ? (ksteps_all - ks0 < p.ksteps_per_split ? ksteps_all - ks0 : p.ksteps_per_split) : ksteps_all;
 
+    // IF4: codes in the padding of K don't count, whatever they are (a tensor rotated along a ragged width has some there):
+    // the scales of those blocks are taken for zeros.  Applied where a step's scales are used first, not at their
+    // load, which would be waited for there.
+    auto drop_tail = [&](int64_t ks, uint32_t &scales) {
+        if constexpr (IF4) scales &= ks0 + ks + 1 >= ksteps_all ? p.k_tail : 0xffffffffu;
+    };
+    auto drop_b_tail = [&](int64_t ks, Staged<WN> &s) {
+        if constexpr (IF4) {
+#pragma unroll
+            for (int j = 0; j < WN; ++j) drop_tail(ks, s.sb[j]);
+        }
+    };
+
     typedef Staged<WN> StagedT;
     auto fetch = [&](int64_t ks, StagedT &s) {
         const uint32_t kq = (uint32_t)(ks0 + ks) * 32u, ksf = (uint32_t)(ks0 + ks) * kScaleStep;
@@ -386,6 +400,8 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
     StagedT bcur;                  // the step being multiplied: its B rows (st[] is refilled two steps ahead)
     half8_t fa[2][WM], fb[2][WN];  // MFMA fragments of the current and the next 16-wide K slice
     fetch(0, st[0]);
+    drop_tail(0, st[0].sa);
+    drop_b_tail(0, st[0]);
 #pragma unroll
     for (int q = 0; q < 4; ++q) stage_quarter(st[0], 0, q);
     b_frags(st[0], 0, fb[0]);
@@ -416,6 +432,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
                 read_frags(buf, kk + 1, fa[(kk + 1) & 1]);
                 b_frags(bcur, kk + 1, fb[(kk + 1) & 1]);
             }
+            if (have_next && kk == 0) drop_tail(ks + 1, nxt.sa);
             if (have_next) stage_quarter(nxt, buf ^ 1, kk);
             const bool at_barrier = have_next && kk + 1 == BK / 16;
             auto mfmas = [&](int i_begin, int i_end) {
@@ -438,6 +455,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
                 mfmas(WM / 2, WM);
                 // the next step's B rows become the current ones (fb[0] is free: slice 3 used fb[1])
                 bcur = nxt;
+                drop_b_tail(ks + 1, bcur);
                 b_frags(bcur, 0, fb[0]);
             } else {
                 mfmas(0, WM);
@@ -1266,7 +1284,7 @@ extern "C" size_t fos_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
                            const float *alpha, const float *amax_a, const float *amax_b, double denominator,
                            int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
-                           void *workspace, size_t workspace_bytes, fos_stream_t stream, bool if4 = false, int64_t rows = -1) {
+                           void *workspace, size_t workspace_bytes, fos_stream_t stream, bool if4 = false, int64_t rows = -1, int64_t depth = -1) {
     if (!A || !B || !sfA || !sfB || !D) return FOS_E_NULL_POINTER;
     if (((uintptr_t)d_amax & 3) || ((uintptr_t)bias & 7)) return FOS_E_BAD_ALIGNMENT;
     if (!alpha && (!amax_a || !amax_b)) return FOS_E_NULL_POINTER;
@@ -1284,6 +1302,8 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     p.two_factors = if4;
     p.M = M; p.N = N; p.K = K; p.ldd = ldd;
     p.rows = rows < 0 ? M : rows;
+    // (blocks of the last 64 codes that lie below `depth`: 8 bits of the mask each)
+    p.k_tail = depth < 0 || K - depth < 16 ? 0xffffffffu : (1u << (8 * ((depth - (K - 64)) / 16))) - 1u;
     hipStream_t s = (hipStream_t)stream;
     GemmPlan g = plan_gemm(M, N, K, if4);
     if (M < 128 && g.kind != kPlanSkinny) return FOS_E_BAD_SHAPE;
@@ -1381,12 +1401,13 @@ extern "C" int fos_gemm_if4(const uint8_t *A, const uint8_t *B, const uint8_t *s
 
 extern "C" int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
                                     const float *amax_a, const float *amax_b, double denominator,
-                                    int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
+                                    int64_t M, int64_t rows, int64_t N, int64_t K, int64_t depth, void *D, int out_type, int64_t ldd, const void *bias,
                                     float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream) {
     if (!amax_a || !amax_b) return FOS_E_NULL_POINTER;
     if (dtype != FOS_DTYPE_NVFP4 && dtype != FOS_DTYPE_IF4) return FOS_E_UNSUPPORTED;
     const bool if4 = dtype == FOS_DTYPE_IF4;
     if (!(denominator > 0.0) || rows < 0 || rows > M || (if4 && M % 128 != 0)) return FOS_E_BAD_SHAPE;
+    if (depth > K || depth <= K - 64 || (depth != K && (!if4 || depth % 16 != 0))) return FOS_E_BAD_SHAPE;
     return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, workspace,
-                           workspace_bytes, stream, if4, rows);
+                           workspace_bytes, stream, if4, rows, depth);
 }

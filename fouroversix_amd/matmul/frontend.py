@@ -125,7 +125,9 @@ def _gemm_record(q: QuantizedTensor) -> tuple:
 
 
 def _if4_gemm_applies(input: QuantizedTensor, other: QuantizedTensor, out_dtype: DataType) -> bool:
-    """Two IF4 tensors as ``quantize`` lays them out (row-major scales), on one GPU, for the IF4 GEMM."""
+    """Two IF4 tensors as ``quantize`` lays them out (row-major scales), on one GPU, for the IF4 GEMM.  It leaves out
+    whole blocks that are padding of the inner dimension; a block with some elements of padding, which may hold values
+    (a ragged width that was rotated), takes the dequantized form, which crops."""
 
     def fits(q: QuantizedTensor) -> bool:
         return (
@@ -151,6 +153,8 @@ def _if4_gemm_applies(input: QuantizedTensor, other: QuantizedTensor, out_dtype:
         and fits(other)
         and input.values.device == other.values.device
         and input.padded_shape[1] == other.padded_shape[1]
+        and input.original_shape[1] % 16 == 0
+        and input.padded_shape[1] - 64 < input.original_shape[1] <= input.padded_shape[1]
         and not torch.compiler.is_compiling()
     )
 
@@ -328,7 +332,7 @@ def quantized_matmul(
             out = ops.gemm_if4(
                 input.values, other.values, input.scale_factors, other.scale_factors, input.amax, other.amax,
                 dequantize_divisor(input) * dequantize_divisor(other), out_dtype.torch_dtype, d_amax,
-                bias.detach() if fused_bias else None, input.original_shape[0],
+                bias.detach() if fused_bias else None, input.original_shape[0], input.original_shape[1],
             )
             out_shape = (input.original_shape[0], other.original_shape[0])
             out = out if tuple(out.shape) == out_shape else out[: out_shape[0], : out_shape[1]]

@@ -310,11 +310,13 @@ size_t fos_gemm_if4_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /*
  * fos_gemm_nvfp4_linear (dtype FOS_DTYPE_NVFP4) or fos_gemm_if4 (FOS_DTYPE_IF4) for an A whose rows from `rows` on are
  * padding: all M rows of D are written, and d_amax receives the maximum over the first `rows` alone (with a bias the
- * padding rows of D are not zeros but hold the bias).
+ * padding rows of D are not zeros but hold the bias).  `depth`: K, or for IF4 the multiple of 16 above K - 64 from which
+ * on the codes of a row are padding that does not count (a tensor whose ragged width was rotated holds values there,
+ * which its dequantization leaves out).
  */
 int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
                          const float *amax_a, const float *amax_b, double denominator,
-                         int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
+                         int64_t M, int64_t rows, int64_t N, int64_t K, int64_t depth, void *D, int out_type, int64_t ldd, const void *bias,
                          float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream);
 
 /*

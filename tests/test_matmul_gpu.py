@@ -444,6 +444,43 @@ def test_product_with_a_bias_that_is_differentiated(dtype):
     assert torch.equal(both, torch.stack([expect, fos.quantized_matmul(qa, qb) + 2 * bias]))
 
 
+@pytest.mark.parametrize("env", [{}, {"FOS_GEMM_TILE": "128"}, {"FOS_GEMM_TILE": "129"}, {"FOS_GEMM_TILE": "256"},
+                                 {"FOS_GEMM_TILE": "128", "FOS_GEMM_SPLITK": "2"}], ids=str)
+@pytest.mark.parametrize("k", [1, 16, 48, 80, 100, 112, 127, 192, 336])
+def test_if4_product_leaves_out_the_padding_of_the_inner_dimension(monkeypatch, k, env):
+    """Codes and scales (a NaN scale among them) in the padding of both operands: the product of the dequantized, cropped
+    operands.  Bound as for all codes and scales."""
+    for name, value in env.items():
+        monkeypatch.setenv(name, value)
+    g = torch.Generator("cpu").manual_seed(k)
+    rows_p, cols_p = 256, -(-k // 64) * 64
+
+    def operand(rows, amax):
+        codes = torch.randint(0, 256, (rows_p, cols_p // 2), generator=g, dtype=torch.uint8)
+        scales = torch.randint(0, 127, (rows_p, cols_p // 16), generator=g, dtype=torch.uint8)
+        scales[:, -(-k // 16):] = 0x7F
+        return fos.QuantizedTensor(codes.cuda(), scales.flatten().cuda().view(torch.float8_e4m3fn), torch.tensor(amax, device="cuda"),
+                                   fos.DataType.if4, (rows, k), fos.ScaleRule.mse, fos.RoundStyle.nearest, padded_shape=(rows_p, cols_p),
+                                   scale_factors_are_in_blackwell_layout=False)
+
+    qa, qb = operand(200, 2.0), operand(256, 1.0)
+    a, b = (fos.dequantize(q, dtype=torch.float32).double().cpu() for q in (qa, qb))
+    exact, size = a @ b.T, a.abs() @ b.abs().T
+    out = fos.quantized_matmul(qa, qb).double().cpu()
+    assert bool(((out - exact).abs() <= 2.0 ** -8 * exact.abs() + 2 * k * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("tokens", [7, 16, 100, 128, 200])
+def test_if4_weight_gradient_of_ragged_token_counts(tokens):
+    """Both operands rotated along the tokens, which leaves values in the padding: as the dequantized product."""
+    cfg = fos.QuantizationConfig(dtype="if4", transpose=True, rht=True)
+    qg, qx = (fos.quantize(make_input("randn", (tokens, cols), cols).cuda(), cfg) for cols in (256, 384))
+    a, b = (fos.dequantize(q, dtype=torch.float32).double() for q in (qg, qx))
+    exact, size = a @ b.T, a.abs() @ b.abs().T
+    out = fos.quantized_matmul(qg, qx).double()
+    assert bool(((out - exact).abs() <= 2.0 ** -8 * exact.abs() + 2 * tokens * 2.0 ** -24 * size).all())
+
+
 def test_linear_forward_replays_in_a_hip_graph():
     """A decode-sized forward (quantize -> alpha -> weight-streaming GEMM, twice) captured in
     a HIP graph: every replay, interleaved with eager work and synchronisations, equals
