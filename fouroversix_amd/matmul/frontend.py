@@ -124,6 +124,10 @@ def _gemm_record(q: QuantizedTensor) -> tuple:
     return rec
 
 
+# The GEMM's 32-bit offsets inside a panel of 256 rows; longer rows, and empty operands, take the dequantized form.
+_IF4_GEMM_DEPTH = 1 << 22
+
+
 def _if4_gemm_applies(input: QuantizedTensor, other: QuantizedTensor, out_dtype: DataType) -> bool:
     """Two IF4 tensors as ``quantize`` lays them out (row-major scales), on one GPU, for the IF4 GEMM.  It leaves out
     whole blocks that are padding of the inner dimension; a block with some elements of padding, which may hold values
@@ -153,8 +157,10 @@ def _if4_gemm_applies(input: QuantizedTensor, other: QuantizedTensor, out_dtype:
         and fits(other)
         and input.values.device == other.values.device
         and input.padded_shape[1] == other.padded_shape[1]
+        and input.original_shape[1] > 0
         and input.original_shape[1] % 16 == 0
-        and input.padded_shape[1] - 64 < input.original_shape[1] <= input.padded_shape[1]
+        and input.padded_shape[1] - 64 < input.original_shape[1] <= input.padded_shape[1] <= _IF4_GEMM_DEPTH
+        and input.original_shape[0] > 0 < other.original_shape[0]
         and not torch.compiler.is_compiling()
     )
 

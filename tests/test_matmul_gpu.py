@@ -481,6 +481,24 @@ def test_if4_weight_gradient_of_ragged_token_counts(tokens):
     assert bool(((out - exact).abs() <= 2.0 ** -8 * exact.abs() + 2 * tokens * 2.0 ** -24 * size).all())
 
 
+@pytest.mark.parametrize(("m", "n", "k"), [(0, 128, 256), (4, 0, 256), (4, 8, 0), (1, 2, (1 << 22) + 64)])
+def test_if4_products_that_the_kernel_does_not_take(m, n, k):
+    """Empty operands and rows beyond the kernel's offsets: the dequantized form, as other formats without a kernel."""
+    cfg = fos.QuantizationConfig(dtype="if4")
+    qa, qb = (fos.quantize(torch.randn(rows, k, generator=torch.Generator("cpu").manual_seed(rows)).bfloat16().cuda(), cfg) for rows in (m, n))
+    out = fos.quantized_matmul(qa, qb)
+    a, b = (fos.dequantize(q, dtype=torch.float32).double() for q in (qa, qb))
+    exact = a @ b.T
+    assert out.shape == (m, n) and out.dtype == torch.bfloat16
+    assert bool(((out - exact).abs() <= 2.0 ** -8 * exact.abs() + 2 * k * 2.0 ** -24 * (a.abs() @ b.abs().T)).all())
+    if m == 0:
+        model = nn.Sequential(nn.Linear(k, n, device="cuda", dtype=torch.bfloat16))
+        fos.quantize_model(model, fos.ModelQuantizationConfig(dtype="if4"))
+        model[0].quantize_weight_()
+        with torch.no_grad():
+            assert model(torch.empty(2, 0, k, device="cuda", dtype=torch.bfloat16)).shape == (2, 0, n)
+
+
 def test_linear_forward_replays_in_a_hip_graph():
     """A decode-sized forward (quantize -> alpha -> weight-streaming GEMM, twice) captured in
     a HIP graph: every replay, interleaved with eager work and synchronisations, equals
