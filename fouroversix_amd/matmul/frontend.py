@@ -333,15 +333,21 @@ def quantized_matmul(
             # the dequantized operands' product (src/fouroversix/matmul/pytorch.py:33-52) without forming them: fp16
             # values as the dequantization defines them, the tensor maxima in the output scale
             device = input.values.device
+            m, n = input.original_shape[0], other.original_shape[0]
             fused_bias = _fusable_bias(bias, out_dtype.torch_dtype, other.values.shape[0], device)
-            d_amax = _fresh_amax_word(device) if emit_amax and (bias is None or fused_bias) else None
+            whole_rows = n == other.values.shape[0]
+            d_amax = _fresh_amax_word(device) if emit_amax and whole_rows and (bias is None or fused_bias) else None
             out = ops.gemm_if4(
                 input.values, other.values, input.scale_factors, other.scale_factors, input.amax, other.amax,
                 dequantize_divisor(input) * dequantize_divisor(other), out_dtype.torch_dtype, d_amax,
-                bias.detach() if fused_bias else None, input.original_shape[0], input.original_shape[1],
+                bias.detach() if fused_bias else None, m, input.original_shape[1],
             )
-            out_shape = (input.original_shape[0], other.original_shape[0])
-            out = out if tuple(out.shape) == out_shape else out[: out_shape[0], : out_shape[1]]
+            # (contiguous, as the product of the dequantized matrices is; whatever the padding columns hold is not in
+            # the maximum, which is recorded for whole rows only)
+            if not whole_rows:
+                out = out[:m, :n].contiguous()
+            elif m != out.shape[0]:
+                out = out[:m]
             if d_amax is not None:
                 attach_known_amax(out, d_amax)
             return out if bias is None or fused_bias else out + bias

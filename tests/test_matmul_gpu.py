@@ -481,6 +481,16 @@ def test_if4_weight_gradient_of_ragged_token_counts(tokens):
     assert bool(((out - exact).abs() <= 2.0 ** -8 * exact.abs() + 2 * tokens * 2.0 ** -24 * size).all())
 
 
+@pytest.mark.parametrize(("m", "n"), [(1, 300), (100, 256), (128, 144), (200, 300)])
+def test_if4_product_is_contiguous(m, n):
+    """Sizes that get padding: the result is the plain matrix that the dequantized form returns."""
+    cfg = fos.QuantizationConfig(dtype="if4")
+    qa, qb = (fos.quantize(make_input("randn", (rows, 128), rows).cuda(), cfg) for rows in (m, n))
+    for bias in (None, torch.ones(n, device="cuda", dtype=torch.bfloat16)):
+        out = fos.quantized_matmul(qa, qb, bias=bias, emit_amax=True)
+        assert out.is_contiguous() and out.view(-1).shape == (m * n,)
+
+
 @pytest.mark.parametrize(("m", "n", "k"), [(0, 128, 256), (4, 0, 256), (4, 8, 0), (1, 2, (1 << 22) + 64)])
 def test_if4_products_that_the_kernel_does_not_take(m, n, k):
     """Empty operands and rows beyond the kernel's offsets: the dequantized form, as other formats without a kernel."""
