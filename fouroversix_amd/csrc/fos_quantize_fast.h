@@ -46,7 +46,8 @@ FOS_DEVICE float amax_norm(float amax) {
     return u2f((254u - (e < 1u ? 1u : (e > 253u ? 253u : e))) << 23);
 }
 
-// Entry for scale byte `s` (0..127); built with the reference's operations.
+// Entry for scale byte `s` (0..127); built with the reference's operations.  Looked up with the byte's low seven bits: the
+// scale of a block with an infinite element is a NaN of either sign (under a given, finite tensor maximum).
 template <bool PRODUCT_FORM = false>
 FOS_DEVICE FastLutEntry make_lut_entry(uint32_t s, const QuantConsts &k) {
     FastLutEntry e;
@@ -516,7 +517,7 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_fast(const Block16 &blk, const QuantCon
         // and sub-normal scales alike -- is exact on the fast path.
         // The stochastic style clamps to 6 in the reference as well, so only the zero scale
         // byte is left out there.
-        const FastLutEntry A = lut[s6];
+        const FastLutEntry A = lut[s6 & 0x7fu];
         if (SR ? s6 != 0u : (s6 >= 8u || (s6 != 0u && bmax * A.inv < 7.0f))) {
             if constexpr (SR) {
                 // scaled values, hardware stochastic rounding (one Philox call per block);
@@ -529,7 +530,7 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_fast(const Block16 &blk, const QuantCon
                 uint32_t a0, a1;
                 sr_pack16(xa, pA, a0, a1);
                 if (STATIC) return BlockOut{a0, a1, s6};
-                const FastLutEntry B = lut[s4];
+                const FastLutEntry B = lut[s4 & 0x7fu];
                 float xb[16];
 #pragma unroll
                 for (int i = 0; i < 16; ++i) xb[i] = scaled(x[i], B.inv);
@@ -579,7 +580,7 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_fast(const Block16 &blk, const QuantCon
                 });
                 return BlockOut{c0, c1, s6};
             }
-            const FastLutEntry B = lut[s4];
+            const FastLutEntry B = lut[s4 & 0x7fu];
             uint32_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;
             float SA = 0.0f, SB = 0.0f, GA = 0.0f, GB = 0.0f;  // (product form: SA / SB hold F)
             static_for<0, 8>([&](auto jc) {
@@ -688,10 +689,10 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_f32(const Block16F &blk, const QuantCon
         const float s_hp6 = (bmax / k.qdiv) * enc, s_hp4 = s_hp6 * 1.5f;
         const uint32_t pk = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(s_hp6, s_hp4, 0, false);
         const uint32_t s6 = pk & 0xffu, s4 = (pk >> 8) & 0xffu;
-        const FastLutEntry A = lut[s6];
+        const FastLutEntry A = lut[s6 & 0x7fu];
         // (the exclusions of quantize_block_nvfp4_fast; a given maximum may be below the tensor's own: beyond 7 as well)
         if (s6 != 0u && bmax * A.inv < 7.0f) {
-            const FastLutEntry B = STATIC ? A : lut[s4];
+            const FastLutEntry B = STATIC ? A : lut[s4 & 0x7fu];
             uint32_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;
             float SA = 0.0f, SB = 0.0f;
             static_for<0, 8>([&](auto jc) {
@@ -787,7 +788,7 @@ FOS_DEVICE BlockOut quantize_block_if4_mse(const Block16 &blk, const QuantConsts
         if (TWO_D) bmax = row16_max(bmax);
         const float s_hp = div_const(bmax, k.qdiv, rq) * enc;
         const uint32_t s = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(s_hp, 0.0f, 0, false) & 0xffu;
-        const FastLutEntry A = lut[s];
+        const FastLutEntry A = lut[s & 0x7fu];
         // same exclusions as the NVFP4 path: the unclamped E2M1 value 8 and the zero scale byte
         if (s >= 8u || (s != 0u && bmax * A.inv < 7.0f)) {
             uint32_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;

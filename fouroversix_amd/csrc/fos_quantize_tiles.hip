@@ -512,9 +512,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
             const float s_hp4 = s_hp6 * 1.5f;
             const uint32_t pk = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(s_hp6, s_hp4, 0, false);
             const uint32_t s6 = pk & 0xffu, s4 = (pk >> 8) & 0xffu;
-            const FastLutEntry A = lut[s6];
+            const FastLutEntry A = lut[s6 & 0x7fu];
             FastLutEntry B = A;
-            if (ADAPTIVE && !IF4) B = lut[s4];
+            if (ADAPTIVE && !IF4) B = lut[s4 & 0x7fu];
             // the hardware convert saturates at 6 where the reference's unclamped rounding gives 8:
             // that needs a sub-normal scale byte rounded down by more than 7/6; a zero scale byte
             // of a non-zero tile has no scaled domain.  (The stochastic styles clamp to 6 in the

@@ -506,6 +506,37 @@ def test_element_wise_fast_form_bit_exact(oracle, dtype, two_d, rule):
     assert_same_quantization(q, oracle.quantize(y, **cfg, amax=float(np.float32(given))), "given maximum")
 
 
+@pytest.mark.parametrize("split", ["1", "2"])
+@pytest.mark.parametrize("two_d", [False, True])
+@pytest.mark.parametrize("dtype", ["nvfp4", "if4"])
+def test_blocks_with_an_infinite_element_under_a_given_maximum(monkeypatch, dtype, two_d, split):
+    """Their scale byte is a NaN, of either sign: their codes are those on the number that its low seven bits spell (480),
+    and the other blocks do not depend on them."""
+    monkeypatch.setenv("FOS_QUANT_SPLIT", split)
+    x = make_input("randn", (64, 512), 19)
+    with_inf = x.clone()
+    with_inf[::16, 4::64] = float("inf")
+    with_inf[1::16, 38::64] = -float("inf")
+    blocks = torch.isinf(with_inf.float()).view(64, -1, 16).any(-1)
+    if two_d:
+        blocks = blocks.view(4, 16, -1).any(1).repeat_interleave(16, 0)
+    for given in (5.0, 3.0):
+        cfg = fos.QuantizationConfig(dtype=dtype, scale_rule="mse" if dtype == "if4" else "static_6", block_scale_2d=two_d, kwargs={"amax": torch.tensor(given, device="cuda")})
+        q, plain = fos.quantize(with_inf.cuda(), cfg), fos.quantize(x.cuda(), cfg)
+        codes, expect = (t.values[:64].view(64, -1, 8).cpu() for t in (q, plain))
+        assert torch.equal(codes[~blocks], expect[~blocks])
+        if dtype == "nvfp4":
+            # (elements that are no tie of two codes)
+            scaled = with_inf.float().view(64, -1, 16) / (480 * given / 2688)
+            grid = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6])
+            clear = ((scaled.abs()[..., None] - (grid[1:] + grid[:-1]) / 2).abs().amin(-1) > 1e-3) & scaled.isfinite()
+            nibbles = torch.stack([codes & 15, codes >> 4], -1).view(64, -1, 16).long()
+            read = grid[nibbles & 7] * (1 - 2 * (nibbles >> 3).float())
+            nearest = grid[(scaled.abs()[..., None] - grid).abs().argmin(-1)] * scaled.sign()
+            pick = blocks[..., None] & clear
+            assert torch.equal(read[pick], nearest[pick])
+
+
 @pytest.mark.parametrize("shape", [(3, 17), (129, 301), (64, 1025)])
 def test_unaligned_bf16_rows(oracle, shape):
     for offset in (0, 1, 3):  # rows that start at any element of the buffer
