@@ -822,8 +822,10 @@ FOS_DEVICE BlockOut quantize_block_if4_mse(const Block16 &blk, const QuantConsts
             if (cmp > 0) return BlockOut{b0, b1, s | 0x80u};
             if (cmp < 0) return BlockOut{a0, a1, s};
             // undecided (uniform over the 16 lanes of a tile when TWO_D: both sums are tile sums)
+            // (not with a NaN among the elements, nor with the NaN scale byte of a given maximum that is too small, whose
+            // scaled values the conversions saturate and the operation-by-operation form does not)
             if constexpr (!TWO_D) {
-                if (k.shortcut_ok && k.errdiv == 2688.0f && (f2u(k.amax) & 0xffffu) == 0) {
+                if (k.shortcut_ok && k.errdiv == 2688.0f && (f2u(k.amax) & 0xffffu) == 0 && s < 0x7fu && SA == SA) {
                     const bool pickB = exact_pick_integer_1d(x, a0, a1, b0, b1, A, e4m3_decode(s) * k.amax);
                     return BlockOut{pickB ? b0 : a0, pickB ? b1 : a1, pickB ? s | 0x80u : s};
                 }

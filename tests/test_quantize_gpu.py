@@ -537,6 +537,21 @@ def test_blocks_with_an_infinite_element_under_a_given_maximum(monkeypatch, dtyp
             assert torch.equal(read[pick], nearest[pick])
 
 
+@pytest.mark.parametrize("shape", [(64, 256), (33, 70), (130, 272)])
+@pytest.mark.parametrize(("given", "special"), [(8.0, True), (5.0, True), (1.0, False)])
+def test_if4_blocks_outside_the_exact_decision(shape, given, special):
+    """A given maximum with NaN elements, or one so small that scales become NaN, in blocks whose candidates nearly tie (one
+    large element): the bytes of the operation-by-operation form, which fp32 inputs take."""
+    x = make_input("randn", shape, 92).float() * (0.02 if special else 0.004)
+    x[:, 5::16] = 1 + torch.arange(x[:, 5::16].numel()).view(x.shape[0], -1) % 128 / 128
+    if special:
+        x[::3, 2::32] = float("nan")
+    cfg = fos.QuantizationConfig(dtype="if4", kwargs={"amax": torch.tensor(given, device="cuda")})
+    q, expect = fos.quantize(x.bfloat16().cuda(), cfg), fos.quantize(x.bfloat16().float().cuda(), cfg)
+    assert torch.equal(q.scale_factors.view(torch.uint8), expect.scale_factors.view(torch.uint8))
+    assert torch.equal(q.values, expect.values)
+
+
 @pytest.mark.parametrize("shape", [(3, 17), (129, 301), (64, 1025)])
 def test_unaligned_bf16_rows(oracle, shape):
     for offset in (0, 1, 3):  # rows that start at any element of the buffer
