@@ -709,7 +709,16 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_f32(const Block16F &blk, const QuantCon
                     accumulate_scaled<RULE>(fb.x - xb0, fb.y - xb1, SB);
                 }
             });
-            if (STATIC) return BlockOut{a0, a1, s6};
+            if (STATIC) {
+                // (a NaN element, under a given maximum, has its code from the operation-by-operation form; the rules that
+                // compare find it in SA)
+                float nan = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) nan = __builtin_fmaf(x[i], 0.0f, nan);
+                if (TWO_D) nan = row16_max(nan == nan ? 0.0f : 1.0f);
+                if (nan == 0.0f) return BlockOut{a0, a1, s6};
+                return generic_block_f32<RULE, TWO_D>(blk, k);
+            }
             if (TWO_D) {
                 SA = row16_sum_lane0(SA);
                 SB = row16_sum_lane0(SB);
@@ -717,7 +726,7 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_f32(const Block16F &blk, const QuantCon
             int cmp = k.shortcut_ok ? shortcut_compare<RULE, TWO_D>(SA, shortcut_weight<RULE>(A), SB, shortcut_weight<RULE>(B)) : 0;
             if (cmp == 0) {
                 // (codes that stand for the same numbers: an exact tie, the first candidate wins)
-                bool tie = e4m3_decode(s4) == 1.5f * e4m3_decode(s6) && (tie_violations(a0, b0) | tie_violations(a1, b1)) == 0;
+                bool tie = SA == SA && e4m3_decode(s4) == 1.5f * e4m3_decode(s6) && (tie_violations(a0, b0) | tie_violations(a1, b1)) == 0;
                 if (TWO_D) tie = row16_max(tie ? 0.0f : 1.0f) == 0.0f;
                 if (tie) cmp = -1;
             }

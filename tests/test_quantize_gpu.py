@@ -552,6 +552,27 @@ def test_if4_blocks_outside_the_exact_decision(shape, given, special):
     assert torch.equal(q.values, expect.values)
 
 
+@pytest.mark.parametrize("rule", ["mse", "mae", "static_6", "static_4"])
+@pytest.mark.parametrize("two_d", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_element_wise_fast_form_with_nan_elements(dtype, two_d, rule):
+    """Under a given maximum: a NaN gets the code 0 of the operation-by-operation form, the elements beside it the codes that
+    they have beside a zero (under the rules with one candidate), blocks without a NaN all of their bytes."""
+    x = make_input("randn", (33, 71), 93).to(dtype)  # (odd rows: the element-wise kernel for fp16 too)
+    x[:, 3::5] = torch.round(x[:, 3::5] * 2) / 2
+    nan, zero = x.clone(), x.clone()
+    nan[::17, 4::33], zero[::17, 4::33] = float("nan"), 0.0
+    cfg = fos.QuantizationConfig(scale_rule=rule, block_scale_2d=two_d, kwargs={"amax": torch.tensor(5.0, device="cuda")})
+    q, expect = fos.quantize(nan.cuda(), cfg), fos.quantize(zero.cuda(), cfg)
+    codes, other = (torch.stack([t.values & 15, t.values >> 4], -1).view(128, 128).cpu() for t in (q, expect))
+    assert bool((codes[:33, :71][nan.isnan()] == 0).all())
+    blocks = torch.nn.functional.pad(nan.isnan(), (0, 57, 0, 95)).view(128, 8, 16).any(-1)
+    if two_d:
+        blocks = blocks.view(8, 16, 8).any(1).repeat_interleave(16, 0)
+    keep = torch.ones_like(blocks) if rule.startswith("static") else ~blocks
+    assert torch.equal(codes.view(128, 8, 16)[keep], other.view(128, 8, 16)[keep])
+
+
 @pytest.mark.parametrize("shape", [(3, 17), (129, 301), (64, 1025)])
 def test_unaligned_bf16_rows(oracle, shape):
     for offset in (0, 1, 3):  # rows that start at any element of the buffer
