@@ -1254,6 +1254,9 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool if4) {
     return g;
 }
 
+int check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
+                      double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax);
+
 }  // namespace fos
 
 using namespace fos;
@@ -1284,7 +1287,8 @@ extern "C" size_t fos_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
                            const float *alpha, const float *amax_a, const float *amax_b, double denominator,
                            int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
-                           void *workspace, size_t workspace_bytes, fos_stream_t stream, bool if4 = false, int64_t rows = -1, int64_t depth = -1) {
+                           void *workspace, size_t workspace_bytes, fos_stream_t stream, bool if4 = false, int64_t rows = -1, int64_t depth = -1,
+                           bool check_only = false) {
     if (!A || !B || !sfA || !sfB || !D) return FOS_E_NULL_POINTER;
     if (((uintptr_t)d_amax & 3) || ((uintptr_t)bias & 7)) return FOS_E_BAD_ALIGNMENT;
     if (!alpha && (!amax_a || !amax_b)) return FOS_E_NULL_POINTER;
@@ -1309,6 +1313,7 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     if (M < 128 && g.kind != kPlanSkinny) return FOS_E_BAD_SHAPE;
     // the tile kernels store whole rows of their output tiles, 16 bytes per lane
     if (g.kind != kPlanSkinny && (((uintptr_t)D & 15) || (ldd % 8 != 0))) return FOS_E_BAD_ALIGNMENT;  // partial bands only through the weight-streaming kernel
+    if (check_only) return FOS_OK;
     if (g.splits > 1 && !(workspace && !((uintptr_t)workspace & 15) &&
                           workspace_bytes >= (size_t)g.splits * (size_t)M * (size_t)N * sizeof(float))) {
         // no (or too small a) workspace: run unsplit
@@ -1397,6 +1402,15 @@ extern "C" int fos_gemm_if4(const uint8_t *A, const uint8_t *B, const uint8_t *s
     if (!(denominator > 0.0) || M % 128 != 0) return FOS_E_BAD_SHAPE;
     return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, workspace,
                            workspace_bytes, stream, true);
+}
+
+// The argument checks of an NVFP4 fos_gemm_linear_rows, nothing launched: for a caller that launches something ahead of it.
+int fos::check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a,
+                           const float *amax_b, double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd,
+                           const void *bias, float *d_amax) {
+    if (!(denominator > 0.0)) return FOS_E_BAD_SHAPE;
+    return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, nullptr, 0,
+                           nullptr, false, -1, -1, true);
 }
 
 extern "C" int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,

@@ -509,6 +509,11 @@ extern "C" int fos_quantize(const void *x, int x_type, int64_t rows, int64_t col
                          amax, amax_is_input, workspace, workspace_bytes, stream, nullptr, 0);
 }
 
+namespace fos {
+int check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
+                      double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax);
+}
+
 // Scratch of fos_linear_nvfp4: codes, scales, tensor maximum, pass-1 partials and split-K partials, each from a
 // 256-byte boundary on.
 namespace {
@@ -550,7 +555,11 @@ extern "C" int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t
     if (scratch_bytes < at.total) return FOS_E_WORKSPACE;
     uint8_t *base = static_cast<uint8_t *>(scratch);
     float *amax = x_amax ? const_cast<float *>(x_amax) : reinterpret_cast<float *>(base + at.amax);
-    const int rc = quantize_impl(x, x_type, rows, cols, ld, FOS_DTYPE_NVFP4, rule, FOS_ROUND_NEAREST, 0, 0, 0, FOS_SF_TILED_128X4,
+    // (a call that the product refuses has written nothing, d_amax included)
+    int rc = check_gemm_linear(base + at.codes, W, base + at.sf, sfW, amax, w_amax, denominator, LinearScratch::gemm_rows(rows, cols), N,
+                               fos_padded_cols(cols), D, out_type, ldd, bias, d_amax);
+    if (rc != FOS_OK) return rc;
+    rc = quantize_impl(x, x_type, rows, cols, ld, FOS_DTYPE_NVFP4, rule, FOS_ROUND_NEAREST, 0, 0, 0, FOS_SF_TILED_128X4,
                                  base + at.codes, base + at.sf, amax, x_amax != nullptr, base + at.partials, at.gemm - at.partials, stream,
                                  nullptr, 0, nullptr, 0, d_amax);
     if (rc != FOS_OK) return rc;

@@ -103,6 +103,22 @@ def test_argument_checks_need_no_device(native):
     assert d(inter=0) == -3  # value x scale meets in fp16 or fp32 only
 
 
+def test_linear_layer_checks_all_arguments_before_it_launches(native):
+    """What the product refuses is refused before the quantize kernel, which clears the recorded maximum."""
+    L = native.lib()
+    buf = ctypes.create_string_buffer(1 << 17)
+    p = (ctypes.addressof(buf) + 255) & ~255
+    f = lambda **kw: L.fos_linear_nvfp4(  # noqa: E731
+        kw.get("x", p), 0, kw.get("rows", 129), 64, kw.get("ld", 64), 3, None, kw.get("W", p), p, kw.get("w_amax", p),
+        kw.get("den", 2.0), kw.get("N", 128), kw.get("D", p), kw.get("out", 0), kw.get("ldd", 128), kw.get("bias"), kw.get("d_amax", p),
+        p, kw.get("bytes", 1 << 16), None)
+    assert f(W=None) == f(D=None) == f(w_amax=None) == f(x=None) == -4
+    assert f(N=100) == f(ldd=64) == f(den=0.0) == f(rows=0) == f(ld=32) == -1
+    assert f(D=p + 2) == f(D=p + 8) == f(bias=p + 2) == f(d_amax=p + 1) == f(ldd=132) == -2
+    assert f(out=2) == -3
+    assert f(bytes=16) == -5
+
+
 @pytest.mark.parametrize("tile", ["1", "128", "129", "256"])
 def test_workspace_query_of_a_small_batch_on_forced_tiles(native, monkeypatch, tile):
     """Fewer rows than a tile has, with the weight-streaming kernels switched off: the query answers (the product itself
