@@ -307,9 +307,10 @@ Tensor gemm_nvfp4_amax(const Tensor &a, const Tensor &b, const Tensor &a_sf, con
                        bias.has_value() ? &*bias : nullptr, rows);
 }
 
-// A word for a recorded maximum: one of a block of 4096 per (device, stream), each handed out once, so that the block is
-// not given back, and the word not overwritten, while a reader on another stream may still be at work on a result whose
-// lifetime was extended without this word's.  Inside a capture a tensor of its own (the graph's private pool).
+// A word for a recorded maximum: one of a block of 4096 per (device, stream), each handed out once, so that no word is
+// overwritten while a reader may still be at work on it.  A block lives as long as one of its words is held; a reader on
+// another stream keeps it from reuse itself (the frontend's known_amax).  Inside a capture a tensor of its own (the graph's
+// private pool).
 Tensor amax_word(const Tensor &like, fos_stream_t stream) {
     const auto opts = like.options().dtype(at::kFloat);
     if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return at::empty({1}, opts);

@@ -99,15 +99,19 @@ def attach_known_amax(x: torch.Tensor, amax: torch.Tensor) -> torch.Tensor:
     version = _version_or_none(x)
     if version is not None:
         # (address and shape as well: a tag copied along with the object's attributes onto other storage is not believed)
-        setattr(x, _KNOWN_AMAX, (amax, version, x.data_ptr(), x.shape))
+        setattr(x, _KNOWN_AMAX, (amax, version, x.data_ptr(), x.shape, nat.current_stream(amax.device) if amax.is_cuda else None))
     return x
 
 
 def known_amax(x: torch.Tensor) -> torch.Tensor | None:
-    """The maximum recorded by ``attach_known_amax`` if ``x`` has not been written since."""
+    """The maximum recorded by ``attach_known_amax`` if ``x`` has not been written since.  On another stream than the one it
+    was attached on, its memory is kept from reuse until what this stream does with it is done: the caller looks
+    after ``x`` (``record_stream``), but does not see this word."""
     tag = getattr(x, _KNOWN_AMAX, None)
     if tag is None or tag[0].device != x.device or tag[1] != _version_or_none(x) or tag[2] != x.data_ptr() or tag[3] != x.shape:
         return None
+    if tag[4] is not None and tag[4] != nat.current_stream(x.device):
+        tag[0].record_stream(torch.cuda.current_stream(x.device))
     return tag[0]
 
 

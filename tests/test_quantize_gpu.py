@@ -573,6 +573,30 @@ def test_element_wise_fast_form_with_nan_elements(dtype, two_d, rule):
     assert torch.equal(codes.view(128, 8, 16)[keep], other.view(128, 8, 16)[keep])
 
 
+@pytest.mark.parametrize("pseudo", [False, True])
+def test_recorded_maximum_outlives_a_reader_on_another_stream(pseudo):
+    """The word is dropped, and its size allocated again, while the reader's stream is still busy: not the same memory."""
+    from fouroversix_amd.quantize import attach_known_amax
+
+    x = make_input("randn", (64, 256), 3).cuda()
+    word = x.abs().max().float().reshape(1) + torch.zeros(1, device="cuda")
+    address = word.data_ptr()
+    expect = fos.quantize(x)
+    attach_known_amax(x, word)
+    del word
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    x.record_stream(other)
+    with torch.cuda.stream(other):
+        torch.cuda._sleep(20_000_000)
+        q = fos.quantize(x, fos.QuantizationConfig(pseudo_quantize=pseudo))
+    del x
+    again = [torch.full((1,), 1e30, device="cuda") for _ in range(64)]
+    assert address not in [t.data_ptr() for t in again]
+    torch.cuda.synchronize()
+    assert torch.equal(q, fos.dequantize(expect)) if pseudo else torch.equal(q.values, expect.values)
+
+
 @pytest.mark.parametrize("shape", [(3, 17), (129, 301), (64, 1025)])
 def test_unaligned_bf16_rows(oracle, shape):
     for offset in (0, 1, 3):  # rows that start at any element of the buffer
