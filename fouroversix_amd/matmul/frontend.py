@@ -10,6 +10,7 @@ padded result is cropped to ``(M, N)``.
 
 from __future__ import annotations
 
+import threading
 from typing import Any
 
 import torch
@@ -202,17 +203,19 @@ def _unit_alpha(device: torch.device) -> torch.Tensor:
 # captured call gets a word of its own with its own fill, which replays with it.
 _AMAX_WORDS = 4096
 _AMAX_POOL: dict = {}
+_AMAX_LOCK = threading.Lock()
 
 
 def _fresh_amax_word(device: torch.device) -> torch.Tensor:
     if torch.cuda.is_current_stream_capturing():
         return torch.zeros(1, dtype=torch.float32, device=device)
     key = (device, nat.current_stream(device))
-    slot = _AMAX_POOL.get(key)
-    if slot is None or slot[1] == _AMAX_WORDS:
-        slot = _AMAX_POOL[key] = [torch.zeros(_AMAX_WORDS, dtype=torch.float32, device=device), 0]
-    word = slot[0][slot[1] : slot[1] + 1]
-    slot[1] += 1
+    with _AMAX_LOCK:  # (threads that share a stream)
+        slot = _AMAX_POOL.get(key)
+        if slot is None or slot[1] == _AMAX_WORDS:
+            slot = _AMAX_POOL[key] = [torch.zeros(_AMAX_WORDS, dtype=torch.float32, device=device), 0]
+        word = slot[0][slot[1] : slot[1] + 1]
+        slot[1] += 1
     return word
 
 

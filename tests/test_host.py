@@ -173,6 +173,41 @@ def test_reference_import_name_and_rht_matrix(oracle):
     assert torch.equal(plain[0].float(), torch.full((16,), 0.25)) and torch.equal(plain.float(), plain.float().T)
 
 
+def test_threads_on_one_stream_get_words_of_their_own(monkeypatch):
+    """Each recorded maximum has its own word, also where threads that share a stream take words at the same time (an
+    allocation in between gives the interpreter to another thread)."""
+    import threading
+    import time
+
+    from fouroversix_amd.matmul import frontend
+
+    monkeypatch.setattr(frontend.nat, "current_stream", lambda device: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(frontend, "_AMAX_POOL", {})
+    zeros = torch.zeros
+
+    def slow_zeros(*args, **kwargs):
+        time.sleep(0.05)
+        return zeros(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "zeros", slow_zeros)
+    words, start = [], threading.Barrier(4)
+
+    def take():
+        start.wait()
+        words.append(frontend._fresh_amax_word(torch.device("cpu")))
+
+    for _ in range(4096 - 2):  # the next block is due within the four threads' words
+        words.append(frontend._fresh_amax_word(torch.device("cpu")))
+    threads = [threading.Thread(target=take) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len({w.data_ptr() for w in words}) == len(words) == 4098
+    assert len(frontend._AMAX_POOL) == 1 and next(iter(frontend._AMAX_POOL.values()))[1] == 2
+
+
 def test_layers_without_gradients_keep_the_autograd_function_where_it_is_seen():
     """The direct forward pass is for plain calls: a functorch transform and forward-mode differentiation (on under
     no_grad as well) still meet the autograd function."""
