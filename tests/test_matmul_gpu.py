@@ -250,7 +250,11 @@ def test_layer_in_one_call_equals_quantize_and_matmul(tokens, inf, outf, dtype):
         model[0].quantize_weight_()
         wide = make_input("outlier", (max(tokens, 1), 2 * inf), 81).to(dtype).cuda()
         for x in (wide[:tokens, :inf].contiguous(), wide[:tokens, :inf], wide[:tokens, ::2]):
-            if tokens == 0:
+            if tokens == 0:  # (refused by either form, as the product of an NVFP4 tensor without rows is)
+                with torch.no_grad(), pytest.raises(RuntimeError):
+                    model(x)
+                with pytest.raises(RuntimeError):
+                    fos.quantized_matmul(x, model[0].quantized_weight(), emit_amax=True, bias=model[0].bias)
                 continue
             with torch.no_grad():
                 out = model(x)

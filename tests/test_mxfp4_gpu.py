@@ -180,15 +180,14 @@ def test_mxfp4_gemm(oracle, m, n, k, out_dtype):
 
 @pytest.mark.parametrize("k", [128, 256, 384, 1152, 4224])
 def test_mxfp4_gemm_kernels_agree_bitwise(monkeypatch, k):
-    """The big-tile kernel that loads operands straight into LDS (four stages), the
-    register-staged big-tile kernel and the small-tile kernel contract K in the same order
-    with the same matrix instruction: whole outputs are bit-identical.  K covers fewer steps
-    than stages, a partial last round of stages, and many rounds."""
+    """The kernel's three tiles (256 x 256, 128 x 256, 128 x 128; operands straight into LDS, four stages) contract K in
+    the same order with the same matrix instruction: whole outputs are bit-identical, and so is that of the tile
+    chosen by size.  K covers fewer steps than stages, a partial last round of stages, and many rounds."""
     m = n = 4096
     qa = fos.quantize(make_input("randn", (m, k), 21).cuda(), mx_config())
     qb = fos.quantize(make_input("outlier", (n, k), 22).cuda(), mx_config("static_4"))
     outs = []
-    for tile in (None, "256", "128"):
+    for tile in (None, "256", "129", "128"):
         if tile is None:
             monkeypatch.delenv("FOS_MX_TILE", raising=False)
         else:
@@ -196,7 +195,7 @@ def test_mxfp4_gemm_kernels_agree_bitwise(monkeypatch, k):
         outs.append(fos.quantized_matmul(qa, qb))
         torch.cuda.synchronize()
     assert not torch.isnan(outs[0].float()).any()
-    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert all(torch.equal(outs[0], out) for out in outs[1:])
 
 
 @pytest.mark.parametrize(("m", "n", "k"), [(128, 128, 128), (384, 384, 256), (256, 640, 1152), (640, 256, 640)])
