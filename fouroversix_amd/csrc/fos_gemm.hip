@@ -523,6 +523,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
     __syncthreads();  // every wavefront is done reading the A buffers
     uint8_t *epi = reinterpret_cast<uint8_t *>(lds) + wave * 32 * kEpiPitch;
     constexpr int kLanesPerRow = kRowBytes / 16, kRowsPerPass = 64 / kLanesPerRow;
+    const int real_rows = (int)(p.rows - m0 < BM ? p.rows - m0 : BM);  // (negative for a tile of padding)
     uint32_t umax = 0u;
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
@@ -543,7 +544,8 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
                     pack_outputs<OUT_BF16>(v, p.bias, n0 + wn * WN * 32 + nl, um);
             }
         }
-        if (um > umax && m0 + wm * WM * 32 + i * 32 + (lane & 31) < p.rows) umax = um;
+        um = wm * WM * 32 + i * 32 + (lane & 31) < real_rows ? um : 0u;
+        umax = um > umax ? um : umax;
         // (LDS operations of one wavefront complete in order: its own writes are visible to its reads)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();

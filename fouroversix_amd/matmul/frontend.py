@@ -167,13 +167,11 @@ def _if4_gemm_applies(input: QuantizedTensor, other: QuantizedTensor, out_dtype:
 
 
 def _fusable_bias(bias: torch.Tensor | None, dtype: torch.dtype, columns: int, device: torch.device) -> bool:
-    """Whether the GEMM's epilogue can add ``bias`` (``columns``: the weight's rows with their padding).  It reads the
-    memory of ``bias``: a sum that something differentiates or transforms stays a sum of torch's."""
+    """Whether the GEMM's epilogue can add ``bias`` (``columns``: the weight's rows with their padding), unless backward
+    is to see the sum."""
     return (
         bias is not None
-        and (type(bias) is torch.Tensor or type(bias) is torch.nn.Parameter)
         and not (bias.requires_grad and torch.is_grad_enabled())
-        and not seen_by_autograd_functions()
         and bias.dtype == dtype
         and bias.dim() == 1
         and bias.shape[0] == columns  # (no row padding of the weight between the bias and the product)
@@ -181,6 +179,12 @@ def _fusable_bias(bias: torch.Tensor | None, dtype: torch.dtype, columns: int, d
         and bias.is_contiguous()
         and bias.data_ptr() % 8 == 0
     )
+
+
+def _plain(bias: torch.Tensor | None) -> bool:
+    """Whether the memory of ``bias`` is all there is to it: a sum that something maps, traces or differentiates forward
+    stays a sum of torch's.  (A layer's call has asked that itself, or is inside an autograd function.)"""
+    return type(bias) in (torch.Tensor, torch.nn.Parameter) and not seen_by_autograd_functions()
 
 
 _UNIT_ALPHA: dict = {}
@@ -316,7 +320,7 @@ def quantized_matmul(
         and not torch.compiler.is_compiling()
     ):
         torch_dtype = torch.bfloat16 if out_dtype is DataType.bfloat16 else torch.float16
-        fused_bias = _fusable_bias(bias, torch_dtype, rb[0].shape[0], ra[6])
+        fused_bias = _plain(bias) and _fusable_bias(bias, torch_dtype, rb[0].shape[0], ra[6])
         d_amax = _fresh_amax_word(ra[6]) if emit_amax and (bias is None or fused_bias) else None
         m, n = input.original_shape[0], other.original_shape[0]
         out = ops.gemm_nvfp4_from_amax(
@@ -337,7 +341,7 @@ def quantized_matmul(
             # values as the dequantization defines them, the tensor maxima in the output scale
             device = input.values.device
             m, n = input.original_shape[0], other.original_shape[0]
-            fused_bias = _fusable_bias(bias, out_dtype.torch_dtype, other.values.shape[0], device)
+            fused_bias = _plain(bias) and _fusable_bias(bias, out_dtype.torch_dtype, other.values.shape[0], device)
             whole_rows = n == other.values.shape[0]
             d_amax = _fresh_amax_word(device) if emit_amax and whole_rows and (bias is None or fused_bias) else None
             out = ops.gemm_if4(

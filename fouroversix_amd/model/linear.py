@@ -22,7 +22,7 @@ import torch.nn as nn
 from fouroversix_amd.matmul import quantized_matmul
 from fouroversix_amd.matmul.frontend import nvfp4_linear
 from fouroversix_amd.quantize import QuantizedTensor, dequantize, quantize
-from fouroversix_amd.quantize.frontend import attach_known_amax, known_amax
+from fouroversix_amd.quantize.frontend import carry_known_amax
 from fouroversix_amd.utils import DataType, RoundStyle
 from fouroversix_amd.utils import seen_by_autograd_functions as _seen_by_autograd_functions
 
@@ -42,16 +42,15 @@ def fp4_linear(
     else:
         if isinstance(weight, torch.Tensor):
             weight = quantize(weight.data if isinstance(weight, nn.Parameter) else weight, config.get_weight_config())
-        flat = input.reshape(-1, input.shape[-1])
+        # (a parameter or another subclass becomes a plain view)
+        flat = input if type(input) is torch.Tensor and input.dim() == 2 else input.reshape(-1, input.shape[-1])
         if config.pseudo_quantize:
             out = torch.matmul(quantize(flat, config.get_activation_config()), weight.T)
             out = out.reshape(*input.shape[:-1], weight.shape[0])
         else:
             # (a maximum recorded on `input` by the layer that produced it survives the flattening:
             # a view shares the version counter)
-            amax_in = known_amax(input)
-            if amax_in is not None and flat is not input:
-                attach_known_amax(flat, amax_in)
+            carry_known_amax(input, flat)
             # (the bias goes into the GEMM's epilogue with the two roundings of `out + bias`; the recorded
             # maximum is then that of the sum)
             out2d = None
@@ -72,10 +71,10 @@ def fp4_linear(
                     emit_amax=config.emit_output_amax,
                     bias=bias,
                 )
+            if input.dim() == 2:
+                return out2d
             out = out2d.reshape(*input.shape[:-1], weight.original_shape[0])
-            amax_out = known_amax(out2d)
-            if amax_out is not None and out is not out2d:
-                attach_known_amax(out, amax_out)
+            carry_known_amax(out2d, out)
             return out
     if bias is not None:
         out = out + bias

@@ -82,6 +82,7 @@ def _quantize_meta(x: torch.Tensor, config: QuantizationConfig) -> QuantizedTens
 # Tensors made under ``torch.inference_mode()`` have no version counter: they are never tagged and
 # ``quantize`` finds their maximum itself.
 _KNOWN_AMAX = "_fos_known_amax"
+_raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 def _version_or_none(x: torch.Tensor) -> int | None:
@@ -93,24 +94,47 @@ def _version_or_none(x: torch.Tensor) -> int | None:
         return None
 
 
+def _stream_of(t: torch.Tensor) -> int | None:
+    """Handle of the current stream on the tensor's GPU, None for a tensor elsewhere."""
+    index = t.get_device()
+    return _raw_stream(index) if index >= 0 else None
+
+
 def attach_known_amax(x: torch.Tensor, amax: torch.Tensor) -> torch.Tensor:
     """Record ``amax`` (device f32[1] = max|x|) on ``x`` for a later ``quantize(x)``; without effect
     on tensors that have no version counter (inference tensors)."""
     version = _version_or_none(x)
     if version is not None:
         # (address and shape as well: a tag copied along with the object's attributes onto other storage is not believed)
-        setattr(x, _KNOWN_AMAX, (amax, version, x.data_ptr(), x.shape, nat.current_stream(amax.device) if amax.is_cuda else None))
+        setattr(x, _KNOWN_AMAX, (amax, version, x.data_ptr(), x.shape, _stream_of(amax)))
     return x
+
+
+def _standing_tag(x: torch.Tensor) -> tuple | None:
+    tag = getattr(x, _KNOWN_AMAX, None)
+    if tag is None or tag[0].device != x.device or tag[1] != _version_or_none(x) or tag[2] != x.data_ptr() or tag[3] != x.shape:
+        return None
+    return tag
+
+
+def carry_known_amax(x: torch.Tensor, view: torch.Tensor) -> None:
+    """The maximum recorded on ``x``, if it still holds, on ``view`` as well: another shape of all of ``x`` (a view shares
+    the version counter; a copy starts with its own)."""
+    tag = _standing_tag(x) if view is not x else None
+    if tag is not None:
+        version = _version_or_none(view)
+        if version is not None:
+            setattr(view, _KNOWN_AMAX, (tag[0], version, view.data_ptr(), view.shape, tag[4]))
 
 
 def known_amax(x: torch.Tensor) -> torch.Tensor | None:
     """The maximum recorded by ``attach_known_amax`` if ``x`` has not been written since.  On another stream than the one it
     was attached on, its memory is kept from reuse until what this stream does with it is done: the caller looks
     after ``x`` (``record_stream``), but does not see this word."""
-    tag = getattr(x, _KNOWN_AMAX, None)
-    if tag is None or tag[0].device != x.device or tag[1] != _version_or_none(x) or tag[2] != x.data_ptr() or tag[3] != x.shape:
+    tag = _standing_tag(x)
+    if tag is None:
         return None
-    if tag[4] is not None and tag[4] != nat.current_stream(x.device):
+    if tag[4] != _stream_of(tag[0]):
         tag[0].record_stream(torch.cuda.current_stream(x.device))
     return tag[0]
 

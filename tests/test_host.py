@@ -173,6 +173,22 @@ def test_reference_import_name_and_rht_matrix(oracle):
     assert torch.equal(plain[0].float(), torch.full((16,), 0.25)) and torch.equal(plain.float(), plain.float().T)
 
 
+def test_recorded_maximum_on_another_shape_of_the_tensor():
+    """carry_known_amax: on views and copies of all of a tensor, as long as the record stands."""
+    from fouroversix_amd.quantize.frontend import attach_known_amax, carry_known_amax, known_amax
+
+    x = torch.arange(24.0).view(2, 3, 4)
+    word = torch.tensor([23.0])
+    attach_known_amax(x, word)
+    flat, copy, late = x.reshape(-1, 4), x.reshape(-1, 4).clone(), x.reshape(-1)
+    carry_known_amax(x, flat)
+    carry_known_amax(x, copy)
+    assert known_amax(flat) is word and known_amax(copy) is word
+    x.add_(1)  # (seen through the view; the copy is what was measured)
+    carry_known_amax(x, late)
+    assert known_amax(x) is None and known_amax(flat) is None and known_amax(late) is None and known_amax(copy) is word
+
+
 def test_threads_on_one_stream_get_words_of_their_own(monkeypatch):
     """Each recorded maximum has its own word, also where threads that share a stream take words at the same time (an
     allocation in between gives the interpreter to another thread)."""
