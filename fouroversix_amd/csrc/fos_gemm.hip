@@ -1190,6 +1190,9 @@ constexpr int kTargetWorkgroups = 256;
 //   2560 x 4096 x 14336 (160) 275 -> 253, 6144 x 2560 x 2048 (240) 65 -> 55,
 //   1280 x 14336 x 4096 (280: a second generation nearly empty) 168 -> 141, 2560 x 8192 x 8192 (320) 322 -> 292.
 // A 256-wide tile over the edge of the output counts as a whole one.
+// IF4 operands, whose conversions take longer, are slower on all three by much the same factor: on 22 shapes with the tile
+// forced this choice is the fastest or within 1 % of it (2048 x 4096 x 4096 on 128 / 128 x 256 / 256: 115 / 97 / 116 us,
+// 1024 x 14336 x 4096 210 / 175 / 142, 512 x 4096 x 4096 67 / 77 / 110).
 static int pick_tile(int64_t M, int64_t N, int forced) {
     const int64_t m128 = M / 128, n128 = N / 128, m256 = (m128 + 1) / 2, n256 = (n128 + 1) / 2;
     if (forced == 128 || M < 128) return kPlanSmall;
@@ -1206,7 +1209,7 @@ static int pick_tile(int64_t M, int64_t N, int forced) {
 static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool if4) {
     GemmPlan g;
     g.narrow = g.wide = 0;
-    const int tile = tuning().gemm_tile;  // tuning / tests: 128 = small tile, 129 = 128 x 256 tile and 256 = 256 x 256 tile wherever M and N allow, 1 = no weight-streaming kernel
+    const int tile = tuning().gemm_tile;  // tuning / tests: 128 = small tile, 129 = 128 x 256 tile, 256 = 256 x 256 tile, 1 = no weight-streaming kernel
     int64_t steps, tiles;
     if (!if4 && M <= 128 && K % 256 == 0 && (tile == 0 || tile == 16 || tile == 32 || tile == 64)) {
         // one 128-row band: weight streaming, steps of 256 along K shared by 8 wavefronts

@@ -792,8 +792,8 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
                                      m0 + wm * WM * 32, n0 + wn * WN * 32, rows_a - wm * WM * 32, wn * WN * 32 < rows_b);
 }
 
-// Tile size: the cheapest by what its generations take (us at K = 4096; all scale with K).  136 and 102 KB of LDS:
-// 256 workgroups of the 256 x 256 and 128 x 256 tiles at a time; 70 KB: 512 of the 128 x 128 tile.  Measured with the
+// Tile size: the cheapest by what its generations take (us at K = 4096; all scale with K).  136 and 104 KiB of LDS:
+// 256 workgroups of the 256 x 256 and 128 x 256 tiles at a time; 72 KiB: 512 of the 128 x 128 tile.  Measured with the
 // tile forced on 60 shapes, 128 ... 8192 rows; against "256 x 256 from 256 tiles on, else 128 x 128 through registers":
 // 2048 x 4096 x 14336 (128 / 256 / 512 tiles) 82.7 -> 69.2 us on 128 x 256, 2560 x 4096 x 4096 35.7 -> 30.9 and
 // 1024 x 14336 x 4096 45.2 -> 35.3 on 256 x 256, 128 x 4096 x 14336 46.8 -> 39.1 on 128 x 128.

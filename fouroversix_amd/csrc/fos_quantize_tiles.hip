@@ -631,7 +631,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
 // measured best at 8192 x 8192 (43.9 us against 45.9 with 1024).  FOS_QUANT_GRID overrides for
 // tuning runs.  Few tiles: in four parts each, as the 1x16 kernel's.  Pass 2 of bf16, 4/6-MSE,
 // whole / in four (us): 128 x 4096 (8 tiles) 11.9 / 5.9, 2048 x 4096 (128) 12.2 / 7.9, 4096 x 4096 (256) 13.3 / 11.0,
-// 2048 x 14336 (448) 19.9 / 16.7.
+// 2048 x 14336 (448) 19.9 / 16.7, 4096 x 8192 (512) 21.5 / 20.0, 2560 x 16384 (640) 25.0 / 23.4, 4096 x 12288 (768) 26.3 / 26.7.
+// The line is the static rules', which have the least to do per tile: 448 tiles 13.7 / 13.6, 512 15.5 / 15.8, 768 21.6 / 23.5.
 template <int RULE, bool PSEUDO, bool IF4, bool SR>
 static void launch_tiles(QuantParams &p, hipStream_t s) {
     constexpr int64_t kSplitTiles = 448;

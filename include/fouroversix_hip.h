@@ -52,7 +52,7 @@ int fos_version(void);
 const char *fos_error_string(int code);
 
 /* Kernel-choice overrides for tuning runs and tests (FOS_GEMM_TILE, FOS_GEMM_SPLITK,
- * FOS_MX_TILE, FOS_QUANT_GRID, FOS_AMAX_GRID) are read from the environment once, at the
+ * FOS_MX_TILE, FOS_QUANT_GRID, FOS_QUANT_SPLIT, FOS_AMAX_GRID and the others of Tuning) are read from the environment once, at the
  * first call that needs them; this reads them again.  No counterpart in the reference. */
 void fos_tuning_reload(void);
 
@@ -256,7 +256,7 @@ int fos_gemm_nvfp4_amax(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, 
  * fos_gemm_nvfp4_amax that also folds max|D| -- of the values as stored, in the output type --
  * into d_amax[0] (device f32[1]): every workgroup does an unsigned atomic max on the value's
  * bits, so the caller sets d_amax[0] to 0 before the call (or leaves an earlier maximum there to
- * extend it).  A NaN among the outputs is recorded as NaN (its bits lie above every number's), as the
+ * extend it).  All M rows count (fos_gemm_linear_rows: the ones that are no padding).  A NaN among the outputs is recorded as NaN (its bits lie above every number's), as the
  * reference's `x.abs().max()` would report it.  The next layer's activation quantization can then take d_amax as its
  * `amax` input (amax_is_input = 1) and skip its own pass over D.  No counterpart in the
  * reference, whose quantize op always reduces its input
