@@ -120,7 +120,7 @@ def lib() -> ctypes.CDLL:
     L.fos_linear_nvfp4_scratch_bytes.restype = ctypes.c_size_t
     L.fos_gemm_if4.argtypes = [vp, vp, vp, vp, vp, vp, dbl, i64, i64, i64, vp, i32, i64, vp, vp, vp, ctypes.c_size_t, vp]
     L.fos_gemm_if4.restype = i32
-    L.fos_gemm_linear_rows.argtypes = [i32, vp, vp, vp, vp, vp, vp, dbl, i64, i64, i64, i64, i64, vp, i32, i64, vp, vp, vp, ctypes.c_size_t, vp]
+    L.fos_gemm_linear_rows.argtypes = [i32, vp, vp, vp, vp, vp, vp, dbl, i64, i64, i64, i64, i64, i64, vp, i32, i64, vp, vp, vp, ctypes.c_size_t, vp]
     L.fos_gemm_linear_rows.restype = i32
     L.fos_gemm_if4_workspace_bytes.argtypes = [i64, i64, i64]
     L.fos_gemm_if4_workspace_bytes.restype = ctypes.c_size_t

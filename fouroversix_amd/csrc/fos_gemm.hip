@@ -61,6 +61,7 @@ struct GemmParams {
     float *d_amax;             // optional: max|D| as stored is folded into d_amax[0] (unsigned atomic max on the bits)
     int64_t M, N, K, ldd;
     uint32_t k_tail;           // IF4: mask on the scale bytes of the last 64 codes of a row, 0 for blocks that are padding
+    int64_t cols;              // IF4: columns of D that exist, a multiple of 8 (the rest of N is padding that is not written)
     int64_t rows;              // rows 0 ... rows - 1 of D count for d_amax: padding rows hold the bias, not zeros
     int tiles_m, tiles_n;
     // split-K: workgroup (tile, blockIdx.y) contracts K steps [y * ksteps_per_split, ...) and
@@ -523,6 +524,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
     __syncthreads();  // every wavefront is done reading the A buffers
     uint8_t *epi = reinterpret_cast<uint8_t *>(lds) + wave * 32 * kEpiPitch;
     constexpr int kLanesPerRow = kRowBytes / 16, kRowsPerPass = 64 / kLanesPerRow;
+    const int real_cols = (int)(p.cols - n0 < BN ? p.cols - n0 : BN);
     const int real_rows = (int)(p.rows - m0 < BM ? p.rows - m0 : BM);  // (negative for a tile of padding)
     uint32_t umax = 0u;
 #pragma unroll
@@ -555,7 +557,8 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
             const int row = t * kRowsPerPass + lane / kLanesPerRow, c16 = lane % kLanesPerRow;
             const uint4 v = *reinterpret_cast<const uint4 *>(epi + row * kEpiPitch + c16 * 16);
             const int64_t m = m0 + wm * WM * 32 + i * 32 + row;
-            *reinterpret_cast<uint4 *>(D + m * p.ldd + n0 + wn * WN * 32 + c16 * 8) = v;
+            if (!IF4 || wn * WN * 32 + c16 * 8 < real_cols)
+                *reinterpret_cast<uint4 *>(D + m * p.ldd + n0 + wn * WN * 32 + c16 * 8) = v;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -1110,7 +1113,7 @@ __global__ __launch_bounds__(kReduceThreads) void gemm_reduce_kernel(const GemmP
     const float v[4] = {(alpha * s.x) * post, (alpha * s.y) * post, (alpha * s.z) * post, (alpha * s.w) * post};
     uint32_t um = 0u;
     const uint2 o = pack_outputs<OUT_BF16>(v, p.bias, n, um);
-    if (mine) *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.D) + m * p.ldd + n) = o;
+    if (mine && n < p.cols) *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.D) + m * p.ldd + n) = o;
     if (p.d_amax) fold_amax<OUT_BF16, kReduceThreads / 64>(p.d_amax, mine && m < p.rows ? um : 0u, words);
 }
 
@@ -1293,12 +1296,13 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
                            const float *alpha, const float *amax_a, const float *amax_b, double denominator,
                            int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
                            void *workspace, size_t workspace_bytes, fos_stream_t stream, bool if4 = false, int64_t rows = -1, int64_t depth = -1,
-                           bool check_only = false) {
+                           bool check_only = false, int64_t cols = -1) {
     if (!A || !B || !sfA || !sfB || !D) return FOS_E_NULL_POINTER;
     if (((uintptr_t)d_amax & 3) || ((uintptr_t)bias & 7)) return FOS_E_BAD_ALIGNMENT;
     if (!alpha && (!amax_a || !amax_b)) return FOS_E_NULL_POINTER;
     if (!alpha && (((uintptr_t)amax_a & 3) || ((uintptr_t)amax_b & 3))) return FOS_E_BAD_ALIGNMENT;
-    if (M <= 0 || N <= 0 || K <= 0 || (M > 128 && M % 128 != 0) || N % 128 != 0 || K % 64 != 0 || ldd < N) return FOS_E_BAD_SHAPE;
+    if (M <= 0 || N <= 0 || K <= 0 || (M > 128 && M % 128 != 0) || N % 128 != 0 || K % 64 != 0 || ldd < (cols < 0 ? N : cols))
+        return FOS_E_BAD_SHAPE;
     if (M < 128 && K % 256 != 0) return FOS_E_BAD_SHAPE;  // partial bands only through the weight-streaming kernel
     if (out_type != FOS_T_BF16 && out_type != FOS_T_F16) return FOS_E_UNSUPPORTED;
     if (((uintptr_t)A & 15) || ((uintptr_t)B & 15) || ((uintptr_t)sfA & 15) || ((uintptr_t)sfB & 15) ||
@@ -1311,6 +1315,7 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     p.two_factors = if4;
     p.M = M; p.N = N; p.K = K; p.ldd = ldd;
     p.rows = rows < 0 ? M : rows;
+    p.cols = cols < 0 ? N : cols;
     // (blocks of the last 64 codes that lie below `depth`: 8 bits of the mask each)
     p.k_tail = depth < 0 || K - depth < 16 ? 0xffffffffu : (1u << (8 * ((depth - (K - 64)) / 16))) - 1u;
     hipStream_t s = (hipStream_t)stream;
@@ -1420,13 +1425,14 @@ int fos::check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sf
 
 extern "C" int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
                                     const float *amax_a, const float *amax_b, double denominator,
-                                    int64_t M, int64_t rows, int64_t N, int64_t K, int64_t depth, void *D, int out_type, int64_t ldd, const void *bias,
-                                    float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream) {
+                                    int64_t M, int64_t rows, int64_t N, int64_t cols, int64_t K, int64_t depth, void *D, int out_type,
+                                    int64_t ldd, const void *bias, float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream) {
     if (!amax_a || !amax_b) return FOS_E_NULL_POINTER;
     if (dtype != FOS_DTYPE_NVFP4 && dtype != FOS_DTYPE_IF4) return FOS_E_UNSUPPORTED;
     const bool if4 = dtype == FOS_DTYPE_IF4;
     if (!(denominator > 0.0) || rows < 0 || rows > M || (if4 && M % 128 != 0)) return FOS_E_BAD_SHAPE;
+    if (cols > N || cols <= N - 128 || (cols != N && (!if4 || cols % 8 != 0 || bias || d_amax))) return FOS_E_BAD_SHAPE;
     if (depth > K || depth <= K - 64 || (depth != K && (!if4 || depth % 16 != 0))) return FOS_E_BAD_SHAPE;
     return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, workspace,
-                           workspace_bytes, stream, if4, rows, depth);
+                           workspace_bytes, stream, if4, rows, depth, false, cols);
 }

@@ -564,7 +564,7 @@ extern "C" int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t
                                  nullptr, 0, nullptr, 0, d_amax);
     if (rc != FOS_OK) return rc;
     return fos_gemm_linear_rows(FOS_DTYPE_NVFP4, base + at.codes, W, base + at.sf, sfW, amax, w_amax, denominator,
-                                LinearScratch::gemm_rows(rows, cols), rows, N, fos_padded_cols(cols), fos_padded_cols(cols), D, out_type, ldd,
+                                LinearScratch::gemm_rows(rows, cols), rows, N, N, fos_padded_cols(cols), fos_padded_cols(cols), D, out_type, ldd,
                                 bias, d_amax, at.total > at.gemm ? base + at.gemm : nullptr, at.total - at.gemm, stream);
 }
 

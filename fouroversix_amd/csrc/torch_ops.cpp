@@ -265,7 +265,7 @@ Tensor gemm_launch(const Tensor &a, const Tensor &b, const Tensor &a_sf, const T
                         "gemm: bias must be a contiguous [N] tensor of the output type");
         }
         rc = fos_gemm_linear_rows(FOS_DTYPE_NVFP4, A, B, sA, sB, amax_a->data_ptr<float>(), amax_b->data_ptr<float>(), denominator, m,
-                                  rows < 0 || rows > m ? m : rows, n, k, k, out.data_ptr(), out_type, n, bias ? bias->data_ptr() : nullptr,
+                                  rows < 0 || rows > m ? m : rows, n, n, k, k, out.data_ptr(), out_type, n, bias ? bias->data_ptr() : nullptr,
                                   d_amax ? d_amax->data_ptr<float>() : nullptr, wsp, ws_bytes, stream);
     } else {
         rc = fos_gemm_nvfp4_amax(A, B, sA, sB, amax_a->data_ptr<float>(), amax_b->data_ptr<float>(), denominator, m, n, k,
@@ -366,10 +366,10 @@ std::tuple<Tensor, c10::optional<Tensor>> linear_nvfp4(const Tensor &x, int64_t 
 }
 
 // IF4 x IF4 (row-major E4M3 scales), output scale from the two maxima, optional bias and recorded maximum (of the first
-// `rows` rows) as above.  `depth`: what of K is no padding (negative: all).
+// `rows` rows) as above.  `depth`, `cols`: what of K and of N is no padding (negative: all); the result has `cols` columns.
 Tensor gemm_if4(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tensor &b_sf, const Tensor &amax_a, const Tensor &amax_b,
                 double denominator, at::ScalarType out_dtype, const c10::optional<Tensor> &d_amax, const c10::optional<Tensor> &bias,
-                int64_t rows, int64_t depth) {
+                int64_t rows, int64_t depth, int64_t cols) {
     const Tensor *scales[2] = {&amax_a, &amax_b};
     const char *names[2] = {"amax_a", "amax_b"};
     check_gemm_operands(a, b, a_sf, b_sf, scales, 2, names);
@@ -382,14 +382,15 @@ Tensor gemm_if4(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tens
         TORCH_CHECK(bias->scalar_type() == out_dtype && bias->dim() == 1 && bias->size(0) == n && bias->is_contiguous(),
                     "gemm: bias must be a contiguous [N] tensor of the output type");
     }
-    Tensor out = at::empty({m, n}, a.options().dtype(out_dtype));
+    const int64_t width = cols < 0 ? n : cols;
+    Tensor out = at::empty({m, width}, a.options().dtype(out_dtype));
     const size_t ws_bytes = fos_gemm_if4_workspace_bytes(m, n, k);
     const DeviceGuard guard(a.device());
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
     check(fos_gemm_linear_rows(FOS_DTYPE_IF4, a.data_ptr<uint8_t>(), b.data_ptr<uint8_t>(), static_cast<const uint8_t *>(a_sf.data_ptr()),
                                static_cast<const uint8_t *>(b_sf.data_ptr()), amax_a.data_ptr<float>(), amax_b.data_ptr<float>(),
-                               denominator, m, rows < 0 || rows > m ? m : rows, n, k, depth < 0 ? k : depth, out.data_ptr(), out_type, n,
+                               denominator, m, rows < 0 || rows > m ? m : rows, n, width, k, depth < 0 ? k : depth, out.data_ptr(), out_type, width,
                                bias.has_value() ? bias->data_ptr() : nullptr, d_amax.has_value() ? d_amax->data_ptr<float>() : nullptr,
                                ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, current_stream(a)),
           "fouroversix::gemm_if4");

@@ -347,11 +347,11 @@ def quantized_matmul(
             out = ops.gemm_if4(
                 input.values, other.values, input.scale_factors, other.scale_factors, input.amax, other.amax,
                 dequantize_divisor(input) * dequantize_divisor(other), out_dtype.torch_dtype, d_amax,
-                bias.detach() if fused_bias else None, m, input.original_shape[1],
+                bias.detach() if fused_bias else None, m, input.original_shape[1], n if n % 8 == 0 and not whole_rows else -1,
             )
             # (contiguous, as the product of the dequantized matrices is; whatever the padding columns hold is not in
             # the maximum, which is recorded for whole rows only)
-            if not whole_rows:
+            if out.shape[1] != n:
                 out = out[:m, :n].contiguous()
             elif m != out.shape[0]:
                 out = out[:m]

@@ -126,10 +126,11 @@ def linear_nvfp4(x, selection_rule, x_amax, w, w_sf, w_amax, denominator, out_dt
     return _C.linear_nvfp4(x, selection_rule, x_amax, w, w_sf, w_amax, denominator, out_dtype, emit_amax, bias)
 
 
-def gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax=None, bias=None, rows=-1, depth=-1):
+def gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax=None, bias=None, rows=-1, depth=-1, cols=-1):
     """IF4 x IF4 product with the output scale of ``gemm_nvfp4_from_amax``; ``d_amax``, ``bias`` and ``rows`` as there.
-    ``depth`` (a multiple of 16; negative: all of K): where the padding of K begins, whose codes don't count."""
-    return _C.gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, bias, rows, depth)
+    ``depth`` (a multiple of 16; negative: all of K): where the padding of K begins, whose codes don't count.  ``cols``
+    (a multiple of 8, without ``d_amax`` and ``bias``; negative: all of N): columns of the result."""
+    return _C.gemm_if4(a, b, a_sf, b_sf, amax_a, amax_b, denominator, out_dtype, d_amax, bias, rows, depth, cols)
 
 
 def gemm_alpha_into(amax_a, amax_b, denominator, alpha):

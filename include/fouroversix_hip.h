@@ -312,12 +312,13 @@ size_t fos_gemm_if4_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * padding: all M rows of D are written, and d_amax receives the maximum over the first `rows` alone (with a bias the
  * padding rows of D are not zeros but hold the bias).  `depth`: K, or for IF4 the multiple of 16 above K - 64 from which
  * on the codes of a row are padding that does not count (a tensor whose ragged width was rotated holds values there,
- * which its dequantization leaves out).
+ * which its dequantization leaves out).  `cols`: N, or for IF4 without bias and d_amax the multiple of 8 above N - 128 from
+ * which on the columns of D don't exist (ldd >= cols).
  */
 int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
                          const float *amax_a, const float *amax_b, double denominator,
-                         int64_t M, int64_t rows, int64_t N, int64_t K, int64_t depth, void *D, int out_type, int64_t ldd, const void *bias,
-                         float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream);
+                         int64_t M, int64_t rows, int64_t N, int64_t cols, int64_t K, int64_t depth, void *D, int out_type, int64_t ldd,
+                         const void *bias, float *d_amax, void *workspace, size_t workspace_bytes, fos_stream_t stream);
 
 /*
  * alpha[0] = (amax_a[0] * amax_b[0]) * f32(1 / denominator), in fp32 on the device: the

@@ -119,6 +119,24 @@ def test_linear_layer_checks_all_arguments_before_it_launches(native):
     assert f(bytes=16) == -5
 
 
+def test_products_with_padding_check_their_arguments(native):
+    """What of M, N and K is padding: only what the kernels leave out, and nothing for NVFP4's N and K."""
+    L = native.lib()
+    buf = ctypes.create_string_buffer(1 << 16)
+    p = (ctypes.addressof(buf) + 255) & ~255
+    f = lambda dtype=1, out=9, **kw: L.fos_gemm_linear_rows(  # noqa: E731  (out type 9: refused after the sizes)
+        dtype, p, p, p, p, p, p, 2.0, 128, kw.get("rows", 128), 256, kw.get("cols", 256), 256, kw.get("depth", 256), p, out,
+        kw.get("ldd", 256), kw.get("bias"), kw.get("d_amax"), None, 0, None)
+    assert f(dtype=2) == -3
+    for dtype in (0, 1):
+        assert f(dtype) == f(dtype, rows=1) == -3
+        assert f(dtype, rows=-1) == f(dtype, rows=129) == f(dtype, cols=264) == f(dtype, depth=320) == f(dtype, ldd=128) == -1
+    assert f(depth=208) == f(cols=136, ldd=136) == -3
+    assert f(depth=200) == f(depth=192) == f(cols=130) == f(cols=128) == -1  # (a whole tile of padding does not exist)
+    assert f(cols=136, bias=p) == f(cols=136, d_amax=p) == f(cols=136, ldd=128) == -1
+    assert f(0, depth=240) == f(0, cols=136) == -1
+
+
 @pytest.mark.parametrize("tile", ["1", "128", "129", "256"])
 def test_workspace_query_of_a_small_batch_on_forced_tiles(native, monkeypatch, tile):
     """Fewer rows than a tile has, with the weight-streaming kernels switched off: the query answers (the product itself

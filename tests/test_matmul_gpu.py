@@ -485,14 +485,23 @@ def test_if4_weight_gradient_of_ragged_token_counts(tokens):
     assert bool(((out - exact).abs() <= 2.0 ** -8 * exact.abs() + 2 * tokens * 2.0 ** -24 * size).all())
 
 
-@pytest.mark.parametrize(("m", "n"), [(1, 300), (100, 256), (128, 144), (200, 300)])
-def test_if4_product_is_contiguous(m, n):
+@pytest.mark.parametrize("env", [{}, {"FOS_GEMM_TILE": "128"}, {"FOS_GEMM_TILE": "129"}, {"FOS_GEMM_TILE": "256"},
+                                 {"FOS_GEMM_TILE": "128", "FOS_GEMM_SPLITK": "2"}], ids=str)
+@pytest.mark.parametrize(("m", "n"), [(1, 300), (100, 256), (128, 144), (200, 300), (300, 8), (300, 264), (257, 392)])
+def test_if4_product_is_contiguous(monkeypatch, m, n, env):
     """Sizes that get padding: the result is the plain matrix that the dequantized form returns."""
+    for name, value in env.items():
+        monkeypatch.setenv(name, value)
     cfg = fos.QuantizationConfig(dtype="if4")
     qa, qb = (fos.quantize(make_input("randn", (rows, 128), rows).cuda(), cfg) for rows in (m, n))
     for bias in (None, torch.ones(n, device="cuda", dtype=torch.bfloat16)):
         out = fos.quantized_matmul(qa, qb, bias=bias, emit_amax=True)
         assert out.is_contiguous() and out.view(-1).shape == (m * n,)
+        a, b = (fos.dequantize(q, dtype=torch.float32).double() for q in (qa, qb))
+        exact, size = a @ b.T, a.abs() @ b.abs().T
+        if bias is not None:
+            exact, size = exact + 1, size + 1
+        assert bool(((out.double() - exact).abs() <= 2.0 ** -7 * (exact.abs() + 1) + 2 * 128 * 2.0 ** -24 * size).all())
 
 
 @pytest.mark.parametrize(("m", "n", "k"), [(0, 128, 256), (4, 0, 256), (4, 8, 0), (1, 2, (1 << 22) + 64)])
