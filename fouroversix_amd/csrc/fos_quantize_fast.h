@@ -46,8 +46,8 @@ FOS_DEVICE float amax_norm(float amax) {
     return u2f((254u - (e < 1u ? 1u : (e > 253u ? 253u : e))) << 23);
 }
 
-// Entry for scale byte `s` (0..127); built with the reference's operations.  Looked up with the byte's low seven bits: the
-// scale of a block with an infinite element is a NaN of either sign (under a given, finite tensor maximum).
+// Entry for scale byte `s` (0..127); built with the reference's operations.  The tables have it under byte s + 128 as well:
+// the scale of a block with an infinite element is a NaN of either sign (under a given, finite tensor maximum).
 template <bool PRODUCT_FORM = false>
 FOS_DEVICE FastLutEntry make_lut_entry(uint32_t s, const QuantConsts &k) {
     FastLutEntry e;
@@ -517,7 +517,7 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_fast(const Block16 &blk, const QuantCon
         // and sub-normal scales alike -- is exact on the fast path.
         // The stochastic style clamps to 6 in the reference as well, so only the zero scale
         // byte is left out there.
-        const FastLutEntry A = lut[s6 & 0x7fu];
+        const FastLutEntry A = lut[s6];
         if (SR ? s6 != 0u : (s6 >= 8u || (s6 != 0u && bmax * A.inv < 7.0f))) {
             if constexpr (SR) {
                 // scaled values, hardware stochastic rounding (one Philox call per block);
@@ -530,7 +530,7 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_fast(const Block16 &blk, const QuantCon
                 uint32_t a0, a1;
                 sr_pack16(xa, pA, a0, a1);
                 if (STATIC) return BlockOut{a0, a1, s6};
-                const FastLutEntry B = lut[s4 & 0x7fu];
+                const FastLutEntry B = lut[s4];
                 float xb[16];
 #pragma unroll
                 for (int i = 0; i < 16; ++i) xb[i] = scaled(x[i], B.inv);
@@ -580,7 +580,7 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_fast(const Block16 &blk, const QuantCon
                 });
                 return BlockOut{c0, c1, s6};
             }
-            const FastLutEntry B = lut[s4 & 0x7fu];
+            const FastLutEntry B = lut[s4];
             uint32_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;
             float SA = 0.0f, SB = 0.0f, GA = 0.0f, GB = 0.0f;  // (product form: SA / SB hold F)
             static_for<0, 8>([&](auto jc) {
@@ -678,7 +678,8 @@ __device__ __attribute__((noinline)) BlockOut generic_block_f32(Block16F blk, Qu
 }
 
 template <int RULE, bool TWO_D>
-FOS_DEVICE BlockOut quantize_block_nvfp4_f32(const Block16F &blk, const QuantConsts &k, float enc, bool in_range, const FastLutEntry *lut) {
+FOS_DEVICE BlockOut quantize_block_nvfp4_f32(const Block16F &blk, const QuantConsts &k, float enc, bool in_range, bool given,
+                                             const FastLutEntry *lut) {
     constexpr bool STATIC = RULE == FOS_RULE_STATIC_6 || RULE == FOS_RULE_STATIC_4;
     if (in_range) {
         const float *x = blk.x;
@@ -689,10 +690,10 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_f32(const Block16F &blk, const QuantCon
         const float s_hp6 = (bmax / k.qdiv) * enc, s_hp4 = s_hp6 * 1.5f;
         const uint32_t pk = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(s_hp6, s_hp4, 0, false);
         const uint32_t s6 = pk & 0xffu, s4 = (pk >> 8) & 0xffu;
-        const FastLutEntry A = lut[s6 & 0x7fu];
+        const FastLutEntry A = lut[s6];
         // (the exclusions of quantize_block_nvfp4_fast; a given maximum may be below the tensor's own: beyond 7 as well)
         if (s6 != 0u && bmax * A.inv < 7.0f) {
-            const FastLutEntry B = STATIC ? A : lut[s4 & 0x7fu];
+            const FastLutEntry B = STATIC ? A : lut[s4];
             uint32_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;
             float SA = 0.0f, SB = 0.0f;
             static_for<0, 8>([&](auto jc) {
@@ -711,7 +712,8 @@ FOS_DEVICE BlockOut quantize_block_nvfp4_f32(const Block16F &blk, const QuantCon
             });
             if (STATIC) {
                 // (a NaN element, under a given maximum, has its code from the operation-by-operation form; the rules that
-                // compare find it in SA)
+                // compare find it in SA.  The tensor's own maximum would be NaN, out of range)
+                if (!given) return BlockOut{a0, a1, s6};
                 float nan = 0.0f;
 #pragma unroll
                 for (int i = 0; i < 16; ++i) nan = __builtin_fmaf(x[i], 0.0f, nan);
@@ -797,7 +799,7 @@ FOS_DEVICE BlockOut quantize_block_if4_mse(const Block16 &blk, const QuantConsts
         if (TWO_D) bmax = row16_max(bmax);
         const float s_hp = div_const(bmax, k.qdiv, rq) * enc;
         const uint32_t s = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(s_hp, 0.0f, 0, false) & 0xffu;
-        const FastLutEntry A = lut[s & 0x7fu];
+        const FastLutEntry A = lut[s];
         // same exclusions as the NVFP4 path: the unclamped E2M1 value 8 and the zero scale byte
         if (s >= 8u || (s != 0u && bmax * A.inv < 7.0f)) {
             uint32_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
     __shared__ uint32_t red[4];
     // per wavefront: 4 scale tiles x 128 bytes (pseudo-quantize: the 2 KiB of a step's output instead)
     __shared__ __attribute__((aligned(16))) uint32_t sf_stage[4][PSEUDO ? 512 : 128];
-    __shared__ __attribute__((aligned(16))) FastLutEntry lut[128];
+    __shared__ __attribute__((aligned(16))) FastLutEntry lut[256];
     // undecided blocks are evaluated exactly one at a time, spread over the wavefront (whole tiles only: every
     // lane takes part); per wavefront 16 words of staging
     constexpr bool kSpread = FULL && !IF4 && (RULE == FOS_RULE_MSE || RULE == FOS_RULE_MAE);
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
     const bool deq_lut = PSEUDO && in_range && fast_c && (amax_bits & 0xffffu) == 0 && kt.errdiv == p.c;
     // the MSE decision in its product form (bf16 elements, round to nearest)
     constexpr bool kProduct = RULE == FOS_RULE_MSE && !SR && !IF4 && !F16;
-    if (threadIdx.x < 128) lut[threadIdx.x] = make_lut_entry<kProduct>(threadIdx.x, kt);
+    lut[threadIdx.x] = make_lut_entry<kProduct>(threadIdx.x & 127u, kt);
     __syncthreads();
 
     auto process = [&](const RowsTile &t, int g, const Block16 &b) __attribute__((always_inline)) {

@@ -27,7 +27,7 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(const QuantParams p)
     // MSE: 81.8 -> 42.5 us)
     constexpr bool TYPED = !FAST && !ALIGNED;
     constexpr bool FAST_F32 = TYPED && DT == FOS_DTYPE_NVFP4 && ROUND == FOS_ROUND_NEAREST && RULE != FOS_RULE_ABS_MAX;
-    __shared__ __attribute__((aligned(16))) FastLutEntry lut[FAST || FAST_F32 ? 128 : 1];
+    __shared__ __attribute__((aligned(16))) FastLutEntry lut[FAST || FAST_F32 ? 256 : 1];
 
     const uint32_t amax_bits = reduce_partials(p, red);
     QuantConsts k;
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(const QuantParams p)
     k.rerr = 1.0f / k.errdiv;
     k.fast_div = in_range && (k.errdiv == 1536.0f || k.errdiv == 2688.0f);
     if (FAST || FAST_F32) {
-        if (threadIdx.x < 128) lut[threadIdx.x] = make_lut_entry(threadIdx.x, k);
+        lut[threadIdx.x] = make_lut_entry(threadIdx.x & 127u, k);
         __syncthreads();
     }
 
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(const QuantParams p)
             codes[1] = o.c1;
             sbyte = o.s;
         } else if constexpr (FAST_F32) {
-            const BlockOut o = quantize_block_nvfp4_f32<RULE, TWO_D>(xf[it], k, enc_fast, in_range, lut);
+            const BlockOut o = quantize_block_nvfp4_f32<RULE, TWO_D>(xf[it], k, enc_fast, in_range, p.n_partials == 0, lut);
             codes[0] = o.c0;
             codes[1] = o.c1;
             sbyte = o.s;

@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
     constexpr bool ADAPTIVE = !STATIC;            // 4/6 with the MSE, MAE or abs-max rule
     constexpr bool MAXRULE = RULE == FOS_RULE_ABS_MAX;  // the error is the largest term, not the sum
     __shared__ uint32_t red[4];
-    __shared__ __attribute__((aligned(16))) FastLutEntry lut[128];
+    __shared__ __attribute__((aligned(16))) FastLutEntry lut[256];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // (scalar: what derives from it stays in scalar registers)
     const int par = wave & 1, half = wave >> 1;
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
     // (the 3-operation division is exact for these divisors only; the unbiased stochastic style rescales them)
     const bool fast_c = p.c == 1536.0f || p.c == 1792.0f || p.c == 2688.0f;
     const bool deq_lut = PSEUDO && in_range && fast_c && (amax_bits & 0xffffu) == 0 && kt.errdiv == p.c;
-    if (threadIdx.x < 128) lut[threadIdx.x] = make_lut_entry(threadIdx.x, kt);
+    lut[threadIdx.x] = make_lut_entry(threadIdx.x & 127u, kt);
     __syncthreads();
 
     // one quantised block (row `rstep` rows below the share's first, + li) to memory
@@ -512,9 +512,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
             const float s_hp4 = s_hp6 * 1.5f;
             const uint32_t pk = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(s_hp6, s_hp4, 0, false);
             const uint32_t s6 = pk & 0xffu, s4 = (pk >> 8) & 0xffu;
-            const FastLutEntry A = lut[s6 & 0x7fu];
+            const FastLutEntry A = lut[s6];
             FastLutEntry B = A;
-            if (ADAPTIVE && !IF4) B = lut[s4 & 0x7fu];
+            if (ADAPTIVE && !IF4) B = lut[s4];
             // the hardware convert saturates at 6 where the reference's unclamped rounding gives 8:
             // that needs a sub-normal scale byte rounded down by more than 7/6; a zero scale byte
             // of a non-zero tile has no scaled domain.  (The stochastic styles clamp to 6 in the
