@@ -38,207 +38,12 @@
 #include <type_traits>
 
 #include "fos_device.h"
+#include "fos_gemm_common.h"
 #include "fos_gemm_tiles.h"
 #include "fos_tuning.h"
 #include "fouroversix_hip.h"
 
 namespace fos {
-
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
-
-struct GemmParams {
-    const uint8_t *A, *B;      // [M, K/2], [N, K/2]
-    const uint8_t *sfA, *sfB;  // 128x4-tiled E4M3 bytes
-    const float *alpha;        // output scale on the device, or null: (amax_a * amax_b) * inv_den
-    const float *amax_a, *amax_b;
-    float inv_den;
-    int two_factors;           // an output scale outside fp32's normal range is applied in two factors (load_alpha)
-    void *D;
-    const void *bias;          // optional: N values of the output type, added to the rounded product and rounded again
-    float *d_amax;             // optional: max|D| as stored is folded into d_amax[0] (unsigned atomic max on the bits)
-    int64_t M, N, K, ldd;
-    uint32_t k_tail;           // IF4: mask on the scale bytes of the last 64 codes of a row, 0 for blocks that are padding
-    int64_t cols;              // IF4: columns of D that exist, a multiple of 8 (the rest of N is padding that is not written)
-    int64_t rows;              // rows 0 ... rows - 1 of D count for d_amax: padding rows hold the bias, not zeros
-    int tiles_m, tiles_n;
-    // split-K: workgroup (tile, blockIdx.y) contracts K steps [y * ksteps_per_split, ...) and
-    // writes its FP32 partial tile to partials[y][M][N]; splits == 1 writes D directly
-    float *partials;
-    int splits, ksteps_per_split;
-};
-
-// Output scale: read from the device, or formed from the two tensor maxima with the
-// arithmetic of gemm_alpha_kernel (product, then times the fp32 reciprocal of the divisor).
-// `post`: with two_factors, what is left to multiply alpha * acc with (1 otherwise).  Maxima whose product, divided by
-// the denominator, would be a sub-normal number with a few bits are multiplied 2^64 times too large; finite maxima
-// whose product overflows, 2^64 times too small (with an infinite scale a sum of zero would become NaN and a small
-// one infinite).  What still overflows then is a scale of 2^192 or more: any sum but zero, 2^-20 at least, is infinite
-// with the largest number in its place too.
-FOS_DEVICE float load_alpha(const GemmParams &p, float &post) {
-    constexpr float kMax = 0x1.fffffep127f;
-    post = 1.0f;
-    if (p.alpha) return *p.alpha;
-    const float a = *p.amax_a, b = *p.amax_b;
-    if (p.two_factors && a * b < 0x1p-90f) {
-        post = 0x1p-64f;
-        return ((fminf(a, b) * 0x1p64f) * fmaxf(a, b)) * p.inv_den;
-    }
-    if (p.two_factors && a * b > kMax && a <= kMax && b <= kMax) {
-        post = 0x1p64f;
-        return fminf(((fmaxf(a, b) * 0x1p-64f) * fminf(a, b)) * p.inv_den, kMax);
-    }
-    return (a * b) * p.inv_den;
-}
-
-// One value of the result as stored: alpha * acc rounded to the output type (16 bits returned).
-template <bool OUT_BF16>
-FOS_DEVICE uint32_t round_out(float v) {
-    if (OUT_BF16) {
-        uint32_t u = f2u(v);
-        u += 0x7fffu + ((u >> 16) & 1u);
-        return u >> 16;
-    }
-    // (v is a product already rounded to fp32 -- the reference's epilogue multiplies in fp32, then converts -- and
-    // must stay one: left to itself the compiler folds the multiplication into the conversion, v_fma_mixlo_f16,
-    // which rounds the exact product once and differs from the two roundings in one output in 10^5)
-    asm("" : "+v"(v));
-    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v);
-}
-template <bool OUT_BF16>
-FOS_DEVICE float widen_out(uint32_t bits) {
-    if (OUT_BF16) return u2f(bits << 16);
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
-}
-
-// Four consecutive outputs (columns n .. n + 3, n % 4 == 0) from their scaled accumulators: rounded to the output
-// type, and with a bias rounded, added to bias[n ..] in fp32 and rounded again -- the two roundings of the
-// reference's `out + bias` on the GEMM's result (src/fouroversix/model/modules/linear.py:83-92).  The magnitude
-// bits of what goes into the last rounding are folded into `umax` as unsigned integers, which order finite
-// values, infinity and NaN (largest) alike: a NaN in the output ends up as the recorded maximum, as it does
-// in the reference's x.abs().max().
-template <bool OUT_BF16>
-FOS_DEVICE uint32_t finish_output(float f, bool with_bias, uint32_t bias16, uint32_t &umax) {
-    if (with_bias) f = widen_out<OUT_BF16>(round_out<OUT_BF16>(f)) + widen_out<OUT_BF16>(bias16);
-    const uint32_t mag = f2u(f) & 0x7fffffffu;
-    umax = mag > umax ? mag : umax;
-    return round_out<OUT_BF16>(f);
-}
-template <bool OUT_BF16>
-FOS_DEVICE uint2 pack_outputs(const float *v, const void *bias, int64_t n, uint32_t &umax) {
-    uint2 bw = make_uint2(0u, 0u);
-    if (bias) bw = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(bias) + n);
-    const uint32_t o0 = finish_output<OUT_BF16>(v[0], bias != nullptr, bw.x & 0xffffu, umax);
-    const uint32_t o1 = finish_output<OUT_BF16>(v[1], bias != nullptr, bw.x >> 16, umax);
-    const uint32_t o2 = finish_output<OUT_BF16>(v[2], bias != nullptr, bw.y & 0xffffu, umax);
-    const uint32_t o3 = finish_output<OUT_BF16>(v[3], bias != nullptr, bw.y >> 16, umax);
-    return make_uint2(o0 | (o1 << 16), o2 | (o3 << 16));
-}
-// ... two consecutive outputs (n % 2 == 0)
-template <bool OUT_BF16>
-FOS_DEVICE uint32_t pack_outputs2(float v0, float v1, const void *bias, int64_t n, uint32_t &umax) {
-    uint32_t bw = 0u;
-    if (bias) bw = *reinterpret_cast<const uint32_t *>(static_cast<const uint16_t *>(bias) + n);
-    const uint32_t o0 = finish_output<OUT_BF16>(v0, bias != nullptr, bw & 0xffffu, umax);
-    const uint32_t o1 = finish_output<OUT_BF16>(v1, bias != nullptr, bw >> 16, umax);
-    return o0 | (o1 << 16);
-}
-
-// max|D| for the caller that quantizes D next: `umax` holds the magnitude bits of the largest value this
-// lane stored, before its rounding to the output type (0 for a lane that stored nothing).  Rounding is
-// monotonic, so the rounded maximum is the maximum of the rounded values.  At most one vector atomic per
-// workgroup on the unsigned image of the value (non-negative floats order like their bits, NaN above all);
-// every lane of the WAVES wavefronts must call it.  `words`: WAVES words of LDS nobody else uses any more.
-//
-// The atomics of a launch all go to one address and are served one after the other, about 12 ns each:
-// bound by that chain, not by the reduction.  Workgroups of one generation end together, so that almost
-// all of them find a smaller maximum in the word: with one atomic per wavefront a 2048 x 4096 x 4096 product
-// took 75 us against 64 without the maximum (1024 wavefronts), and the reduction of a 128 x 4096 output's two partials
-// 25 us (2048).  One per workgroup after a maximum in LDS: whole linear layers, quantization of the activation
-// included, 128 x 14336 -> 4096 53.6 -> 39.9 us and 2048 x 4096 -> 4096 79.4 -> 76.2 us.
-template <bool OUT_BF16, int WAVES>
-FOS_DEVICE void fold_amax(float *d_amax, uint32_t umax, uint32_t *words) {
-    uint32_t r;
-    if (umax > 0x7f800000u) r = 0x7fc00000u;
-    else r = f2u(widen_out<OUT_BF16>(round_out<OUT_BF16>(u2f(umax))));
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const uint32_t other = (uint32_t)__shfl_xor((int)r, off);
-        r = other > r ? other : r;
-    }
-    if constexpr (WAVES > 1) {
-        if ((threadIdx.x & 63) == 0) words[threadIdx.x >> 6] = r;
-        __syncthreads();
-        if (threadIdx.x < 64) {
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) r = words[w] > r ? words[w] : r;
-        }
-    }
-    // (a workgroup first looks whether its value would change anything: a late one's seldom does)
-    if (threadIdx.x == 0) {
-        unsigned int *word = reinterpret_cast<unsigned int *>(d_amax);
-        if (r > __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(word, r);
-    }
-}
-
-// The two E4M3 bytes in the low 16 bits of `w` -> fp16 pair {s0, s1} (one hardware
-// convert; exact, sub-normals included -- checked against the OCP decode of all 256 bytes).
-FOS_DEVICE half2_t e4m3x2_to_half2(uint32_t w) {
-    return __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, false);
-}
-
-// 8 packed codes (one 32-bit word) times a block scale -> 8 fp16 in k order.
-FOS_DEVICE half8_t dequant8(uint32_t word, half2_t s) {
-    half2_t p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 0) * s;
-    half2_t p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 1) * s;
-    half2_t p2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 2) * s;
-    half2_t p3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 3) * s;
-    half8_t r = {p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
-    return r;
-}
-
-// 8 packed IF4 codes times their block scale -> 8 fp16 in k order.  A block holds E2M1 codes or (`integer`) two's
-// complement integers q with the value RN16(6/7 q), and the product with the scale is rounded to fp16: the
-// numbers the dequantization of the format is defined by (src/fouroversix/quantize/backend.py:89-160).
-// Blocks differ from lane to lane, so both decodings are formed and one is selected: 34 instructions a word
-// against 8 for E2M1 alone, and what bounds the product (2048 x 4096 x 4096 99 us, NVFP4 61;
-// two dequantize kernels, a library fp32 product and the conversion of its result took 570).  Integers: q + 8 = nibble ^ 8 is a byte 0 .. 15, which E4M3 reads as (q + 8) / 512 (the
-// sub-normals run on into the first normal binade); 6/7 q is then formed from a two-part constant, equal to the rounded
-// product for all 16 integers.
-FOS_DEVICE half8_t dequant8_if4(uint32_t word, half2_t s, bool integer) {
-    const uint32_t u = word ^ 0x88888888u, even = u & 0x0f0f0f0fu, odd = (u >> 4) & 0x0f0f0f0fu;
-    const uint32_t pairs[2] = {__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u)};
-    constexpr _Float16 hi = (_Float16)(6.0 / 7.0), lo = (_Float16)(6.0 / 7.0 - (double)hi);
-    const half2_t k512 = {(_Float16)512.0f, (_Float16)512.0f}, m8 = {(_Float16)-8.0f, (_Float16)-8.0f}, hi2 = {hi, hi}, lo2 = {lo, lo};
-    auto sevenths = [&](half2_t x) {
-        const half2_t q = __builtin_elementwise_fma(x, k512, m8);
-        return __builtin_elementwise_fma(q, hi2, q * lo2);
-    };
-    auto pick = [&](half2_t i, half2_t f) {
-        return __builtin_bit_cast(half2_t, integer ? __builtin_bit_cast(uint32_t, i) : __builtin_bit_cast(uint32_t, f)) * s;
-    };
-    const half2_t p0 = pick(sevenths(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pairs[0], 1.0f, false)),
-                            __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 0));
-    const half2_t p1 = pick(sevenths(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pairs[0], 1.0f, true)),
-                            __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 1));
-    const half2_t p2 = pick(sevenths(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pairs[1], 1.0f, false)),
-                            __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 2));
-    const half2_t p3 = pick(sevenths(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pairs[1], 1.0f, true)),
-                            __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, 3));
-    half8_t r = {p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
-    return r;
-}
-
-// One word of block `blk` (0, 1) of the two whose scale bytes are the low 16 bits of `two`.
-template <bool IF4>
-FOS_DEVICE half8_t dequant_word(uint32_t word, uint32_t two, int blk) {
-    const half2_t s2 = e4m3x2_to_half2(IF4 ? two & 0x7f7fu : two);
-    const half2_t s = blk ? __builtin_shufflevector(s2, s2, 1, 1) : __builtin_shufflevector(s2, s2, 0, 0);
-    if constexpr (IF4) return dequant8_if4(word, s, (two & (blk ? 0x8000u : 0x80u)) != 0);
-    else return dequant8(word, s);
-}
 
 constexpr int BK = 64;
 constexpr int kPitch = BK + 8;  // halfs per LDS row (144 bytes: conflict-free 128-bit accesses)
@@ -265,8 +70,6 @@ struct Staged {
 // is fed from the B matrix (rows n) and the "B" operand from the A matrix (rows m), so
 // that a lane's four consecutive accumulator registers are four consecutive n of one
 // output row and can be stored as 8 bytes.
-enum { kOutF16 = 0, kOutBF16 = 1, kOutPartial = 2 };
-
 // QUARTER (4 * BM == threads): every thread stages a quarter row of A (16 codes) instead of the first 2 * BM threads
 // half a row each, so that all wavefronts carry the same conversion work.
 // IF4: operands in the IF4 format, whose scale bytes lie row-major (K / 16 a row) with bit 7 marking integer blocks,
@@ -548,7 +351,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void gemm_nvfp4_kernel(const
             }
         }
         um = wm * WM * 32 + i * 32 + (lane & 31) < real_rows ? um : 0u;
-        umax = um > umax ? um : umax;
+        umax = max_pairs(umax, um);
         // (LDS operations of one wavefront complete in order: its own writes are visible to its reads)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -909,7 +712,7 @@ __global__ __launch_bounds__(64 * skinny_waves(WN), (WN == 2 && MT == 2) ? 2 : 1
                 *reinterpret_cast<uint2 *>(D + (int64_t)m * p.ldd + n) = pack_outputs<OUT == kOutBF16>(v, p.bias, n, um);
             }
         }
-        if (um > umax && m < p.rows) umax = um;
+        if (m < p.rows) umax = max_pairs(umax, um);
     }
     if (OUT != kOutPartial && p.d_amax) {
         __syncthreads();  // every wavefront has summed its share of the slots
@@ -1084,7 +887,7 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams
         uint32_t um = 0u;
         const uint2 o = pack_outputs<OUT == kOutBF16>(v, p.bias, n_out + 32 * b, um);
         if (row_ok) {
-            if (um > umax && c < p.rows) umax = um;
+            if (c < p.rows) umax = max_pairs(umax, um);
             *reinterpret_cast<uint2 *>(D + (int64_t)c * p.ldd + n_out + 32 * b) = o;
         }
     }
