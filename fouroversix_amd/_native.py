@@ -50,6 +50,7 @@ EXPORTS = (
     "fos_gemm_alpha",
     "fos_padded_cols_for",
     "fos_gemm_workspace_bytes",
+    "fos_gemm_scratch_bytes",
     "fos_dequantize",
 )
 
@@ -132,6 +133,8 @@ def lib() -> ctypes.CDLL:
     L.fos_padded_cols_for.restype = i64
     L.fos_gemm_workspace_bytes.argtypes = [i64, i64, i64]
     L.fos_gemm_workspace_bytes.restype = ctypes.c_size_t
+    L.fos_gemm_scratch_bytes.argtypes = [i32, i64, i64, i64]
+    L.fos_gemm_scratch_bytes.restype = ctypes.c_size_t
     L.fos_dequantize.argtypes = [vp, vp, vp, i32, i32, dbl, i64, i64, i64, i64, vp, i32, i64, i32, vp]
     L.fos_dequantize.restype = i32
     _lib = L

@@ -39,6 +39,7 @@
 
 #include "fos_device.h"
 #include "fos_gemm_common.h"
+#include "fos_gemm_half.h"
 #include "fos_gemm_tiles.h"
 #include "fos_tuning.h"
 #include "fouroversix_hip.h"
@@ -1000,17 +1001,23 @@ constexpr int kTargetWorkgroups = 256;
 // IF4 operands, whose conversions take longer, are slower on all three by much the same factor: on 22 shapes with the tile
 // forced this choice is the fastest or within 1 % of it (2048 x 4096 x 4096 on 128 / 128 x 256 / 256: 115 / 97 / 116 us,
 // 1024 x 14336 x 4096 210 / 175 / 142, 512 x 4096 x 4096 67 / 77 / 110).
-static int pick_tile(int64_t M, int64_t N, int forced) {
+static float tile_cost(int64_t M, int64_t N, int *kind) {
     const int64_t m128 = M / 128, n128 = N / 128, m256 = (m128 + 1) / 2, n256 = (n128 + 1) / 2;
-    if (forced == 128 || M < 128) return kPlanSmall;
-    if (forced == 129) return kPlanWide;
-    if (forced == 256) return kPlanBig;
     static const float big[8] = {69, 69, 70, 75, 79, 86, 94, 104}, wide[8] = {42, 43, 43, 44, 46, 49.5f, 54, 59},
                        small[8] = {24, 34, 36.5f, 38.5f, 53, 56, 60, 64.5f};
     const float cost_big = tiles_cost(m256 * n256, 256, 92, big), cost_wide = tiles_cost(m128 * n256, 256, 56, wide),
                 cost_small = tiles_cost(m128 * n128, 512, 59, small);
-    if (cost_big <= cost_wide && cost_big <= cost_small) return kPlanBig;
-    return cost_wide < cost_small ? kPlanWide : kPlanSmall;
+    const bool is_big = cost_big <= cost_wide && cost_big <= cost_small;
+    if (kind) *kind = is_big ? kPlanBig : cost_wide < cost_small ? kPlanWide : kPlanSmall;
+    return is_big ? cost_big : cost_wide < cost_small ? cost_wide : cost_small;
+}
+static int pick_tile(int64_t M, int64_t N, int forced) {
+    if (forced == 128 || M < 128) return kPlanSmall;
+    if (forced == 129) return kPlanWide;
+    if (forced == 256) return kPlanBig;
+    int kind;
+    tile_cost(M, N, &kind);
+    return kind;
 }
 
 static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool if4) {
@@ -1066,8 +1073,65 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool if4) {
     return g;
 }
 
-int check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
-                      double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax);
+// The product with A converted ahead into fragments (fos_gemm_half.hip), for callers that lend the scratch for them: its
+// tile (0: the kernels above are faster) and split of K.
+struct HalfPlan {
+    int tile = 0, splits = 1, chunks_per_split = 0;
+    size_t partials = 0, bytes = 0;  // scratch: fragments, then from `partials` on the FP32 partials
+};
+
+// Time of `tiles` output tiles (us at K = 4096, without what a launch takes at any K): 256 workgroups of the 256 x 256 tile
+// run at a time, 512 of the others.  Measured with the fragments given, 128 ... 8192 rows, N = 1024 ... 14336, K = 1024 ... 14336.
+static float half_cost(int tile, int64_t tiles, float k) {
+    static const float big[8] = {65, 66, 67, 70, 71.5f, 75.5f, 79.5f, 86}, wide[8] = {42, 43.5f, 46, 50, 77, 79, 83, 89},
+                       small[8] = {28.5f, 29, 30, 32, 43, 45.5f, 48, 52};
+    if (tile == kHalf256) return k * tiles_cost(tiles, 256, 86, big);
+    if (tile == kHalfWide) return k * tiles_cost(tiles, 512, 87, wide);
+    return k * tiles_cost(tiles, 512, 50, small);
+}
+
+// `expand`: the fragments have to be formed from codes and scales first (a layer's quantize kernel writes them instead, at
+// little more than it takes to write the codes).  With the fragments given the product is the faster one from 256 rows on,
+// on all but a few of 400 shapes, which tie: 1024 x 14336 x 4096 97 -> 83 us, 8192 x 4096 x 4096 207 -> 178,
+// 6144 x 4096 x 4096 (384 tiles of 256 x 256) 180 -> 138, 2048 x 1024 x 4096 36 -> 28 in two splits, 1024 x 1024 x 14336
+// 49 -> 44 in four.  With the pass in front it has to make up for 4 us and 0.32 us per 2^20 elements of A: that
+// leaves the larger products.
+static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand) {
+    HalfPlan h;
+    const int forced = tuning().gemm_tile;  // tuning / tests: 1000 + tile; another kernel's tile excludes this one
+    if (M < 128 || M % 128 || N % 128 || K % 64 || K > (1 << 20) || if4 || (forced && forced <= 1000) || (!forced && M < 256)) return h;
+    if (fragment_bytes(M, K) > ((size_t)8 << 30)) return h;  // (a call with an operand that large keeps to the smaller workspace)
+    const int64_t chunks = (K + 127) / 128, m128 = M / 128, n128 = N / 128, m256 = (m128 + 1) / 2, n256 = (n128 + 1) / 2;
+    const int forced_splits = tuning().gemm_splitk;
+    int64_t splits = 1;
+    if (forced) {
+        h.tile = forced - 1000;
+        splits = forced_splits > 0 ? forced_splits : 1;
+    } else {
+        float best = 3e38f;
+        for (int tile = kHalf256; tile <= kHalfSmall; ++tile) {
+            const int64_t tiles = tile == kHalf256 ? m256 * n256 : tile == kHalfWide ? m128 * n256 : m128 * n128;
+            for (int s = 1; s <= 16; s = s < 4 ? s + 1 : s * 2) {
+                if (s > 1 && (chunks < 2 * s || tiles > 512)) break;
+                if (forced_splits && s != forced_splits) continue;
+                // (a split's partials are written and read again by a kernel of their own)
+                const float cost = half_cost(tile, tiles * s, (float)((chunks + s - 1) / s) / 32) + (s > 1 ? 5.5f + 0.25e-6f * 4 * s * M * N : 0.0f);
+                if (cost < best) best = cost, h.tile = tile, splits = s;
+            }
+        }
+        if (expand && h.tile) {
+            const GemmPlan g = plan_gemm(M, N, K, false);
+            if (g.splits > 1 || best + 5 + 4 + 0.32e-6f * M * K > tile_cost(M, N, nullptr) * (float)K / 4096) h.tile = 0;
+        }
+        if (!h.tile) return h;
+    }
+    if (splits > chunks) splits = chunks;
+    h.chunks_per_split = (int)((chunks + splits - 1) / splits);
+    h.splits = (int)((chunks + h.chunks_per_split - 1) / h.chunks_per_split);
+    h.partials = fragment_bytes(M, K);
+    h.bytes = h.partials + (h.splits > 1 ? (size_t)h.splits * (size_t)M * (size_t)N * sizeof(float) : 0);
+    return h;
+}
 
 }  // namespace fos
 
@@ -1096,11 +1160,15 @@ extern "C" size_t fos_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     return g.splits > 1 ? (size_t)g.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
+// Where the fragments of A come from, for products that read them: codes and scales; the same, in a layer's call, whose
+// plan is that of fragments given; the scratch holds them.
+enum Fragments { kFromCodes, kOfLayer, kGiven };
+
 static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB,
                            const float *alpha, const float *amax_a, const float *amax_b, double denominator,
                            int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
                            void *workspace, size_t workspace_bytes, fos_stream_t stream, bool if4 = false, int64_t rows = -1, int64_t depth = -1,
-                           bool check_only = false, int64_t cols = -1) {
+                           bool check_only = false, int64_t cols = -1, Fragments fragments = kFromCodes) {
     if (!A || !B || !sfA || !sfB || !D) return FOS_E_NULL_POINTER;
     if (((uintptr_t)d_amax & 3) || ((uintptr_t)bias & 7)) return FOS_E_BAD_ALIGNMENT;
     if (!alpha && (!amax_a || !amax_b)) return FOS_E_NULL_POINTER;
@@ -1121,6 +1189,7 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     p.rows = rows < 0 ? M : rows;
     p.cols = cols < 0 ? N : cols;
     // (blocks of the last 64 codes that lie below `depth`: 8 bits of the mask each)
+    p.depth = depth < 0 ? K : depth;
     p.k_tail = depth < 0 || K - depth < 16 ? 0xffffffffu : (1u << (8 * ((depth - (K - 64)) / 16))) - 1u;
     hipStream_t s = (hipStream_t)stream;
     GemmPlan g = plan_gemm(M, N, K, if4);
@@ -1128,6 +1197,19 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     // the tile kernels store whole rows of their output tiles, 16 bytes per lane
     if (g.kind != kPlanSkinny && (((uintptr_t)D & 15) || (ldd % 8 != 0))) return FOS_E_BAD_ALIGNMENT;  // partial bands only through the weight-streaming kernel
     if (check_only) return FOS_OK;
+    if (const HalfPlan h = plan_half(M, N, K, if4, fragments == kFromCodes); h.tile && workspace && !((uintptr_t)workspace & 15) && workspace_bytes >= h.bytes) {
+        uint8_t *scratch = static_cast<uint8_t *>(workspace);
+        if (fragments != kGiven) {
+            const int rc = launch_expand_fragments(ExpandParams{A, sfA, scratch, M, K, p.depth}, if4, s);
+            if (rc != FOS_OK) return rc;
+        }
+        p.frags = scratch;
+        p.partials = h.splits > 1 ? reinterpret_cast<float *>(scratch + h.partials) : nullptr;
+        p.splits = h.splits;
+        p.ksteps_per_split = h.chunks_per_split;
+        const int rc = launch_gemm_half(p, h.tile, if4, out_type, s);
+        return rc != FOS_OK || h.splits == 1 ? rc : launch_reduce(p, out_type, s);
+    }
     if (g.splits > 1 && !(workspace && !((uintptr_t)workspace & 15) &&
                           workspace_bytes >= (size_t)g.splits * (size_t)M * (size_t)N * sizeof(float))) {
         // no (or too small a) workspace: run unsplit
@@ -1207,6 +1289,13 @@ extern "C" int fos_gemm_nvfp4_linear(const uint8_t *A, const uint8_t *B, const u
                            workspace_bytes, stream);
 }
 
+extern "C" size_t fos_gemm_scratch_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || (dtype != FOS_DTYPE_NVFP4 && dtype != FOS_DTYPE_IF4)) return 0;
+    const HalfPlan h = plan_half(M, N, K, dtype == FOS_DTYPE_IF4, true);
+    if (h.tile) return h.bytes;
+    return dtype == FOS_DTYPE_IF4 ? fos_gemm_if4_workspace_bytes(M, N, K) : fos_gemm_workspace_bytes(M, N, K);
+}
+
 extern "C" size_t fos_gemm_if4_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M % 128 != 0 || N % 128 != 0 || K % 64 != 0) return 0;
     const GemmPlan g = plan_gemm(M, N, K, true);
@@ -1223,7 +1312,6 @@ extern "C" int fos_gemm_if4(const uint8_t *A, const uint8_t *B, const uint8_t *s
                            workspace_bytes, stream, true);
 }
 
-// The argument checks of an NVFP4 fos_gemm_linear_rows, nothing launched: for a caller that launches something ahead of it.
 int fos::check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a,
                            const float *amax_b, double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd,
                            const void *bias, float *d_amax) {
@@ -1244,4 +1332,18 @@ extern "C" int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *
     if (depth > K || depth <= K - 64 || (depth != K && (!if4 || depth % 16 != 0))) return FOS_E_BAD_SHAPE;
     return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, workspace,
                            workspace_bytes, stream, if4, rows, depth, false, cols);
+}
+
+size_t fos::linear_scratch_bytes(int64_t M, int64_t N, int64_t K) {
+    const HalfPlan h = plan_half(M, N, K, false, false);
+    return h.tile ? h.bytes : fos_gemm_workspace_bytes(M, N, K);
+}
+bool fos::linear_reads_fragments(int64_t M, int64_t N, int64_t K) { return plan_half(M, N, K, false, false).tile != 0; }
+int fos::gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
+                     double denominator, int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
+                     float *d_amax, void *scratch, size_t scratch_bytes, fos_stream_t stream) {
+    const Fragments fragments = A ? kOfLayer : kGiven;
+    if (!A) A = sfA = static_cast<const uint8_t *>(scratch);  // (not read)
+    return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, scratch,
+                           scratch_bytes, stream, false, rows, -1, false, -1, fragments);
 }

@@ -18,6 +18,7 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 struct GemmParams {
     const uint8_t *A, *B;      // [M, K/2], [N, K/2]
     const uint8_t *sfA, *sfB;  // 128x4-tiled E4M3 bytes
+    const uint8_t *frags;      // A as fp16 fragments (fos_gemm_half.h), for the kernels that read it that way
     const float *alpha;        // output scale on the device, or null: (amax_a * amax_b) * inv_den
     const float *amax_a, *amax_b;
     float inv_den;
@@ -26,6 +27,7 @@ struct GemmParams {
     const void *bias;          // optional: N values of the output type, added to the rounded product and rounded again
     float *d_amax;             // optional: max|D| as stored is folded into d_amax[0] (unsigned atomic max on the bits)
     int64_t M, N, K, ldd;
+    int64_t depth;             // columns of A and B from here on are padding (K % 64 == 0, K - depth < 64)
     uint32_t k_tail;           // IF4: mask on the scale bytes of the last 64 codes of a row, 0 for blocks that are padding
     int64_t cols;              // IF4: columns of D that exist, a multiple of 8 (the rest of N is padding that is not written)
     int64_t rows;              // rows 0 ... rows - 1 of D count for d_amax: padding rows hold the bias, not zeros

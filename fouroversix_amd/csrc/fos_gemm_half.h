@@ -1,0 +1,45 @@
+// Products with A converted ahead (fos_gemm_half.hip): its layout, the pass that produces it from codes and scales, the launch.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "fos_gemm_common.h"
+
+namespace fos {
+
+// 1 KiB fragments of 16 rows x 32 k: eight make a step of a band of 128 rows, four steps a chunk of 128 k.
+constexpr int kFragmentStep = 8192, kBandChunkBytes = 32768;
+
+// Byte of the fragments of [rows, K] at which the eight values k ... k + 7 (k % 8 == 0) of a row begin.
+FOS_DEVICE int64_t fragment_offset(int64_t row, int64_t k, int64_t chunks) {
+    return ((row >> 7) * chunks + (k >> 7)) * kBandChunkBytes + ((k >> 3) & 3) * kFragmentStep + ((row & 127) >> 4) * 1024 +
+           (((k >> 5) & 3) * 16 + (row & 15)) * 16;
+}
+inline size_t fragment_bytes(int64_t rows, int64_t K) { return (size_t)((rows + 127) / 128) * (size_t)((K + 127) / 128) * kBandChunkBytes; }
+
+struct ExpandParams {
+    const uint8_t *codes, *sf;
+    uint8_t *out;
+    int64_t rows, K, depth;  // K % 64 == 0; blocks from `depth` on are padding
+};
+int launch_expand_fragments(const ExpandParams &p, bool if4, hipStream_t s);
+
+// Output tiles of the product: 256 x 256 (eight wavefronts), 128 x 256 and 128 x 128 (four).
+enum { kHalf256 = 1, kHalfWide, kHalfSmall };
+// p: frags, B, sfB, ... ; with splits > 1 every split takes ksteps_per_split chunks of 128 k and the caller sums the partials.
+int launch_gemm_half(GemmParams &p, int tile, bool if4, int out_type, hipStream_t s);
+
+// The argument checks of an NVFP4 fos_gemm_linear_rows, nothing launched: for a caller that launches something ahead of it.
+int check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
+                      double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax);
+// The product of a layer's call.  Its plan is made for fragments that the quantize kernel writes: linear_reads_fragments says
+// whether the shape takes them, at the beginning of the scratch; A null: they are there, otherwise codes and scales to
+// form them from (inputs that the streaming quantize kernels don't read).  Arguments checked by check_gemm_linear.
+size_t linear_scratch_bytes(int64_t M, int64_t N, int64_t K);
+bool linear_reads_fragments(int64_t M, int64_t N, int64_t K);
+int gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
+                double denominator, int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
+                float *d_amax, void *scratch, size_t scratch_bytes, fos_stream_t stream);
+
+}  // namespace fos

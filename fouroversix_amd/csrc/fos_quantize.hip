@@ -14,6 +14,7 @@
 #include <cstdlib>
 
 #include "fos_quantize_kernel.h"
+#include "fos_gemm_half.h"
 #include "fos_tuning.h"
 
 namespace fos {
@@ -379,7 +380,14 @@ extern "C" int fos_pseudo_quantize_is_fused(int x_type, int dtype, int rule, int
            (rule == FOS_RULE_MSE || rule == FOS_RULE_STATIC_6 || rule == FOS_RULE_STATIC_4);
 }
 
-// Shared body of fos_quantize and fos_pseudo_quantize (pseudo_out != null: bf16 round trip
+// The streaming kernels address a 128-row tile with 32-bit byte offsets: a row pitch of 2^23
+// elements or more (16 MiB rows) takes the element-wise kernel like an unaligned input.
+constexpr int64_t kMaxPitch = int64_t{1} << 23;
+static bool streamable(const void *x, int64_t cols, int64_t ld) {
+    return ((uintptr_t)x & 15) == 0 && ld % 8 == 0 && cols % 16 == 0 && ld < kMaxPitch;
+}
+
+// Shared body of fos_quantize and fos_pseudo_quantize (frags != null: fragments of a product's operand; pseudo_out != null: bf16 round trip
 // instead of codes / scales).
 static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld,
                          int dtype, int rule, int round_style, int block2d,
@@ -387,8 +395,8 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
                          uint8_t *codes, uint8_t *sf, float *amax, int amax_is_input,
                          void *workspace, size_t workspace_bytes, fos_stream_t stream,
                          uint16_t *pseudo_out, int64_t ldo, const uint64_t *key = nullptr, int ready_partials = 0,
-                         float *zero_out = nullptr) {
-    if (!x || !amax || (!pseudo_out && (!codes || !sf))) return FOS_E_NULL_POINTER;
+                         float *zero_out = nullptr, uint8_t *frags = nullptr) {
+    if (!x || !amax || (!pseudo_out && !frags && (!codes || !sf))) return FOS_E_NULL_POINTER;
     if ((uintptr_t)key & 7) return FOS_E_BAD_ALIGNMENT;
     if (dtype == FOS_DTYPE_MXFP4) {
         // one streaming kernel; no tensor maximum, no workspace
@@ -420,12 +428,11 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
     uint32_t *partials = (uint32_t *)workspace;
     // (fp32 inputs, and fp16 ones outside the case below, take the element-wise kernel: they are treated as
     // unaligned throughout)
-    // The streaming kernels address a 128-row tile with 32-bit byte offsets: a row pitch of 2^23
-    // elements or more (16 MiB rows) takes the element-wise kernel like an unaligned input.
-    constexpr int64_t kMaxPitch = int64_t{1} << 23;
     // fp16 input has a streaming form for NVFP4 codes with 1x16 blocks and round to nearest
     const bool f16_streams = x_type == FOS_T_F16 && dtype == FOS_DTYPE_NVFP4 && round_style == FOS_ROUND_NEAREST && !block2d;
-    const bool aligned = (x_type == FOS_T_BF16 || f16_streams) && (((uintptr_t)x & 15) == 0) && (ld % 8 == 0) && (cols % 16 == 0) && ld < kMaxPitch;
+    const bool aligned = (x_type == FOS_T_BF16 || f16_streams) && streamable(x, cols, ld);
+    if (frags && (!aligned || block2d || round_style != FOS_ROUND_NEAREST || (dtype == FOS_DTYPE_IF4 && rule != FOS_RULE_MSE)))
+        return FOS_E_UNSUPPORTED;
     if (pseudo_out) {
         // only the streaming kernels have the fused epilogue
         if (!aligned) return FOS_E_UNSUPPORTED;
@@ -444,6 +451,7 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
     p.seed = seed; p.offset = offset;
     p.key = key;
     p.zero_out = zero_out;
+    p.frags = frags;
     p.sf_layout = sf_layout;
 
     if (ready_partials > 0) {
@@ -509,11 +517,6 @@ extern "C" int fos_quantize(const void *x, int x_type, int64_t rows, int64_t col
                          amax, amax_is_input, workspace, workspace_bytes, stream, nullptr, 0);
 }
 
-namespace fos {
-int check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
-                      double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax);
-}
-
 // Scratch of fos_linear_nvfp4: codes, scales, tensor maximum, pass-1 partials and split-K partials, each from a
 // 256-byte boundary on.
 namespace {
@@ -526,7 +529,7 @@ struct LinearScratch {
         amax = sf + up(elems / 16);
         partials = amax + 256;
         gemm = partials + up(fos_quantize_workspace_bytes(rows, cols));
-        total = gemm + fos_gemm_workspace_bytes(gemm_rows(rows, cols), N, fos_padded_cols(cols));
+        total = gemm + fos::linear_scratch_bytes(gemm_rows(rows, cols), N, fos_padded_cols(cols));
     }
     // rows the product is made for: a small batch's own where the weight-streaming kernels take it
     static int64_t gemm_rows(int64_t rows, int64_t cols) {
@@ -559,13 +562,16 @@ extern "C" int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t
     int rc = check_gemm_linear(base + at.codes, W, base + at.sf, sfW, amax, w_amax, denominator, LinearScratch::gemm_rows(rows, cols), N,
                                fos_padded_cols(cols), D, out_type, ldd, bias, d_amax);
     if (rc != FOS_OK) return rc;
+    const int64_t gemm_rows = LinearScratch::gemm_rows(rows, cols), depth = fos_padded_cols(cols);
+    void *gemm = at.total > at.gemm ? base + at.gemm : nullptr;
+    // what a streaming quantize kernel reads, and the product wants converted, goes straight into the product's scratch
+    const bool direct = x_type != FOS_T_F32 && streamable(x, cols, ld) && fos::linear_reads_fragments(gemm_rows, N, depth);
     rc = quantize_impl(x, x_type, rows, cols, ld, FOS_DTYPE_NVFP4, rule, FOS_ROUND_NEAREST, 0, 0, 0, FOS_SF_TILED_128X4,
-                                 base + at.codes, base + at.sf, amax, x_amax != nullptr, base + at.partials, at.gemm - at.partials, stream,
-                                 nullptr, 0, nullptr, 0, d_amax);
+                       direct ? nullptr : base + at.codes, direct ? nullptr : base + at.sf, amax, x_amax != nullptr, base + at.partials,
+                       at.gemm - at.partials, stream, nullptr, 0, nullptr, 0, d_amax, direct ? base + at.gemm : nullptr);
     if (rc != FOS_OK) return rc;
-    return fos_gemm_linear_rows(FOS_DTYPE_NVFP4, base + at.codes, W, base + at.sf, sfW, amax, w_amax, denominator,
-                                LinearScratch::gemm_rows(rows, cols), rows, N, N, fos_padded_cols(cols), fos_padded_cols(cols), D, out_type, ldd,
-                                bias, d_amax, at.total > at.gemm ? base + at.gemm : nullptr, at.total - at.gemm, stream);
+    return fos::gemm_linear(direct ? nullptr : base + at.codes, W, base + at.sf, sfW, amax, w_amax, denominator, gemm_rows, rows, N, depth, D,
+                            out_type, ldd, bias, d_amax, gemm, at.total - at.gemm, stream);
 }
 
 extern "C" int fos_quantize_devkey(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld,

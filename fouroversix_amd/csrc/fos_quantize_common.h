@@ -36,6 +36,7 @@ struct QuantParams {
     float c, qdiv, errdiv;       // f32(qmax*smax*adj), f32(qmax*adj), selection divisor
     uint16_t *pseudo_out;        // fused quantize -> dequantize: bf16 [rows, cols] output instead of codes / sf
     int64_t ldo;                 // its leading dimension
+    uint8_t *frags = nullptr;    // codes times scales as the fragments of a product's operand (fos_gemm_half.h) instead of codes / sf
 };
 
 // Order in which the streaming kernels walk their tiles.  Workgroups are dealt to the eight

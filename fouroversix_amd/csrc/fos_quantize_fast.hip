@@ -10,6 +10,7 @@
 #include <cstdlib>
 
 #include "fos_buffer.h"
+#include "fos_gemm_half.h"
 #include "fos_quantize_kernel.h"
 #include "fos_tuning.h"
 
@@ -44,7 +45,10 @@ struct RowsTile {
 // F16: fp16 elements instead of bf16 (NVFP4, round to nearest, codes out).
 // SPLIT: a workgroup covers 32 rows (one q) of a tile instead of 128, and one tile only: tensors with few tiles
 // otherwise run one workgroup a compute unit at most, eight steps one after the other (see launch_rows).
-template <int RULE, bool FULL, bool PSEUDO, bool SR, bool IF4 = false, bool F16 = false, bool SPLIT = false>
+// FRAG: the product's operand out, fp16(value * scale) as fragments, instead of codes and scales (2 bytes per element written
+// instead of 0.5625, where a pass over the codes would read and write 2.5625): a wavefront's store covers 64 bytes of each of 16
+// fragments, whose lines the next step and the neighbouring wavefront complete in L2.
+template <int RULE, bool FULL, bool PSEUDO, bool SR, bool IF4 = false, bool F16 = false, bool SPLIT = false, bool FRAG = false>
 // (the stochastic instantiations hold two sets of scaled values and the Philox state: with 128
 // registers they spilled -- 30 MB of scratch traffic per launch at 8192 x 8192 -- and the launch
 // grid of three workgroups per compute unit leaves 168; the IF4 instantiation spilled as well)
@@ -63,10 +67,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
     const int64_t sf_cols = p.cols_p >> 4;
     const int lb = lane & 15;               // block column inside the tile
     const int rl = wave * 8 + (lane >> 4);  // this lane's row in step 0
-    const bool tiled = !PSEUDO && p.sf_layout == FOS_SF_TILED_128X4;
+    const bool tiled = !PSEUDO && !FRAG && p.sf_layout == FOS_SF_TILED_128X4;
     const int64_t code_pitch = p.cols_p >> 1;
     const uint32_t n_tiles = (uint32_t)(p.rows_p >> 7) * (uint32_t)p.tiles_x;
-    static_assert(!(SPLIT && PSEUDO), "split tiles: codes and scales out");
+    static_assert(!(SPLIT && PSEUDO) && !(FRAG && (PSEUDO || SR)), "split tiles: codes and scales, or fragments, out");
+    // fragments: chunks of 128 columns, written whole (a tile's 256 columns are two of them)
+    const int64_t chunks = (p.cols_p + 127) >> 7, blocks_out = FRAG ? chunks * 8 : sf_cols;
+    const uint32_t f_lane = (uint32_t)((lb >> 3) * kBandChunkBytes + (lb & 1) * 2 * kFragmentStep + (wave >> 1) * 1024 + ((lb >> 1) & 3) * 256 +
+                                       ((wave & 1) * 8 + (lane >> 4)) * 16);
     const uint32_t sub = SPLIT ? blockIdx.x / n_tiles : 0u;  // (the four parts of a tile on one die where n_tiles % 8 == 0)
     // byte offsets inside a tile (the host checked that a tile spans less than 2^31 bytes);
     // step g starts 32 (g >> 1) + 4 (g & 1) rows below step 0
@@ -94,7 +102,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
         }
         t.x_bytes = __builtin_amdgcn_readfirstlane(x_bytes);
         t.x_base = uniform64((uint64_t)(p.x + t.row_base * p.ld + col_base));
-        t.codes_base = PSEUDO ? 0 : uniform64((uint64_t)(p.codes + t.row_base * code_pitch + col_base / 2));
+        t.codes_base = FRAG ? uniform64((uint64_t)(p.frags + ((int64_t)t.tile_y * chunks + 2 * t.tile_x) * kBandChunkBytes + 2048 * sub))
+                       : PSEUDO ? 0 : uniform64((uint64_t)(p.codes + t.row_base * code_pitch + col_base / 2));
         t.out_base = PSEUDO ? uniform64((uint64_t)(p.pseudo_out + t.row_base * p.ldo + col_base)) : 0;
         t.x_off = (FULL || t.cb * 16 < p.cols) ? x_lane : 0x80000000u;
         return t;
@@ -169,7 +178,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
     __syncthreads();
 
     auto process = [&](const RowsTile &t, int g, const Block16 &b) __attribute__((always_inline)) {
-        if (!FULL && t.cb >= sf_cols) return;  // past the padded width
+        if (!FULL && t.cb >= blocks_out) return;  // past the padded width
         const int64_t row = t.row_base + step_row(g) + rl;
         // a step that lies wholly in the row padding (decode-sized inputs: most steps) only
         // writes its zero codes and scales
@@ -236,6 +245,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
                 __builtin_amdgcn_raw_buffer_store_b128(d0, rout, o_off, 0, 0);
                 __builtin_amdgcn_raw_buffer_store_b128(d1, rout, o_off + 16u, 0, 0);
             }
+            return;
+        }
+        if constexpr (FRAG) {
+            // rows 32 (g >> 1) + 4 (g & 1) + ... of the tile: two fragments, or four rows inside them, per step
+            const BufferRsrc rfrags = make_rsrc(reinterpret_cast<const void *>(uniform64(t.codes_base)), 0xffffffffu);
+            const uint32_t step = (uint32_t)(2048 * (g >> 1) + 64 * (g & 1));
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dequant_word<IF4>(o.c0, o.s, 0)), rfrags, f_lane + step, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dequant_word<IF4>(o.c1, o.s, 0)), rfrags,
+                                                   f_lane + step + kFragmentStep, 0, 0);
             return;
         }
         const u32x2 c01 = {o.c0, o.c1};
@@ -315,8 +333,8 @@ void launch_quantize_nvfp4_tiles(QuantParams &p, hipStream_t s);
 // 2048 x 4096 (256) 9.2 / 6.6, 3072 x 4096 (384) 10.0 / 8.1, 4096 x 4096 (512) 10.4 / 10.2 (IF4 12.1 / 13.2),
 // 6144 x 4096 (768) 13.9 / 16.4.
 constexpr int64_t kSplitTiles = 384;
-template <int RULE, bool PSEUDO, bool SR, bool IF4, bool F16>
-static void launch_rows(QuantParams &p, hipStream_t s) {
+template <int RULE, bool PSEUDO, bool SR, bool IF4, bool F16, bool FRAG>
+static void launch_rows_as(QuantParams &p, hipStream_t s) {
     p.tiles_x = (int)((p.cols_p + 255) / 256);
     const int64_t n = (p.rows_p / 128) * p.tiles_x;
     p.tile_map = kMapRowMajor;
@@ -326,16 +344,24 @@ static void launch_rows(QuantParams &p, hipStream_t s) {
         const int split = tuning().quant_split;  // tuning / tests: 1 = never, 2 = always
         if (split == 2 ? 4 * n <= 0x7fffffff : (split == 0 && n <= kSplitTiles)) {
             const dim3 grid((unsigned)(4 * n));
-            if (full) hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, true, false, SR, IF4, F16, true>), grid, dim3(kThreads), 0, s, p);
-            else hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, false, false, SR, IF4, F16, true>), grid, dim3(kThreads), 0, s, p);
+            if (full) hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, true, false, SR, IF4, F16, true, FRAG>), grid, dim3(kThreads), 0, s, p);
+            else hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, false, false, SR, IF4, F16, true, FRAG>), grid, dim3(kThreads), 0, s, p);
             return;
         }
     }
     int64_t grid = 768;
     if (const int forced = tuning().quant_grid) grid = forced > 0 ? forced : grid;
     if (grid > n) grid = n;
-    if (full) hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, true, PSEUDO, SR, IF4, F16>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-    else hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, false, PSEUDO, SR, IF4, F16>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+    if (full) hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, true, PSEUDO, SR, IF4, F16, false, FRAG>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+    else hipLaunchKernelGGL((quantize_nvfp4_rows_kernel<RULE, false, PSEUDO, SR, IF4, F16, false, FRAG>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+}
+
+template <int RULE, bool PSEUDO, bool SR, bool IF4, bool F16>
+static void launch_rows(QuantParams &p, hipStream_t s) {
+    if constexpr (!PSEUDO && !SR) {
+        if (p.frags) return launch_rows_as<RULE, PSEUDO, SR, IF4, F16, true>(p, s);
+    }
+    launch_rows_as<RULE, PSEUDO, SR, IF4, F16, false>(p, s);
 }
 
 template <int RULE, bool PSEUDO, bool SR>

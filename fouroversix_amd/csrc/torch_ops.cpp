@@ -244,9 +244,9 @@ Tensor gemm_launch(const Tensor &a, const Tensor &b, const Tensor &a_sf, const T
                    int64_t rows = -1) {
     const int64_t m = a.size(0), n = b.size(0), k = a.size(1) * 2;
     Tensor out = at::empty({m, n}, a.options().dtype(out_dtype));
-    const size_t ws_bytes = fos_gemm_workspace_bytes(m, n, k);
+    const size_t ws_bytes = fos_gemm_scratch_bytes(FOS_DTYPE_NVFP4, m, n, k);
     const DeviceGuard guard(a.device());
-    // split-K partial tiles of small-M shapes; from torch's caching allocator, which keeps the block tied to the current stream
+    // split-K partial tiles of small-M shapes, A in fp16 of larger ones; from torch's caching allocator, which keeps the block tied to the current stream
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
     void *wsp = ws_bytes ? ws.data_ptr() : nullptr;
@@ -384,7 +384,7 @@ Tensor gemm_if4(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tens
     }
     const int64_t width = cols < 0 ? n : cols;
     Tensor out = at::empty({m, width}, a.options().dtype(out_dtype));
-    const size_t ws_bytes = fos_gemm_if4_workspace_bytes(m, n, k);
+    const size_t ws_bytes = fos_gemm_scratch_bytes(FOS_DTYPE_IF4, m, n, k);
     const DeviceGuard guard(a.device());
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));

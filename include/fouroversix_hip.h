@@ -336,6 +336,13 @@ int fos_gemm_alpha(const float *amax_a, const float *amax_b, double denominator,
 size_t fos_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
+ * Workspace with which the products run fastest (dtype FOS_DTYPE_NVFP4 or FOS_DTYPE_IF4): for larger M it also takes A
+ * converted to fp16, 2 bytes per element of the padded operand; elsewhere it is what the queries above return.  Every
+ * product call accepts either size (or none); K is summed in another order with this one.
+ */
+size_t fos_gemm_scratch_bytes(int dtype, int64_t M, int64_t N, int64_t K);
+
+/*
  * MXFP4 counterpart of fos_gemm_nvfp4: D = alpha * sum_k (A 2^(sfA-127)) (B 2^(sfB-127)) on
  * the native scaled FP4 matrix instruction.  Stands in for
  * torch.ops.fouroversix.gemm_mxfp4mxfp4_accum_fp32_out_bf16_tnt

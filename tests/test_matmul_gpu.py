@@ -886,3 +886,66 @@ def test_recorded_maximum_of_an_output_with_nan_is_nan():
     assert bool(torch.isnan(known_amax(out)).all())
     q = fos.quantize(out)
     assert bool(torch.isnan(q.amax).all())
+
+
+@pytest.mark.parametrize("splits", ["1", "3"])
+@pytest.mark.parametrize("tile", ["1001", "1002", "1003"])
+@pytest.mark.parametrize(("m", "n", "k"), [(128, 128, 64), (128, 256, 128), (384, 640, 192), (256, 384, 1088), (640, 256, 320), (300, 200, 1040)])
+def test_product_with_a_converted_ahead(monkeypatch, m, n, k, tile, splits):
+    """256 x 256, 128 x 256 and 128 x 128 tiles inside and over the edges of the output, one chunk of K and more, half a
+    chunk at the end, splits of unequal length: every code under every finite scale against the fp64 product.  Error bound:
+    fp32 accumulation over K (K 2^-24 of the sum of magnitudes, doubled for the output scale) plus half a unit of bf16."""
+    from fouroversix_amd.quantize import known_amax
+
+    monkeypatch.setenv("FOS_GEMM_TILE", tile)
+    monkeypatch.setenv("FOS_GEMM_SPLITK", splits)
+    g = torch.Generator("cpu").manual_seed(m + n + k)
+
+    def operand(rows):
+        rows_p, cols_p = -(-rows // 128) * 128, -(-k // 64) * 64
+        codes = torch.randint(0, 256, (rows_p, cols_p // 2), generator=g, dtype=torch.uint8)
+        scales = torch.randint(0, 127, (rows_p * cols_p // 16,), generator=g, dtype=torch.uint8)
+        codes[rows:] = 0
+        codes[:, k // 2:] = 0
+        return fos.QuantizedTensor(codes.cuda(), scales.cuda().view(torch.float8_e4m3fn), torch.tensor(1.5, device="cuda"), fos.DataType.nvfp4,
+                                   (rows, k), fos.ScaleRule.mse, fos.RoundStyle.nearest, padded_shape=(rows_p, cols_p))
+
+    qa, qb = operand(m), operand(n)
+    a, b = (fos.dequantize(q, dtype=torch.float32).double().cpu() for q in (qa, qb))
+    exact, size = a @ b.T, a.abs() @ b.abs().T
+    out = fos.quantized_matmul(qa, qb)
+    assert out.shape == (m, n)
+    assert bool(((out.double().cpu() - exact).abs() <= 2.0 ** -8 * exact.abs() + 2 * k * 2.0 ** -24 * size).all())
+    if n % 128 == 0:
+        bias = torch.linspace(-1, 1, n, device="cuda").bfloat16()
+        with_bias = fos.quantized_matmul(qa, qb, bias=bias, emit_amax=True)
+        assert torch.equal(with_bias, out + bias)
+        assert float(known_amax(with_bias)) == float(with_bias.abs().max())
+
+
+@pytest.mark.parametrize("quant_split", ["1", "2"])
+@pytest.mark.parametrize("rule", ["static_6", "mse", "mae", "abs_max"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize(("tokens", "inf"), [(130, 64), (256, 1040), (384, 512), (257, 4096)])
+def test_layer_with_operands_written_by_the_quantizer(monkeypatch, tokens, inf, dtype, rule, quant_split):
+    """An aligned input is quantized straight into the product's operand; the same values at an odd address become codes and
+    scales first, which are then converted: the same bits, and the codes' own product within a rounding."""
+    monkeypatch.setenv("FOS_QUANT_SPLIT", quant_split)
+    g = torch.Generator("cpu").manual_seed(tokens + inf)
+    model = nn.Sequential(nn.Linear(inf, 384, device="cuda", dtype=dtype))
+    fos.quantize_model(model, fos.ModelQuantizationConfig(activation_scale_rule=rule))
+    model[0].quantize_weight_()
+    x = torch.randn(tokens, inf, generator=g).to(dtype)
+    x[tokens // 2:] *= 30
+    aligned = x.cuda()
+    moved = torch.empty(tokens * inf + 1, dtype=dtype, device="cuda")[1:].view(tokens, inf)
+    moved.copy_(aligned)
+    with torch.no_grad():
+        out = model(aligned)
+        assert torch.equal(out, model(moved))
+    qx = fos.quantize(aligned, fos.QuantizationConfig(scale_rule=rule))
+    a, b = (fos.dequantize(q, dtype=torch.float32).double() for q in (qx, model[0].quantized_weight()))
+    exact, size = a @ b.T + model[0].bias.double(), a.abs() @ b.abs().T
+    # (the product rounded to the output type, then the sum)
+    bound = 2.0 ** -8 * (exact.abs() + (a @ b.T).abs()) * (1 + 2.0 ** -8) + 2 * inf * 2.0 ** -24 * size
+    assert bool(((out.double() - exact).abs() <= bound).all())
