@@ -521,7 +521,7 @@ extern "C" int fos_quantize(const void *x, int x_type, int64_t rows, int64_t col
 // 256-byte boundary on.
 namespace {
 struct LinearScratch {
-    size_t codes = 0, sf, amax, partials, gemm, total;
+    size_t codes = 0, sf, amax, partials, gemm, least, total;  // (least: without room for the operand as fragments)
     LinearScratch(int64_t rows, int64_t cols, int64_t N) {
         auto up = [](size_t v) { return (v + 255) / 256 * 256; };
         const size_t elems = (size_t)fos_padded_rows(rows) * (size_t)fos_padded_cols(cols);
@@ -529,6 +529,7 @@ struct LinearScratch {
         amax = sf + up(elems / 16);
         partials = amax + 256;
         gemm = partials + up(fos_quantize_workspace_bytes(rows, cols));
+        least = gemm + fos_gemm_workspace_bytes(gemm_rows(rows, cols), N, fos_padded_cols(cols));
         total = gemm + fos::linear_scratch_bytes(gemm_rows(rows, cols), N, fos_padded_cols(cols));
     }
     // rows the product is made for: a small batch's own where the weight-streaming kernels take it
@@ -555,7 +556,7 @@ extern "C" int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t
     if (rows <= 0 || cols <= 0 || N <= 0) return FOS_E_BAD_SHAPE;
     if (((uintptr_t)scratch & 255) || ((uintptr_t)d_amax & 3)) return FOS_E_BAD_ALIGNMENT;
     const LinearScratch at(rows, cols, N);
-    if (scratch_bytes < at.total) return FOS_E_WORKSPACE;
+    if (scratch_bytes < (at.least < at.total ? at.least : at.total)) return FOS_E_WORKSPACE;
     uint8_t *base = static_cast<uint8_t *>(scratch);
     float *amax = x_amax ? const_cast<float *>(x_amax) : reinterpret_cast<float *>(base + at.amax);
     // (a call that the product refuses has written nothing, d_amax included)
@@ -563,15 +564,17 @@ extern "C" int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t
                                fos_padded_cols(cols), D, out_type, ldd, bias, d_amax);
     if (rc != FOS_OK) return rc;
     const int64_t gemm_rows = LinearScratch::gemm_rows(rows, cols), depth = fos_padded_cols(cols);
-    void *gemm = at.total > at.gemm ? base + at.gemm : nullptr;
+    void *gemm = scratch_bytes > at.gemm ? base + at.gemm : nullptr;
+    const size_t gemm_bytes = scratch_bytes - at.gemm;
     // what a streaming quantize kernel reads, and the product wants converted, goes straight into the product's scratch
-    const bool direct = x_type != FOS_T_F32 && streamable(x, cols, ld) && fos::linear_reads_fragments(gemm_rows, N, depth);
+    const bool direct = scratch_bytes >= at.total && x_type != FOS_T_F32 && streamable(x, cols, ld) &&
+                        fos::linear_reads_fragments(gemm_rows, N, depth);
     rc = quantize_impl(x, x_type, rows, cols, ld, FOS_DTYPE_NVFP4, rule, FOS_ROUND_NEAREST, 0, 0, 0, FOS_SF_TILED_128X4,
                        direct ? nullptr : base + at.codes, direct ? nullptr : base + at.sf, amax, x_amax != nullptr, base + at.partials,
                        at.gemm - at.partials, stream, nullptr, 0, nullptr, 0, d_amax, direct ? base + at.gemm : nullptr);
     if (rc != FOS_OK) return rc;
     return fos::gemm_linear(direct ? nullptr : base + at.codes, W, base + at.sf, sfW, amax, w_amax, denominator, gemm_rows, rows, N, depth, D,
-                            out_type, ldd, bias, d_amax, gemm, at.total - at.gemm, stream);
+                            out_type, ldd, bias, d_amax, gemm, gemm_bytes, stream);
 }
 
 extern "C" int fos_quantize_devkey(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld,

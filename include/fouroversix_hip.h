@@ -286,7 +286,8 @@ int fos_gemm_nvfp4_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA
  * fos_quantize followed by fos_gemm_nvfp4_linear gives it.  D has fos_linear_nvfp4_rows(rows, cols) rows (the padded
  * ones, or `rows` where the product skips the padding of a small batch).  d_amax, when given, is set to max|D| (unlike
  * there it needs no initial value: the quantize kernel clears it), over the first `rows` rows.  `scratch`: fos_linear_nvfp4_scratch_bytes bytes,
- * 256-byte aligned, in use until the product is done.
+ * 256-byte aligned, in use until the product is done (with less, down to what codes, scales and fos_gemm_workspace_bytes
+ * take, the product runs as fos_gemm_nvfp4_linear does).
  */
 size_t fos_linear_nvfp4_scratch_bytes(int64_t rows, int64_t cols, int64_t N);
 int64_t fos_linear_nvfp4_rows(int64_t rows, int64_t cols);
