@@ -1077,7 +1077,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool if4) {
 // tile (0: the kernels above are faster) and split of K.
 struct HalfPlan {
     int tile = 0, splits = 1, chunks_per_split = 0;
-    size_t partials = 0, bytes = 0;  // scratch: fragments, then from `partials` on the FP32 partials
+    size_t b = 0, partials = 0, bytes = 0;  // scratch: fragments of A, (IF4) from `b` on those of B, then the FP32 partials
 };
 
 // Time of `tiles` output tiles (us at K = 4096, without what a launch takes at any K): 256 workgroups of the 256 x 256 tile
@@ -1095,11 +1095,13 @@ static float half_cost(int tile, int64_t tiles, float k) {
 // on all but a few of 400 shapes, which tie: 1024 x 14336 x 4096 97 -> 83 us, 8192 x 4096 x 4096 207 -> 178,
 // 6144 x 4096 x 4096 (384 tiles of 256 x 256) 180 -> 138, 2048 x 1024 x 4096 36 -> 28 in two splits, 1024 x 1024 x 14336
 // 49 -> 44 in four.  With the pass in front it has to make up for 4 us and 0.32 us per 2^20 elements of A: that
-// leaves the larger products.
+// leaves the larger products.  IF4, both of whose operands are converted ahead, pays for B as well, against kernels that take
+// 1.7 times NVFP4's times: whole products of 2048 x 4096 x 4096 117 -> 70 us, 512 x 4096 x 4096 69 -> 39,
+// 256 x 14336 x 4096 76 -> 61; 384 x 8192 x 1024 stays (26 against 28).
 static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand) {
     HalfPlan h;
     const int forced = tuning().gemm_tile;  // tuning / tests: 1000 + tile; another kernel's tile excludes this one
-    if (M < 128 || M % 128 || N % 128 || K % 64 || K > (1 << 20) || if4 || (forced && forced <= 1000) || (!forced && M < 256)) return h;
+    if (M < 128 || M % 128 || N % 128 || K % 64 || K > (1 << 20) || (forced && forced <= 1000) || (!forced && M < 256)) return h;
     if (fragment_bytes(M, K) > ((size_t)8 << 30)) return h;  // (a call with an operand that large keeps to the smaller workspace)
     const int64_t chunks = (K + 127) / 128, m128 = M / 128, n128 = N / 128, m256 = (m128 + 1) / 2, n256 = (n128 + 1) / 2;
     const int forced_splits = tuning().gemm_splitk;
@@ -1119,16 +1121,20 @@ static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand
                 if (cost < best) best = cost, h.tile = tile, splits = s;
             }
         }
-        if (expand && h.tile) {
+        const float other = tile_cost(M, N, nullptr) * (float)K / 4096;
+        if (if4) {
+            if (best + 9 + 0.32e-6f * (M + N) * K > 1.7f * other) h.tile = 0;
+        } else if (expand && h.tile) {
             const GemmPlan g = plan_gemm(M, N, K, false);
-            if (g.splits > 1 || best + 5 + 4 + 0.32e-6f * M * K > tile_cost(M, N, nullptr) * (float)K / 4096) h.tile = 0;
+            if (g.splits > 1 || best + 5 + 4 + 0.32e-6f * M * K > other) h.tile = 0;
         }
         if (!h.tile) return h;
     }
     if (splits > chunks) splits = chunks;
     h.chunks_per_split = (int)((chunks + splits - 1) / splits);
     h.splits = (int)((chunks + h.chunks_per_split - 1) / h.chunks_per_split);
-    h.partials = fragment_bytes(M, K);
+    h.b = fragment_bytes(M, K);
+    h.partials = h.b + (if4 ? fragment_bytes(N, K) : 0);
     h.bytes = h.partials + (h.splits > 1 ? (size_t)h.splits * (size_t)M * (size_t)N * sizeof(float) : 0);
     return h;
 }
@@ -1200,10 +1206,13 @@ static int gemm_nvfp4_impl(const uint8_t *A, const uint8_t *B, const uint8_t *sf
     if (const HalfPlan h = plan_half(M, N, K, if4, fragments == kFromCodes); h.tile && workspace && !((uintptr_t)workspace & 15) && workspace_bytes >= h.bytes) {
         uint8_t *scratch = static_cast<uint8_t *>(workspace);
         if (fragments != kGiven) {
-            const int rc = launch_expand_fragments(ExpandParams{A, sfA, scratch, M, K, p.depth}, if4, s);
+            ExpandParams e{K, p.depth, {{A, sfA, scratch, M}}};
+            if (if4) e.operand[1] = {B, sfB, scratch + h.b, N};
+            const int rc = launch_expand_fragments(e, if4, s);
             if (rc != FOS_OK) return rc;
         }
         p.frags = scratch;
+        p.frags_b = scratch + h.b;  // (IF4)
         p.partials = h.splits > 1 ? reinterpret_cast<float *>(scratch + h.partials) : nullptr;
         p.splits = h.splits;
         p.ksteps_per_split = h.chunks_per_split;

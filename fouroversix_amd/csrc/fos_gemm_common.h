@@ -18,7 +18,7 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 struct GemmParams {
     const uint8_t *A, *B;      // [M, K/2], [N, K/2]
     const uint8_t *sfA, *sfB;  // 128x4-tiled E4M3 bytes
-    const uint8_t *frags;      // A as fp16 fragments (fos_gemm_half.h), for the kernels that read it that way
+    const uint8_t *frags, *frags_b;  // A, for IF4 B too, as fp16 fragments (fos_gemm_half.h), for the kernels that read them that way
     const float *alpha;        // output scale on the device, or null: (amax_a * amax_b) * inv_den
     const float *amax_a, *amax_b;
     float inv_den;

@@ -18,16 +18,22 @@ FOS_DEVICE int64_t fragment_offset(int64_t row, int64_t k, int64_t chunks) {
 }
 inline size_t fragment_bytes(int64_t rows, int64_t K) { return (size_t)((rows + 127) / 128) * (size_t)((K + 127) / 128) * kBandChunkBytes; }
 
-struct ExpandParams {
-    const uint8_t *codes, *sf;
-    uint8_t *out;
-    int64_t rows, K, depth;  // K % 64 == 0; blocks from `depth` on are padding
+// One operand, or two of the same inner dimension (rows 0: none).
+struct ExpandOperand {
+    const uint8_t *codes = nullptr, *sf = nullptr;
+    uint8_t *out = nullptr;
+    int64_t rows = 0;
 };
-int launch_expand_fragments(const ExpandParams &p, bool if4, hipStream_t s);
+struct ExpandParams {
+    int64_t K, depth;  // K % 64 == 0; blocks from `depth` on are padding
+    ExpandOperand operand[2];
+    int groups = 0;    // blocks of 16 rows of the first one (launch_expand_fragments)
+};
+int launch_expand_fragments(ExpandParams p, bool if4, hipStream_t s);
 
 // Output tiles of the product: 256 x 256 (eight wavefronts), 128 x 256 and 128 x 128 (four).
 enum { kHalf256 = 1, kHalfWide, kHalfSmall };
-// p: frags, B, sfB, ... ; with splits > 1 every split takes ksteps_per_split chunks of 128 k and the caller sums the partials.
+// p: frags, B, sfB (NVFP4), or frags and frags_b (IF4), ... ; with splits > 1 every split takes ksteps_per_split chunks of 128 k and the caller sums the partials.
 int launch_gemm_half(GemmParams &p, int tile, bool if4, int out_type, hipStream_t s);
 
 // The argument checks of an NVFP4 fos_gemm_linear_rows, nothing launched: for a caller that launches something ahead of it.

@@ -50,30 +50,34 @@ FOS_DEVICE uint32_t tail_mask(int left) { return left <= 0 ? 0u : left == 1 ? 0x
 // ---------------------------------------------------------------------------------------
 // Codes and scales -> fragments.  Memory-bound: 0.5625 bytes read and 2 written per element; 16384 x 4096 27 us = 6.4 TB/s.
 // A workgroup takes 16 rows and four chunks, a wavefront a chunk: 64 contiguous bytes of each of 16 rows in, four whole
-// KiB out.  Rows from `rows` on (a band is written whole) and blocks from `depth` on are zeros.
+// KiB out.  Rows from `rows` on (a band is written whole) and blocks from `depth` on are zeros.  A second operand follows
+// in the same launch (blocks of rows from p.groups on).
 template <bool IF4>
 __global__ __launch_bounds__(256) void expand_fragments_kernel(const ExpandParams p) {
     const int64_t chunks = (p.K + 127) >> 7, chunk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (chunk >= chunks) return;
+    const int second = blockIdx.y >= (unsigned)p.groups;  // (uniform)
+    const ExpandOperand &o = p.operand[second];
     const int lane = threadIdx.x & 63, q = lane >> 4;
-    const int64_t row = (int64_t)blockIdx.y * 16 + (lane & 15), k0 = chunk * 128 + q * 32;
+    const int64_t row = (int64_t)(blockIdx.y - (second ? p.groups : 0)) * 16 + (lane & 15), k0 = chunk * 128 + q * 32;
     uint4 w = make_uint4(0u, 0u, 0u, 0u);
     uint32_t s = 0u;
-    if (row < p.rows && k0 < p.K) {
-        w = *reinterpret_cast<const uint4 *>(p.codes + row * (p.K >> 1) + (k0 >> 1));
+    if (row < o.rows && k0 < p.K) {
+        w = *reinterpret_cast<const uint4 *>(o.codes + row * (p.K >> 1) + (k0 >> 1));
         const int64_t at = IF4 ? row * (p.K >> 4) + (k0 >> 4)
                                : ((row >> 7) * (p.K >> 6) + (k0 >> 6)) * 512 + (row & 31) * 16 + ((row & 127) >> 5) * 4 + ((k0 >> 4) & 3);
-        s = *reinterpret_cast<const uint16_t *>(p.sf + at) & tail_mask((int)((p.depth - k0 + 15) >> 4));
+        s = *reinterpret_cast<const uint16_t *>(o.sf + at) & tail_mask((int)((p.depth - k0 + 15) >> 4));
     }
-    uint8_t *out = p.out + ((row >> 7) * chunks + chunk) * kBandChunkBytes + ((row & 127) >> 4) * 1024 + lane * 16;
+    uint8_t *out = o.out + ((row >> 7) * chunks + chunk) * kBandChunkBytes + ((row & 127) >> 4) * 1024 + lane * 16;
     *reinterpret_cast<half8_t *>(out) = dequant_word<IF4>(w.x, s, 0);
     *reinterpret_cast<half8_t *>(out + kFragmentStep) = dequant_word<IF4>(w.y, s, 0);
     *reinterpret_cast<half8_t *>(out + 2 * kFragmentStep) = dequant_word<IF4>(w.z, s, 1);
     *reinterpret_cast<half8_t *>(out + 3 * kFragmentStep) = dequant_word<IF4>(w.w, s, 1);
 }
 
-int launch_expand_fragments(const ExpandParams &p, bool if4, hipStream_t s) {
-    const dim3 grid((unsigned)((p.K + 511) / 512), (unsigned)((p.rows + 127) / 128 * 8));
+int launch_expand_fragments(ExpandParams p, bool if4, hipStream_t s) {
+    p.groups = (int)((p.operand[0].rows + 127) / 128 * 8);
+    const dim3 grid((unsigned)((p.K + 511) / 512), (unsigned)(p.groups + (p.operand[1].rows + 127) / 128 * 8));
     if (if4) hipLaunchKernelGGL(expand_fragments_kernel<true>, grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL(expand_fragments_kernel<false>, grid, dim3(256), 0, s, p);
     return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;
@@ -94,32 +98,30 @@ int launch_expand_fragments(const ExpandParams &p, bool if4, hipStream_t s) {
 // read behind a load into LDS that it knows about.  No other vector-memory load is in the loop, so the waits by hand are all there are.
 constexpr int kSlotsA = 4, kSlotsB = 2;
 
-constexpr int half_lds_bytes(int BM, int BN) {
-    const int loop = kSlotsA * BM * 64 + kSlotsB * BN * 72, epilogue = BM * BN / 8192 * 32 * 144;
+constexpr int half_lds_bytes(int BM, int BN, bool if4) {
+    const int loop = kSlotsA * BM * 64 + (if4 ? kSlotsA * BN * 64 : kSlotsB * BN * 72), epilogue = BM * BN / 8192 * 32 * 144;
     return loop > epilogue ? loop : epilogue;
 }
 
-template <int I, bool IF4>
-FOS_DEVICE void convert_pair(half8_t &f, uint32_t word, uint32_t (&pairs)[2], half2_t s, bool integer) {
-    half2_t v = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, I);
-    if constexpr (IF4) {
-        if (I == 0) if4_integer_bytes(word, pairs);
-        const half2_t i = if4_sevenths(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pairs[I >> 1], 1.0f, (I & 1) != 0));
-        v = __builtin_bit_cast(half2_t, integer ? __builtin_bit_cast(uint32_t, i) : __builtin_bit_cast(uint32_t, v));
-    }
-    v = v * s;
+template <int I>
+FOS_DEVICE void convert_pair(half8_t &f, uint32_t word, half2_t s) {
+    const half2_t v = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, I) * s;
     f[2 * I] = v.x;
     f[2 * I + 1] = v.y;
 }
 
+// IF4: B as fragments too, loaded and read as A is.  Its conversion takes 34 instructions a word and in the loop bounded the
+// product (2048 x 4096 x 4096 123 us on 128 x 128 tiles, the others spilled; 95 in gemm_nvfp4_kernel); ahead of it, it
+// is bound by memory.
 template <int WAVES_M, int WAVES_N, int WM, int BAR, int OCC, int OUT, bool IF4>
 __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(const GemmParams p) {
     constexpr bool OUT_BF16 = OUT == kOutBF16;
     constexpr int WN = 4, NW = WAVES_M * WAVES_N, BM = 16 * WM * WAVES_M, BN = 64 * WAVES_N, MFMAS = WM * WN;
-    constexpr int kSlotA = BM * 64, kCodesB = BN * 64, kSlotB = BN * 72, kBaseB = kSlotsA * kSlotA;
-    // a wavefront's loads: of A per step; of B's codes (16 rows each) and scales (256 bytes each) per chunk
-    constexpr int LA = BM / 16 / NW, LB = BN / 16 / NW, LS = BN / 32 / NW;
-    static_assert((LA == 1 || LA == 2) && LB >= 1 && LS >= 1 && (WM == 4 || WM == 8), "shares of the loads");
+    constexpr int kSlotA = BM * 64, kCodesB = BN * 64, kSlotB = IF4 ? BN * 64 : BN * 72, kBaseB = kSlotsA * kSlotA;
+    // a wavefront's loads: of A per step, and of B per step (IF4) or of B's codes (16 rows each) and scales (256 bytes each)
+    // per chunk
+    constexpr int LA = BM / 16 / NW, LB = BN / 16 / NW, LS = IF4 ? 0 : BN / 32 / NW, LSTEP = IF4 ? LA + LB : LA, LCHUNK = IF4 ? 0 : LB + LS;
+    static_assert(LA == 2 && LB >= 1 && (WM == 4 || WM == 8), "shares of the loads");
     extern __shared__ __attribute__((aligned(16))) uint8_t half_lds[];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4;
@@ -133,18 +135,24 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
     const int chunks = OUT == kOutPartial ? (chunks_all - c0 < p.ksteps_per_split ? chunks_all - c0 : p.ksteps_per_split) : chunks_all;
     const int steps = 4 * chunks;
     const uint32_t band = (uint32_t)chunks_all * kBandChunkBytes, kbytes = (uint32_t)(p.K >> 1);
-    const uint32_t scale_band = IF4 ? 0u : (uint32_t)p.K * 8u, scale_row = (uint32_t)(p.K >> 4);
+    const uint32_t scale_band = (uint32_t)p.K * 8u;
     const int4v ra = raw_rsrc(p.frags + (m0 >> 7) * (int64_t)band, (uint32_t)(rows_a >> 7) * band);
-    const int4v rb = raw_rsrc(p.B + n0 * kbytes, (uint32_t)rows_b * kbytes);
-    const int4v rs = raw_rsrc(p.sfB + n0 * scale_row, (uint32_t)rows_b * scale_row);  // (the same extent in either layout)
+    const int4v rb = IF4 ? raw_rsrc(p.frags_b + (n0 >> 7) * (int64_t)band, (uint32_t)(rows_b >> 7) * band)
+                         : raw_rsrc(p.B + n0 * kbytes, (uint32_t)rows_b * kbytes);
+    const int4v rs = raw_rsrc(p.sfB + (n0 >> 7) * (int64_t)scale_band, (uint32_t)(rows_b >> 7) * scale_band);  // (NVFP4)
     const uint32_t lds_base = (uint32_t)(uintptr_t)(LdsPtr)half_lds;
-    const uint32_t va = lane * 16, vb = (lane & 15) * kbytes + q * 16, vs = IF4 ? (lane >> 1) * scale_row + (lane & 1) * 4 : lane * 4;
+    const uint32_t va = lane * 16, vb = (lane & 15) * kbytes + q * 16, vs = lane * 4;
 
     // m0 = LDS address of the run a wavefront fills (lane i: unit i); one wait state between a write of m0 and its use
     auto load16 = [&](uint32_t to, uint32_t offset, const int4v &r, uint32_t base) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to), "v"(offset), "s"(r), "s"(base) : "memory");
     };
-    auto load_a = [&](int step, int slot, int t) {
+    auto load_step = [&](int step, int slot, int t) {
+        if (t >= LA) {  // (IF4)
+            const uint32_t f = wave * LB + t - LA;
+            load16(lds_base + kBaseB + slot * kSlotB + f * 1024, va, rb, (f >> 3) * band + (uint32_t)(c0 * 4 + step) * kFragmentStep + (f & 7) * 1024);
+            return;
+        }
         const uint32_t f = wave * LA + t;
         load16(lds_base + slot * kSlotA + f * 1024, va, ra, (f >> 3) * band + (uint32_t)(c0 * 4 + step) * kFragmentStep + (f & 7) * 1024);
     };
@@ -155,7 +163,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
             load16(base + g * 1024, vb, rb, g * 16 * kbytes + (uint32_t)(c0 + chunk) * 64);
         } else {
             const uint32_t g = wave * LS + t - LB;
-            const uint32_t from = IF4 ? g * 32 * scale_row + (uint32_t)(c0 + chunk) * 8 : (g >> 2) * scale_band + (uint32_t)(c0 + chunk) * 1024 + (g & 3) * 256;
+            const uint32_t from = (g >> 2) * scale_band + (uint32_t)(c0 + chunk) * 1024 + (g & 3) * 256;
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
                          ::"s"(base + kCodesB + g * 256), "v"(vs), "s"(rs), "s"(from) : "memory");
         }
@@ -165,33 +173,31 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
     const uint8_t *lds_a = half_lds + wm * WM * 1024 + lane * 16;
     const uint8_t *lds_b = half_lds + kBaseB + wn * 4096 + lane * 16;
     // scale bytes of column 64 wn + 16 j + (lane & 15), blocks 2 q and 2 q + 1 of the chunk
-    const uint8_t *lds_s = half_lds + kBaseB + kCodesB +
-                           (IF4 ? (wn * 64 + (lane & 15)) * 8 + q * 2
-                                : (wn >> 1) * 1024 + (q >> 1) * 512 + (lane & 15) * 16 + (wn & 1) * 8 + (q & 1) * 2);
-    half8_t fa[2][WM], fb[2];
+    const uint8_t *lds_s = half_lds + kBaseB + kCodesB + (wn >> 1) * 1024 + (q >> 1) * 512 + (lane & 15) * 16 + (wn & 1) * 8 + (q & 1) * 2;
+    half8_t fa[2][WM], fb[2][IF4 ? WN : 1];  // (NVFP4: the current and the next 16 columns; IF4: the current and the next step)
     uint4 codes[2][WN];
-    uint32_t scales[2][WN], pairs[2];
+    uint32_t scales[2][WN];
     half2_t s2[WN];
-    auto read_a = [&](int slot, int set, int t) { fa[set][t] = *reinterpret_cast<const half8_t *>(lds_a + slot * kSlotA + t * 1024); };
-    auto read_b = [&](int slot, int set, int t) {
+    auto read_step = [&](int slot, int set, int t) {
+        if (t < WM) fa[set][t] = *reinterpret_cast<const half8_t *>(lds_a + slot * kSlotA + t * 1024);
+        else if constexpr (IF4) fb[set][t - WM] = *reinterpret_cast<const half8_t *>(lds_b + slot * kSlotB + (t - WM) * 1024);
+    };
+    auto read_chunk = [&](int slot, int set, int t) {
         if (t < WN) codes[set][t] = *reinterpret_cast<const uint4 *>(lds_b + slot * kSlotB + t * 1024);
-        else scales[set][t - WN] = *reinterpret_cast<const uint16_t *>(lds_s + slot * kSlotB + (IF4 ? (t - WN) * 128 : ((t - WN) & 1) * 256 + ((t - WN) >> 1) * 4));
+        else scales[set][t - WN] = *reinterpret_cast<const uint16_t *>(lds_s + slot * kSlotB + ((t - WN) & 1) * 256 + ((t - WN) >> 1) * 4);
     };
     const uint32_t last_mask = tail_mask((int)((p.depth - (int64_t)(chunks_all - 1) * 128 + 15) >> 4) - 2 * q);
     auto widen_scales = [&](int chunk, int set) {
         const uint32_t mask = c0 + chunk + 1 >= chunks_all ? last_mask : 0xffffu;
 #pragma unroll
-        for (int t = 0; t < WN; ++t) {
-            scales[set][t] &= mask;
-            s2[t] = e4m3x2_to_half2(IF4 ? scales[set][t] & 0x7f7fu : scales[set][t]);
-        }
+        for (int t = 0; t < WN; ++t) s2[t] = e4m3x2_to_half2(scales[set][t] & mask);
     };
     // pair i (0 .. 3) of word w of the next fragment: columns j of the chunk in register set `set`
     auto convert = [&](auto ic, half8_t &f, int set, int j, int w) {
         const uint4 &c = codes[set][j];
         const uint32_t word = w == 0 ? c.x : w == 1 ? c.y : w == 2 ? c.z : c.w;
         const half2_t s = w >= 2 ? __builtin_shufflevector(s2[j], s2[j], 1, 1) : __builtin_shufflevector(s2[j], s2[j], 0, 0);
-        convert_pair<decltype(ic)::value, IF4>(f, word, pairs, s, IF4 && (scales[set][j] & (w >= 2 ? 0x8000u : 0x80u)) != 0);
+        convert_pair<decltype(ic)::value>(f, word, s);
     };
 
     float4v acc[WM][WN];
@@ -203,22 +209,29 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
             for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.0f;
 
     // chunks 0, 1 of B and steps 0 .. 3 of A in flight (past the end: the last ones once more, into slots nobody reads)
+    if constexpr (!IF4) {
 #pragma unroll
-    for (int c = 0; c < kSlotsB; ++c)
+        for (int c = 0; c < kSlotsB; ++c)
 #pragma unroll
-        for (int t = 0; t < LB + LS; ++t) load_b(c < chunks ? c : chunks - 1, c, t);
+            for (int t = 0; t < LCHUNK; ++t) load_b(c < chunks ? c : chunks - 1, c, t);
+    }
 #pragma unroll
     for (int k = 0; k < kSlotsA; ++k)
 #pragma unroll
-        for (int t = 0; t < LA; ++t) load_a(k, k, t);
+        for (int t = 0; t < LSTEP; ++t) load_step(k, k, t);
 #define FOS_HALF_WAIT(n) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(n) : "memory")
-    FOS_HALF_WAIT((kSlotsA - 1) * LA);
+    FOS_HALF_WAIT((kSlotsA - 1) * LSTEP);
+    constexpr int READS = WM + (IF4 ? WN : 0);  // fragments a wavefront reads per step
+    if constexpr (!IF4) {
 #pragma unroll
-    for (int t = 0; t < 2 * WN; ++t) read_b(0, 0, t);
+        for (int t = 0; t < 2 * WN; ++t) read_chunk(0, 0, t);
+    }
 #pragma unroll
-    for (int t = 0; t < WM; ++t) read_a(0, 0, t);
-    widen_scales(0, 0);
-    static_for<0, 4>([&](auto ic) { convert(ic, fb[0], 0, 0, 0); });
+    for (int t = 0; t < READS; ++t) read_step(0, 0, t);
+    if constexpr (!IF4) {
+        widen_scales(0, 0);
+        static_for<0, 4>([&](auto ic) { convert(ic, fb[0][0], 0, 0, 0); });
+    }
 
     int slot_b = 0;
     // (a chunk's four steps use the four slots of A in order; its codes are in register set CUR)
@@ -233,40 +246,41 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
                 if constexpr (m == BAR) {
                     // newer than the loads of step k + 1: two steps of A, and from the second step of a chunk on its B
                     // (issued behind A in the first step; a chunk is asked for seven steps ahead of its use)
-                    FOS_HALF_WAIT(LA * (kSlotsA - 2) + (w >= 1 ? LB + LS : 0));
+                    FOS_HALF_WAIT(LSTEP * (kSlotsA - 2) + (w >= 1 ? LCHUNK : 0));
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[j & 1], fa[set][i], acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(IF4 ? fb[set][IF4 ? j : 0] : fb[j & 1][0], fa[set][i], acc[i][j], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 // conversion of the next fragment of B: the next columns of this step, or the first ones of the next step
-                if constexpr (i % (WM / 4) == 0) {
+                if constexpr (!IF4 && i % (WM / 4) == 0) {
                     constexpr int jn = (j + 1) % WN, wn_next = j + 1 == WN ? (w + 1) & 3 : w, from = j + 1 == WN && w == 3 ? CUR ^ 1 : CUR;
                     if constexpr (from != CUR && i == 0) widen_scales(c + 1, from);
-                    convert(std::integral_constant<int, i / (WM / 4)>{}, fb[(j & 1) ^ 1], from, jn, wn_next);
+                    convert(std::integral_constant<int, i / (WM / 4)>{}, fb[(j & 1) ^ 1][0], from, jn, wn_next);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 if constexpr (m >= BAR) {
                     // the reads of step k + 1, spread; ahead of the last step's the next chunk's codes and scales, which
                     // are converted from the last columns on
-                    constexpr int x = m - BAR, nb = w == 3 ? 2 * WN : 0, reads = WM + nb, span = (w == 3 ? 3 * WM - 2 : MFMAS) - BAR;
+                    constexpr int x = m - BAR, nb = !IF4 && w == 3 ? 2 * WN : 0, reads = READS + nb, span = (nb ? 3 * WM - 2 : MFMAS) - BAR;
                     constexpr int first = x * reads / span < reads ? x * reads / span : reads,
                                   end = (x + 1) * reads / span < reads ? (x + 1) * reads / span : reads;
                     static_for<first, end>([&](auto tc) {
                         constexpr int t = decltype(tc)::value;
-                        if constexpr (t < nb) read_b(slot_b ^ 1, CUR ^ 1, t);
-                        else read_a((w + 1) & 3, set ^ 1, t - nb);
+                        if constexpr (t < nb) read_chunk(slot_b ^ 1, CUR ^ 1, t);
+                        else read_step((w + 1) & 3, set ^ 1, IF4 ? (t + WM) % READS : t - nb);  // (IF4: B's first)
                         __builtin_amdgcn_sched_barrier(0);
                     });
-                    constexpr int gap = WM == 8 ? 4 : 2;
-                    if constexpr (x == 1 || (LA == 2 && x == 1 + gap)) {
-                        load_a(k_next, w, x == 1 ? 0 : 1);
+                    constexpr int gap = IF4 ? 2 : WM == 8 ? 4 : 2;
+                    if constexpr (x >= 1 && (x - 1) % gap == 0 && (x - 1) / gap < LSTEP) {
+                        load_step(k_next, w, (x - 1) / gap);
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                    if constexpr (w == 0 && x >= 2 + gap && x < 2 + gap + LB + LS) {
-                        load_b(c_next, slot_b, x - 2 - gap);
+                    constexpr int behind = 2 + gap * (LSTEP - 1);
+                    if constexpr (w == 0 && x >= behind && x < behind + LCHUNK) {
+                        load_b(c_next, slot_b, x - behind);
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                    static_assert(BAR + 2 + gap + LB + LS <= MFMAS && span > 0, "room for the loads and reads behind the barrier");
+                    static_assert(BAR + behind + LCHUNK <= MFMAS && span > 0, "room for the loads and reads behind the barrier");
                 }
             });
         });
@@ -345,7 +359,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
 
 template <int WAVES_M, int WAVES_N, int WM, int BAR, int OCC, bool IF4>
 static int launch_tiles(GemmParams &p, int out_type, hipStream_t s) {
-    constexpr int BM = 16 * WM * WAVES_M, BN = 64 * WAVES_N, lds_bytes = half_lds_bytes(BM, BN);
+    constexpr int BM = 16 * WM * WAVES_M, BN = 64 * WAVES_N, lds_bytes = half_lds_bytes(BM, BN, IF4);
     p.tiles_m = (int)((p.M + BM - 1) / BM);
     p.tiles_n = (int)((p.N + BN - 1) / BN);
     auto kernel = p.splits > 1             ? gemm_half_kernel<WAVES_M, WAVES_N, WM, BAR, OCC, kOutPartial, IF4>

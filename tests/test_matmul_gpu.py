@@ -949,3 +949,15 @@ def test_layer_with_operands_written_by_the_quantizer(monkeypatch, tokens, inf, 
     # (the product rounded to the output type, then the sum)
     bound = 2.0 ** -8 * (exact.abs() + (a @ b.T).abs()) * (1 + 2.0 ** -8) + 2 * inf * 2.0 ** -24 * size
     assert bool(((out.double() - exact).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("tile", ["1001", "1002", "1003"])
+@pytest.mark.parametrize(("m", "n", "k"), [(128, 128, 64), (384, 640, 192), (300, 200, 1088), (256, 256, 128)])
+def test_if4_product_with_both_operands_converted_ahead(monkeypatch, m, n, k, tile):
+    """The same codes, scales and bounds as the kernels that convert in the loop, whole and split."""
+    test_if4_gemm_over_all_codes_and_scales(monkeypatch, m, n, k, tile, (1.0, 7.5) if k != 128 else (2.0 ** -100, 2.0 ** -20))
+    monkeypatch.setenv("FOS_GEMM_SPLITK", "2")
+    test_if4_gemm_over_all_codes_and_scales(monkeypatch, m, n, k, tile, (1.0, 1.0))
+    for depth in (16, 112, 127, 192, 336):
+        test_if4_product_leaves_out_the_padding_of_the_inner_dimension(monkeypatch, depth, {"FOS_GEMM_TILE": tile})
+    test_if4_product_is_contiguous(monkeypatch, 257, 392, {"FOS_GEMM_TILE": tile})
