@@ -41,6 +41,7 @@ EXPORTS = (
     "fos_gemm_nvfp4_amax_out",
     "fos_gemm_nvfp4_linear",
     "fos_linear_nvfp4",
+    "fos_linear_nvfp4_into_zero",
     "fos_linear_nvfp4_rows",
     "fos_linear_nvfp4_scratch_bytes",
     "fos_gemm_if4",
@@ -115,6 +116,8 @@ def lib() -> ctypes.CDLL:
     L.fos_gemm_nvfp4_linear.restype = i32
     L.fos_linear_nvfp4.argtypes = [vp, i32, i64, i64, i64, i32, vp, vp, vp, vp, dbl, i64, vp, i32, i64, vp, vp, vp, ctypes.c_size_t, vp]
     L.fos_linear_nvfp4.restype = i32
+    L.fos_linear_nvfp4_into_zero.argtypes = [vp, i32, i64, i64, i64, i32, vp, vp, vp, vp, dbl, i64, vp, i32, i64, vp, vp, i32, vp, ctypes.c_size_t, vp]
+    L.fos_linear_nvfp4_into_zero.restype = i32
     L.fos_linear_nvfp4_rows.argtypes = [i64, i64]
     L.fos_linear_nvfp4_rows.restype = i64
     L.fos_linear_nvfp4_scratch_bytes.argtypes = [i64, i64, i64]

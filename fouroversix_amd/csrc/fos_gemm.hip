@@ -37,10 +37,12 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "fos_buffer.h"
 #include "fos_device.h"
 #include "fos_gemm_common.h"
 #include "fos_gemm_half.h"
 #include "fos_gemm_tiles.h"
+#include "fos_quantize_fast.h"
 #include "fos_tuning.h"
 #include "fouroversix_hip.h"
 
@@ -48,13 +50,6 @@ namespace fos {
 
 constexpr int BK = 64;
 constexpr int kPitch = BK + 8;  // halfs per LDS row (144 bytes: conflict-free 128-bit accesses)
-
-// Buffer resource (V#) over [base, base + bytes): raw 32-bit offsets, no swizzle.
-typedef __amdgpu_buffer_rsrc_t BufferRsrc;
-typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
-FOS_DEVICE BufferRsrc make_rsrc(const void *base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
-}
 
 // Packed operands of one K step as a thread holds them: the half row of A that it turns into
 // fp16 in LDS for the whole workgroup, and, per 32-row tile of its wavefront's B columns, the
@@ -744,6 +739,15 @@ __global__ __launch_bounds__(64 * skinny_waves(WN), (WN == 2 && MT == 2) ? 2 : 1
 // NB = 1 halves the workgroup to 16 rows (n128 + 32 q + r0 + i, i = 0..3, r0 = 4 (blockIdx.x % 8);
 // lane row c: q = c >> 2, i = c & 3): twice the workgroups for narrow outputs (N <= 4096), which
 // would otherwise split K and pay a reduction kernel.  acc[0][e] is then D[c][n128 + 32 g + r0 + e].
+// NB = 4 doubles it to 64 rows (n128 + 32 b + r0 + c, r0 = 16 (blockIdx.x % 2)): acc[b][e] is D[c][n128 + 32 b + r0 + 4 g + e].
+//
+// RULE >= 0: a layer's call in one launch.  A is x, bf16, quantized here (1x16 blocks, round to nearest, scale rule RULE):
+// every workgroup finds the tensor's maximum (or is given it), quantizes the columns of its share of K and keeps them in LDS as
+// fp16(value * scale) in the order the matrix instructions read them.  A kernel of its own in front cost a launch, its
+// latency and, at 16 rows, 9 us in which 64 workgroups scanned the tensor while the weight could have been on its way: here
+// it is in flight behind x.  What each workgroup quantizes again is what bounds it, so K is split
+// where that is more than kFusedElements (plan_decode).  Layers, us a call / in a graph: 1 x 4096 -> 4096 14.4 / 12.6 -> 12.1 / 11.0,
+// 16 x 4096 -> 4096 17.6 / 15.3 -> 14.9 / 16.4, 1 x 14336 -> 4096 19.2 / 17.7 -> 13.1 / 13.5.
 template <int NB>
 struct DecodeRegs {
     uint4 b[NB][2];   // 64 codes of NB rows of B
@@ -751,14 +755,129 @@ struct DecodeRegs {
     uint32_t sb[NB];  // their scale groups (NB = 2: adjacent words of one 16-byte unit)
     uint32_t sa;
 };
+struct DecodeInput {
+    const uint16_t *x;    // [M, cols], contiguous rows of whole 16-byte units
+    const float *amax;    // max|x| if known, or null
+    int64_t cols;         // a multiple of 16, padded to K with zeros
+    float c, qdiv, errdiv;
+    float *amax_out, *zero_out;  // with splits: the maximum, for the reduction; set to 0 here, the reduction folds a maximum into it
+};
+constexpr int decode_reduce_bytes(int NB) { return 4 * (4 * NB) * 64 * (int)sizeof(float); }
+constexpr int kDecodeSetupBytes = 256 * (int)sizeof(FastLutEntry) + 64;
 
-template <int NB, int OUT>
-__global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams p) {
+// x[0 .. M) quantized, columns 256 s_begin ... 256 s_end, to `frags`: 16-byte units [step][slice x][lane group g][row].
+// In two parts, between which the caller asks for the weight: loads return in order, and the chain that begins with x is the
+// longer one.
+struct DecodeQuantizer {
+    static constexpr int kThreadsQ = 512;
+    const DecodeInput &in;
+    int M, per_row, blocks, block0;  // blocks of a row and of all rows in this share of K, the first one's column
+    bool few;                        // (K unsplit and few blocks: those a thread loads first are the tensor)
+    Block16 first[2];                // the first blocks this thread quantizes
+    uint32_t bytes;                  // of the tensor
+    float known;                     // the maximum where it is given
+    uint32_t m = 0;                  // magnitude bits of two columns' maxima, over what this thread scanned
+
+    // (buffer loads: what lies past the tensor reads as zeros without a branch, and a load under a branch is waited for there)
+    FOS_DEVICE Block16 load(int i) const {
+        const int row = i / per_row, col = (block0 + i - row * per_row) * 16;
+        const uint32_t at = i < blocks && col < in.cols ? (uint32_t)(row * (int)in.cols + col) * 2u : 0x80000000u;
+        const BufferRsrc r = make_rsrc(in.x, bytes);
+        const u32x4 lo = __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0), hi = __builtin_amdgcn_raw_buffer_load_b128(r, at + 16u, 0, 0);
+        Block16 blk;
+        blk.w[0] = lo.x; blk.w[1] = lo.y; blk.w[2] = lo.z; blk.w[3] = lo.w;
+        blk.w[4] = hi.x; blk.w[5] = hi.y; blk.w[6] = hi.z; blk.w[7] = hi.w;
+        return blk;
+    }
+
+    // `somewhere`: a word to read in the place of a maximum that is not known
+    FOS_DEVICE DecodeQuantizer(const DecodeInput &in_, int M_, int64_t s_begin, int64_t s_end, bool all_here, const float *somewhere)
+        : in(in_), M(M_), per_row((int)(s_end - s_begin) * 16), blocks(M_ * per_row), block0((int)s_begin * 16),
+          few(all_here && blocks <= 2 * kThreadsQ), bytes((uint32_t)(M_ * in_.cols) * 2u) {
+        const int tid = threadIdx.x;
+        known = *(in.amax ? in.amax : somewhere);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) first[u] = load(tid + u * kThreadsQ);
+        if (in.amax || few) return;
+        const BufferRsrc r = make_rsrc(in.x, bytes);
+        constexpr int U = 8;  // loads in flight per thread
+        for (uint32_t base = 0; base < bytes; base += U * kThreadsQ * 16) {
+            u32x4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = __builtin_amdgcn_raw_buffer_load_b128(r, base + (uint32_t)(u * kThreadsQ + tid) * 16u, 0, 0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                m = pk_max_u16(m, v[u].x & 0x7fff7fffu);
+                m = pk_max_u16(m, v[u].y & 0x7fff7fffu);
+                m = pk_max_u16(m, v[u].z & 0x7fff7fffu);
+                m = pk_max_u16(m, v[u].w & 0x7fff7fffu);
+            }
+        }
+    }
+
+    // Returns the tensor's maximum.  `setup`: kDecodeSetupBytes of LDS.
+    template <int RULE>
+    FOS_DEVICE float quantize(uint8_t *setup, uint8_t *frags);
+};
+
+template <int RULE>
+FOS_DEVICE float DecodeQuantizer::quantize(uint8_t *setup, uint8_t *frags) {
+    FastLutEntry *lut = reinterpret_cast<FastLutEntry *>(setup);
+    uint32_t *red = reinterpret_cast<uint32_t *>(setup + 256 * sizeof(FastLutEntry));
+    const int tid = threadIdx.x;
+    uint32_t amax_bits;
+    if (in.amax) {
+        amax_bits = f2u(known);
+    } else {
+        if (few) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) m = pk_max_u16(m, first[u].w[i] & 0x7fff7fffu);
+        }
+        m = wave_max_u32((m & 0xffffu) > (m >> 16) ? (m & 0xffffu) : (m >> 16));
+        if ((tid & 63) == 0) red[tid >> 6] = m;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kThreadsQ / 64; ++w) m = red[w] > m ? red[w] : m;
+        amax_bits = m << 16;  // bf16 magnitude bits -> fp32 bits
+    }
+    QuantConsts k;
+    k.amax = u2f(amax_bits);
+    k.enc = in.c / k.amax;
+    k.dec = 1.0f / (in.c / k.amax);
+    k.qdiv = in.qdiv;
+    k.errdiv = in.errdiv;
+    k.exact_ok = k.errdiv == 1536.0f && (amax_bits & 0xffffu) == 0;
+    k.shortcut_ok = shortcut_range(k.amax);
+    const bool in_range = k.amax >= 0x1p-100f && k.amax <= 0x1p100f;
+    const float enc_fast = in_range ? k.enc : 0.0f, rq = 1.0f / k.qdiv;
+    constexpr bool kProduct = RULE == FOS_RULE_MSE;
+    if (tid < 256) lut[tid] = make_lut_entry<kProduct>(tid & 127u, k);
+    __syncthreads();
+    auto emit = [&](int i, const Block16 &blk) {
+        const int row = i / per_row, b = i - row * per_row;
+        const BlockOut o = quantize_block_nvfp4_fast<RULE, false, false, false, kProduct>(blk, k, enc_fast, rq, in_range, lut, 0, 0, 0);
+        const int unit = ((b >> 4) * 8 + 2 * (b & 3)) * 4 + ((b >> 2) & 3);
+        half8_t *dst = reinterpret_cast<half8_t *>(frags + ((size_t)unit * M + row) * 16);
+        dst[0] = dequant_word<false>(o.c0, o.s, 0);
+        dst[4 * M] = dequant_word<false>(o.c1, o.s, 0);
+    };
+    if (tid < blocks) emit(tid, first[0]);
+    if (tid + kThreadsQ < blocks) emit(tid + kThreadsQ, first[1]);
+    for (int i = tid + 2 * kThreadsQ; i < blocks; i += kThreadsQ) emit(i, load(i));
+    __syncthreads();
+    return k.amax;
+}
+
+template <int NB, int OUT, int RULE = -1>
+__global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams p, const DecodeInput in) {
     constexpr int kWaves = 8, kDepth = 3;
+    constexpr bool kFused = RULE >= 0;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
-    const int64_t n128 = (int64_t)(blockIdx.x >> (NB == 2 ? 2 : 3)) * 128;
-    const int r0 = NB == 2 ? (int)(blockIdx.x & 3) * 8 : (int)(blockIdx.x & 7) * 4;
+    const int64_t n128 = (int64_t)(blockIdx.x >> (NB == 4 ? 1 : NB == 2 ? 2 : 3)) * 128;
+    const int r0 = NB == 4 ? (int)(blockIdx.x & 1) * 16 : NB == 2 ? (int)(blockIdx.x & 3) * 8 : (int)(blockIdx.x & 7) * 4;
     const int64_t kbytes = p.K >> 1, sf_groups = p.K >> 6;
     const int64_t steps_all = p.K >> 8;
     const int64_t s_begin = OUT == kOutPartial ? (int64_t)blockIdx.y * p.ksteps_per_split : 0;
@@ -780,11 +899,13 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams
     const BufferRsrc rsb = make_rsrc(p.sfB + (n128 >> 7) * sf_groups * 512, (uint32_t)(sf_groups * 512));
     const BufferRsrc r_none = make_rsrc(p.A, 0);
     const uint32_t qa_off = (uint32_t)(c * kbytes + g * 32);
-    const uint32_t qb_off = NB == 2 ? (uint32_t)((64 * (c >> 3) + r0 + (c & 7)) * kbytes + g * 32)  // b = 1: 32 rows further
-                                    : (uint32_t)((32 * (c >> 2) + r0 + (c & 3)) * kbytes + g * 32);
+    const uint32_t qb_off = NB == 4   ? (uint32_t)((r0 + c) * kbytes + g * 32)
+                            : NB == 2 ? (uint32_t)((64 * (c >> 3) + r0 + (c & 7)) * kbytes + g * 32)  // b = 1: 32 rows further
+                                      : (uint32_t)((32 * (c >> 2) + r0 + (c & 3)) * kbytes + g * 32);
     const uint32_t sa_off = (uint32_t)(g * 512 + c * 16);
-    const uint32_t sb_off = NB == 2 ? (uint32_t)(g * 512 + (r0 + (c & 7)) * 16 + (c >> 3) * 8)
-                                    : (uint32_t)(g * 512 + (r0 + (c & 3)) * 16 + (c >> 2) * 4);
+    const uint32_t sb_off = NB == 4   ? (uint32_t)(g * 512 + (r0 + c) * 16)
+                            : NB == 2 ? (uint32_t)(g * 512 + (r0 + (c & 7)) * 16 + (c >> 3) * 8)
+                                      : (uint32_t)(g * 512 + (r0 + (c & 3)) * 16 + (c >> 2) * 4);
 
     auto fetch = [&](int64_t j, DecodeRegs<NB> &s) {
         const bool ok = j < nsteps;
@@ -795,11 +916,13 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams
 #pragma unroll
             for (int u = 0; u < 2; ++u)
                 s.b[b][u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(qb, (int)(qb_off + b * 32 * kbytes + u * 16), kq, 0));
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-            s.a[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(qa, (int)(qa_off + u * 16), kq, 0));
         load_words<NB>(s.sb, fb, (int)sb_off, ksf);
-        s.sa = __builtin_amdgcn_raw_buffer_load_b32(fa, (int)sa_off, ksf, 0);
+        if constexpr (!kFused) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                s.a[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(qa, (int)(qa_off + u * 16), kq, 0));
+            s.sa = __builtin_amdgcn_raw_buffer_load_b32(fa, (int)sa_off, ksf, 0);
+        }
     };
 
     float4_t acc[NB];
@@ -811,10 +934,15 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams
         const half2_t s2 = e4m3x2_to_half2((x & 4) ? w >> 16 : w);
         return ((x >> 1) & 1) ? __builtin_shufflevector(s2, s2, 1, 1) : __builtin_shufflevector(s2, s2, 0, 0);
     };
-    auto compute = [&](const DecodeRegs<NB> &s) {
+    // (lanes beyond the last row multiply that one again, into outputs that are not stored)
+    const uint8_t *frags = smem + decode_reduce_bytes(NB) + kDecodeSetupBytes;
+    const int a_row = g * (int)p.M + (c < (int)p.M ? c : (int)p.M - 1);
+    auto compute = [&](const DecodeRegs<NB> &s, int64_t j) {
 #pragma unroll
         for (int x = 0; x < 8; ++x) {
-            const half8_t fa = dequant8(word_of(s.a[x >> 2], x & 3), scale_of(s.sa, x));
+            half8_t fa;
+            if constexpr (kFused) fa = *reinterpret_cast<const half8_t *>(frags + (((int)(phys(j) - s_begin) * 8 + x) * 4 * (int)p.M + a_row) * 16);
+            else fa = dequant8(word_of(s.a[x >> 2], x & 3), scale_of(s.sa, x));
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 const half8_t fb = dequant8(word_of(s.b[b][x >> 2], x & 3), scale_of(s.sb[b], x));
@@ -825,16 +953,31 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams
 
     // read now, used in the epilogue: short launches would otherwise end on this latency
     float post;  // (1: NVFP4)
-    const float alpha = OUT == kOutPartial ? 0.0f : load_alpha(p, post);
+    float alpha = OUT == kOutPartial || kFused ? 0.0f : load_alpha(p, post);
+    const float amax_b = kFused && OUT != kOutPartial ? *p.amax_b : 0.0f;
 
     DecodeRegs<NB> st[kDepth];
     int64_t step = wave;  // counts this workgroup's steps, see phys()
+    auto fetch_first = [&]() {
 #pragma unroll
-    for (int d = 0; d < kDepth; ++d) fetch(step + d * kWaves, st[d]);
+        for (int d = 0; d < kDepth; ++d) fetch(step + d * kWaves, st[d]);
+    };
+    if constexpr (!kFused) {
+        fetch_first();
+    } else {
+        if (in.zero_out && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *in.zero_out = 0.0f;
+        DecodeQuantizer quantizer(in, (int)p.M, s_begin, s_end, OUT != kOutPartial, p.amax_b);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_first();
+        __builtin_amdgcn_sched_barrier(0);
+        const float amax = quantizer.template quantize<RULE>(smem + decode_reduce_bytes(NB), smem + decode_reduce_bytes(NB) + kDecodeSetupBytes);
+        alpha = (amax * amax_b) * p.inv_den;
+        if (in.amax_out && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *in.amax_out = amax;
+    }
     for (; step + (kDepth - 1) * kWaves < nsteps; step += kDepth * kWaves) {
 #pragma unroll
         for (int d = 0; d < kDepth; ++d) {
-            compute(st[d]);
+            compute(st[d], step + d * kWaves);
             // the refill goes out here: the scheduler may not collect the loads at the loop's end
             __builtin_amdgcn_sched_barrier(0);
             fetch(step + (d + kDepth) * kWaves, st[d]);
@@ -843,7 +986,7 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams
     }
 #pragma unroll
     for (int d = 0; d + 1 < kDepth; ++d)
-        if (step + d * kWaves < nsteps) compute(st[d]);  // the last, incomplete round
+        if (step + d * kWaves < nsteps) compute(st[d], step + d * kWaves);  // the last, incomplete round
 
     // tree reduction of the 8 wavefronts' accumulators (fixed order, hence deterministic)
     float *red = reinterpret_cast<float *>(smem);
@@ -869,8 +1012,9 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_decode_kernel(const GemmParams
     if (wave != 0) return;
     const bool row_ok = c < p.M;  // rows beyond M are padding of the band and are not written
 
-    const int64_t n_out = NB == 2 ? n128 + 64 * (g >> 1) + r0 + 4 * (g & 1)  // column of acc[0][0]; acc[1] is 32 further
-                                  : n128 + 32 * g + r0;
+    const int64_t n_out = NB == 4   ? n128 + r0 + 4 * g                        // column of acc[0][0]; acc[b] is 32 b further
+                          : NB == 2 ? n128 + 64 * (g >> 1) + r0 + 4 * (g & 1)
+                                    : n128 + 32 * g + r0;
     if (OUT == kOutPartial) {
         float *P = p.partials + (int64_t)blockIdx.y * p.M * p.N;
         if (row_ok) {
@@ -971,11 +1115,25 @@ static int launch_skinny(GemmParams &p, int out_type, hipStream_t s, int row_gro
 
 template <int NB>
 static int launch_decode(GemmParams &p, int out_type, hipStream_t s) {
-    constexpr size_t lds_bytes = (size_t)4 * (4 * NB) * 64 * sizeof(float);
+    constexpr size_t lds_bytes = decode_reduce_bytes(NB);
     dim3 grid((unsigned)(p.N / (16 * NB)), (unsigned)p.splits);
     auto kernel = p.splits > 1 ? gemm_nvfp4_decode_kernel<NB, kOutPartial>
                   : out_type == FOS_T_BF16 ? gemm_nvfp4_decode_kernel<NB, kOutBF16> : gemm_nvfp4_decode_kernel<NB, kOutF16>;
-    hipLaunchKernelGGL(kernel, grid, dim3(512), lds_bytes, s, p);
+    hipLaunchKernelGGL(kernel, grid, dim3(512), lds_bytes, s, p, DecodeInput{});
+    if (hipGetLastError() != hipSuccess) return FOS_E_LAUNCH;
+    return p.splits > 1 ? launch_reduce(p, out_type, s) : FOS_OK;
+}
+
+template <int NB, int RULE>
+static int launch_decode_fused(GemmParams &p, const DecodeInput &in, int out_type, hipStream_t s) {
+    const int steps = p.splits > 1 ? p.ksteps_per_split : (int)(p.K >> 8);
+    const size_t lds_bytes = (size_t)decode_reduce_bytes(NB) + kDecodeSetupBytes + (size_t)p.M * steps * 512;
+    dim3 grid((unsigned)(p.N / (16 * NB)), (unsigned)p.splits);
+    auto kernel = p.splits > 1 ? gemm_nvfp4_decode_kernel<NB, kOutPartial, RULE>
+                  : out_type == FOS_T_BF16 ? gemm_nvfp4_decode_kernel<NB, kOutBF16, RULE> : gemm_nvfp4_decode_kernel<NB, kOutF16, RULE>;
+    if (lds_bytes > 64 * 1024 && hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
+        return FOS_E_LAUNCH;
+    hipLaunchKernelGGL(kernel, grid, dim3(512), lds_bytes, s, p, in);
     if (hipGetLastError() != hipSuccess) return FOS_E_LAUNCH;
     return p.splits > 1 ? launch_reduce(p, out_type, s) : FOS_OK;
 }
@@ -1343,9 +1501,71 @@ extern "C" int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *
                            workspace_bytes, stream, if4, rows, depth, false, cols);
 }
 
+// A layer's call in one launch (splits == 1), or with K split: at most 16 rows, K in whole steps, an input that
+// every workgroup can scan, and quantize its share of.  One workgroup per compute unit: the quantization is done by
+// each of them, so there are as few as fill the chip, of 16, 32 or 64 rows of B.  Beyond 8192 columns a workgroup's share of B
+// takes longer than a launch saves (1 x 4096 -> 14336: 15.0 / 17 us a call / in a graph, two launches 15.3 / 14.4), and beyond
+// 65536 elements the quantization does (8 x 14336 -> 4096 20.5 / 22.5 and 20.3 / 20.5, 4 x 14336 17.5 / 19.4 and 25.0 / 21.1).
+struct DecodePlan {
+    int splits = 0, steps = 0, nb = 0;  // (splits 0: not taken)
+};
+constexpr int64_t kFusedElements = 16384;
+static DecodePlan plan_decode(int64_t M, int64_t N, int64_t K) {
+    DecodePlan d;
+    if (M > 16 || N % 128 || N > 8192 || K % 256 || M * K > 4 * kFusedElements || tuning().gemm_tile) return d;
+    const int64_t steps = K / 256;
+    int64_t splits = (M * K + kFusedElements - 1) / kFusedElements, most = kTargetWorkgroups / (N / 64);
+    if (most < 1) most = 1;
+    if (splits > most) splits = most;
+    if (const int forced = tuning().gemm_splitk) splits = forced;
+    if (splits > steps) splits = steps;
+    d.steps = (int)((steps + splits - 1) / splits);
+    d.splits = (int)((steps + d.steps - 1) / d.steps);
+    d.nb = N / 16 * d.splits <= kTargetWorkgroups ? 1 : N / 32 * d.splits <= kTargetWorkgroups ? 2 : 4;
+    return d;
+}
+bool fos::linear_is_one_launch(int64_t M, int64_t N, int64_t K) { return plan_decode(M, N, K).splits == 1; }
+
+template <int RULE>
+static int launch_decode_layer(GemmParams &p, const DecodeInput &in, int nb, int out_type, hipStream_t s) {
+    if (nb == 1) return launch_decode_fused<1, RULE>(p, in, out_type, s);
+    if (nb == 2) return launch_decode_fused<2, RULE>(p, in, out_type, s);
+    return launch_decode_fused<4, RULE>(p, in, out_type, s);
+}
+int fos::gemm_decode_linear(const void *x, int64_t cols, int rule, const float *x_amax, const uint8_t *B, const uint8_t *sfB,
+                            const float *amax_b, double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd,
+                            const void *bias, float *d_amax, float *amax_word, void *partials, size_t partials_bytes, fos_stream_t stream) {
+    const DecodePlan d = plan_decode(M, N, K);
+    const int splits = d.splits;
+    if (!splits || (splits > 1 && partials_bytes < (size_t)splits * (size_t)M * (size_t)N * sizeof(float))) return kNotTaken;
+    GemmParams p{};
+    p.B = B; p.sfB = sfB; p.D = D; p.bias = bias; p.d_amax = d_amax;
+    p.amax_a = x_amax ? x_amax : amax_word;  // (read by the reduction)
+    p.amax_b = amax_b;
+    p.inv_den = (float)(1.0 / denominator);
+    p.M = p.rows = M; p.N = p.cols = N; p.K = p.depth = K; p.ldd = ldd;
+    p.k_tail = 0xffffffffu;
+    p.splits = splits;
+    p.ksteps_per_split = d.steps;
+    p.partials = splits > 1 ? static_cast<float *>(partials) : nullptr;
+    DecodeInput in{static_cast<const uint16_t *>(x), x_amax, cols, 0.0f, 0.0f, 1536.0f,
+                   splits > 1 && !x_amax ? amax_word : nullptr, splits > 1 ? d_amax : nullptr};
+    const bool is_static = rule == FOS_RULE_STATIC_6 || rule == FOS_RULE_STATIC_4;
+    in.qdiv = rule == FOS_RULE_STATIC_4 ? 4.0f : 6.0f;
+    in.c = in.qdiv * (is_static ? 448.0f : 256.0f);
+    hipStream_t s = (hipStream_t)stream;
+    if (is_static) return launch_decode_layer<FOS_RULE_STATIC_6>(p, in, d.nb, out_type, s);
+    if (rule == FOS_RULE_MAE) return launch_decode_layer<FOS_RULE_MAE>(p, in, d.nb, out_type, s);
+    if (rule == FOS_RULE_MSE) return launch_decode_layer<FOS_RULE_MSE>(p, in, d.nb, out_type, s);
+    return launch_decode_layer<FOS_RULE_ABS_MAX>(p, in, d.nb, out_type, s);
+}
+
 size_t fos::linear_scratch_bytes(int64_t M, int64_t N, int64_t K) {
     const HalfPlan h = plan_half(M, N, K, false, false);
-    return h.tile ? h.bytes : fos_gemm_workspace_bytes(M, N, K);
+    if (h.tile) return h.bytes;
+    const int splits = plan_decode(M, N, K).splits;
+    const size_t other = fos_gemm_workspace_bytes(M, N, K), partials = splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+    return partials > other ? partials : other;
 }
 bool fos::linear_reads_fragments(int64_t M, int64_t N, int64_t K) { return plan_half(M, N, K, false, false).tile != 0; }
 int fos::gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,

@@ -48,4 +48,13 @@ int gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const ui
                 double denominator, int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
                 float *d_amax, void *scratch, size_t scratch_bytes, fos_stream_t stream);
 
+// A layer's call for a few rows of bf16 input (contiguous, 16-byte aligned, cols % 16 == 0), quantization included, in one
+// launch or, with K split, that and the reduction; kNotTaken where the shape is none for it.  In one launch d_amax has to be zero
+// before (or an earlier maximum to extend).
+constexpr int kNotTaken = 1;
+bool linear_is_one_launch(int64_t M, int64_t N, int64_t K);
+int gemm_decode_linear(const void *x, int64_t cols, int rule, const float *x_amax, const uint8_t *B, const uint8_t *sfB,
+                       const float *amax_b, double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd,
+                       const void *bias, float *d_amax, float *amax_word, void *partials, size_t partials_bytes, fos_stream_t stream);
+
 }  // namespace fos

@@ -548,10 +548,20 @@ extern "C" int64_t fos_linear_nvfp4_rows(int64_t rows, int64_t cols) {
     return rows <= 0 || cols <= 0 ? 0 : LinearScratch::gemm_rows(rows, cols);
 }
 
+__global__ void clear_word_kernel(float *word) { *word = 0.0f; }
+
 extern "C" int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int rule, const float *x_amax,
                                 const uint8_t *W, const uint8_t *sfW, const float *w_amax, double denominator, int64_t N,
                                 void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
                                 void *scratch, size_t scratch_bytes, fos_stream_t stream) {
+    return fos_linear_nvfp4_into_zero(x, x_type, rows, cols, ld, rule, x_amax, W, sfW, w_amax, denominator, N, D, out_type, ldd, bias, d_amax, 0,
+                                      scratch, scratch_bytes, stream);
+}
+
+extern "C" int fos_linear_nvfp4_into_zero(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int rule, const float *x_amax,
+                                          const uint8_t *W, const uint8_t *sfW, const float *w_amax, double denominator, int64_t N,
+                                          void *D, int out_type, int64_t ldd, const void *bias, float *d_amax, int d_amax_is_zero,
+                                          void *scratch, size_t scratch_bytes, fos_stream_t stream) {
     if (!scratch) return FOS_E_NULL_POINTER;
     if (rows <= 0 || cols <= 0 || N <= 0) return FOS_E_BAD_SHAPE;
     if (((uintptr_t)scratch & 255) || ((uintptr_t)d_amax & 3)) return FOS_E_BAD_ALIGNMENT;
@@ -566,6 +576,17 @@ extern "C" int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t
     const int64_t gemm_rows = LinearScratch::gemm_rows(rows, cols), depth = fos_padded_cols(cols);
     void *gemm = scratch_bytes > at.gemm ? base + at.gemm : nullptr;
     const size_t gemm_bytes = scratch_bytes - at.gemm;
+    // a few rows: quantized by the product itself (the checks of quantize_impl first)
+    if (x_type == FOS_T_BF16 && rows == gemm_rows && rows <= 16 && ld == cols && x && streamable(x, cols, ld) &&
+        rule >= FOS_RULE_STATIC_6 && rule <= FOS_RULE_ABS_MAX && !((uintptr_t)x_amax & 3) && tuning().quant_passes != 1) {
+        if (d_amax && !d_amax_is_zero && fos::linear_is_one_launch(rows, N, depth)) {
+            hipLaunchKernelGGL(clear_word_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, d_amax);
+            if (hipGetLastError() != hipSuccess) return FOS_E_LAUNCH;
+        }
+        rc = fos::gemm_decode_linear(x, cols, rule, x_amax, W, sfW, w_amax, denominator, rows, N, depth, D, out_type, ldd, bias, d_amax,
+                                     reinterpret_cast<float *>(base + at.amax), gemm, gemm_bytes, stream);
+        if (rc != fos::kNotTaken) return rc;
+    }
     // what a streaming quantize kernel reads, and the product wants converted, goes straight into the product's scratch
     const bool direct = scratch_bytes >= at.total && x_type != FOS_T_F32 && streamable(x, cols, ld) &&
                         fos::linear_reads_fragments(gemm_rows, N, depth);

@@ -115,17 +115,16 @@ FOS_DEVICE uint32_t reduce_partials(const QuantParams &p, uint32_t *smem) {
         // small contiguous input: no pass 1 was launched and every workgroup scans the
         // whole tensor itself (rows * cols / 8 aligned 128-bit vectors, 128 KiB out of L2 at
         // most), which costs less than a launch and its dependency
-        const uint4 *v4 = reinterpret_cast<const uint4 *>(p.x);
-        const int n_vec = (int)((p.rows * p.cols) >> 3);
+        // (buffer loads, zeros past the end: under a branch each load was waited for before the next was issued)
+        const uint32_t bytes = (uint32_t)(p.rows * p.cols) * 2u;
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(p.x), 0, (int)bytes, 0x00020000);
+        typedef uint32_t words4 __attribute__((ext_vector_type(4)));
         uint32_t m = 0;
         constexpr int U = 16;  // loads in flight per thread: the scan is latency-bound
-        for (int base = 0; base < n_vec; base += U * kThreads) {
-            uint4 v[U];
+        for (uint32_t base = 0; base < bytes; base += U * kThreads * 16) {
+            words4 v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = base + u * kThreads + (int)threadIdx.x;
-                v[u] = i < n_vec ? v4[i] : make_uint4(0u, 0u, 0u, 0u);
-            }
+            for (int u = 0; u < U; ++u) v[u] = __builtin_amdgcn_raw_buffer_load_b128(r, base + (uint32_t)(u * kThreads + threadIdx.x) * 16u, 0, 0);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 m = pk_max_u16(m, v[u].x & 0x7fff7fffu);

@@ -307,13 +307,13 @@ Tensor gemm_nvfp4_amax(const Tensor &a, const Tensor &b, const Tensor &a_sf, con
                        bias.has_value() ? &*bias : nullptr, rows);
 }
 
-// A word for a recorded maximum: one of a block of 4096 per (device, stream), each handed out once, so that no word is
+// A word for a recorded maximum and whether it is zero: one of a block of 4096 per (device, stream), each handed out once, so that no word is
 // overwritten while a reader may still be at work on it.  A block lives as long as one of its words is held; a reader on
 // another stream keeps it from reuse itself (the frontend's known_amax).  Inside a capture a tensor of its own (the graph's
-// private pool).
-Tensor amax_word(const Tensor &like, fos_stream_t stream) {
+// private pool), which the call clears itself where nothing else does.
+std::pair<Tensor, bool> amax_word(const Tensor &like, fos_stream_t stream) {
     const auto opts = like.options().dtype(at::kFloat);
-    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return at::empty({1}, opts);
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return {at::empty({1}, opts), false};
     constexpr int64_t kWords = 4096;
     struct Block {
         Tensor words;
@@ -324,10 +324,10 @@ Tensor amax_word(const Tensor &like, fos_stream_t stream) {
     std::lock_guard<std::mutex> lock(mutex);
     Block &b = blocks[((uint64_t)(uintptr_t)stream << 8) ^ (uint64_t)like.get_device()];
     if (b.used == kWords) {
-        b.words = at::empty({kWords}, opts);
+        b.words = at::zeros({kWords}, opts);  // (filled on this stream, ahead of every use of its words)
         b.used = 0;
     }
-    return b.words.narrow(0, b.used++, 1);
+    return {b.words.narrow(0, b.used++, 1), true};
 }
 
 // A linear layer in one call: x quantized to NVFP4 (1x16 blocks, round to nearest), times the quantized weight.  What the
@@ -352,14 +352,19 @@ std::tuple<Tensor, c10::optional<Tensor>> linear_nvfp4(const Tensor &x, int64_t 
     const DeviceGuard guard(x.device());
     const fos_stream_t stream = current_stream(x);
     c10::optional<Tensor> d_amax;
-    if (emit_amax) d_amax = amax_word(x, stream);
+    bool is_zero = false;
+    if (emit_amax) {
+        auto word = amax_word(x, stream);
+        d_amax = std::move(word.first);
+        is_zero = word.second;
+    }
     // (one block for the quantized input and the workspaces, from the caching allocator on the current stream)
     const size_t bytes = fos_linear_nvfp4_scratch_bytes(rows, cols, n);
     const Tensor scratch = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
-    check(fos_linear_nvfp4(x.data_ptr(), type_id(x.scalar_type(), "linear: x"), rows, cols, x.stride(0), (int)rule,
+    check(fos_linear_nvfp4_into_zero(x.data_ptr(), type_id(x.scalar_type(), "linear: x"), rows, cols, x.stride(0), (int)rule,
                            x_amax.has_value() ? known.data_ptr<float>() : nullptr, w.data_ptr<uint8_t>(),
                            static_cast<const uint8_t *>(w_sf.data_ptr()), w_amax.data_ptr<float>(), denominator, n, out.data_ptr(), out_type,
-                           n, bias.has_value() ? bias->data_ptr() : nullptr, emit_amax ? d_amax->data_ptr<float>() : nullptr,
+                           n, bias.has_value() ? bias->data_ptr() : nullptr, emit_amax ? d_amax->data_ptr<float>() : nullptr, is_zero ? 1 : 0,
                            scratch.data_ptr(), bytes, stream),
           "fouroversix::linear_nvfp4");
     return {out, d_amax};

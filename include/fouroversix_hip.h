@@ -295,6 +295,12 @@ int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t cols, int6
                      const uint8_t *W, const uint8_t *sfW, const float *w_amax, double denominator, int64_t N,
                      void *D, int out_type, int64_t ldd, const void *bias, float *d_amax,
                      void *scratch, size_t scratch_bytes, fos_stream_t stream);
+/* ... for a caller whose d_amax is zero already (d_amax_is_zero != 0): a call of few rows, which runs in one launch, then
+ * needs no other one to clear it. */
+int fos_linear_nvfp4_into_zero(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int rule, const float *x_amax,
+                               const uint8_t *W, const uint8_t *sfW, const float *w_amax, double denominator, int64_t N,
+                               void *D, int out_type, int64_t ldd, const void *bias, float *d_amax, int d_amax_is_zero,
+                               void *scratch, size_t scratch_bytes, fos_stream_t stream);
 
 /*
  * IF4 x IF4 product: as fos_gemm_nvfp4_linear for operands in the IF4 format (row-major scale bytes, bit 7 = integer

@@ -961,3 +961,51 @@ def test_if4_product_with_both_operands_converted_ahead(monkeypatch, m, n, k, ti
     for depth in (16, 112, 127, 192, 336):
         test_if4_product_leaves_out_the_padding_of_the_inner_dimension(monkeypatch, depth, {"FOS_GEMM_TILE": tile})
     test_if4_product_is_contiguous(monkeypatch, 257, 392, {"FOS_GEMM_TILE": tile})
+
+
+@pytest.mark.parametrize("rule", ["static_6", "static_4", "mse", "mae", "abs_max"])
+@pytest.mark.parametrize(("tokens", "inf", "outf", "scale"), [
+    (1, 256, 128, 1.0), (1, 4096, 4096, 1.0), (3, 2032, 384, 1.0),  # one launch; a width that ends inside a step
+    (5, 8192, 256, 1.0), (16, 4096, 1024, 1.0), (16, 1024, 8192, 1.0),  # K split, 64 rows of the weight a workgroup
+    (16, 768, 2176, 1.0),                                               # 32 rows
+    (2, 512, 256, 2.0 ** -115), (2, 512, 256, 0.0),                     # outside the fast range; zeros
+])
+def test_layer_of_few_rows_in_one_launch(tokens, inf, outf, scale, rule):
+    """Quantization and product in one kernel: the product of what the quantizer writes, with the bias, the recorded maximum
+    and a maximum recorded on the input; twice, so that a word that is not zero would show.  Bounds as for the layers above."""
+    from fouroversix_amd.quantize import attach_known_amax, known_amax
+
+    g = torch.Generator("cpu").manual_seed(tokens + inf + outf)
+    model = nn.Sequential(nn.Linear(inf, outf, device="cuda", dtype=torch.bfloat16))
+    with torch.no_grad():
+        model[0].bias.mul_(scale)
+    fos.quantize_model(model, fos.ModelQuantizationConfig(activation_scale_rule=rule))
+    model[0].quantize_weight_()
+    for part in range(2):
+        x = (torch.randn(tokens, inf, generator=g) * scale).bfloat16()
+        x[:, part::7] *= 8
+        x = x.cuda()
+        qx = fos.quantize(x, fos.QuantizationConfig(scale_rule=rule))
+        if part:
+            attach_known_amax(x, qx.amax.clone())
+        with torch.no_grad():
+            out = model(x)
+        assert out.shape == (tokens, outf) and float(known_amax(out)) == float(out.abs().max())
+        a, b = (fos.dequantize(q, dtype=torch.float32).double() for q in (qx, model[0].quantized_weight()))
+        product, size = a @ b.T, a.abs() @ b.abs().T
+        exact = product + model[0].bias.double()
+        bound = 2.0 ** -8 * (exact.abs() + product.abs()) * (1 + 2.0 ** -8) + 2 * inf * 2.0 ** -24 * size + 2.0 ** -133
+        assert bool(((out.double() - exact).abs() <= bound).all())
+
+
+def test_layer_of_few_rows_with_an_element_that_is_no_number():
+    for value in (float("nan"), float("inf")):
+        model = nn.Sequential(nn.Linear(512, 256, bias=False, device="cuda", dtype=torch.bfloat16))
+        fos.quantize_model(model, fos.ModelQuantizationConfig())
+        model[0].quantize_weight_()
+        x = make_input("randn", (3, 512), 91).cuda()
+        x[1, 100] = value
+        with torch.no_grad():
+            out = model(x)
+        expect = fos.quantized_matmul(fos.quantize(x), model[0].quantized_weight())
+        assert torch.equal(out.isnan(), expect.isnan()) and torch.equal(out.isinf(), expect.isinf())
