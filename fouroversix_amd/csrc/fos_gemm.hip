@@ -1181,7 +1181,7 @@ static int pick_tile(int64_t M, int64_t N, int forced) {
 static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool if4) {
     GemmPlan g;
     g.narrow = g.wide = 0;
-    const int tile = tuning().gemm_tile;  // tuning / tests: 128 = small tile, 129 = 128 x 256 tile, 256 = 256 x 256 tile, 1 = no weight-streaming kernel
+    const int tile = tuning().gemm_tile > 1000 ? 0 : (int)tuning().gemm_tile;  // tuning / tests: 128 = small tile, 129 = 128 x 256 tile, 256 = 256 x 256 tile, 1 = no weight-streaming kernel
     int64_t steps, tiles;
     if (!if4 && M <= 128 && K % 256 == 0 && (tile == 0 || tile == 16 || tile == 32 || tile == 64)) {
         // one 128-row band: weight streaming, steps of 256 along K shared by 8 wavefronts
@@ -1259,7 +1259,17 @@ static float half_cost(int tile, int64_t tiles, float k) {
 static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand) {
     HalfPlan h;
     const int forced = tuning().gemm_tile;  // tuning / tests: 1000 + tile; another kernel's tile excludes this one
-    if (M < 128 || M % 128 || N % 128 || K % 64 || K > (1 << 20) || (forced && forced <= 1000) || (!forced && M < 256)) return h;
+    if ((M > 128 && M % 128) || N % 128 || K % 64 || K > (1 << 20) || (forced && forced <= 1000)) return h;
+    // 65 ... 128 rows: the streaming form where K is long and the outputs are narrow, in as many splits as leave a wavefront two
+    // chunks.  Products with the fragments given, and of packed operands (us), 128 rows: 14336 -> 4096 23.5 and 28.5,
+    // 14336 -> 1024 17.6 and 21.3, but 4096 -> 4096 15.2 and 14.3, 14336 -> 8192 36.6 and 36.4; of fewer rows whole layers
+    // are slower with it (64 x 4096 -> 4096 19.6 and 17.8 in a graph).
+    const bool streams = M > 64 && M <= 128 && N <= 4096 && K >= 8192 && !if4 && !expand;
+    if (forced == 1000 + kHalfStream) {
+        if (M <= 64 || M > 128 || if4) return h;
+    } else if (M < 128 || (M == 128 && !forced)) {
+        if (!streams) return h;
+    }
     if (fragment_bytes(M, K) > ((size_t)8 << 30)) return h;  // (a call with an operand that large keeps to the smaller workspace)
     const int64_t chunks = (K + 127) / 128, m128 = M / 128, n128 = N / 128, m256 = (m128 + 1) / 2, n256 = (n128 + 1) / 2;
     const int forced_splits = tuning().gemm_splitk;
@@ -1267,6 +1277,12 @@ static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand
     if (forced) {
         h.tile = forced - 1000;
         splits = forced_splits > 0 ? forced_splits : 1;
+    } else if (M <= 128) {
+        h.tile = kHalfStream;
+        splits = kTargetWorkgroups / (N / 64) < chunks / 8 ? kTargetWorkgroups / (N / 64) : chunks / 8;
+        if (splits > 8) splits = 8;
+        if (forced_splits > 0) splits = forced_splits;
+        if (splits < 1) splits = 1;
     } else {
         float best = 3e38f;
         for (int tile = kHalf256; tile <= kHalfSmall; ++tile) {

@@ -31,8 +31,9 @@ struct ExpandParams {
 };
 int launch_expand_fragments(ExpandParams p, bool if4, hipStream_t s);
 
-// Output tiles of the product: 256 x 256 (eight wavefronts), 128 x 256 and 128 x 128 (four).
-enum { kHalf256 = 1, kHalfWide, kHalfSmall };
+// Output tiles of the product: 256 x 256 (eight wavefronts), 128 x 256 and 128 x 128 (four); kHalfStream: up to 128 rows
+// (NVFP4), the weight streamed once.
+enum { kHalf256 = 1, kHalfWide, kHalfSmall, kHalfStream };
 // p: frags, B, sfB (NVFP4), or frags and frags_b (IF4), ... ; with splits > 1 every split takes ksteps_per_split chunks of 128 k and the caller sums the partials.
 int launch_gemm_half(GemmParams &p, int tile, bool if4, int out_type, hipStream_t s);
 

@@ -357,6 +357,137 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// M <= 128: the weight is streamed once, a workgroup owns 64 columns (and a share of K, blockIdx.y), its four wavefronts take
+// the chunks of K in turn, each with all rows: 128 rows x 64 columns of accumulators a wavefront, one wavefront per SIMD.  Nothing
+// is shared in the loop: fragments of A are whole KiB out of L2 into registers, B's codes 64 contiguous bytes of 16
+// rows, both a chunk ahead, no barrier.  A kernel that reads A packed is bound by its conversion, which every 64 columns
+// repeat (gemm_nvfp4_skinny_kernel); this one by what a compute unit reads of A out of L2, about 30 bytes a cycle.
+// (Eight wavefronts with A a step ahead: 24.5 us at 128 x 4096 x 14336 in four splits, 23.5 here.)
+// The accumulators are summed over the wavefronts in two halves through LDS, in fixed order.
+template <int OUT>
+__global__ __launch_bounds__(256, 1) void gemm_half_stream_kernel(const GemmParams p) {
+    constexpr bool OUT_BF16 = OUT == kOutBF16;
+    constexpr int WM = 8, WN = 4, kWaves = 4, HALF = WM * WN / 2;  // HALF: groups of four accumulators a lane hands over at a time
+    extern __shared__ __attribute__((aligned(16))) uint8_t half_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), q = lane >> 4;
+    const int64_t n0 = (int64_t)blockIdx.x * 64;
+    const int chunks_all = (int)((p.K + 127) >> 7);
+    const int c0 = OUT == kOutPartial ? (int)blockIdx.y * p.ksteps_per_split : 0;
+    const int c1 = OUT == kOutPartial ? (c0 + p.ksteps_per_split < chunks_all ? c0 + p.ksteps_per_split : chunks_all) : chunks_all;
+    const uint32_t kbytes = (uint32_t)(p.K >> 1), scale_band = (uint32_t)p.K * 8u;
+    const BufferRsrc ra = make_rsrc(p.frags, (uint32_t)chunks_all * kBandChunkBytes);
+    const BufferRsrc rb = make_rsrc(p.B + n0 * kbytes, 64u * kbytes);
+    const BufferRsrc rs = make_rsrc(p.sfB + (n0 >> 7) * (int64_t)scale_band, scale_band);
+    const uint32_t va = lane * 16, vb = (lane & 15) * kbytes + q * 16;
+    // (rows n0 % 128 + 16 j + (lane & 15): two adjacent words of 32-row groups, 256 bytes apart for the odd j)
+    const uint32_t vs = (q >> 1) * 512 + (lane & 15) * 16 + ((uint32_t)(n0 & 127) >> 5) * 4 + (q & 1) * 2;
+
+    half8_t fa[4][WM];  // a chunk; refilled one at a time with the next chunk's, behind the matrix instructions that read it last
+    u32x4 codes[2][WN];
+    uint32_t scales[2][WN];
+    auto load_a = [&](int chunk, int w, int i) {
+        const uint32_t at = (uint32_t)chunk * kBandChunkBytes + (uint32_t)w * kFragmentStep;
+        fa[w][i] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(va + i * 1024), (int)at, 0));
+    };
+    auto load_b = [&](int chunk, int set) {
+#pragma unroll
+        for (int j = 0; j < WN; ++j) codes[set][j] = __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(vb + j * 16 * kbytes), chunk * 64, 0);
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+            scales[set][j] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)(vs + (j & 1) * 256 + (j >> 1) * 4), chunk * 1024, 0);
+    };
+    const uint32_t last_mask = tail_mask((int)((p.depth - (int64_t)(chunks_all - 1) * 128 + 15) >> 4) - 2 * q);
+
+    float4v acc[WM][WN];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // (past the end: the last chunk once more, which nobody multiplies)
+    auto clamp = [&](int c) { return c < c1 ? c : c1 - 1; };
+    load_b(clamp(c0 + wave), 0);
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+        for (int i = 0; i < WM; ++i) load_a(clamp(c0 + wave), w, i);
+    auto chunk_steps = [&](int c, auto cur_c) {
+        constexpr int CUR = decltype(cur_c)::value;
+        load_b(clamp(c + kWaves), CUR ^ 1);
+        half2_t s2[WN];
+        const uint32_t mask = c + 1 == chunks_all ? last_mask : 0xffffu;
+#pragma unroll
+        for (int j = 0; j < WN; ++j) s2[j] = e4m3x2_to_half2(scales[CUR][j] & mask);
+        static_for<0, 4>([&](auto wc) {
+            constexpr int w = decltype(wc)::value;
+            half8_t fb[WN];
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                const uint32_t word = w == 0 ? codes[CUR][j].x : w == 1 ? codes[CUR][j].y : w == 2 ? codes[CUR][j].z : codes[CUR][j].w;
+                fb[j] = dequant8(word, w >= 2 ? __builtin_shufflevector(s2[j], s2[j], 1, 1) : __builtin_shufflevector(s2[j], s2[j], 0, 0));
+            }
+#pragma unroll
+            for (int i = 0; i < WM; ++i) {
+#pragma unroll
+                for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[j], fa[w][i], acc[i][j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                load_a(clamp(c + kWaves), w, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        });
+    };
+    int c = c0 + wave;
+    for (; c + kWaves < c1; c += 2 * kWaves) {
+        chunk_steps(c, std::integral_constant<int, 0>{});
+        chunk_steps(c + kWaves, std::integral_constant<int, 1>{});
+    }
+    if (c < c1) chunk_steps(c, std::integral_constant<int, 0>{});
+
+    // Sum over the wavefronts: of either half of the rows' fragments every wavefront leaves its HALF groups in LDS, then sums
+    // its share of them over all wavefronts in order and stores those.
+    float post;
+    const float alpha = OUT == kOutPartial ? 0.0f : load_alpha(p, post);
+    constexpr int kMine = HALF / kWaves;
+    uint32_t umax = 0u;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < HALF; ++f)
+            *reinterpret_cast<float4v *>(half_lds + ((wave * HALF + f) * 64 + lane) * 16) = acc[h * (WM / 2) + f / WN][f % WN];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < kMine; ++u) {
+            const int f = wave * kMine + u, i = h * (WM / 2) + f / WN, j = f % WN;
+            float4v sum = *reinterpret_cast<const float4v *>(half_lds + (f * 64 + lane) * 16);
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) sum += *reinterpret_cast<const float4v *>(half_lds + ((w * HALF + f) * 64 + lane) * 16);
+            const int64_t m = 16 * i + (lane & 15), n = n0 + 16 * j + 4 * q;
+            if (m >= p.M) continue;
+            if (OUT == kOutPartial) {
+                *reinterpret_cast<float4v *>(p.partials + ((int64_t)blockIdx.y * p.M + m) * p.N + n) = sum;
+            } else {
+                const float v[4] = {alpha * sum[0], alpha * sum[1], alpha * sum[2], alpha * sum[3]};
+                uint32_t um = 0u;
+                *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(p.D) + m * p.ldd + n) = pack_outputs<OUT_BF16>(v, p.bias, n, um);
+                if (m < p.rows) umax = max_pairs(umax, um);
+            }
+        }
+    }
+    if (OUT != kOutPartial && p.d_amax) {
+        __syncthreads();
+        fold_amax<OUT_BF16, kWaves>(p.d_amax, umax, reinterpret_cast<uint32_t *>(half_lds));
+    }
+}
+
+static int launch_stream(GemmParams &p, int out_type, hipStream_t s) {
+    constexpr int lds_bytes = 64 * 1024;  // half the accumulators of four wavefronts
+    auto kernel = p.splits > 1 ? gemm_half_stream_kernel<kOutPartial> : out_type == FOS_T_BF16 ? gemm_half_stream_kernel<kOutBF16> : gemm_half_stream_kernel<kOutF16>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(p.N / 64), (unsigned)p.splits), dim3(256), lds_bytes, s, p);
+    return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;
+}
+
 template <int WAVES_M, int WAVES_N, int WM, int BAR, int OCC, bool IF4>
 static int launch_tiles(GemmParams &p, int out_type, hipStream_t s) {
     constexpr int BM = 16 * WM * WAVES_M, BN = 64 * WAVES_N, lds_bytes = half_lds_bytes(BM, BN, IF4);
@@ -377,6 +508,7 @@ int launch_gemm_half(GemmParams &p, int tile, bool if4, int out_type, hipStream_
         if (tile == kHalfWide) return launch_tiles<1, 4, 8, 12, 2, true>(p, out_type, s);
         return launch_tiles<2, 2, 4, 4, 2, true>(p, out_type, s);
     }
+    if (tile == kHalfStream) return launch_stream(p, out_type, s);
     if (tile == kHalf256) return launch_tiles<2, 4, 8, 12, 2, false>(p, out_type, s);
     if (tile == kHalfWide) return launch_tiles<1, 4, 8, 12, 2, false>(p, out_type, s);
     return launch_tiles<2, 2, 4, 4, 2, false>(p, out_type, s);

@@ -923,10 +923,17 @@ def test_product_with_a_converted_ahead(monkeypatch, m, n, k, tile, splits):
         assert float(known_amax(with_bias)) == float(with_bias.abs().max())
 
 
+@pytest.mark.parametrize("splits", ["1", "3"])
+@pytest.mark.parametrize(("tokens", "n", "k"), [(65, 128, 256), (100, 384, 2560), (127, 256, 8192), (128, 256, 64), (128, 128, 1600)])
+def test_streaming_product_with_a_converted_ahead(monkeypatch, tokens, n, k, splits):
+    """The form for up to 128 rows: padding rows, fewer chunks of K than wavefronts and more, half a chunk at the end."""
+    test_product_with_a_converted_ahead(monkeypatch, tokens, n, k, "1004", splits)
+
+
 @pytest.mark.parametrize("quant_split", ["1", "2"])
 @pytest.mark.parametrize("rule", ["static_6", "mse", "mae", "abs_max"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize(("tokens", "inf"), [(130, 64), (256, 1040), (384, 512), (257, 4096)])
+@pytest.mark.parametrize(("tokens", "inf"), [(130, 64), (256, 1040), (384, 512), (257, 4096), (100, 8192), (128, 8320)])
 def test_layer_with_operands_written_by_the_quantizer(monkeypatch, tokens, inf, dtype, rule, quant_split):
     """An aligned input is quantized straight into the product's operand; the same values at an odd address become codes and
     scales first, which are then converted: the same bits, and the codes' own product within a rounding."""
