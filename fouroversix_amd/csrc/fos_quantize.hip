@@ -293,6 +293,21 @@ void launch_typed(QuantParams &p, bool two_d, hipStream_t s) {
     else hipLaunchKernelGGL((quantize_kernel<false, DT, RULE, ROUND, false, 1, false>), grid, dim3(kThreads), 0, s, p);
 }
 
+void launch_nvfp4_tiles(QuantParams &p, int rule, hipStream_t s) {
+    const bool f16 = p.x_type == FOS_T_F16;
+    switch (rule) {
+        case FOS_RULE_STATIC_6:
+        case FOS_RULE_STATIC_4:
+            return f16 ? launch_quantize_nvfp4_tiles_f16<FOS_RULE_STATIC_6>(p, s) : launch_quantize_nvfp4_tiles<FOS_RULE_STATIC_6, false, false>(p, s);
+        case FOS_RULE_MAE:
+            return f16 ? launch_quantize_nvfp4_tiles_f16<FOS_RULE_MAE>(p, s) : launch_quantize_nvfp4_tiles<FOS_RULE_MAE, false, false>(p, s);
+        case FOS_RULE_MSE:
+            return f16 ? launch_quantize_nvfp4_tiles_f16<FOS_RULE_MSE>(p, s) : launch_quantize_nvfp4_tiles<FOS_RULE_MSE, false, false>(p, s);
+        default:
+            return f16 ? launch_quantize_nvfp4_tiles_f16<FOS_RULE_ABS_MAX>(p, s) : launch_quantize_nvfp4_tiles<FOS_RULE_ABS_MAX, false, false>(p, s);
+    }
+}
+
 template <int DT, int RULE>
 void dispatch_round(QuantParams &p, int round_style, bool two_d, bool aligned, hipStream_t s) {
     if (p.x_type != FOS_T_BF16 && !(aligned && p.x_type == FOS_T_F16)) {
@@ -383,9 +398,8 @@ extern "C" int fos_pseudo_quantize_is_fused(int x_type, int dtype, int rule, int
 // The streaming kernels address a 128-row tile with 32-bit byte offsets: a row pitch of 2^23
 // elements or more (16 MiB rows) takes the element-wise kernel like an unaligned input.
 constexpr int64_t kMaxPitch = int64_t{1} << 23;
-static bool streamable(const void *x, int64_t cols, int64_t ld) {
-    return ((uintptr_t)x & 15) == 0 && ld % 8 == 0 && cols % 16 == 0 && ld < kMaxPitch;
-}
+static bool aligned_rows(const void *x, int64_t ld) { return ((uintptr_t)x & 15) == 0 && ld % 8 == 0 && ld < kMaxPitch; }
+static bool streamable(const void *x, int64_t cols, int64_t ld) { return aligned_rows(x, ld) && cols % 16 == 0; }
 
 // Shared body of fos_quantize and fos_pseudo_quantize (frags != null: fragments of a product's operand; pseudo_out != null: bf16 round trip
 // instead of codes / scales).
@@ -477,6 +491,11 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
 
     if (tuning().quant_passes == 1) return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;  // timing runs: pass 1 alone
 
+    // 16x16 tiles of NVFP4, round to nearest: fp16 elements, and (either type) a row that ends with half a block, have the
+    // streaming form too where the maximum is not the caller's (elements beyond it may be NaN)
+    const bool tiles = block2d && dtype == FOS_DTYPE_NVFP4 && round_style == FOS_ROUND_NEAREST && !pseudo_out && x_type != FOS_T_F32 &&
+                       !amax_is_input && cols % 8 == 0 && aligned_rows(x, ld);
+
     // (qmax, smax): static_6 (6,448); static_4 (4,448); adaptive NVFP4 (6,256); IF4 (6,448).
     const double adj = round_style == FOS_ROUND_STOCHASTIC_UNBIASED ? 16.0 / 17.0 : 1.0;
     const double qmax = rule == FOS_RULE_STATIC_4 ? 4.0 : 6.0;
@@ -487,6 +506,10 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
     p.errdiv = dtype == FOS_DTYPE_IF4 ? (float)(6.0 * 448.0 * adj) : (float)(6.0 * 256.0 * adj);
 
     const bool two_d = block2d != 0;
+    if (tiles && !aligned) {
+        launch_nvfp4_tiles(p, rule, s);
+        return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;
+    }
     if (dtype == FOS_DTYPE_IF4) {
         switch (rule) {
             case FOS_RULE_MAE: dispatch_round<FOS_DTYPE_IF4, FOS_RULE_MAE>(p, round_style, two_d, aligned, s); break;

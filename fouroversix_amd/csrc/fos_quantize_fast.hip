@@ -319,10 +319,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
     }
 }
 
-// 16x16 tiles on the row-contiguous mapping (fos_quantize_tiles.hip): every rule and rounding style.
-template <int RULE, bool PSEUDO, bool SR>
-void launch_quantize_nvfp4_tiles(QuantParams &p, hipStream_t s);
-
 // Launch of the streaming kernel.
 // Three workgroups per compute unit (256 CUs), each walking several tiles: measured at
 // 8192 x 8192 with the 4/6-MSE rule, 768 workgroups take 31.6 us where 1024 take 33.2 and the

@@ -192,6 +192,11 @@ void launch_quantize(QuantParams &p, bool aligned, hipStream_t s) {
 void launch_quantize_nvfp4_fast(QuantParams &p, int rule, bool two_d, bool aligned, bool sr, hipStream_t s);
 void launch_quantize_if4_mse_rows(QuantParams &p, hipStream_t s);
 void launch_quantize_if4_mse_tiles(QuantParams &p, hipStream_t s);
+// 16x16 tiles of NVFP4 (fos_quantize_tiles.hip): rows of whole 16-byte units, cols % 8 == 0; fp16 with round to nearest.
+template <int RULE, bool PSEUDO, bool SR>
+void launch_quantize_nvfp4_tiles(QuantParams &p, hipStream_t s);
+template <int RULE>
+void launch_quantize_nvfp4_tiles_f16(QuantParams &p, hipStream_t s);
 
 // MXFP4 (fos_mxfp4.hip)
 int launch_quantize_mxfp4(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int rule, int sf_layout, uint8_t *codes,

@@ -61,15 +61,25 @@ FOS_DEVICE uint32_t tile_or(uint32_t v) {
     return a | b;
 }
 
+// The two elements of a word: bf16, or fp16 (F16).
+template <bool F16>
+FOS_DEVICE float low_element(uint32_t w) {
+    return F16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)w) : u2f(w << 16);
+}
+template <bool F16>
+FOS_DEVICE float high_element(uint32_t w) {
+    return F16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)) : u2f(w & 0xffff0000u);
+}
+
 // Both candidates of one block in the scaled domain: codes, and (adaptive rules) the rule's
 // reduction of the rounding residuals added to SA / SB.
-template <int RULE>
+template <int RULE, bool F16>
 FOS_DEVICE void block_candidates(const Block16 &blk, float invA, float invB, uint32_t &a0, uint32_t &a1, uint32_t &b0,
                                  uint32_t &b1, float &SA, float &SB) {
     a0 = a1 = b0 = b1 = 0;
     static_for<0, 8>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
-        const float x0 = u2f(blk.w[j] << 16), x1 = u2f(blk.w[j] & 0xffff0000u);
+        const float x0 = low_element<F16>(blk.w[j]), x1 = high_element<F16>(blk.w[j]);
         const float xa0 = scaled(x0, invA), xa1 = scaled(x1, invA);
         if (j < 4) a0 = pack_fp4<(j & 3)>(a0, xa0, xa1);
         else a1 = pack_fp4<(j & 3)>(a1, xa0, xa1);
@@ -147,7 +157,7 @@ FOS_DEVICE void block_candidates_if4(const Block16 &blk, float inv, uint32_t &a0
 struct TilesPos {
     uint64_t x_base, codes_base, out_base;  // first input element / code byte / output element of the wavefront's share
     uint32_t x_bytes;    // extent of the input descriptor
-    uint32_t x_off;      // this lane's offset into it (beyond the descriptor for a lane past the last column)
+    uint32_t x_off, x_off_hi;  // this lane's offsets into it, of either half of a block (beyond the descriptor past the last column)
     int32_t row0;        // first row of the wavefront's share of the tile (rows_p < 2^31: checked by the host)
     int32_t cb;          // this lane's block column in the tensor
     int64_t unit_base;   // offset of scale unit 16 (w & 1) of the wavefront's first scale tile
@@ -166,13 +176,19 @@ FOS_DEVICE uint32_t quad_bytes(uint32_t l0, uint32_t l1, uint32_t l2, uint32_t l
 // SR: a stochastic rounding style (NVFP4); its two sets of scaled values and the Philox state take the
 // registers of three wavefronts per SIMD.
 // SPLIT: a workgroup covers one group (q) of a tile, one tile only (tensors with few tiles; launch_tiles).
-template <int RULE, bool FULL, bool PSEUDO, bool IF4 = false, bool SR = false, bool SPLIT = false>
+// F16: fp16 elements (NVFP4, round to nearest, codes out, the maximum found by pass 1: there is no NaN where it is finite).
+// Nothing in the fast formulation depends on the element type beyond the conversion to f32, see quantize_block_nvfp4_fast.
+// The element-wise kernel that took them, with 24-bit maxima, an IEEE division a block and no loads ahead, read 5000 x 3000 in
+// 26 us; with the read-back the call pair takes 41.4 us there and 32.6 here.
+// Columns: a multiple of 16; for NVFP4, round to nearest, codes out, of 8 (the last block of a row may be half a block).
+template <int RULE, bool FULL, bool PSEUDO, bool IF4 = false, bool SR = false, bool SPLIT = false, bool F16 = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3 : 4, SR ? 3 : 8))) void quantize_nvfp4_tiles_kernel(
     const QuantParams p) {
-    static_assert(!(SR && IF4), "stochastic styles: NVFP4");
+    static_assert(!(SR && IF4) && !(F16 && (SR || IF4 || PSEUDO)), "stochastic styles, fp16: NVFP4");
     constexpr bool STATIC = RULE == FOS_RULE_STATIC_6;
     constexpr bool ADAPTIVE = !STATIC;            // 4/6 with the MSE, MAE or abs-max rule
     constexpr bool MAXRULE = RULE == FOS_RULE_ABS_MAX;  // the error is the largest term, not the sum
+    constexpr bool kHalfBlocks = !FULL && !IF4 && !SR && !PSEUDO;  // (the others: cols % 16 == 0)
     __shared__ uint32_t red[4];
     __shared__ __attribute__((aligned(16))) FastLutEntry lut[256];
 
@@ -180,7 +196,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
     const int par = wave & 1, half = wave >> 1;
     const int lb = lane & 15, li = lane >> 4;
     const int64_t sf_cols = p.cols_p >> 4;
-    const int32_t rows32 = (int32_t)p.rows, cols16 = (int32_t)(p.cols >> 4);  // (cols % 16 == 0 on this path)
+    const int32_t rows32 = (int32_t)p.rows, cols16 = (int32_t)((p.cols + 15) >> 4), cols8 = (int32_t)(p.cols >> 3);
     const bool tiled = !PSEUDO && p.sf_layout == FOS_SF_TILED_128X4;
     const int64_t code_pitch = p.cols_p >> 1;
     const uint32_t n_tiles = (uint32_t)(p.rows_p >> 7) * (uint32_t)p.tiles_x;
@@ -216,6 +232,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
         t.codes_base = PSEUDO ? 0 : uniform64((uint64_t)(p.codes + (int64_t)t.row0 * code_pitch + col0 / 2));
         t.out_base = PSEUDO ? uniform64((uint64_t)(p.pseudo_out + (int64_t)t.row0 * p.ldo + col0)) : 0;
         t.x_off = (FULL || t.cb < cols16) ? x_lane : 0x80000000u;
+        t.x_off_hi = 2 * t.cb + 1 < cols8 ? x_lane + 16u : 0x80000000u;
         t.unit_base = ((int64_t)tile_y * (sf_cols >> 2) + (col0 >> 6)) * 512 + 256 * par;
         return t;
     };
@@ -230,7 +247,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
         } else {
             // the range check covers the per-lane offset only: keep the step inside it
             lo = __builtin_amdgcn_raw_buffer_load_b128(rx, t.x_off + step, 0, 0);
-            hi = __builtin_amdgcn_raw_buffer_load_b128(rx, t.x_off + step + 16u, 0, 0);
+            hi = __builtin_amdgcn_raw_buffer_load_b128(rx, (kHalfBlocks ? t.x_off_hi : t.x_off + 16u) + step, 0, 0);
         }
         b.w[0] = lo.x; b.w[1] = lo.y; b.w[2] = lo.z; b.w[3] = lo.w;
         b.w[4] = hi.x; b.w[5] = hi.y; b.w[6] = hi.z; b.w[7] = hi.w;
@@ -341,10 +358,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
         const uint32_t gbase = (FULL || cb_tile < cols16) ? 32u * q * x_row + tl * 32u : 0x80000000u;
         const uint32_t c = lane & 15, rp = (lane >> 4) & 1;
         const bool cand_b = lane >= 32;
+        // (the second half of a row's last block may lie past the last column)
+        const uint32_t cbase = (!kHalfBlocks || c < 8 || 2 * cb_tile + 1 < cols8) ? gbase : 0x80000000u;
         float x[8];
 #pragma unroll
         for (int m = 0; m < 8; ++m)
-            x[m] = u2f((uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rx, gbase + (rp + 2 * m) * x_row + c * 2u, 0, 0) << 16);
+            x[m] = low_element<F16>((uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rx, cbase + (rp + 2 * m) * x_row + c * 2u, 0, 0));
         float bmax = 0.0f;
 #pragma unroll
         for (int m = 0; m < 8; ++m) bmax = fmaxf(bmax, fabsf(x[m]));
@@ -399,13 +418,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
         const uint32_t s_out = IF4 && pickB ? sP + 128u : sP;  // what goes into the scale byte
         // codes: lane = (row, four columns)
         const uint32_t r = lane >> 2, cq = lane & 3;
-        const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(rx, gbase + r * x_row + cq * 8u, 0, 0);
+        const uint32_t qbase = (!kHalfBlocks || cq < 2 || 2 * cb_tile + 1 < cols8) ? gbase : 0x80000000u;
+        const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(rx, qbase + r * x_row + cq * 8u, 0, 0);
         uint32_t nibs = 0;
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t word = i < 2 ? w.x : w.y;
-            const float xe = (i & 1) ? u2f(word & 0xffff0000u) : u2f(word << 16);
+            const float xe = (i & 1) ? high_element<F16>(word) : low_element<F16>(word);
             const float xs = (sP != 0) ? xe * invP : 0.0f;
             uint32_t nib = e2m1_mag_code(e2m1_round(fabsf(xs))) | (xs < 0.0f ? 8u : 0u);
             if (IF4 && pickB) nib = (uint32_t)((int)int4_round<false>(xs * 1.16666666f, 0.0f)) & 0xfu;
@@ -498,12 +518,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
             // max|x|: the high element of a word is compared with its neighbour's bits still
             // below it, which the final truncation removes (truncation is monotonic)
             float bmax = 0.0f;
+            if constexpr (F16) {
+                uint32_t m = 0u;  // magnitude bits order like the values
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+                for (int s = 0; s < 4; ++s)
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    bmax = fmaxf(fmaxf(fabsf(u2f(blk[s].w[j] << 16)), fabsf(u2f(blk[s].w[j]))), bmax);
-            bmax = tile_max(u2f(f2u(bmax) & 0xffff0000u));
+                    for (int j = 0; j < 8; ++j) m = pk_max_u16(m, blk[s].w[j] & 0x7fff7fffu);
+                bmax = tile_max(fmaxf(low_element<true>(m), high_element<true>(m)));
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        bmax = fmaxf(fmaxf(fabsf(u2f(blk[s].w[j] << 16)), fabsf(u2f(blk[s].w[j]))), bmax);
+                bmax = tile_max(u2f(f2u(bmax) & 0xffff0000u));
+            }
             // (the 3-operation division is exact for the divisors 6 and 4; the unbiased stochastic style rescales them)
             float bq;
             if (SR && k.qdiv != 6.0f && k.qdiv != 4.0f) bq = bmax / k.qdiv;
@@ -528,7 +557,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
                 else if constexpr (SR)
                     block_candidates_sr<RULE>(blk[s], A.inv, B.inv, key_seed, key_offset, (uint64_t)((int64_t)(grow + 4 * s + li) * sf_cols + t.cb),
                                               oc[s][0], oc[s][1], cB[s][0], cB[s][1], SA, SB);
-                else block_candidates<RULE>(blk[s], A.inv, B.inv, oc[s][0], oc[s][1], cB[s][0], cB[s][1], SA, SB);
+                else block_candidates<RULE, F16>(blk[s], A.inv, B.inv, oc[s][0], oc[s][1], cB[s][0], cB[s][1], SA, SB);
                 load(nt, 32 * nq + 4 * s, blk[s]);
             }
             int cmp = -1;
@@ -633,7 +662,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SR ? 3
 // whole / in four (us): 128 x 4096 (8 tiles) 11.9 / 5.9, 2048 x 4096 (128) 12.2 / 7.9, 4096 x 4096 (256) 13.3 / 11.0,
 // 2048 x 14336 (448) 19.9 / 16.7, 4096 x 8192 (512) 21.5 / 20.0, 2560 x 16384 (640) 25.0 / 23.4, 4096 x 12288 (768) 26.3 / 26.7.
 // The line is the static rules', which have the least to do per tile: 448 tiles 13.7 / 13.6, 512 15.5 / 15.8, 768 21.6 / 23.5.
-template <int RULE, bool PSEUDO, bool IF4, bool SR>
+template <int RULE, bool PSEUDO, bool IF4, bool SR, bool F16 = false>
 static void launch_tiles(QuantParams &p, hipStream_t s) {
     constexpr int64_t kSplitTiles = 448;
     p.tiles_x = (int)((p.cols_p + 511) / 512);
@@ -645,20 +674,28 @@ static void launch_tiles(QuantParams &p, hipStream_t s) {
         const int split = tuning().quant_split;  // tuning / tests: 1 = never, 2 = always
         if (split == 2 ? 4 * n <= 0x7fffffff : (split == 0 && n <= kSplitTiles)) {
             const dim3 grid((unsigned)(4 * n));
-            if (full) hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, true, false, IF4, SR, true>), grid, dim3(kThreads), 0, s, p);
-            else hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, false, false, IF4, SR, true>), grid, dim3(kThreads), 0, s, p);
+            if (full) hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, true, false, IF4, SR, true, F16>), grid, dim3(kThreads), 0, s, p);
+            else hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, false, false, IF4, SR, true, F16>), grid, dim3(kThreads), 0, s, p);
             return;
         }
     }
     int64_t grid = 768;
     if (const int forced = tuning().quant_grid) grid = forced > 0 ? forced : grid;
     if (grid > n) grid = n;
-    if (full) hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, true, PSEUDO, IF4, SR>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-    else hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, false, PSEUDO, IF4, SR>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+    if (full) hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, true, PSEUDO, IF4, SR, false, F16>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+    else hipLaunchKernelGGL((quantize_nvfp4_tiles_kernel<RULE, false, PSEUDO, IF4, SR, false, F16>), dim3((unsigned)grid), dim3(kThreads), 0, s, p);
 }
 
 template <int RULE, bool PSEUDO, bool SR>
 void launch_quantize_nvfp4_tiles(QuantParams &p, hipStream_t s) { launch_tiles<RULE, PSEUDO, false, SR>(p, s); }
+
+// fp16 elements, NVFP4, round to nearest.
+template <int RULE>
+void launch_quantize_nvfp4_tiles_f16(QuantParams &p, hipStream_t s) { launch_tiles<RULE, false, false, false, true>(p, s); }
+template void launch_quantize_nvfp4_tiles_f16<FOS_RULE_STATIC_6>(QuantParams &, hipStream_t);
+template void launch_quantize_nvfp4_tiles_f16<FOS_RULE_MSE>(QuantParams &, hipStream_t);
+template void launch_quantize_nvfp4_tiles_f16<FOS_RULE_MAE>(QuantParams &, hipStream_t);
+template void launch_quantize_nvfp4_tiles_f16<FOS_RULE_ABS_MAX>(QuantParams &, hipStream_t);
 
 // IF4 with the MSE rule, round to nearest, 16x16 tiles, aligned input.
 void launch_quantize_if4_mse_tiles(QuantParams &p, hipStream_t s) { launch_tiles<FOS_RULE_MSE, false, true, false>(p, s); }

@@ -1288,3 +1288,26 @@ def test_transform_reads_unaligned_rows():
     assert torch.equal(t, x.T) and float(amax) == float(x.abs().max())
     h, _ = ops.transform(x, False, True)
     assert torch.equal(h, ops.transform(x.contiguous(), False, True)[0])
+
+
+@pytest.mark.parametrize("split", ["1", "2"])
+@pytest.mark.parametrize("rule", ["static_6", "static_4", "mse", "mae", "abs_max"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize(("rows", "cols"), [(16, 8), (100, 24), (128, 512), (130, 520), (257, 1032), (512, 1000), (31, 72)])
+def test_tiles_of_rows_that_end_with_half_a_block(monkeypatch, oracle, rows, cols, dtype, rule, split):
+    """fp16 elements and widths that are odd multiples of 8 on the streaming 16x16 kernel: the oracle's bytes, values far
+    from 1 and undecided tiles among them; every tensor's rows also with a pitch of their own."""
+    monkeypatch.setenv("FOS_QUANT_SPLIT", split)
+    g = torch.Generator("cpu").manual_seed(rows + cols)
+    x = torch.randn(rows, cols, generator=g)
+    x[:, cols // 2:] = torch.randint(-4, 5, (rows, cols - cols // 2), generator=g).float()  # ties
+    x[: rows // 3] *= 2.0 ** -9
+    x = x.to(dtype)
+    expect = oracle.quantize(x, scale_rule=rule, block_scale_2d=True)
+    wide = torch.full((rows, cols + 16), 1000.0, dtype=dtype, device="cuda")
+    wide[:, :cols].copy_(x)
+    for given in (x.cuda(), wide[:, :cols]):
+        q = fos.quantize(given, fos.QuantizationConfig(scale_rule=rule, block_scale_2d=True))
+        assert float(q.amax) == float(expect.amax)
+        assert np.array_equal(u8(q.values), expect.values)
+        assert np.array_equal(u8(q.scale_factors), expect.scale_factors)
