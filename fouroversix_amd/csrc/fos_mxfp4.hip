@@ -18,6 +18,7 @@
 #include <stdint.h>
 
 #include <cstdlib>
+#include <type_traits>
 
 #include "fos_buffer.h"
 #include "fos_gemm_tiles.h"
@@ -532,8 +533,6 @@ struct MxGemmParams {
     int tiles_m, tiles_n;
 };
 
-constexpr int kMxBK = 128;    // codes per K step
-
 FOS_DEVICE mx_v8i frag_of(const uint4 &q) {
     mx_v8i v = {(int)q.x, (int)q.y, (int)q.z, (int)q.w, 0, 0, 0, 0};  // FP4 operands use the first four registers
     return v;
@@ -590,21 +589,21 @@ FOS_DEVICE void mx_store_rows(const mx_v16f (&acc)[WM][WN], uint8_t *lds, int wa
 }
 
 // ---------------------------------------------------------------------------------------
-// Tiles of 256 x 256, 128 x 256 or 128 x 128 outputs and K steps of 128 codes (64 bytes a row, one scale chunk).  The
+// Tiles of 256 x 256, 128 x 256 or 128 x 128 outputs and K steps of 256 codes (128 bytes a row, two scale chunks).  The
 // operands go from global memory straight into LDS (buffer_load ... lds: lane i of a wavefront fills the i-th 16-byte unit
-// of a 1 KiB run), so no registers stage them and four LDS stages keep three K steps in flight.  (A form that
-// staged through registers had one step of latency cover, and a step lasted as long as a load takes: 2048 x 4096 x 14336
-// 82.7 us on its 128 x 128 tile against 69.2 here on 128 x 256.)
+// of a 1 KiB run), so no registers stage them and two LDS stages (three on 128 x 256) keep the next steps in flight.
+// What bounds a step is the arrival of its operands, not the matrix instructions (1024 cycles a step of about 2500 on
+// 128 x 256).  With steps of 128 codes each load took half of every 128-byte line and the next step's came back for the
+// other half: 2048 x 14336 x 4096 73.4 us on 128 x 256, 8192^3 261 on 256 x 256, 1024 x 4096 x 4096 15.0 on 128 x 128;
+// whole lines 66.8, 242 and 14.4.  (The barrier in the middle of a step, the next step's first fragments read
+// behind it: 72.6 against 74.2 us there, but 84.0 against 79.9 at 2048 x 4096 x 14336.)
 //
-// A stage holds the rows of both operands, 64 bytes each without padding, and the 512-byte
-// scale tiles of the step (fetched the same way, 4 bytes per lane); the 16-byte unit c of
-// row rho sits at unit c ^ ((rho >> 2) & 3).  A 128-bit LDS read serves 16 lanes per cycle
+// A stage holds the rows of both operands, 128 bytes each without padding, and the two 512-byte
+// scale tiles of the step (fetched the same way); the 16-byte unit c of
+// row rho sits at unit c ^ ((rho >> 1) & 7).  A 128-bit LDS read serves 16 lanes per cycle
 // from 64 banks, i.e. the 16 rows a quarter-wave reads must differ in address bits 7:4:
-// those are 4 (rho & 3) + (c ^ ((rho >> 2) & 3)), all 16 values.  (With (rho >> 1) & 3, which
-// serves 8 lanes from 32 banks, the counters showed every fragment read taking twice as
-// long.)  The load of lane i therefore fetches unit (i & 3) ^ ((i >> 4) & 3) of row i >> 2 of
-// its 16-row run.
-constexpr int kDmaStages = 4;
+// those are 8 (rho & 1) + (c ^ ((rho >> 1) & 7)), all 16 values.  The load of lane i therefore fetches unit
+// (i & 7) ^ ((row >> 1) & 7) of row i >> 3 of its 8-row run.
 
 // N consecutive 32-bit words (N = 1, 2, 4) with one LDS read.
 template <int N>
@@ -620,7 +619,8 @@ FOS_DEVICE void lds_words(uint32_t (&dst)[N], const uint8_t *src) {
         dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
     }
 }
-constexpr int dma_stage_bytes(int BM, int BN) { return (BM + BN) * 64 + 2048; }  // + the step's scales: 512 bytes per 128 rows of A, then of B
+constexpr int dma_stage_bytes(int BM, int BN) { return (BM + BN) * 128 + (BM + BN) / 128 * 1024; }  // + the step's scales: 1 KiB per 128 rows of A, then of B
+constexpr int dma_stages(int BM, int BN) { return BM != BN ? 3 : 2; }  // (136 KiB, 153 KiB and 68 KiB of LDS, the last twice in a CU)
 typedef __attribute__((address_space(3))) void *MxLdsPtr;
 typedef int mx_v4i __attribute__((ext_vector_type(4)));
 
@@ -639,8 +639,10 @@ FOS_DEVICE mx_v4i mx_raw_rsrc(const void *base, uint32_t bytes) {
 template <int BM, int BN, bool OUT_BF16>
 __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams p) {
     constexpr int WAVES_N = 4, WM = BM / 64, WN = BN / 128;
-    constexpr int PA = BM / 128, PB = BN / 128;  // load instructions per wavefront and step: 16 rows each
-    constexpr int kABytes = BM * 64, kOperandBytes = (BM + BN) * 64, kStageBytes = dma_stage_bytes(BM, BN);
+    constexpr int STAGES = dma_stages(BM, BN), kRow = 128;  // bytes of a row in a stage
+    constexpr int PA = BM / 64, PB = BN / 64;  // load instructions per wavefront and step: 8 rows each
+    constexpr int kTilesA = BM / 128, kTilesB = BN / 128;
+    constexpr int kABytes = BM * kRow, kOperandBytes = (BM + BN) * kRow, kStageBytes = dma_stage_bytes(BM, BN);
     extern __shared__ __attribute__((aligned(16))) uint8_t mx_lds[];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -649,39 +651,44 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
     tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
     const int64_t kbytes = p.K >> 1;
-    const int64_t ksteps = p.K / kMxBK;
+    const int64_t chunks = p.K >> 7;  // scale tiles along K, two a step
+    const int ksteps = (int)((chunks + 1) >> 1);
 
     // The loads into LDS are written as inline assembly: the compiler orders a wait for ALL
     // loads in flight before any LDS read that follows such a load it knows about, which would
     // undo the pipelining.  Every global load of the loop is of this kind (the scales too), so
     // the compiler places no vector-memory waits of its own there and the one wait per step
-    // is placed by hand in kstep().
+    // is placed by hand.
     // (M and N are multiples of 128: a 256-wide tile may hang over the last 128 rows or columns.  The descriptors end
-    // there; whatever LDS holds in the place of the rows beyond goes into outputs beyond the edge only, which are not stored)
+    // there; whatever LDS holds in the place of the rows beyond goes into outputs beyond the edge only, which are not stored.
+    // Of a last step that K fills by half, the other half is other rows' codes: nobody reads it)
     const int rows_a = (int)(p.M - m0 < BM ? p.M - m0 : BM), rows_b = (int)(p.N - n0 < BN ? p.N - n0 : BN);
     const mx_v4i ra = mx_raw_rsrc(p.A + m0 * kbytes, (uint32_t)(rows_a * kbytes));
     const mx_v4i rb = mx_raw_rsrc(p.B + n0 * kbytes, (uint32_t)(rows_b * kbytes));
-    // wavefront w loads rows BM / 8 w ... of A and BN / 8 w ... of B, 16 rows per instruction
-    const int ld_row = lane >> 2, ld_unit = ((lane & 3) ^ ((ld_row >> 2) & 3)) * 16;
+    // wavefront w loads rows BM / 8 w ... of A and BN / 8 w ... of B, 8 per instruction
+    const int ld_row = lane >> 3, ld_unit = ((lane & 7) ^ (ld_row >> 1)) * 16;
     const uint32_t lda_off = (uint32_t)((wave * (BM / 8) + ld_row) * kbytes + ld_unit);
     const uint32_t ldb_off = (uint32_t)((wave * (BN / 8) + ld_row) * kbytes + ld_unit);
-    const int ld_half = (int)(16 * kbytes);
-    // ... and 256 bytes of the step's scales (a 512-byte tile per 128 rows and K step): half w & 1 of tile w >> 1,
-    // A's tiles first.  With fewer tiles than four the last wavefronts load the last one once more, into bytes that
-    // nobody reads: every wavefront has the same number of loads in flight.
-    const int sf_tile = (wave >> 1) < PA + PB ? wave >> 1 : PA + PB - 1;
-    const int sf_rows = 128 * (sf_tile < PA ? sf_tile : sf_tile - PA);  // first row of the scale tile, inside the operand's tile
-    const bool sf_inside = sf_rows < (sf_tile < PA ? rows_a : rows_b);
-    const uint8_t *sf_src = sf_tile < PA ? p.sfA + ((m0 + (sf_inside ? sf_rows : 0)) >> 7) * ksteps * 512
-                                         : p.sfB + ((n0 + (sf_inside ? sf_rows : 0)) >> 7) * ksteps * 512;
-    const mx_v4i rs = mx_raw_rsrc(sf_src, (uint32_t)(ksteps * 512));
-    const uint32_t sf_off = (uint32_t)((wave & 1) * 256 + lane * 4);
+    // (every other load starts at row 8 of 16: bit 2 of the swizzle)
+    const uint32_t flip = (uint32_t)((ld_unit ^ 64) - ld_unit);
+    const uint32_t lda_odd = lda_off + flip, ldb_odd = ldb_off + flip;
+    const int ld_next = (int)(8 * kbytes);
+    // ... and the step's scales of 128 rows (a 512-byte tile per 128 codes): wavefront w those of the w-th 128 rows, A's
+    // first; the wavefronts beyond write the same bytes once more.  Every wavefront has the same number of loads in flight.
+    const int sf_tile = wave % (kTilesA + kTilesB);
+    const int sf_rows = 128 * (sf_tile < kTilesA ? sf_tile : sf_tile - kTilesA);  // first row of the scale tile, inside the operand's tile
+    const bool sf_inside = sf_rows < (sf_tile < kTilesA ? rows_a : rows_b);
+    const uint8_t *sf_src = sf_tile < kTilesA ? p.sfA + ((m0 + (sf_inside ? sf_rows : 0)) >> 7) * chunks * 512
+                                              : p.sfB + ((n0 + (sf_inside ? sf_rows : 0)) >> 7) * chunks * 512;
+    const mx_v4i rs = mx_raw_rsrc(sf_src, (uint32_t)(chunks * 512));
+    const uint32_t sf_off = (uint32_t)(lane * 16);
+    const uint32_t sf_to = (uint32_t)(kOperandBytes + sf_tile * 1024);
     const uint32_t lds_base = (uint32_t)(uintptr_t)(MxLdsPtr)mx_lds;
-    auto issue = [&](int64_t ks, int stage) {
-        const int kq = (int)(ks * (kMxBK / 2)), ksf = (int)(ks * 512);
+    auto issue = [&](int ks, int stage) {
+        const int kq = ks * kRow, ksf = ks * 1024;
         const uint32_t base = lds_base + (uint32_t)(stage * kStageBytes);
-        const uint32_t run_a = base + (uint32_t)(wave * (BM / 8) * 64), run_b = base + (uint32_t)(kABytes + wave * (BN / 8) * 64);
-        const uint32_t sf_run = base + (uint32_t)(kOperandBytes + wave * 256);
+        const uint32_t run_a = base + (uint32_t)(wave * (BM / 8) * kRow), run_b = base + (uint32_t)(kABytes + wave * (BN / 8) * kRow);
+        const uint32_t sf_run = base + sf_to;
         // m0 = LDS address of the run a wavefront fills (lane i: unit i); one wait state
         // between a write of m0 and its use.  (m0 is reserved: the compiler never keeps a
         // value in it across other code, it writes it right before each use of its own.)
@@ -689,15 +696,15 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
         for (int t = 0; t < PA; ++t)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                          :
-                         : "s"(run_a + t * 1024), "v"(lda_off), "s"(ra), "s"(kq + t * ld_half)
+                         : "s"(run_a + t * 1024), "v"(t & 1 ? lda_odd : lda_off), "s"(ra), "s"(kq + t * ld_next)
                          : "memory");
 #pragma unroll
         for (int t = 0; t < PB; ++t)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                          :
-                         : "s"(run_b + t * 1024), "v"(ldb_off), "s"(rb), "s"(kq + t * ld_half)
+                         : "s"(run_b + t * 1024), "v"(t & 1 ? ldb_odd : ldb_off), "s"(rb), "s"(kq + t * ld_next)
                          : "memory");
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :
                      : "s"(sf_run), "v"(sf_off), "s"(rs), "s"(ksf)
                      : "memory");
@@ -713,77 +720,83 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-    const uint32_t fa_off = (uint32_t)((wm * WM * 32 + r) * 64), fb_off = (uint32_t)(kABytes + (wn * WN * 32 + r) * 64);
-    const int swz = (r >> 2) & 3;
-    auto read_frags = [&](int stage, int kk, uint4 *fa, uint4 *fb) {
-        const uint8_t *base = mx_lds + stage * kStageBytes + (((kk * 2 + h) ^ swz) * 16);
+    const uint32_t fa_off = (uint32_t)((wm * WM * 32 + r) * kRow), fb_off = (uint32_t)(kABytes + (wn * WN * 32 + r) * kRow);
+    const int swz = (r >> 1) & 7;
+    auto read_frags = [&](const uint8_t *st, int kk, uint4 *fa, uint4 *fb) {
+        const uint8_t *base = st + (((kk * 2 + h) ^ swz) * 16);
 #pragma unroll
-        for (int i = 0; i < WM; ++i) fa[i] = *reinterpret_cast<const uint4 *>(base + fa_off + i * 32 * 64);
+        for (int i = 0; i < WM; ++i) fa[i] = *reinterpret_cast<const uint4 *>(base + fa_off + i * 32 * kRow);
 #pragma unroll
-        for (int j = 0; j < WN; ++j) fb[j] = *reinterpret_cast<const uint4 *>(base + fb_off + j * 32 * 64);
+        for (int j = 0; j < WN; ++j) fb[j] = *reinterpret_cast<const uint4 *>(base + fb_off + j * 32 * kRow);
     };
     // scale words of this wavefront's row tiles: the 16-byte unit of row r holds those of rows
     // r, r + 32, r + 64, r + 96 of a 128-row tile, of which a wavefront uses WM (WN) in a row
-    auto unit_of = [&](int row) { return (row >> 7) * 512 + r * 16 + ((row & 127) >> 5) * 4; };
+    auto unit_of = [&](int row) { return (row >> 7) * 1024 + r * 16 + ((row & 127) >> 5) * 4; };
     const uint32_t sa_off = (uint32_t)(kOperandBytes + unit_of(wm * WM * 32));
-    const uint32_t sb_off = (uint32_t)(kOperandBytes + PA * 512 + unit_of(wn * WN * 32));
+    const uint32_t sb_off = (uint32_t)(kOperandBytes + kTilesA * 1024 + unit_of(wn * WN * 32));
 
-    // steps 0 .. 2 in flight (past the end: the last step once more, into stages nobody reads)
+    // all stages but one in flight (past the end: the last step once more, into stages nobody reads)
 #pragma unroll
-    for (int s = 0; s < kDmaStages - 1; ++s) issue(s < ksteps ? s : ksteps - 1, s);
+    for (int s = 0; s < STAGES - 1; ++s) issue(s < ksteps ? s : ksteps - 1, s);
 
-    // One K step.  On entry the loads of step ks are the oldest in flight; behind them are
-    // those of steps ks + 1 and ks + 2.  After the barrier every wavefront has its share of
+    // One K step, or its first half.  On entry the loads of step ks are the oldest in flight; behind them are
+    // those of the following STAGES - 2 steps.  After the barrier every wavefront has its share of
     // step ks in LDS and has read the last fragments of step ks - 1, whose stage the loads of
-    // step ks + 3 may overwrite.  (Moving the barrier between the two slices, with the next
-    // step's first fragments read behind it, measured slower -- 341 against 320 us at 8192^3:
-    // it asks for a step's operands half a step earlier, and their arrival is what a step
-    // waits for.)
-    for (int64_t ks = 0; ks < ksteps; ++ks) {
-        const int stage = (int)(ks & (kDmaStages - 1));
-        MX_WAIT_VMCNT(2 * kLoadsPerStep);
+    // step ks + STAGES - 1 may overwrite.
+    int stage = 0;
+    auto kstep = [&](int ks, auto chunks_c) {
+        constexpr int CHUNKS = decltype(chunks_c)::value, SLICES = 2 * CHUNKS;
+        MX_WAIT_VMCNT((STAGES - 2) * kLoadsPerStep);
         __syncthreads();
-        issue(ks + 3 < ksteps ? ks + 3 : ksteps - 1, (stage + 3) & (kDmaStages - 1));
+        issue(ks + STAGES - 1 < ksteps ? ks + STAGES - 1 : ksteps - 1, stage == 0 ? STAGES - 1 : stage - 1);
         const uint8_t *st = mx_lds + stage * kStageBytes;
-        uint32_t sha[WM], shb[WN];
-        lds_words<WM>(sha, st + sa_off);
-        lds_words<WN>(shb, st + sb_off);
-        // lanes of the upper half use the next byte: after the shift, byte 0 / byte 2 of every
-        // lane's register are the scales of the K blocks it feeds in slice 0 / slice 1
+        stage = stage + 1 == STAGES ? 0 : stage + 1;
+        uint32_t sha[CHUNKS][WM], shb[CHUNKS][WN];
+        uint4 fa[SLICES][WM], fb[SLICES][WN];
 #pragma unroll
-        for (int i = 0; i < WM; ++i) sha[i] >>= 8 * h;
+        for (int c = 0; c < CHUNKS; ++c) {
+            lds_words<WM>(sha[c], st + sa_off + c * 512);
+            lds_words<WN>(shb[c], st + sb_off + c * 512);
+            // lanes of the upper half use the next byte: after the shift, byte 0 / byte 2 of every
+            // lane's register are the scales of the K blocks it feeds in slice 0 / slice 1
 #pragma unroll
-        for (int j = 0; j < WN; ++j) shb[j] >>= 8 * h;
-        uint4 fa[2][WM], fb[2][WN];
-        read_frags(stage, 0, fa[0], fb[0]);
-        read_frags(stage, 1, fa[1], fb[1]);
+            for (int i = 0; i < WM; ++i) sha[c][i] >>= 8 * h;
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
+            for (int j = 0; j < WN; ++j) shb[c][j] >>= 8 * h;
+            read_frags(st, 2 * c, fa[2 * c], fb[2 * c]);
+            read_frags(st, 2 * c + 1, fa[2 * c + 1], fb[2 * c + 1]);
 #pragma unroll
-            for (int i = 0; i < WM; ++i)
+            for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
-                for (int j = 0; j < WN; ++j) {
-                    if (kk == 1)
-                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                            frag_of(fb[1][j]), frag_of(fa[1][i]), acc[i][j], 4, 4, 2, (int)shb[j], 2, (int)sha[i]);
-                    else
-                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                            frag_of(fb[0][j]), frag_of(fa[0][i]), acc[i][j], 4, 4, 0, (int)shb[j], 0, (int)sha[i]);
-                }
+                for (int i = 0; i < WM; ++i)
+#pragma unroll
+                    for (int j = 0; j < WN; ++j) {
+                        if (kk == 1)
+                            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                                frag_of(fb[2 * c + 1][j]), frag_of(fa[2 * c + 1][i]), acc[i][j], 4, 4, 2, (int)shb[c][j], 2, (int)sha[c][i]);
+                        else
+                            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                                frag_of(fb[2 * c][j]), frag_of(fa[2 * c][i]), acc[i][j], 4, 4, 0, (int)shb[c][j], 0, (int)sha[c][i]);
+                    }
+            }
         }
-        // issue order: the scale words and the first slice's fragments, then the second slice's
+        // issue order: the scale words and the first slice's fragments, then the other slices'
         // fragment reads one at a time between the first MFMAs -- with all reads ahead
         // of the first MFMA a step began with a longer wait (256 x 256 tile, 8192^3: 271 -> 263 us,
         // 2048 x 14336 x 4096: 70.8 -> 68.0 us in alternating series)
-        constexpr int kReads = WM + WN, kMfmas = 2 * WM * WN;
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 + kReads, 0);
+        constexpr int kReads = WM + WN, kMfmas = SLICES * WM * WN, kRest = (SLICES - 1) * kReads + 2 * (CHUNKS - 1),
+                      kSpread = kRest < kMfmas ? kRest : kMfmas;
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 + kReads + kRest - kSpread, 0);
 #pragma unroll
-        for (int i = 0; i < kReads; ++i) {
+        for (int i = 0; i < kSpread; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, kMfmas - kReads, 0);
-    }
+        __builtin_amdgcn_sched_group_barrier(0x008, kMfmas - kSpread, 0);
+    };
+    const int full = (int)(chunks >> 1);
+    for (int ks = 0; ks < full; ++ks) kstep(ks, std::integral_constant<int, 2>{});
+    if (full < ksteps) kstep(full, std::integral_constant<int, 1>{});
     // loads still in flight write LDS: drain them before the stages are used again
     MX_WAIT_VMCNT(0);
     __syncthreads();  // ... those of every wavefront, and all fragment reads are done
@@ -792,11 +805,11 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
                                      m0 + wm * WM * 32, n0 + wn * WN * 32, rows_a - wm * WM * 32, wn * WN * 32 < rows_b);
 }
 
-// Tile size: the cheapest by what its generations take (us at K = 4096; all scale with K).  136 and 104 KiB of LDS:
-// 256 workgroups of the 256 x 256 and 128 x 256 tiles at a time; 72 KiB: 512 of the 128 x 128 tile.  Measured with the
-// tile forced on 60 shapes, 128 ... 8192 rows; against "256 x 256 from 256 tiles on, else 128 x 128 through registers":
-// 2048 x 4096 x 14336 (128 / 256 / 512 tiles) 82.7 -> 69.2 us on 128 x 256, 2560 x 4096 x 4096 35.7 -> 30.9 and
-// 1024 x 14336 x 4096 45.2 -> 35.3 on 256 x 256, 128 x 4096 x 14336 46.8 -> 39.1 on 128 x 128.
+// Tile size: the cheapest by what its generations take (us at K = 4096; all scale with K).  136 and 153 KiB of LDS:
+// 256 workgroups of the 256 x 256 and 128 x 256 tiles at a time; 68 KiB: 512 of the 128 x 128 tile.  The rows were
+// measured with steps of 128 codes; with steps of 256 all three tiles are 4 to 18 % faster, and of 80 shapes (128 ... 8192
+// rows, K 1024 ... 14336), each tile forced, the one chosen here is within 5 % of the best on all but one
+// (4096 x 1024 x 4096: 19.2 us on 128 x 256, 17.1 on 256 x 256).
 static int mx_pick_tile(int64_t M, int64_t N) {
     const int forced = tuning().mx_tile;  // tuning / tests: 128, 129 (128 x 256) or 256
     if (forced == 128 || forced == 129 || forced == 256) return forced;
@@ -811,7 +824,7 @@ static int mx_pick_tile(int64_t M, int64_t N) {
 
 template <int BM, int BN>
 static int launch_gemm_mxfp4_dma(MxGemmParams &p, int out_type, hipStream_t s) {
-    constexpr size_t lds_bytes = (size_t)kDmaStages * dma_stage_bytes(BM, BN);
+    constexpr size_t lds_bytes = (size_t)dma_stages(BM, BN) * dma_stage_bytes(BM, BN);
     p.tiles_m = (int)((p.M + BM - 1) / BM);
     p.tiles_n = (int)((p.N + BN - 1) / BN);
     auto kernel = out_type == FOS_T_BF16 ? gemm_mxfp4_dma_kernel<BM, BN, true> : gemm_mxfp4_dma_kernel<BM, BN, false>;

@@ -180,7 +180,7 @@ def test_mxfp4_gemm(oracle, m, n, k, out_dtype):
 
 @pytest.mark.parametrize("k", [128, 256, 384, 1152, 4224])
 def test_mxfp4_gemm_kernels_agree_bitwise(monkeypatch, k):
-    """The kernel's three tiles (256 x 256, 128 x 256, 128 x 128; operands straight into LDS, four stages) contract K in
+    """The kernel's three tiles (256 x 256, 128 x 256, 128 x 128; operands straight into LDS) contract K in
     the same order with the same matrix instruction: whole outputs are bit-identical, and so is that of the tile
     chosen by size.  K covers fewer steps than stages, a partial last round of stages, and many rounds."""
     m = n = 4096
