@@ -591,7 +591,7 @@ FOS_DEVICE void mx_store_rows(const mx_v16f (&acc)[WM][WN], uint8_t *lds, int wa
 // ---------------------------------------------------------------------------------------
 // Tiles of 256 x 256, 128 x 256 or 128 x 128 outputs and K steps of 256 codes (128 bytes a row, two scale chunks).  The
 // operands go from global memory straight into LDS (buffer_load ... lds: lane i of a wavefront fills the i-th 16-byte unit
-// of a 1 KiB run), so no registers stage them and two LDS stages (three on 128 x 256) keep the next steps in flight.
+// of a 1 KiB run), so no registers stage them and two or three LDS stages keep the next steps in flight.
 // What bounds a step is the arrival of its operands, not the matrix instructions (1024 cycles a step of about 2500 on
 // 128 x 256).  With steps of 128 codes each load took half of every 128-byte line and the next step's came back for the
 // other half: 2048 x 14336 x 4096 73.4 us on 128 x 256, 8192^3 261 on 256 x 256, 1024 x 4096 x 4096 15.0 on 128 x 128;
@@ -620,7 +620,6 @@ FOS_DEVICE void lds_words(uint32_t (&dst)[N], const uint8_t *src) {
     }
 }
 constexpr int dma_stage_bytes(int BM, int BN) { return (BM + BN) * 128 + (BM + BN) / 128 * 1024; }  // + the step's scales: 1 KiB per 128 rows of A, then of B
-constexpr int dma_stages(int BM, int BN) { return BM != BN ? 3 : 2; }  // (136 KiB, 153 KiB and 68 KiB of LDS, the last twice in a CU)
 typedef __attribute__((address_space(3))) void *MxLdsPtr;
 typedef int mx_v4i __attribute__((ext_vector_type(4)));
 
@@ -636,10 +635,10 @@ FOS_DEVICE mx_v4i mx_raw_rsrc(const void *base, uint32_t bytes) {
 #define MX_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
 
 // BM, BN = 128 or 256: eight wavefronts, two rows of four, each BM / 2 x BN / 4.
-template <int BM, int BN, bool OUT_BF16>
+template <int BM, int BN, int STAGES, bool OUT_BF16>
 __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams p) {
     constexpr int WAVES_N = 4, WM = BM / 64, WN = BN / 128;
-    constexpr int STAGES = dma_stages(BM, BN), kRow = 128;  // bytes of a row in a stage
+    constexpr int kRow = 128;  // bytes of a row in a stage
     constexpr int PA = BM / 64, PB = BN / 64;  // load instructions per wavefront and step: 8 rows each
     constexpr int kTilesA = BM / 128, kTilesB = BN / 128;
     constexpr int kABytes = BM * kRow, kOperandBytes = (BM + BN) * kRow, kStageBytes = dma_stage_bytes(BM, BN);
@@ -806,7 +805,8 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
 }
 
 // Tile size: the cheapest by what its generations take (us at K = 4096; all scale with K).  136 and 153 KiB of LDS:
-// 256 workgroups of the 256 x 256 and 128 x 256 tiles at a time; 68 KiB: 512 of the 128 x 128 tile.  The rows were
+// 256 workgroups of the 256 x 256 and 128 x 256 tiles at a time; 68 KiB: 512 of the 128 x 128 tile
+// (with two stages; up to 256 of them have three).  The rows were
 // measured with steps of 128 codes; with steps of 256 all three tiles are 4 to 18 % faster, and of 80 shapes (128 ... 8192
 // rows, K 1024 ... 14336), each tile forced, the one chosen here is within 5 % of the best on all but one
 // (4096 x 1024 x 4096: 19.2 us on 128 x 256, 17.1 on 256 x 256).
@@ -822,12 +822,12 @@ static int mx_pick_tile(int64_t M, int64_t N) {
     return cost_wide < cost_small ? 129 : 128;
 }
 
-template <int BM, int BN>
+template <int BM, int BN, int STAGES>
 static int launch_gemm_mxfp4_dma(MxGemmParams &p, int out_type, hipStream_t s) {
-    constexpr size_t lds_bytes = (size_t)dma_stages(BM, BN) * dma_stage_bytes(BM, BN);
+    constexpr size_t lds_bytes = (size_t)STAGES * dma_stage_bytes(BM, BN);
     p.tiles_m = (int)((p.M + BM - 1) / BM);
     p.tiles_n = (int)((p.N + BN - 1) / BN);
-    auto kernel = out_type == FOS_T_BF16 ? gemm_mxfp4_dma_kernel<BM, BN, true> : gemm_mxfp4_dma_kernel<BM, BN, false>;
+    auto kernel = out_type == FOS_T_BF16 ? gemm_mxfp4_dma_kernel<BM, BN, STAGES, true> : gemm_mxfp4_dma_kernel<BM, BN, STAGES, false>;
     if (hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
         return FOS_E_LAUNCH;
     hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(512), lds_bytes, s, p);
@@ -853,8 +853,13 @@ extern "C" int fos_gemm_mxfp4(const uint8_t *A, const uint8_t *B, const uint8_t 
     p.M = M; p.N = N; p.K = K; p.ldd = ldd;
     hipStream_t s = (hipStream_t)stream;
     switch (mx_pick_tile(M, N)) {
-        case 256: return launch_gemm_mxfp4_dma<256, 256>(p, out_type, s);
-        case 129: return launch_gemm_mxfp4_dma<128, 256>(p, out_type, s);
-        default: return launch_gemm_mxfp4_dma<128, 128>(p, out_type, s);
+        case 256: return launch_gemm_mxfp4_dma<256, 256, 2>(p, out_type, s);
+        case 129: return launch_gemm_mxfp4_dma<128, 256, 3>(p, out_type, s);
+        default:
+            // a third stage (102 KiB) where no compute unit gets a second workgroup, which would cover a load's latency: 128 x 128 tiles
+            // of 1024 x 11392 x 3584 38.9 -> 34.3 us, of 1152 x 7680 x 3328 25.7 -> 23.9, of 1024 x 4096 x 4096 15.2 both (a fourth
+            // the same); with more tiles two workgroups are better, 2048 x 11392 x 3584 59.2 against 64.5
+            if ((p.M / 128) * (p.N / 128) <= 256) return launch_gemm_mxfp4_dma<128, 128, 3>(p, out_type, s);
+            return launch_gemm_mxfp4_dma<128, 128, 2>(p, out_type, s);
     }
 }
