@@ -1301,6 +1301,12 @@ static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand
         } else if (expand && h.tile) {
             const GemmPlan g = plan_gemm(M, N, K, false);
             if (g.splits > 1 || best + 5 + 4 + 0.32e-6f * M * K > other) h.tile = 0;
+        } else if (h.tile && K <= 2048) {
+            // a short K is over before the fragments' four times as many bytes are paid for: layers (us) of 2048 x 1024 -> 4096 29.7 from
+            // codes and 32.5, 900 x 576 -> 8192 26.6 and 30.8, 900 x 2048 -> 8192 43.6 and 44.4; but 2048 x 2048 -> 2048 36.4 and
+            // 33.7, 1100 x 1536 -> 14336 60.2 and 53.5, and where the codes' product would split K 1100 x 1024 -> 1024 34.6 and 24.1
+            const GemmPlan g = plan_gemm(M, N, K, false);
+            if (g.splits == 1 && best + (g.kind == kPlanWide ? 5 : 3) + 0.25e-6f * M * K > other) h.tile = 0;
         }
         if (!h.tile) return h;
     }
