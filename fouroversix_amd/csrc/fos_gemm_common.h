@@ -173,8 +173,9 @@ FOS_DEVICE half8_t dequant8(uint32_t word, half2_t s) {
 // complement integers q with the value RN16(6/7 q), and the product with the scale is rounded to fp16: the
 // numbers the dequantization of the format is defined by (src/fouroversix/quantize/backend.py:89-160).
 // Blocks differ from lane to lane, so both decodings are formed and one is selected: 34 instructions a word
-// against 8 for E2M1 alone, and what bounds the product (2048 x 4096 x 4096 99 us, NVFP4 61;
-// two dequantize kernels, a library fp32 product and the conversion of its result took 570).  Integers: q + 8 = nibble ^ 8 is a byte 0 .. 15, which E4M3 reads as (q + 8) / 512 (the
+// against 8 for E2M1 alone, and what bounds a product that converts inside its loop (layer of 2048 x 4096 -> 4096 110 us, with both
+// operands converted ahead 80; two dequantize kernels, a library fp32 product and the conversion of its result took
+// 570).  Integers: q + 8 = nibble ^ 8 is a byte 0 .. 15, which E4M3 reads as (q + 8) / 512 (the
 // sub-normals run on into the first normal binade); 6/7 q is then formed from a two-part constant, equal to the rounded
 // product for all 16 integers.
 FOS_DEVICE void if4_integer_bytes(uint32_t word, uint32_t (&pairs)[2]) {

@@ -492,7 +492,8 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
     if (tuning().quant_passes == 1) return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;  // timing runs: pass 1 alone
 
     // 16x16 tiles of NVFP4, round to nearest: fp16 elements, and (either type) a row that ends with half a block, have the
-    // streaming form too where the maximum is not the caller's (elements beyond it may be NaN)
+    // streaming form too where the maximum is not the caller's (elements beyond it may be NaN): 5000 x 3000 fp16 26 us element by
+    // element, 14 streaming
     const bool tiles = block2d && dtype == FOS_DTYPE_NVFP4 && round_style == FOS_ROUND_NEAREST && !pseudo_out && x_type != FOS_T_F32 &&
                        !amax_is_input && cols % 8 == 0 && aligned_rows(x, ld);
 
