@@ -5,11 +5,9 @@
 #include <stdint.h>
 
 #include "fos_gemm_common.h"
+#include "fos_load_ranges.h"
 
 namespace fos {
-
-// 1 KiB fragments of 16 rows x 32 k: eight make a step of a band of 128 rows, four steps a chunk of 128 k.
-constexpr int kFragmentStep = 8192, kBandChunkBytes = 32768;
 
 // Byte of the fragments of [rows, K] at which the eight values k ... k + 7 (k % 8 == 0) of a row begin.
 FOS_DEVICE int64_t fragment_offset(int64_t row, int64_t k, int64_t chunks) {

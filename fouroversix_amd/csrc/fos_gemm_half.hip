@@ -116,11 +116,10 @@ FOS_DEVICE void convert_pair(half8_t &f, uint32_t word, half2_t s) {
 template <int WAVES_M, int WAVES_N, int WM, int BAR, int OCC, int OUT, bool IF4>
 __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(const GemmParams p) {
     constexpr bool OUT_BF16 = OUT == kOutBF16;
-    constexpr int WN = 4, NW = WAVES_M * WAVES_N, BM = 16 * WM * WAVES_M, BN = 64 * WAVES_N, MFMAS = WM * WN;
+    typedef HalfTile<WAVES_M, WAVES_N, WM, IF4> Tile;
+    constexpr int WN = 4, NW = Tile::NW, BM = Tile::BM, BN = Tile::BN, MFMAS = WM * WN;
     constexpr int kSlotA = BM * 64, kCodesB = BN * 64, kSlotB = IF4 ? BN * 64 : BN * 72, kBaseB = kSlotsA * kSlotA;
-    // a wavefront's loads: of A per step, and of B per step (IF4) or of B's codes (16 rows each) and scales (256 bytes each)
-    // per chunk
-    constexpr int LA = BM / 16 / NW, LB = BN / 16 / NW, LS = IF4 ? 0 : BN / 32 / NW, LSTEP = IF4 ? LA + LB : LA, LCHUNK = IF4 ? 0 : LB + LS;
+    constexpr int LA = Tile::LA, LB = Tile::LB, LS = Tile::LS, LSTEP = IF4 ? LA + LB : LA, LCHUNK = IF4 ? 0 : LB + LS;
     static_assert(LA == 2 && LB >= 1 && (WM == 4 || WM == 8), "shares of the loads");
     extern __shared__ __attribute__((aligned(16))) uint8_t half_lds[];
 
@@ -128,7 +127,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
     int tile_m, tile_n;
     tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
-    // (M and N are multiples of 128: a 256-wide tile may hang over the last 128 rows or columns.  The descriptors end there)
+    // (M and N are multiples of 128: a 256-wide tile may hang over the last 128 rows or columns)
     const int rows_a = (int)(p.M - m0 < BM ? p.M - m0 : BM), rows_b = (int)(p.N - n0 < BN ? p.N - n0 : BN);
     const int chunks_all = (int)((p.K + 127) >> 7);
     const int c0 = OUT == kOutPartial ? (int)blockIdx.y * p.ksteps_per_split : 0;
@@ -136,12 +135,14 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
     const int steps = 4 * chunks;
     const uint32_t band = (uint32_t)chunks_all * kBandChunkBytes, kbytes = (uint32_t)(p.K >> 1);
     const uint32_t scale_band = (uint32_t)p.K * 8u;
-    const int4v ra = raw_rsrc(p.frags + (m0 >> 7) * (int64_t)band, (uint32_t)(rows_a >> 7) * band);
-    const int4v rb = IF4 ? raw_rsrc(p.frags_b + (n0 >> 7) * (int64_t)band, (uint32_t)(rows_b >> 7) * band)
-                         : raw_rsrc(p.B + n0 * kbytes, (uint32_t)rows_b * kbytes);
-    const int4v rs = raw_rsrc(p.sfB + (n0 >> 7) * (int64_t)scale_band, (uint32_t)(rows_b >> 7) * scale_band);  // (NVFP4)
+    // a wavefront's descriptors end with its own share of a tile, or are empty where that lies past the edge
+    const int fa0 = wave * LA, fb0 = wave * LB, gs0 = wave * LS;
+    const int4v ra = raw_rsrc(p.frags + fragment_base(m0, fa0, band), share_bytes(fa0 * 16, rows_a, band));
+    const int4v rb = IF4 ? raw_rsrc(p.frags_b + fragment_base(n0, fb0, band), share_bytes(fb0 * 16, rows_b, band))
+                         : raw_rsrc(p.B + (n0 + fb0 * 16) * kbytes, share_bytes(fb0 * 16, rows_b, LB * 16 * kbytes));
+    const int4v rs = raw_rsrc(p.sfB + scales_base(n0, gs0, scale_band), share_bytes(gs0 * 32, rows_b, scale_band));  // (NVFP4)
     const uint32_t lds_base = (uint32_t)(uintptr_t)(LdsPtr)half_lds;
-    const uint32_t va = lane * 16, vb = (lane & 15) * kbytes + q * 16, vs = lane * 4;
+    const uint32_t va = fragment_lane(lane), vb = codes_lane(lane, kbytes), vs = scales_lane(lane);
 
     // m0 = LDS address of the run a wavefront fills (lane i: unit i); one wait state between a write of m0 and its use
     auto load16 = [&](uint32_t to, uint32_t offset, const int4v &r, uint32_t base) {
@@ -149,23 +150,21 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
     };
     auto load_step = [&](int step, int slot, int t) {
         if (t >= LA) {  // (IF4)
-            const uint32_t f = wave * LB + t - LA;
-            load16(lds_base + kBaseB + slot * kSlotB + f * 1024, va, rb, (f >> 3) * band + (uint32_t)(c0 * 4 + step) * kFragmentStep + (f & 7) * 1024);
+            const int f = fb0 + t - LA;
+            load16(lds_base + kBaseB + slot * kSlotB + f * 1024, va, rb, fragment_scalar(f, c0 * 4 + step));
             return;
         }
-        const uint32_t f = wave * LA + t;
-        load16(lds_base + slot * kSlotA + f * 1024, va, ra, (f >> 3) * band + (uint32_t)(c0 * 4 + step) * kFragmentStep + (f & 7) * 1024);
+        const int f = fa0 + t;
+        load16(lds_base + slot * kSlotA + f * 1024, va, ra, fragment_scalar(f, c0 * 4 + step));
     };
     auto load_b = [&](int chunk, int slot, int t) {
         const uint32_t base = lds_base + kBaseB + slot * kSlotB;
         if (t < LB) {
-            const uint32_t g = wave * LB + t;
-            load16(base + g * 1024, vb, rb, g * 16 * kbytes + (uint32_t)(c0 + chunk) * 64);
+            load16(base + (fb0 + t) * 1024, vb, rb, codes_scalar(t, c0 + chunk, kbytes));
         } else {
-            const uint32_t g = wave * LS + t - LB;
-            const uint32_t from = (g >> 2) * scale_band + (uint32_t)(c0 + chunk) * 1024 + (g & 3) * 256;
+            const int g = gs0 + t - LB;
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-                         ::"s"(base + kCodesB + g * 256), "v"(vs), "s"(rs), "s"(from) : "memory");
+                         ::"s"(base + kCodesB + g * 256), "v"(vs), "s"(rs), "s"(scales_scalar(g, c0 + chunk)) : "memory");
         }
     };
 

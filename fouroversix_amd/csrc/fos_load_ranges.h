@@ -1,0 +1,45 @@
+// Where the loads of the products that go from global memory straight into LDS lie, as plain constexpr functions: the kernels
+// address with them, and a host test walks them over whole operands and finds no load outside.
+//
+// A raw buffer load reads base + lane offset + scalar offset, and its range check compares the LANE offset alone with the
+// size in the descriptor.  What decides whether something exists therefore goes into the descriptor or the lane offset, and
+// a scalar offset only moves a load inside what the check has let pass.
+#pragma once
+
+#include <stdint.h>
+
+namespace fos {
+
+// 1 KiB fragments of 16 rows x 32 k: eight make a step of a band of 128 rows, four steps a chunk of 128 k.
+constexpr int kFragmentStep = 8192, kBandChunkBytes = 32768;
+
+// The tiles of gemm_half_kernel, and a wavefront's loads: of A (and, IF4, of B) fragments per step; of B's codes (16 rows
+// each) and scales (256 bytes each) per chunk.
+template <int WAVES_M, int WAVES_N, int WM, bool IF4>
+struct HalfTile {
+    static constexpr int NW = WAVES_M * WAVES_N, BM = 16 * WM * WAVES_M, BN = 64 * WAVES_N;
+    static constexpr int LA = BM / 16 / NW, LB = BN / 16 / NW, LS = IF4 ? 0 : BN / 32 / NW;
+    // every wavefront has descriptors of its own, of the 128 rows its share lies in (codes: of its own rows)
+    static_assert(LA * NW * 16 == BM && LB * NW * 16 == BN && 8 % LA == 0 && 8 % LB == 0 && (IF4 || 4 % LS == 0), "no share crosses a multiple of 128 rows");
+};
+
+// Size in the descriptor of a share that begins at row `first` of a tile of which `inside` rows exist (a multiple of 128): nothing
+// where the share lies beyond (its loads give zeros without touching memory).
+constexpr uint32_t share_bytes(int first, int inside, uint32_t bytes) { return first < inside ? bytes : 0u; }
+
+// Fragment f (of 16 rows) of the tile at row0; `band`: bytes of 128 rows.
+constexpr int64_t fragment_base(int64_t row0, int f, uint32_t band) { return ((row0 >> 7) + (f >> 3)) * (int64_t)band; }
+constexpr uint32_t fragment_lane(int lane) { return (uint32_t)lane * 16; }
+constexpr uint32_t fragment_scalar(int f, int step) { return (uint32_t)step * kFragmentStep + (uint32_t)(f & 7) * 1024; }
+
+// B's codes, `kbytes` a row: load t of a wavefront's share takes 64 bytes of 16 rows.
+constexpr uint32_t codes_lane(int lane, uint32_t kbytes) { return (uint32_t)(lane & 15) * kbytes + (uint32_t)(lane >> 4) * 16; }
+constexpr uint32_t codes_scalar(int t, int chunk, uint32_t kbytes) { return (uint32_t)t * 16 * kbytes + (uint32_t)chunk * 64; }
+
+// B's scales, of 128 rows in tiles of 512 bytes per 64 k (`band` bytes): run g of the tile at row0 takes 256 bytes, the first two of
+// four those of the first 64 k of a chunk.
+constexpr int64_t scales_base(int64_t row0, int g, uint32_t band) { return ((row0 >> 7) + (g >> 2)) * (int64_t)band; }
+constexpr uint32_t scales_lane(int lane) { return (uint32_t)lane * 4; }
+constexpr uint32_t scales_scalar(int g, int chunk) { return (uint32_t)chunk * 1024 + (uint32_t)(g & 3) * 256; }
+
+}  // namespace fos
