@@ -159,12 +159,13 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
     };
     auto load_b = [&](int chunk, int slot, int t) {
         const uint32_t base = lds_base + kBaseB + slot * kSlotB;
+        const bool half = is_half(c0 + chunk, kbytes);
         if (t < LB) {
-            load16(base + (fb0 + t) * 1024, vb, rb, codes_scalar(t, c0 + chunk, kbytes));
+            load16(base + (fb0 + t) * 1024, whole_or(half, lane, vb), rb, codes_scalar(t, c0 + chunk, kbytes));
         } else {
             const int g = gs0 + t - LB;
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-                         ::"s"(base + kCodesB + g * 256), "v"(vs), "s"(rs), "s"(scales_scalar(g, c0 + chunk)) : "memory");
+                         ::"s"(base + kCodesB + g * 256), "v"(vs), "s"(rs), "s"(scales_scalar(g, c0 + chunk, half)) : "memory");
         }
     };
 
@@ -378,9 +379,7 @@ __global__ __launch_bounds__(256, 1) void gemm_half_stream_kernel(const GemmPara
     const BufferRsrc ra = make_rsrc(p.frags, (uint32_t)chunks_all * kBandChunkBytes);
     const BufferRsrc rb = make_rsrc(p.B + n0 * kbytes, 64u * kbytes);
     const BufferRsrc rs = make_rsrc(p.sfB + (n0 >> 7) * (int64_t)scale_band, scale_band);
-    const uint32_t va = lane * 16, vb = (lane & 15) * kbytes + q * 16;
-    // (rows n0 % 128 + 16 j + (lane & 15): two adjacent words of 32-row groups, 256 bytes apart for the odd j)
-    const uint32_t vs = (q >> 1) * 512 + (lane & 15) * 16 + ((uint32_t)(n0 & 127) >> 5) * 4 + (q & 1) * 2;
+    const uint32_t va = fragment_lane(lane);
 
     half8_t fa[4][WM];  // a chunk; refilled one at a time with the next chunk's, behind the matrix instructions that read it last
     u32x4 codes[2][WN];
@@ -390,11 +389,13 @@ __global__ __launch_bounds__(256, 1) void gemm_half_stream_kernel(const GemmPara
         fa[w][i] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(va + i * 1024), (int)at, 0));
     };
     auto load_b = [&](int chunk, int set) {
-#pragma unroll
-        for (int j = 0; j < WN; ++j) codes[set][j] = __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(vb + j * 16 * kbytes), chunk * 64, 0);
+        const bool half = is_half(chunk, kbytes);
 #pragma unroll
         for (int j = 0; j < WN; ++j)
-            scales[set][j] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)(vs + (j & 1) * 256 + (j >> 1) * 4), chunk * 1024, 0);
+            codes[set][j] = __builtin_amdgcn_raw_buffer_load_b128(rb, (int)stream_codes_lane(lane, j, kbytes, half), chunk * 64, 0);
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+            scales[set][j] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)stream_scales_lane(lane, j, n0, half), chunk * 1024, 0);
     };
     const uint32_t last_mask = tail_mask((int)((p.depth - (int64_t)(chunks_all - 1) * 128 + 15) >> 4) - 2 * q);
 

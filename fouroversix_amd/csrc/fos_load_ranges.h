@@ -32,14 +32,31 @@ constexpr int64_t fragment_base(int64_t row0, int f, uint32_t band) { return ((r
 constexpr uint32_t fragment_lane(int lane) { return (uint32_t)lane * 16; }
 constexpr uint32_t fragment_scalar(int f, int step) { return (uint32_t)step * kFragmentStep + (uint32_t)(f & 7) * 1024; }
 
+// K % 128 = 64: of the last chunk only the first half exists.  A lane of the upper half of a wavefront, which holds the k of the other
+// half, then gets an offset beyond every descriptor; nobody uses what it receives (its scales are masked).
+constexpr uint32_t kNoRead = 0x80000000u;
+constexpr bool is_half(int chunk, uint32_t kbytes) { return (uint32_t)chunk * 64 + 64 > kbytes; }
+constexpr uint32_t whole_or(bool half, int lane, uint32_t offset) { return half && lane >= 32 ? kNoRead : offset; }
+
 // B's codes, `kbytes` a row: load t of a wavefront's share takes 64 bytes of 16 rows.
 constexpr uint32_t codes_lane(int lane, uint32_t kbytes) { return (uint32_t)(lane & 15) * kbytes + (uint32_t)(lane >> 4) * 16; }
 constexpr uint32_t codes_scalar(int t, int chunk, uint32_t kbytes) { return (uint32_t)t * 16 * kbytes + (uint32_t)chunk * 64; }
 
 // B's scales, of 128 rows in tiles of 512 bytes per 64 k (`band` bytes): run g of the tile at row0 takes 256 bytes, the first two of
-// four those of the first 64 k of a chunk.
+// four those of the first 64 k of a chunk.  (Of half a chunk all four take those.)
 constexpr int64_t scales_base(int64_t row0, int g, uint32_t band) { return ((row0 >> 7) + (g >> 2)) * (int64_t)band; }
 constexpr uint32_t scales_lane(int lane) { return (uint32_t)lane * 4; }
-constexpr uint32_t scales_scalar(int g, int chunk) { return (uint32_t)chunk * 1024 + (uint32_t)(g & 3) * 256; }
+constexpr uint32_t scales_scalar(int g, int chunk, bool half) { return (uint32_t)chunk * 1024 + (uint32_t)(g & (half ? 1 : 3)) * 256; }
+
+// gemm_half_stream_kernel: a workgroup's 64 rows from n0, loads j of 16 rows each (scalar offsets: 64 bytes of codes and 1024 of scales
+// a chunk).  A lane's two scales lie in the word of its row, rows n0 % 128 + 16 j + (lane & 15): two adjacent words of 32-row groups, 256
+// bytes apart for the odd j.
+constexpr uint32_t stream_codes_lane(int lane, int j, uint32_t kbytes, bool half) {
+    return whole_or(half, lane, codes_lane(lane, kbytes)) + (uint32_t)j * 16 * kbytes;
+}
+constexpr uint32_t stream_scales_lane(int lane, int j, int64_t n0, bool half) {
+    return whole_or(half, lane, (uint32_t)(lane >> 5) * 512 + (uint32_t)(lane & 15) * 16 + ((uint32_t)(n0 & 127) >> 5) * 4 + (uint32_t)(lane >> 4 & 1) * 2) +
+           (uint32_t)(j & 1) * 256 + (uint32_t)(j >> 1) * 4;
+}
 
 }  // namespace fos

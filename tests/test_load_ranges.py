@@ -63,13 +63,14 @@ static void walk(int M, int N, int K) {
                         const int f0 = wave * T::LB, g0 = wave * T::LS;
                         for (int t = 0; t < T::LB; ++t) {
                             const int row = n0 + (f0 + t) * 16 + (lane & 15), byte = chunk * 64 + (lane >> 4) * 16;
-                            touch("codes", (i64)(n0 + f0 * 16) * kbytes, share_bytes(f0 * 16, rows_b, T::LB * 16 * kbytes), codes_lane(lane, kbytes),
+                            touch("codes", (i64)(n0 + f0 * 16) * kbytes, share_bytes(f0 * 16, rows_b, T::LB * 16 * kbytes),
+                                  whole_or(is_half(chunk, kbytes), lane, codes_lane(lane, kbytes)),
                                   codes_scalar(t, chunk, kbytes), 16, codes, (f0 + t) * 16 < rows_b && byte < (int)kbytes ? (i64)row * kbytes + byte : -1);
                         }
                         for (int t = 0; t < T::LS; ++t) {
                             const int g = g0 + t, tile = 2 * chunk + (g & 3) / 2;  // (64 k each)
                             touch("scales", scales_base(n0, g0, scale_band), share_bytes(g0 * 32, rows_b, scale_band), scales_lane(lane),
-                                  scales_scalar(g, chunk), 4, scales,
+                                  scales_scalar(g, chunk, is_half(chunk, kbytes)), 4, scales,
                                   g * 32 < rows_b && tile * 64 < K ? (i64)((n0 + g * 32) / 128) * scale_band + tile * 512 + (g & 1) * 256 + lane * 4 : -1);
                         }
                     }
@@ -80,7 +81,7 @@ template <int WAVES_M, int WAVES_N, int WM>
 static void tiles() {
     for (int M : {128, 256, 384, 640})
         for (int N : {128, 256, 384, 640})
-            for (int K : {128, 384, 1024}) {
+            for (int K : {64, 128, 192, 384, 1024, 1088}) {
                 walk<HalfTile<WAVES_M, WAVES_N, WM, false>, false>(M, N, K);
                 walk<HalfTile<WAVES_M, WAVES_N, WM, true>, true>(M, N, K);
             }
@@ -93,8 +94,30 @@ int main() {
 }
 """
 
+STREAM = r"""
+int main() {
+    for (int N : {128, 384})
+        for (int K : {8192, 8256, 8320})
+            for (int n0 = 0; n0 < N; n0 += 64) {
+                const uint32_t kbytes = K / 2, scale_band = (uint32_t)K * 8;
+                const i64 codes = (i64)N * kbytes, scales = (i64)(N / 128) * scale_band;
+                for (int chunk = 0; chunk * 128 < K; ++chunk)
+                    for (int lane = 0; lane < 64; ++lane)
+                        for (int j = 0; j < 4; ++j) {
+                            const bool half = is_half(chunk, kbytes);
+                            const int row = n0 + 16 * j + (lane & 15), k = chunk * 128 + (lane >> 4) * 32, in_band = row & 127;
+                            touch("codes", (i64)n0 * kbytes, 64 * kbytes, stream_codes_lane(lane, j, kbytes, half), chunk * 64, 16, codes,
+                                  k < K ? (i64)row * kbytes + k / 2 : -1);
+                            touch("scales", (i64)(n0 / 128) * scale_band, scale_band, stream_scales_lane(lane, j, n0, half), chunk * 1024, 2, scales,
+                                  k < K ? (i64)(row / 128) * scale_band + k / 64 * 512 + (in_band & 31) * 16 + in_band / 32 * 4 + (k & 32) / 16 : -1);
+                        }
+            }
+    puts("inside");
+}
+"""
 
-@pytest.mark.parametrize("source", [HALF], ids=["converted_ahead"])
+
+@pytest.mark.parametrize("source", [HALF, STREAM], ids=["converted_ahead", "weight_streamed"])
 def test_loads_stay_inside_their_operands(tmp_path, source):
     compiler = os.environ.get("CXX") or shutil.which("g++")
     (tmp_path / "walk.cpp").write_text(COMMON + source)
