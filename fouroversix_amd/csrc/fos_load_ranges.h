@@ -59,4 +59,17 @@ constexpr uint32_t stream_scales_lane(int lane, int j, int64_t n0, bool half) {
            (uint32_t)(j & 1) * 256 + (uint32_t)(j >> 1) * 4;
 }
 
+// gemm_mxfp4_dma_kernel: steps of 256 codes (128 bytes a row), 8 rows a load.  The lane that fills 16-byte unit c of row rho fetches unit
+// c ^ ((rho >> 1) & 7), so every other load (rows 8 ... 15 of 16: `odd`) has the units' upper halves exchanged.  Of a last
+// step that K fills by half (K % 256 = 128) the units from 64 bytes on and the second of the two scale tiles don't exist.
+constexpr uint32_t mx_unit(int lane, bool odd) { return (uint32_t)(((lane & 7) ^ (lane >> 4)) * 16) ^ (odd ? 64u : 0u); }
+constexpr bool mx_is_half(int step, uint32_t kbytes) { return (uint32_t)step * 128 + 128 > kbytes; }
+constexpr uint32_t mx_codes_lane(int first_row, int lane, bool odd, uint32_t kbytes) {
+    return (uint32_t)(first_row + (lane >> 3)) * kbytes + mx_unit(lane, odd);
+}
+constexpr uint32_t mx_whole_or(bool half, int lane, bool odd, uint32_t offset) { return half && mx_unit(lane, odd) >= 64 ? kNoRead : offset; }
+constexpr uint32_t mx_codes_scalar(int t, int step, uint32_t kbytes) { return (uint32_t)step * 128 + (uint32_t)t * 8 * kbytes; }
+constexpr uint32_t mx_scales_lane(int lane) { return (uint32_t)lane * 16; }
+constexpr uint32_t mx_scales_scalar(int step) { return (uint32_t)step * 1024; }
+
 }  // namespace fos

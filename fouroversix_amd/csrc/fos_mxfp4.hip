@@ -22,6 +22,7 @@
 
 #include "fos_buffer.h"
 #include "fos_gemm_tiles.h"
+#include "fos_load_ranges.h"
 #include "fos_quantize_fast.h"
 #include "fos_tuning.h"
 #include "fouroversix_hip.h"
@@ -660,18 +661,14 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
     // is placed by hand.
     // (M and N are multiples of 128: a 256-wide tile may hang over the last 128 rows or columns.  The descriptors end
     // there; whatever LDS holds in the place of the rows beyond goes into outputs beyond the edge only, which are not stored.
-    // Of a last step that K fills by half, the other half is other rows' codes: nobody reads it)
+    // Of a last step that K fills by half, nobody reads the other half)
     const int rows_a = (int)(p.M - m0 < BM ? p.M - m0 : BM), rows_b = (int)(p.N - n0 < BN ? p.N - n0 : BN);
     const mx_v4i ra = mx_raw_rsrc(p.A + m0 * kbytes, (uint32_t)(rows_a * kbytes));
     const mx_v4i rb = mx_raw_rsrc(p.B + n0 * kbytes, (uint32_t)(rows_b * kbytes));
     // wavefront w loads rows BM / 8 w ... of A and BN / 8 w ... of B, 8 per instruction
-    const int ld_row = lane >> 3, ld_unit = ((lane & 7) ^ (ld_row >> 1)) * 16;
-    const uint32_t lda_off = (uint32_t)((wave * (BM / 8) + ld_row) * kbytes + ld_unit);
-    const uint32_t ldb_off = (uint32_t)((wave * (BN / 8) + ld_row) * kbytes + ld_unit);
-    // (every other load starts at row 8 of 16: bit 2 of the swizzle)
-    const uint32_t flip = (uint32_t)((ld_unit ^ 64) - ld_unit);
-    const uint32_t lda_odd = lda_off + flip, ldb_odd = ldb_off + flip;
-    const int ld_next = (int)(8 * kbytes);
+    const uint32_t row_bytes = (uint32_t)kbytes;
+    const uint32_t lda_off = mx_codes_lane(wave * (BM / 8), lane, false, row_bytes), lda_odd = mx_codes_lane(wave * (BM / 8), lane, true, row_bytes);
+    const uint32_t ldb_off = mx_codes_lane(wave * (BN / 8), lane, false, row_bytes), ldb_odd = mx_codes_lane(wave * (BN / 8), lane, true, row_bytes);
     // ... and the step's scales of 128 rows (a 512-byte tile per 128 codes): wavefront w those of the w-th 128 rows, A's
     // first; the wavefronts beyond write the same bytes once more.  Every wavefront has the same number of loads in flight.
     const int sf_tile = wave % (kTilesA + kTilesB);
@@ -680,11 +677,13 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
     const uint8_t *sf_src = sf_tile < kTilesA ? p.sfA + ((m0 + (sf_inside ? sf_rows : 0)) >> 7) * chunks * 512
                                               : p.sfB + ((n0 + (sf_inside ? sf_rows : 0)) >> 7) * chunks * 512;
     const mx_v4i rs = mx_raw_rsrc(sf_src, (uint32_t)(chunks * 512));
-    const uint32_t sf_off = (uint32_t)(lane * 16);
+    const uint32_t sf_off = mx_scales_lane(lane);
     const uint32_t sf_to = (uint32_t)(kOperandBytes + sf_tile * 1024);
     const uint32_t lds_base = (uint32_t)(uintptr_t)(MxLdsPtr)mx_lds;
     auto issue = [&](int ks, int stage) {
-        const int kq = ks * kRow, ksf = ks * 1024;
+        const bool half = mx_is_half(ks, row_bytes);
+        const uint32_t a_off[2] = {mx_whole_or(half, lane, false, lda_off), mx_whole_or(half, lane, true, lda_odd)};
+        const uint32_t b_off[2] = {mx_whole_or(half, lane, false, ldb_off), mx_whole_or(half, lane, true, ldb_odd)};
         const uint32_t base = lds_base + (uint32_t)(stage * kStageBytes);
         const uint32_t run_a = base + (uint32_t)(wave * (BM / 8) * kRow), run_b = base + (uint32_t)(kABytes + wave * (BN / 8) * kRow);
         const uint32_t sf_run = base + sf_to;
@@ -695,17 +694,17 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
         for (int t = 0; t < PA; ++t)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                          :
-                         : "s"(run_a + t * 1024), "v"(t & 1 ? lda_odd : lda_off), "s"(ra), "s"(kq + t * ld_next)
+                         : "s"(run_a + t * 1024), "v"(a_off[t & 1]), "s"(ra), "s"(mx_codes_scalar(t, ks, row_bytes))
                          : "memory");
 #pragma unroll
         for (int t = 0; t < PB; ++t)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                          :
-                         : "s"(run_b + t * 1024), "v"(t & 1 ? ldb_odd : ldb_off), "s"(rb), "s"(kq + t * ld_next)
+                         : "s"(run_b + t * 1024), "v"(b_off[t & 1]), "s"(rb), "s"(mx_codes_scalar(t, ks, row_bytes))
                          : "memory");
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :
-                     : "s"(sf_run), "v"(sf_off), "s"(rs), "s"(ksf)
+                     : "s"(sf_run), "v"(whole_or(half, lane, sf_off)), "s"(rs), "s"(mx_scales_scalar(ks))
                      : "memory");
     };
     constexpr int kLoadsPerStep = PA + PB + 1;

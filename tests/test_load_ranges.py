@@ -116,8 +116,43 @@ int main() {
 }
 """
 
+MXFP4 = r"""
+// rows of one operand in a tile of BROWS rows: lane i of a load fills unit i & 7 of row i >> 3
+static void walk(int tile_rows, int rows, int K) {
+    const uint32_t kbytes = K / 2, chunks = K / 128;
+    const int steps = (K + 255) / 256;
+    for (int row0 = 0; row0 < rows; row0 += tile_rows) {
+        const int inside = rows - row0 < tile_rows ? rows - row0 : tile_rows;
+        for (int step = 0; step < steps; ++step)
+            for (int lane = 0; lane < 64; ++lane) {
+                const bool half = mx_is_half(step, kbytes);
+                for (int wave = 0; wave < 8; ++wave)
+                    for (int t = 0; t < tile_rows / 64; ++t) {
+                        const int row = wave * (tile_rows / 8) + t * 8 + lane / 8, byte = step * 128 + (((lane & 7) ^ (row / 2 % 8)) * 16);
+                        touch("codes", (i64)row0 * kbytes, (uint32_t)inside * kbytes,
+                              mx_whole_or(half, lane, t & 1, mx_codes_lane(wave * (tile_rows / 8), lane, t & 1, kbytes)), mx_codes_scalar(t, step, kbytes), 16,
+                              (i64)rows * kbytes, row < inside && byte < (int)kbytes ? (i64)(row0 + row) * kbytes + byte : -1);
+                    }
+                for (int band = 0; band < inside / 128; ++band) {
+                    const i64 at = (i64)(row0 / 128 + band) * chunks * 512, of_step = step * 1024 + lane * 16;
+                    touch("scales", at, chunks * 512, whole_or(half, lane, mx_scales_lane(lane)), mx_scales_scalar(step), 16, (i64)(rows / 128) * chunks * 512,
+                          of_step < (i64)chunks * 512 ? at + of_step : -1);
+                }
+            }
+    }
+}
+int main() {
+    for (int rows : {128, 256, 384, 640})
+        for (int K : {128, 256, 384, 1024, 1152}) {
+            walk(128, rows, K);
+            walk(256, rows, K);
+        }
+    puts("inside");
+}
+"""
 
-@pytest.mark.parametrize("source", [HALF, STREAM], ids=["converted_ahead", "weight_streamed"])
+
+@pytest.mark.parametrize("source", [HALF, STREAM, MXFP4], ids=["converted_ahead", "weight_streamed", "mxfp4"])
 def test_loads_stay_inside_their_operands(tmp_path, source):
     compiler = os.environ.get("CXX") or shutil.which("g++")
     (tmp_path / "walk.cpp").write_text(COMMON + source)
