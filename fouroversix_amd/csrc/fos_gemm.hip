@@ -1270,7 +1270,8 @@ static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand
     } else if (M < 128 || (M == 128 && !forced)) {
         if (!streams) return h;
     }
-    if (fragment_bytes(M, K) > ((size_t)8 << 30)) return h;  // (a call with an operand that large keeps to the smaller workspace)
+    // (a call with operands that large keeps to the smaller workspace)
+    if (fragment_bytes(M, K) + (if4 ? fragment_bytes(N, K) : 0) > ((size_t)8 << 30)) return h;
     const int64_t chunks = (K + 127) / 128, m128 = M / 128, n128 = N / 128, m256 = (m128 + 1) / 2, n256 = (n128 + 1) / 2;
     const int forced_splits = tuning().gemm_splitk;
     int64_t splits = 1;

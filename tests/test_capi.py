@@ -146,3 +146,12 @@ def test_workspace_query_of_a_small_batch_on_forced_tiles(native, monkeypatch, t
     for m in (1, 16, 127, 128):
         assert L.fos_gemm_workspace_bytes(m, 256, 512) >= 0
         assert L.fos_linear_nvfp4_scratch_bytes(m, 512, 256) > 0
+
+
+def test_scratch_for_converted_operands_is_bounded(native):
+    """No more than 8 GiB of operands in fp16, the weight's among them where it is converted too (IF4)."""
+    L = native.lib()
+    most = 1 << 20  # rows of 4096 columns: 8 GiB
+    for m, n in ((most - 2048, 2048), (2048, most - 2048)):
+        assert L.fos_gemm_scratch_bytes(1, m, n, 4096) == 8 << 30
+        assert L.fos_gemm_scratch_bytes(1, m + 128, n, 4096) == L.fos_gemm_scratch_bytes(1, m, n + 128, 4096) == 0
