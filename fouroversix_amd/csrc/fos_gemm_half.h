@@ -25,7 +25,7 @@ struct ExpandOperand {
 struct ExpandParams {
     int64_t K, depth;  // K % 64 == 0; blocks from `depth` on are padding
     ExpandOperand operand[2];
-    int groups = 0;    // blocks of 16 rows of the first one (launch_expand_fragments)
+    int groups = 0, groups_all = 0;  // blocks of 16 rows of the first one and of both (launch_expand_fragments)
 };
 int launch_expand_fragments(ExpandParams p, bool if4, hipStream_t s);
 

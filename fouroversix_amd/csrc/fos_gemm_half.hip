@@ -52,14 +52,17 @@ FOS_DEVICE uint32_t tail_mask(int left) { return left <= 0 ? 0u : left == 1 ? 0x
 // A workgroup takes 16 rows and four chunks, a wavefront a chunk: 64 contiguous bytes of each of 16 rows in, four whole
 // KiB out.  Rows from `rows` on (a band is written whole) and blocks from `depth` on are zeros.  A second operand follows
 // in the same launch (blocks of rows from p.groups on).
+constexpr int kExpandGroupsY = 32768;  // (a grid has at most 65535 workgroups along y and z: more blocks of rows go on along z)
 template <bool IF4>
 __global__ __launch_bounds__(256) void expand_fragments_kernel(const ExpandParams p) {
     const int64_t chunks = (p.K + 127) >> 7, chunk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (chunk >= chunks) return;
-    const int second = blockIdx.y >= (unsigned)p.groups;  // (uniform)
+    const int group = (int)(blockIdx.z * kExpandGroupsY + blockIdx.y);
+    if (group >= p.groups_all) return;
+    const int second = group >= p.groups;  // (uniform)
     const ExpandOperand &o = p.operand[second];
     const int lane = threadIdx.x & 63, q = lane >> 4;
-    const int64_t row = (int64_t)(blockIdx.y - (second ? p.groups : 0)) * 16 + (lane & 15), k0 = chunk * 128 + q * 32;
+    const int64_t row = (int64_t)(group - (second ? p.groups : 0)) * 16 + (lane & 15), k0 = chunk * 128 + q * 32;
     uint4 w = make_uint4(0u, 0u, 0u, 0u);
     uint32_t s = 0u;
     if (row < o.rows && k0 < p.K) {
@@ -77,7 +80,9 @@ __global__ __launch_bounds__(256) void expand_fragments_kernel(const ExpandParam
 
 int launch_expand_fragments(ExpandParams p, bool if4, hipStream_t s) {
     p.groups = (int)((p.operand[0].rows + 127) / 128 * 8);
-    const dim3 grid((unsigned)((p.K + 511) / 512), (unsigned)(p.groups + (p.operand[1].rows + 127) / 128 * 8));
+    p.groups_all = p.groups + (int)((p.operand[1].rows + 127) / 128 * 8);
+    const int along_y = p.groups_all < kExpandGroupsY ? p.groups_all : kExpandGroupsY;
+    const dim3 grid((unsigned)((p.K + 511) / 512), (unsigned)along_y, (unsigned)((p.groups_all + along_y - 1) / along_y));
     if (if4) hipLaunchKernelGGL(expand_fragments_kernel<true>, grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL(expand_fragments_kernel<false>, grid, dim3(256), 0, s, p);
     return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;

@@ -923,6 +923,32 @@ def test_product_with_a_converted_ahead(monkeypatch, m, n, k, tile, splits):
         assert float(known_amax(with_bias)) == float(with_bias.abs().max())
 
 
+@pytest.mark.parametrize("dtype", ["nvfp4", "if4"])
+def test_operands_converted_ahead_of_more_rows_than_a_grid_has_along_one_axis(monkeypatch, dtype):
+    """The pass takes 16 rows a workgroup, and a grid has at most 65535 of them along y: the same bits as for a few rows at
+    the beginning, around the first row of the next layer of the grid, and at the end."""
+    monkeypatch.setenv("FOS_GEMM_TILE", "1001")
+    rows, n, k = 65536 * 16 + 128, 128, 64
+    g = torch.Generator("cuda").manual_seed(rows)
+
+    def operand(rows):
+        codes = torch.randint(0, 256, (rows, k // 2), generator=g, device="cuda", dtype=torch.uint8)
+        return codes, torch.randint(0, 127, (rows * k // 16,), generator=g, device="cuda", dtype=torch.uint8)
+
+    def tensor(codes, scales):
+        return fos.QuantizedTensor(codes, scales.view(torch.float8_e4m3fn), torch.tensor(1.5, device="cuda"), fos.DataType(dtype),
+                                   (codes.shape[0], k), fos.ScaleRule.mse, fos.RoundStyle.nearest, padded_shape=(codes.shape[0], k),
+                                   scale_factors_are_in_blackwell_layout=dtype == "nvfp4")
+
+    codes, scales = operand(rows)
+    b = tensor(*operand(n))
+    out = fos.quantized_matmul(tensor(codes, scales), b)
+    assert out.shape == (rows, n)
+    for first in (0, 32768 * 16 - 128, 65535 * 16 // 128 * 128, rows - 256):
+        part = tensor(codes[first:first + 256], scales[first * k // 16:(first + 256) * k // 16])
+        assert torch.equal(out[first:first + 256], fos.quantized_matmul(part, b))
+
+
 @pytest.mark.parametrize("splits", ["1", "3"])
 @pytest.mark.parametrize(("tokens", "n", "k"), [(65, 128, 256), (100, 384, 2560), (127, 256, 8192), (128, 256, 64), (128, 128, 1600)])
 def test_streaming_product_with_a_converted_ahead(monkeypatch, tokens, n, k, splits):
