@@ -1248,6 +1248,21 @@ static float half_cost(int tile, int64_t tiles, float k) {
     return k * tiles_cost(tiles, 512, 50, small);
 }
 
+// 65 ... 128 rows of a layer: the streaming form, in as many splits as leave a wavefront two chunks, against the weight-streaming kernel
+// of packed operands.  Layers (us) of 65, 96 and 128 rows, K = 8192 ... 53248 in steps of 512 and more, N = 128 ... 4096: narrow
+// outputs gain while the packed kernel has two splits of K (128 x 11264 -> 1024 26.9 -> 22.6), tie where it has three
+// (128 x 14336 -> 1024 29.3 and 29.0) and lose where it has more than the 8 there are here (65 x 28672 -> 512 28.3 and 34.1,
+// 128 x 16384 -> 2048 28.5 and 30.1), unless their columns alone make it few (96 x 16384 -> 2304 8 % faster here).  Wide ones tie up to
+// K = 10240 and gain beyond (128 x 14336 -> 4096 35.6 -> 32.8, 128 x 28672 -> 3072 23 % faster).  Where K % 256 leaves that kernel out
+// (gemm_nvfp4_kernel on a whole tile instead) 5 to 20 % on all but the narrowest of a long K.  Of fewer rows whole layers
+// are slower here (64 x 4096 -> 4096 19.6 and 17.8 in a graph).
+static bool stream_pays(int64_t N, int64_t K) {
+    if (N > 4096 || K < 8192) return false;
+    if (K % 256) return N > 256 || K < 20480;
+    if (N > 2560) return K > 10240;
+    return K < 12288 || (N > 2048 && K >= 16384);
+}
+
 // `expand`: the fragments have to be formed from codes and scales first (a layer's quantize kernel writes them instead, at
 // little more than it takes to write the codes).  With the fragments given the product is the faster one from 256 rows on,
 // on all but a few of 400 shapes, which tie: 1024 x 14336 x 4096 97 -> 83 us, 8192 x 4096 x 4096 207 -> 178,
@@ -1260,11 +1275,7 @@ static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand
     HalfPlan h;
     const int forced = tuning().gemm_tile;  // tuning / tests: 1000 + tile; another kernel's tile excludes this one
     if ((M > 128 && M % 128) || N % 128 || K % 64 || K > (1 << 20) || (forced && forced <= 1000)) return h;
-    // 65 ... 128 rows: the streaming form where K is long and the outputs are narrow, in as many splits as leave a wavefront two
-    // chunks.  Products with the fragments given, and of packed operands (us), 128 rows: 14336 -> 4096 23.5 and 28.5,
-    // 14336 -> 1024 17.6 and 21.3, but 4096 -> 4096 15.2 and 14.3, 14336 -> 8192 36.6 and 36.4; of fewer rows whole layers
-    // are slower with it (64 x 4096 -> 4096 19.6 and 17.8 in a graph).
-    const bool streams = M > 64 && M <= 128 && N <= 4096 && K >= 8192 && !if4 && !expand;
+    const bool streams = M > 64 && M <= 128 && !if4 && !expand && stream_pays(N, K);
     if (forced == 1000 + kHalfStream) {
         if (M <= 64 || M > 128 || if4) return h;
     } else if (M < 128 || (M == 128 && !forced)) {

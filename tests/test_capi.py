@@ -155,3 +155,29 @@ def test_scratch_for_converted_operands_is_bounded(native):
     for m, n in ((most - 2048, 2048), (2048, most - 2048)):
         assert L.fos_gemm_scratch_bytes(1, m, n, 4096) == 8 << 30
         assert L.fos_gemm_scratch_bytes(1, m + 128, n, 4096) == L.fos_gemm_scratch_bytes(1, m, n + 128, 4096) == 0
+
+
+@pytest.fixture
+def converts(native, monkeypatch):
+    """Whether a query answers with room for an operand in fp16: another number than with those kernels switched off."""
+    L = native.lib()
+
+    def ask(query, *args):
+        by_plan = getattr(L, query)(*args)
+        with monkeypatch.context() as m:
+            m.setenv("FOS_GEMM_TILE", "64")  # (the packed kernels as they are chosen by themselves)
+            L.fos_tuning_reload()
+            packed = getattr(L, query)(*args)
+        L.fos_tuning_reload()
+        return by_plan != packed
+
+    yield ask
+
+
+@pytest.mark.parametrize("rows", [65, 96, 128])
+def test_layers_of_up_to_128_rows_stream_the_weight_where_it_pays(converts, rows):
+    """Measured on either route: 5 to 50 % apart, and ties, which stay with the kernel that reads packed operands."""
+    for cols, n in ((8192, 512), (11264, 2048), (11776, 4096), (14336, 4096), (28672, 3072), (53248, 4096), (16384, 2304)):
+        assert converts("fos_linear_nvfp4_scratch_bytes", rows, cols, n), (cols, n)
+    for cols, n in ((28672, 512), (53248, 128), (16384, 2048), (24576, 1024), (14336, 1024), (8192, 4096), (8192, 4224), (7936, 512)):
+        assert not converts("fos_linear_nvfp4_scratch_bytes", rows, cols, n), (cols, n)
