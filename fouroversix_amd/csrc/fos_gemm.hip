@@ -1248,6 +1248,47 @@ static float half_cost(int tile, int64_t tiles, float k) {
     return k * tiles_cost(tiles, 512, 50, small);
 }
 
+// The kernels above, from packed operands, with the plan they have for the shape (us): `unsplit` times what the tiles take, or as
+// many shares of K and their sum.
+static float packed_cost(int64_t M, int64_t N, int64_t K, const GemmPlan &g, float unsplit, float sum, float sum_per_partial) {
+    if (g.splits == 1) return unsplit * tile_cost(M, N, nullptr) * (float)K / 4096;
+    static const float small[8] = {24, 34, 36.5f, 38.5f, 53, 56, 60, 64.5f};
+    return unsplit * tiles_cost(M / 128 * (N / 128) * g.splits, 512, 59, small) * (float)(g.ksteps_per_split * BK) / 4096 + sum +
+           sum_per_partial * 1e-6f * (float)g.splits * M * N;
+}
+
+// Whether the product with operands converted ahead, of `tiles_us` in `splits` over `workgroups` workgroups, is the faster one.
+// `expand`: the fragments have to be formed from codes and scales first (a layer's quantize kernel writes them instead).
+// What it pays beside its tiles: a split's partials and the kernel that adds them; a second workgroup on a few compute units where a
+// split of the small tile has 257 to 384 of them; the pass that forms the fragments; and their bytes, 2 per element written and read
+// where codes and scales take 0.56, which show once they leave the caches.  Constants (us, 10^6 elements): least loss over
+// 1200 layers and 700 products in graphs, each timed from packed operands and with the plan here (128 ... 16384 rows, N = 128 ... 16384,
+// K = 256 ... 16384; bf16 input).  Of the 490 NVFP4 layers among them with N and K from 1024 on six are more than 2 % slower than from packed operands,
+// at most 7 %.  Where fragments were taken for every layer of K > 2048 (us, with them and from packed operands):
+// 15439 x 6912 -> 128 197 and 130, 12053 x 6272 -> 768 214 and 167, 5726 x 9600 -> 1536 235 and 203, 174 x 11904 -> 1152 38.8
+// and 33.7; IF4 444 x 14144 -> 11648 318 and 276.  Where they pay: 1000 x 4096 -> 14336 95 and 110, 2048 x 4096 -> 4096 67 and 75,
+// 515 x 15360 -> 3456 86 and 142; products of 16384 x 4096 x 14336 1216 and 1392.
+static bool half_pays(int64_t M, int64_t N, int64_t K, bool if4, bool expand, float tiles_us, int tile, int64_t workgroups, int64_t splits) {
+    const GemmPlan g = plan_gemm(M, N, K, if4);
+    const auto beyond = [](float v, float from) { return v > from ? v - from : 0.0f; };
+    const float a = 1e-6f * M * K, partials = 1e-6f * (float)splits * M * N;
+    const float crowded = splits > 1 && tile == kHalfSmall && workgroups > 256 && workgroups <= 384 ? 1.0f : 0.0f;
+    const float short_k = K <= 2048 && g.splits == 1 ? 1.0f : 0.0f;
+    if (if4) {
+        const float both = a + 1e-6f * N * K;
+        return tiles_us + 1.5f + 2.0f * short_k + 0.21f * both + 0.7f * beyond(both, 85) + (splits > 1 ? 3.9f + 1.5f * partials : 0.0f) <
+               packed_cost(M, N, K, g, 1.21f, 4.5f, 1.45f);
+    }
+    if (expand) {
+        if (g.splits > 1) return false;  // (the pass and two sums of partials against one)
+        const float packed = packed_cost(M, N, K, g, 1.0f, 0.0f, 0.0f);
+        return tiles_us + 6.0f + 1.2f * short_k + 0.32f * a + 0.8f * beyond(a, 55) + 1.5f * crowded + (splits > 1 ? 1.1f + 1.75f * partials : 0.0f) <
+               0.945f * packed + 0.08f * beyond(packed, 90);
+    }
+    return tiles_us + 2.7f + 2.0f * short_k + 0.05f * a + 0.55f * beyond(a, 21) + 5.0f * crowded + (splits > 1 ? 2.6f + 1.9f * partials : 0.0f) <
+           packed_cost(M, N, K, g, 1.0f, 6.0f, 1.6f);
+}
+
 // 65 ... 128 rows of a layer: the streaming form, in as many splits as leave a wavefront two chunks, against the weight-streaming kernel
 // of packed operands.  Layers (us) of 65, 96 and 128 rows, K = 8192 ... 53248 in steps of 512 and more, N = 128 ... 4096: narrow
 // outputs gain while the packed kernel has two splits of K (128 x 11264 -> 1024 26.9 -> 22.6), tie where it has three
@@ -1263,14 +1304,6 @@ static bool stream_pays(int64_t N, int64_t K) {
     return K < 12288 || (N > 2048 && K >= 16384);
 }
 
-// `expand`: the fragments have to be formed from codes and scales first (a layer's quantize kernel writes them instead, at
-// little more than it takes to write the codes).  With the fragments given the product is the faster one from 256 rows on,
-// on all but a few of 400 shapes, which tie: 1024 x 14336 x 4096 97 -> 83 us, 8192 x 4096 x 4096 207 -> 178,
-// 6144 x 4096 x 4096 (384 tiles of 256 x 256) 180 -> 138, 2048 x 1024 x 4096 36 -> 28 in two splits, 1024 x 1024 x 14336
-// 49 -> 44 in four.  With the pass in front it has to make up for 4 us and 0.32 us per 2^20 elements of A: that
-// leaves the larger products.  IF4, both of whose operands are converted ahead, pays for B as well, against kernels that take
-// 1.7 times NVFP4's times: whole products of 2048 x 4096 x 4096 117 -> 70 us, 512 x 4096 x 4096 69 -> 39,
-// 256 x 14336 x 4096 76 -> 61; 384 x 8192 x 1024 stays (26 against 28).
 static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand) {
     HalfPlan h;
     const int forced = tuning().gemm_tile;  // tuning / tests: 1000 + tile; another kernel's tile excludes this one
@@ -1296,30 +1329,19 @@ static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand
         if (forced_splits > 0) splits = forced_splits;
         if (splits < 1) splits = 1;
     } else {
-        float best = 3e38f;
+        float best = 3e38f, tiles_us = 0.0f;
+        int64_t workgroups = 0;
         for (int tile = kHalf256; tile <= kHalfSmall; ++tile) {
             const int64_t tiles = tile == kHalf256 ? m256 * n256 : tile == kHalfWide ? m128 * n256 : m128 * n128;
             for (int s = 1; s <= 16; s = s < 4 ? s + 1 : s * 2) {
                 if (s > 1 && (chunks < 2 * s || tiles > 512)) break;
                 if (forced_splits && s != forced_splits) continue;
                 // (a split's partials are written and read again by a kernel of their own)
-                const float cost = half_cost(tile, tiles * s, (float)((chunks + s - 1) / s) / 32) + (s > 1 ? 5.5f + 0.25e-6f * 4 * s * M * N : 0.0f);
-                if (cost < best) best = cost, h.tile = tile, splits = s;
+                const float us = half_cost(tile, tiles * s, (float)((chunks + s - 1) / s) / 32), cost = us + (s > 1 ? 5.5f + 0.25e-6f * 4 * s * M * N : 0.0f);
+                if (cost < best) best = cost, tiles_us = us, h.tile = tile, splits = s, workgroups = tiles * s;
             }
         }
-        const float other = tile_cost(M, N, nullptr) * (float)K / 4096;
-        if (if4) {
-            if (best + 9 + 0.32e-6f * (M + N) * K > 1.7f * other) h.tile = 0;
-        } else if (expand && h.tile) {
-            const GemmPlan g = plan_gemm(M, N, K, false);
-            if (g.splits > 1 || best + 5 + 4 + 0.32e-6f * M * K > other) h.tile = 0;
-        } else if (h.tile && K <= 2048) {
-            // a short K is over before the fragments' four times as many bytes are paid for: layers (us) of 2048 x 1024 -> 4096 29.7 from
-            // codes and 32.5, 900 x 576 -> 8192 26.6 and 30.8, 900 x 2048 -> 8192 43.6 and 44.4; but 2048 x 2048 -> 2048 36.4 and
-            // 33.7, 1100 x 1536 -> 14336 60.2 and 53.5, and where the codes' product would split K 1100 x 1024 -> 1024 34.6 and 24.1
-            const GemmPlan g = plan_gemm(M, N, K, false);
-            if (g.splits == 1 && best + (g.kind == kPlanWide ? 5 : 3) + 0.25e-6f * M * K > other) h.tile = 0;
-        }
+        if (h.tile && !half_pays(M, N, K, if4, expand, tiles_us, h.tile, workgroups, splits)) h.tile = 0;
         if (!h.tile) return h;
     }
     if (splits > chunks) splits = chunks;

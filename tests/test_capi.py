@@ -151,10 +151,16 @@ def test_workspace_query_of_a_small_batch_on_forced_tiles(native, monkeypatch, t
 def test_scratch_for_converted_operands_is_bounded(native):
     """No more than 8 GiB of operands in fp16, the weight's among them where it is converted too (IF4)."""
     L = native.lib()
-    most = 1 << 20  # rows of 4096 columns: 8 GiB
-    for m, n in ((most - 2048, 2048), (2048, most - 2048)):
-        assert L.fos_gemm_scratch_bytes(1, m, n, 4096) == 8 << 30
-        assert L.fos_gemm_scratch_bytes(1, m + 128, n, 4096) == L.fos_gemm_scratch_bytes(1, m, n + 128, 4096) == 0
+    m = n = 1 << 19  # rows of 4096 columns, 8 GiB together
+    assert L.fos_gemm_scratch_bytes(1, m, n, 4096) == 8 << 30
+    assert L.fos_gemm_scratch_bytes(1, m + 128, n, 4096) == L.fos_gemm_scratch_bytes(1, m, n + 128, 4096) == 0
+
+
+LAYERS_FROM_CODES = [
+    # narrow outputs of many rows: the fragments' bytes; K split on either side; a second workgroup for a few compute units
+    (15439, 6912, 128), (12053, 6272, 768), (10225, 12544, 640), (5726, 9600, 1536), (4842, 13568, 128), (174, 11904, 1152), (1272, 16128, 256),
+]
+LAYERS_FROM_FRAGMENTS = [(1000, 4096, 14336), (2048, 4096, 4096), (16384, 4096, 14336), (8192, 4096, 4096), (515, 15360, 3456)]
 
 
 @pytest.fixture
@@ -174,9 +180,29 @@ def converts(native, monkeypatch):
     yield ask
 
 
+@pytest.mark.parametrize("shapes", [LAYERS_FROM_CODES, LAYERS_FROM_FRAGMENTS], ids=["codes", "fragments"])
+def test_layers_convert_their_operand_where_it_pays(converts, shapes):
+    """Measured on either route, 7 to 50 % apart."""
+    for shape in shapes:
+        assert converts("fos_linear_nvfp4_scratch_bytes", *shape) == (shapes is LAYERS_FROM_FRAGMENTS), shape
+
+
+@pytest.mark.parametrize(("dtype", "pays", "shapes"), [
+    (1, False, [(512, 11648, 14144), (640, 13056, 12544), (11008, 512, 11776)]),
+    (1, True, [(2048, 4096, 4096), (1280, 13184, 7040), (640, 4224, 13184)]),
+    (0, False, [(9856, 256, 16256), (8320, 1024, 14848), (4864, 2176, 16000), (2048, 1024, 4096)]),
+    (0, True, [(16384, 14336, 4096), (8192, 8192, 8192), (2560, 13952, 10624)]),
+])
+def test_products_convert_their_operands_where_it_pays(converts, dtype, pays, shapes):
+    """(IF4: both; NVFP4: A, by a pass of its own.)  Measured on either route, 8 to 45 % apart, but for 2048 x 1024 x 4096,
+    where the conversion and a split of K save no time and take two launches more."""
+    for shape in shapes:
+        assert converts("fos_gemm_scratch_bytes", dtype, *shape) == pays, shape
+
+
 @pytest.mark.parametrize("rows", [65, 96, 128])
 def test_layers_of_up_to_128_rows_stream_the_weight_where_it_pays(converts, rows):
-    """Measured on either route: 5 to 50 % apart, and ties, which stay with the kernel that reads packed operands."""
+    """As above for the form that streams the weight: 5 to 50 % apart, and ties, which stay with the packed kernel."""
     for cols, n in ((8192, 512), (11264, 2048), (11776, 4096), (14336, 4096), (28672, 3072), (53248, 4096), (16384, 2304)):
         assert converts("fos_linear_nvfp4_scratch_bytes", rows, cols, n), (cols, n)
     for cols, n in ((28672, 512), (53248, 128), (16384, 2048), (24576, 1024), (14336, 1024), (8192, 4096), (8192, 4224), (7936, 512)):
