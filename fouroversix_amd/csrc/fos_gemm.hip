@@ -1617,17 +1617,18 @@ int fos::gemm_decode_linear(const void *x, int64_t cols, int rule, const float *
 }
 
 size_t fos::linear_scratch_bytes(int64_t M, int64_t N, int64_t K) {
+    // (an input the quantizer does not write fragments of may take the codes' plan)
     const HalfPlan h = plan_half(M, N, K, false, false);
-    if (h.tile) return h.bytes;
     const int splits = plan_decode(M, N, K).splits;
     const size_t other = fos_gemm_workspace_bytes(M, N, K), partials = splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
-    return partials > other ? partials : other;
+    const size_t most = partials > other ? partials : other;
+    return h.tile && h.bytes > most ? h.bytes : most;
 }
 bool fos::linear_reads_fragments(int64_t M, int64_t N, int64_t K) { return plan_half(M, N, K, false, false).tile != 0; }
 int fos::gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
                      double denominator, int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
-                     float *d_amax, void *scratch, size_t scratch_bytes, fos_stream_t stream) {
-    const Fragments fragments = A ? kOfLayer : kGiven;
+                     float *d_amax, bool as_given, void *scratch, size_t scratch_bytes, fos_stream_t stream) {
+    const Fragments fragments = !A ? kGiven : as_given ? kOfLayer : kFromCodes;
     if (!A) A = sfA = static_cast<const uint8_t *>(scratch);  // (not read)
     return gemm_nvfp4_impl(A, B, sfA, sfB, nullptr, amax_a, amax_b, denominator, M, N, K, D, out_type, ldd, bias, d_amax, scratch,
                            scratch_bytes, stream, false, rows, -1, false, -1, fragments);

@@ -39,13 +39,14 @@ int launch_gemm_half(GemmParams &p, int tile, bool if4, int out_type, hipStream_
 int check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
                       double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax);
 // The product of a layer's call.  Its plan is made for fragments that the quantize kernel writes: linear_reads_fragments says
-// whether the shape takes them, at the beginning of the scratch; A null: they are there, otherwise codes and scales to
-// form them from (inputs that the streaming quantize kernels don't read).  Arguments checked by check_gemm_linear.
+// whether the shape takes them, at the beginning of the scratch; A null: they are there, otherwise codes and scales, for the
+// same plan (`as_given`: an input that the streaming quantize kernels would read at another address) or for the one of
+// products from codes.  Arguments checked by check_gemm_linear.
 size_t linear_scratch_bytes(int64_t M, int64_t N, int64_t K);
 bool linear_reads_fragments(int64_t M, int64_t N, int64_t K);
 int gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
                 double denominator, int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
-                float *d_amax, void *scratch, size_t scratch_bytes, fos_stream_t stream);
+                float *d_amax, bool as_given, void *scratch, size_t scratch_bytes, fos_stream_t stream);
 
 // A layer's call for a few rows of bf16 input (contiguous, 16-byte aligned, cols % 16 == 0), quantization included, in one
 // launch or, with K split, that and the reduction; kNotTaken where the shape is none for it.  In one launch d_amax has to be zero

@@ -612,14 +612,17 @@ extern "C" int fos_linear_nvfp4_into_zero(const void *x, int x_type, int64_t row
         if (rc != fos::kNotTaken) return rc;
     }
     // what a streaming quantize kernel reads, and the product wants converted, goes straight into the product's scratch
+    // (fp32 elements and ragged widths, which never are, take the plan that counts the pass over the codes: a layer of 3564 x 13184 ->
+    // 2432 in fp32 301 us from packed operands, 330 with that pass; another address or pitch alone changes no bit of the result)
     const bool direct = scratch_bytes >= at.total && x_type != FOS_T_F32 && streamable(x, cols, ld) &&
                         fos::linear_reads_fragments(gemm_rows, N, depth);
+    const bool as_given = x_type != FOS_T_F32 && cols % 16 == 0;
     rc = quantize_impl(x, x_type, rows, cols, ld, FOS_DTYPE_NVFP4, rule, FOS_ROUND_NEAREST, 0, 0, 0, FOS_SF_TILED_128X4,
                        direct ? nullptr : base + at.codes, direct ? nullptr : base + at.sf, amax, x_amax != nullptr, base + at.partials,
                        at.gemm - at.partials, stream, nullptr, 0, nullptr, 0, d_amax, direct ? base + at.gemm : nullptr);
     if (rc != FOS_OK) return rc;
     return fos::gemm_linear(direct ? nullptr : base + at.codes, W, base + at.sf, sfW, amax, w_amax, denominator, gemm_rows, rows, N, depth, D,
-                            out_type, ldd, bias, d_amax, gemm, gemm_bytes, stream);
+                            out_type, ldd, bias, d_amax, as_given, gemm, gemm_bytes, stream);
 }
 
 extern "C" int fos_quantize_devkey(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld,

@@ -986,6 +986,47 @@ def test_layer_with_operands_written_by_the_quantizer(monkeypatch, tokens, inf, 
     assert bool(((out.double() - exact).abs() <= bound).all())
 
 
+def linear_through_c(model, x, d_amax=None, d_amax_is_zero=None, scratch_bytes=None, rule=3):
+    """``fos_linear_nvfp4`` (or ``..._into_zero``) on a converted layer without a bias; the result and the scratch, which held 0xa5."""
+    import ctypes
+
+    from fouroversix_amd import _native
+
+    L, w = _native.lib(), model[0].quantized_weight()
+    rows, cols, n = x.shape[0], x.shape[1], w.values.shape[0]
+    bytes_ = L.fos_linear_nvfp4_scratch_bytes(rows, cols, n) if scratch_bytes is None else scratch_bytes
+    scratch = torch.full((bytes_,), 0xA5, dtype=torch.uint8, device="cuda")
+    out = torch.empty(L.fos_linear_nvfp4_rows(rows, cols), n, dtype=torch.bfloat16, device="cuda")
+    args = [x.data_ptr(), _native.TORCH_TO_T[x.dtype], rows, cols, x.stride(0), rule, None, w.values.data_ptr(), w.scale_factors.data_ptr(),
+            w.amax.data_ptr(), (6.0 * 256) ** 2, n, out.data_ptr(), _native.TORCH_TO_T[torch.bfloat16], n, None,
+            None if d_amax is None else d_amax.data_ptr()]
+    if d_amax_is_zero is not None:
+        args.append(d_amax_is_zero)
+    call = L.fos_linear_nvfp4 if d_amax_is_zero is None else L.fos_linear_nvfp4_into_zero
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert call(*args, scratch.data_ptr(), scratch.numel(), stream) == 0
+    return out[:rows], scratch
+
+
+@pytest.mark.parametrize(("dtype", "inf"), [(torch.float32, 2048), (torch.bfloat16, 2040), (torch.bfloat16, 2048)], ids=["fp32", "ragged", "bf16"])
+def test_layer_whose_input_the_quantizer_does_not_convert(dtype, inf):
+    """fp32 elements and ragged widths become codes, and the layer then has the plan of a product from codes: at this size it
+    leaves the part of the scratch alone that an input converted on the way (bf16, 2048 columns) fills."""
+    g = torch.Generator("cpu").manual_seed(inf)
+    model = nn.Sequential(nn.Linear(inf, 2048, bias=False, device="cuda", dtype=torch.bfloat16))
+    fos.quantize_model(model, fos.ModelQuantizationConfig())
+    model[0].quantize_weight_()
+    x = torch.randn(512, inf, generator=g).to(dtype).cuda()
+    out, scratch = linear_through_c(model, x)
+    written = bool((scratch[-512 * 2048 * 2:] != 0xA5).any())
+    assert written == (dtype == torch.bfloat16 and inf % 16 == 0)
+    with torch.no_grad():
+        assert torch.equal(out, model(x))
+    a, b = (fos.dequantize(q, dtype=torch.float32).double() for q in (fos.quantize(x), model[0].quantized_weight()))
+    exact, size = a @ b.T, a.abs() @ b.abs().T
+    assert bool(((out.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + 2 * 2048 * 2.0 ** -24 * size).all())
+
+
 @pytest.mark.parametrize("tile", ["1001", "1002", "1003"])
 @pytest.mark.parametrize(("m", "n", "k"), [(128, 128, 64), (384, 640, 192), (300, 200, 1088), (256, 256, 128)])
 def test_if4_product_with_both_operands_converted_ahead(monkeypatch, m, n, k, tile):
