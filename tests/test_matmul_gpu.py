@@ -1048,7 +1048,7 @@ def test_if4_product_with_both_operands_converted_ahead(monkeypatch, m, n, k, ti
 ])
 def test_layer_of_few_rows_in_one_launch(tokens, inf, outf, scale, rule):
     """Quantization and product in one kernel: the product of what the quantizer writes, with the bias, the recorded maximum
-    and a maximum recorded on the input; twice, so that a word that is not zero would show.  Bounds as for the layers above."""
+    and, the second time, a maximum recorded on the input.  Bounds as for the layers above."""
     from fouroversix_amd.quantize import attach_known_amax, known_amax
 
     g = torch.Generator("cpu").manual_seed(tokens + inf + outf)
@@ -1072,6 +1072,26 @@ def test_layer_of_few_rows_in_one_launch(tokens, inf, outf, scale, rule):
         exact = product + model[0].bias.double()
         bound = 2.0 ** -8 * (exact.abs() + product.abs()) * (1 + 2.0 ** -8) + 2 * inf * 2.0 ** -24 * size + 2.0 ** -133
         assert bool(((out.double() - exact).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("is_zero", [None, 0, 1])
+@pytest.mark.parametrize(("tokens", "inf", "outf"), [(1, 256, 128), (3, 2048, 384), (5, 8192, 256), (16, 4096, 1024)])
+def test_recorded_maximum_of_few_rows_through_the_c_entries(tokens, inf, outf, is_zero):
+    """Quantized inside the product's kernel (the scratch's room for codes stays as it was), in one launch and with K split: a word
+    that held a large number is cleared by the call, a word that is zero already is only extended."""
+    g = torch.Generator("cpu").manual_seed(tokens + inf + outf)
+    model = nn.Sequential(nn.Linear(inf, outf, bias=False, device="cuda", dtype=torch.bfloat16))
+    fos.quantize_model(model, fos.ModelQuantizationConfig())
+    model[0].quantize_weight_()
+    x = torch.randn(tokens, inf, generator=g).bfloat16().cuda()
+    word = torch.full((1,), 0.0 if is_zero else 1e30, device="cuda")
+    for _ in range(2):
+        out, scratch = linear_through_c(model, x, word, is_zero)
+        assert bool((scratch[:128 * inf // 2] == 0xA5).all())
+        assert float(word) == float(out.abs().max())
+        word.fill_(0.0 if is_zero else 1e30)
+    with torch.no_grad():
+        assert torch.equal(out, model(x))
 
 
 def test_layer_of_few_rows_with_an_element_that_is_no_number():
