@@ -44,6 +44,7 @@ EXPORTS = (
     "fos_linear_nvfp4_into_zero",
     "fos_linear_nvfp4_rows",
     "fos_linear_nvfp4_scratch_bytes",
+    "fos_linear_nvfp4_scratch_for",
     "fos_gemm_if4",
     "fos_gemm_if4_workspace_bytes",
     "fos_gemm_linear_rows",
@@ -120,6 +121,8 @@ def lib() -> ctypes.CDLL:
     L.fos_linear_nvfp4_into_zero.restype = i32
     L.fos_linear_nvfp4_rows.argtypes = [i64, i64]
     L.fos_linear_nvfp4_rows.restype = i64
+    L.fos_linear_nvfp4_scratch_for.argtypes = [vp, i32, i64, i64, i64, i64, ctypes.POINTER(ctypes.c_size_t)]
+    L.fos_linear_nvfp4_scratch_for.restype = ctypes.c_size_t
     L.fos_linear_nvfp4_scratch_bytes.argtypes = [i64, i64, i64]
     L.fos_linear_nvfp4_scratch_bytes.restype = ctypes.c_size_t
     L.fos_gemm_if4.argtypes = [vp, vp, vp, vp, vp, vp, dbl, i64, i64, i64, vp, i32, i64, vp, vp, vp, ctypes.c_size_t, vp]

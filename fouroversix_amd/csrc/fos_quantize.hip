@@ -541,14 +541,14 @@ extern "C" int fos_quantize(const void *x, int x_type, int64_t rows, int64_t col
                          amax, amax_is_input, workspace, workspace_bytes, stream, nullptr, 0);
 }
 
-// Scratch of fos_linear_nvfp4: codes, scales, tensor maximum, pass-1 partials and split-K partials, each from a
-// 256-byte boundary on.
+// Scratch of fos_linear_nvfp4: codes, scales (neither where the quantizer writes fragments: `direct`), tensor maximum, pass-1
+// partials and what the product takes, each from a 256-byte boundary on.
 namespace {
 struct LinearScratch {
     size_t codes = 0, sf, amax, partials, gemm, least, total;  // (least: without room for the operand as fragments)
-    LinearScratch(int64_t rows, int64_t cols, int64_t N) {
+    LinearScratch(int64_t rows, int64_t cols, int64_t N, bool direct = false) {
         auto up = [](size_t v) { return (v + 255) / 256 * 256; };
-        const size_t elems = (size_t)fos_padded_rows(rows) * (size_t)fos_padded_cols(cols);
+        const size_t elems = direct ? 0 : (size_t)fos_padded_rows(rows) * (size_t)fos_padded_cols(cols);
         sf = up(elems / 2);
         amax = sf + up(elems / 16);
         partials = amax + 256;
@@ -566,6 +566,21 @@ struct LinearScratch {
 extern "C" size_t fos_linear_nvfp4_scratch_bytes(int64_t rows, int64_t cols, int64_t N) {
     if (rows <= 0 || cols <= 0 || N <= 0) return 0;
     return LinearScratch(rows, cols, N).total;
+}
+
+// What a streaming quantize kernel reads, and the product wants converted, goes straight into the product's scratch.
+static bool writes_fragments(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int64_t N) {
+    return x_type != FOS_T_F32 && streamable(x, cols, ld) && fos::linear_reads_fragments(LinearScratch::gemm_rows(rows, cols), N, fos_padded_cols(cols));
+}
+
+extern "C" size_t fos_linear_nvfp4_scratch_for(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int64_t N, size_t *least) {
+    const bool sizes = rows > 0 && cols > 0 && N > 0;
+    const LinearScratch at = sizes ? LinearScratch(rows, cols, N) : LinearScratch(1, 1, 1);
+    const size_t fewest = at.least < at.total ? at.least : at.total;
+    size_t best = at.total;
+    if (sizes && writes_fragments(x, x_type, rows, cols, ld, N)) best = LinearScratch(rows, cols, N, true).total;
+    if (least) *least = !sizes ? 0 : fewest < best ? fewest : best;
+    return sizes ? best : 0;
 }
 
 extern "C" int64_t fos_linear_nvfp4_rows(int64_t rows, int64_t cols) {
@@ -589,8 +604,10 @@ extern "C" int fos_linear_nvfp4_into_zero(const void *x, int x_type, int64_t row
     if (!scratch) return FOS_E_NULL_POINTER;
     if (rows <= 0 || cols <= 0 || N <= 0) return FOS_E_BAD_SHAPE;
     if (((uintptr_t)scratch & 255) || ((uintptr_t)d_amax & 3)) return FOS_E_BAD_ALIGNMENT;
-    const LinearScratch at(rows, cols, N);
-    if (scratch_bytes < (at.least < at.total ? at.least : at.total)) return FOS_E_WORKSPACE;
+    const LinearScratch lean(rows, cols, N, true);
+    const bool direct = scratch_bytes >= lean.total && writes_fragments(x, x_type, rows, cols, ld, N);
+    const LinearScratch at = direct ? lean : LinearScratch(rows, cols, N);
+    if (!direct && scratch_bytes < (at.least < at.total ? at.least : at.total)) return FOS_E_WORKSPACE;
     uint8_t *base = static_cast<uint8_t *>(scratch);
     float *amax = x_amax ? const_cast<float *>(x_amax) : reinterpret_cast<float *>(base + at.amax);
     // (a call that the product refuses has written nothing, d_amax included)
@@ -611,11 +628,9 @@ extern "C" int fos_linear_nvfp4_into_zero(const void *x, int x_type, int64_t row
                                      reinterpret_cast<float *>(base + at.amax), gemm, gemm_bytes, stream);
         if (rc != fos::kNotTaken) return rc;
     }
-    // what a streaming quantize kernel reads, and the product wants converted, goes straight into the product's scratch
-    // (fp32 elements and ragged widths, which never are, take the plan that counts the pass over the codes: a layer of 3564 x 13184 ->
-    // 2432 in fp32 301 us from packed operands, 330 with that pass; another address or pitch alone changes no bit of the result)
-    const bool direct = scratch_bytes >= at.total && x_type != FOS_T_F32 && streamable(x, cols, ld) &&
-                        fos::linear_reads_fragments(gemm_rows, N, depth);
+    // (fp32 elements and ragged widths, which are never written as fragments, take the plan that counts the pass over the codes: a layer
+    // of 3564 x 13184 -> 2432 in fp32 301 us from packed operands, 330 with that pass; another address or pitch alone changes no bit of
+    // the result)
     const bool as_given = x_type != FOS_T_F32 && cols % 16 == 0;
     rc = quantize_impl(x, x_type, rows, cols, ld, FOS_DTYPE_NVFP4, rule, FOS_ROUND_NEAREST, 0, 0, 0, FOS_SF_TILED_128X4,
                        direct ? nullptr : base + at.codes, direct ? nullptr : base + at.sf, amax, x_amax != nullptr, base + at.partials,

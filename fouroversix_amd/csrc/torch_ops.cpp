@@ -239,16 +239,29 @@ void check_gemm_operands(const Tensor &a, const Tensor &b, const Tensor &a_sf, c
 // One GEMM launch.  alpha, or (amax_a, amax_b, denominator) for the output scale formed in the kernel;
 // with the latter, d_amax (device f32[1], zero or an earlier maximum) receives max|out| over the first `rows` rows
 // (negative: all).
+// Scratch of `best` bytes from torch's caching allocator, which keeps the block tied to the current stream; where there is not
+// that much memory, the `least` with which the call runs too (from packed operands).
+Tensor scratch_block(const Tensor &like, size_t best, size_t least) {
+    const auto opts = like.options().dtype(at::kByte);
+    if (best > least) {
+        try {
+            return at::empty({(int64_t)best}, opts);
+        } catch (const c10::OutOfMemoryError &) {
+            best = least;
+        }
+    }
+    return best ? at::empty({(int64_t)best}, opts) : Tensor();
+}
+
 Tensor gemm_launch(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tensor &b_sf, const Tensor *alpha, const Tensor *amax_a,
                    const Tensor *amax_b, double denominator, at::ScalarType out_dtype, const Tensor *d_amax, const Tensor *bias = nullptr,
                    int64_t rows = -1) {
     const int64_t m = a.size(0), n = b.size(0), k = a.size(1) * 2;
     Tensor out = at::empty({m, n}, a.options().dtype(out_dtype));
-    const size_t ws_bytes = fos_gemm_scratch_bytes(FOS_DTYPE_NVFP4, m, n, k);
     const DeviceGuard guard(a.device());
-    // split-K partial tiles of small-M shapes, A in fp16 of larger ones; from torch's caching allocator, which keeps the block tied to the current stream
-    Tensor ws;
-    if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
+    // split-K partial tiles of small-M shapes, A in fp16 of larger ones
+    const Tensor ws = scratch_block(a, fos_gemm_scratch_bytes(FOS_DTYPE_NVFP4, m, n, k), fos_gemm_workspace_bytes(m, n, k));
+    const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
     void *wsp = ws_bytes ? ws.data_ptr() : nullptr;
     const int out_type = out_dtype == at::kBFloat16 ? FOS_T_BF16 : FOS_T_F16;
     const fos_stream_t stream = current_stream(a);
@@ -359,13 +372,14 @@ std::tuple<Tensor, c10::optional<Tensor>> linear_nvfp4(const Tensor &x, int64_t 
         is_zero = word.second;
     }
     // (one block for the quantized input and the workspaces, from the caching allocator on the current stream)
-    const size_t bytes = fos_linear_nvfp4_scratch_bytes(rows, cols, n);
-    const Tensor scratch = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+    size_t least = 0;
+    const size_t best = fos_linear_nvfp4_scratch_for(x.data_ptr(), type_id(x.scalar_type(), "linear: x"), rows, cols, x.stride(0), n, &least);
+    const Tensor scratch = scratch_block(x, best, least);
     check(fos_linear_nvfp4_into_zero(x.data_ptr(), type_id(x.scalar_type(), "linear: x"), rows, cols, x.stride(0), (int)rule,
                            x_amax.has_value() ? known.data_ptr<float>() : nullptr, w.data_ptr<uint8_t>(),
                            static_cast<const uint8_t *>(w_sf.data_ptr()), w_amax.data_ptr<float>(), denominator, n, out.data_ptr(), out_type,
                            n, bias.has_value() ? bias->data_ptr() : nullptr, emit_amax ? d_amax->data_ptr<float>() : nullptr, is_zero ? 1 : 0,
-                           scratch.data_ptr(), bytes, stream),
+                           scratch.data_ptr(), (size_t)scratch.numel(), stream),
           "fouroversix::linear_nvfp4");
     return {out, d_amax};
 }
@@ -389,10 +403,9 @@ Tensor gemm_if4(const Tensor &a, const Tensor &b, const Tensor &a_sf, const Tens
     }
     const int64_t width = cols < 0 ? n : cols;
     Tensor out = at::empty({m, width}, a.options().dtype(out_dtype));
-    const size_t ws_bytes = fos_gemm_scratch_bytes(FOS_DTYPE_IF4, m, n, k);
     const DeviceGuard guard(a.device());
-    Tensor ws;
-    if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
+    const Tensor ws = scratch_block(a, fos_gemm_scratch_bytes(FOS_DTYPE_IF4, m, n, k), fos_gemm_if4_workspace_bytes(m, n, k));
+    const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
     check(fos_gemm_linear_rows(FOS_DTYPE_IF4, a.data_ptr<uint8_t>(), b.data_ptr<uint8_t>(), static_cast<const uint8_t *>(a_sf.data_ptr()),
                                static_cast<const uint8_t *>(b_sf.data_ptr()), amax_a.data_ptr<float>(), amax_b.data_ptr<float>(),
                                denominator, m, rows < 0 || rows > m ? m : rows, n, width, k, depth < 0 ? k : depth, out.data_ptr(), out_type, width,

@@ -290,6 +290,9 @@ int fos_gemm_nvfp4_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA
  * take, the product runs as fos_gemm_nvfp4_linear does).
  */
 size_t fos_linear_nvfp4_scratch_bytes(int64_t rows, int64_t cols, int64_t N);
+/* ... for one input: what its call runs fastest with (0.56 bytes per element less where x is converted without codes in
+ * between: bf16 or fp16, 16-byte aligned rows of a multiple of 16 columns), and in `least`, if given, what it needs at least. */
+size_t fos_linear_nvfp4_scratch_for(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int64_t N, size_t *least);
 int64_t fos_linear_nvfp4_rows(int64_t rows, int64_t cols);
 int fos_linear_nvfp4(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int rule, const float *x_amax,
                      const uint8_t *W, const uint8_t *sfW, const float *w_amax, double denominator, int64_t N,

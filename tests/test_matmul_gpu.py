@@ -986,6 +986,34 @@ def test_layer_with_operands_written_by_the_quantizer(monkeypatch, tokens, inf, 
     assert bool(((out.double() - exact).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("call", ["layer", "if4"])
+def test_calls_run_where_there_is_no_memory_for_converted_operands(monkeypatch, call):
+    """A limit on the process's memory that leaves room for the output and the smaller scratch: the result of the kernels that
+    read packed operands."""
+    rows, inf, outf = 8192, 4096, 1024  # 64 MiB and more of operands in fp16
+    dtype = "if4" if call == "if4" else "nvfp4"
+    model = nn.Sequential(nn.Linear(inf, outf, bias=False, device="cuda", dtype=torch.bfloat16))
+    fos.quantize_model(model, fos.ModelQuantizationConfig(dtype=dtype))
+    model[0].quantize_weight_()
+    x = make_input("randn", (rows, inf), 5).cuda()
+    monkeypatch.setenv("FOS_GEMM_TILE", "64")
+    with torch.no_grad():
+        expect = model(x)
+        monkeypatch.delenv("FOS_GEMM_TILE")
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        # (codes, scales and output: 18 + 16 MiB, in blocks of 2 and 20 MiB)
+        room = torch.cuda.memory_reserved() + (56 << 20)
+        torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory)
+        try:
+            with pytest.raises(torch.OutOfMemoryError):
+                torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+            out = model(x)
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(out, expect)
+
+
 def linear_through_c(model, x, d_amax=None, d_amax_is_zero=None, scratch_bytes=None, rule=3):
     """``fos_linear_nvfp4`` (or ``..._into_zero``) on a converted layer without a bias; the result and the scratch, which held 0xa5."""
     import ctypes
