@@ -9,11 +9,6 @@
 
 namespace fos {
 
-// Byte of the fragments of [rows, K] at which the eight values k ... k + 7 (k % 8 == 0) of a row begin.
-FOS_DEVICE int64_t fragment_offset(int64_t row, int64_t k, int64_t chunks) {
-    return ((row >> 7) * chunks + (k >> 7)) * kBandChunkBytes + ((k >> 3) & 3) * kFragmentStep + ((row & 127) >> 4) * 1024 +
-           (((k >> 5) & 3) * 16 + (row & 15)) * 16;
-}
 inline size_t fragment_bytes(int64_t rows, int64_t K) { return (size_t)((rows + 127) / 128) * (size_t)((K + 127) / 128) * kBandChunkBytes; }
 
 // One operand, or two of the same inner dimension (rows 0: none).

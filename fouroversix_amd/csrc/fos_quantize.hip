@@ -445,7 +445,7 @@ static int quantize_impl(const void *x, int x_type, int64_t rows, int64_t cols, 
     // fp16 input has a streaming form for NVFP4 codes with 1x16 blocks and round to nearest
     const bool f16_streams = x_type == FOS_T_F16 && dtype == FOS_DTYPE_NVFP4 && round_style == FOS_ROUND_NEAREST && !block2d;
     const bool aligned = (x_type == FOS_T_BF16 || f16_streams) && streamable(x, cols, ld);
-    if (frags && (!aligned || block2d || round_style != FOS_ROUND_NEAREST || (dtype == FOS_DTYPE_IF4 && rule != FOS_RULE_MSE)))
+    if (frags && (!aligned || block2d || round_style != FOS_ROUND_NEAREST || dtype != FOS_DTYPE_NVFP4))
         return FOS_E_UNSUPPORTED;
     if (pseudo_out) {
         // only the streaming kernels have the fused epilogue

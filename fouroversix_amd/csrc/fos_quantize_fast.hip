@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
     const bool tiled = !PSEUDO && !FRAG && p.sf_layout == FOS_SF_TILED_128X4;
     const int64_t code_pitch = p.cols_p >> 1;
     const uint32_t n_tiles = (uint32_t)(p.rows_p >> 7) * (uint32_t)p.tiles_x;
-    static_assert(!(SPLIT && PSEUDO) && !(FRAG && (PSEUDO || SR)), "split tiles: codes and scales, or fragments, out");
+    static_assert(!(SPLIT && PSEUDO) && !(FRAG && (PSEUDO || SR || IF4)), "split tiles: codes and scales, or fragments, out");
     // fragments: chunks of 128 columns, written whole (a tile's 256 columns are two of them)
     const int64_t chunks = (p.cols_p + 127) >> 7, blocks_out = FRAG ? chunks * 8 : sf_cols;
     const uint32_t f_lane = (uint32_t)((lb >> 3) * kBandChunkBytes + (lb & 1) * 2 * kFragmentStep + (wave >> 1) * 1024 + ((lb >> 1) & 3) * 256 +
@@ -251,8 +251,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((SR ||
             // rows 32 (g >> 1) + 4 (g & 1) + ... of the tile: two fragments, or four rows inside them, per step
             const BufferRsrc rfrags = make_rsrc(reinterpret_cast<const void *>(uniform64(t.codes_base)), 0xffffffffu);
             const uint32_t step = (uint32_t)(2048 * (g >> 1) + 64 * (g & 1));
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dequant_word<IF4>(o.c0, o.s, 0)), rfrags, f_lane + step, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dequant_word<IF4>(o.c1, o.s, 0)), rfrags,
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dequant_word<false>(o.c0, o.s, 0)), rfrags, f_lane + step, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dequant_word<false>(o.c1, o.s, 0)), rfrags,
                                                    f_lane + step + kFragmentStep, 0, 0);
             return;
         }
@@ -354,7 +354,7 @@ static void launch_rows_as(QuantParams &p, hipStream_t s) {
 
 template <int RULE, bool PSEUDO, bool SR, bool IF4, bool F16>
 static void launch_rows(QuantParams &p, hipStream_t s) {
-    if constexpr (!PSEUDO && !SR) {
+    if constexpr (!PSEUDO && !SR && !IF4) {
         if (p.frags) return launch_rows_as<RULE, PSEUDO, SR, IF4, F16, true>(p, s);
     }
     launch_rows_as<RULE, PSEUDO, SR, IF4, F16, false>(p, s);
