@@ -1261,32 +1261,33 @@ static float packed_cost(int64_t M, int64_t N, int64_t K, const GemmPlan &g, flo
 // `expand`: the fragments have to be formed from codes and scales first (a layer's quantize kernel writes them instead).
 // What it pays beside its tiles: a split's partials and the kernel that adds them; a second workgroup on a few compute units where a
 // split of the small tile has 257 to 384 of them; the pass that forms the fragments; and their bytes, 2 per element written and read
-// where codes and scales take 0.56, which show once they leave the caches.  Constants (us, 10^6 elements): least loss over
-// 1200 layers and 700 products in graphs, each timed from packed operands and with the plan here (128 ... 16384 rows, N = 128 ... 16384,
-// K = 256 ... 16384; bf16 input).  Of the 490 NVFP4 layers among them with N and K from 1024 on six are more than 2 % slower than from packed operands,
-// at most 7 %.  Where fragments were taken for every layer of K > 2048 (us, with them and from packed operands):
-// 15439 x 6912 -> 128 197 and 130, 12053 x 6272 -> 768 214 and 167, 5726 x 9600 -> 1536 235 and 203, 174 x 11904 -> 1152 38.8
-// and 33.7; IF4 444 x 14144 -> 11648 318 and 276.  Where they pay: 1000 x 4096 -> 14336 95 and 110, 2048 x 4096 -> 4096 67 and 75,
-// 515 x 15360 -> 3456 86 and 142; products of 16384 x 4096 x 14336 1216 and 1392.
+// where codes and scales take 0.56, which show once they leave the caches, the less the more columns there are to multiply meanwhile.
+// Constants (us, 10^6 elements): least loss over 1400 layers and 1000 products in graphs, each timed from packed operands and with the plan
+// here (128 ... 16384 rows, N = 128 ... 28672, K = 256 ... 28672; bf16 input).  Of the 559 NVFP4 layers among them with N and K from 1024 on
+// nine are more than 2 % slower than from packed operands, at most 7 %.  Where fragments were taken for every layer of K > 2048 (us,
+// with them and from packed operands): 15439 x 6912 -> 128 197 and 130, 12053 x 6272 -> 768 214 and 167, 5726 x 9600 -> 1536 235
+// and 203, 174 x 11904 -> 1152 38.8 and 33.7; IF4 444 x 14144 -> 11648 318 and 276.  Where they pay: 1000 x 4096 -> 14336 95 and 110,
+// 2048 x 4096 -> 4096 67 and 75, 8192 x 14336 -> 4096 725 and 760, 515 x 15360 -> 3456 86 and 142; products of
+// 16384 x 4096 x 14336 1216 and 1392.
 static bool half_pays(int64_t M, int64_t N, int64_t K, bool if4, bool expand, float tiles_us, int tile, int64_t workgroups, int64_t splits) {
     const GemmPlan g = plan_gemm(M, N, K, if4);
     const auto beyond = [](float v, float from) { return v > from ? v - from : 0.0f; };
-    const float a = 1e-6f * M * K, partials = 1e-6f * (float)splits * M * N;
+    const float a = 1e-6f * M * K, partials = 1e-6f * (float)splits * M * N, columns = (float)N / 2500, exposed = 1.0f / (1.0f + columns * columns);
     const float crowded = splits > 1 && tile == kHalfSmall && workgroups > 256 && workgroups <= 384 ? 1.0f : 0.0f;
     const float short_k = K <= 2048 && g.splits == 1 ? 1.0f : 0.0f;
     if (if4) {
         const float both = a + 1e-6f * N * K;
-        return tiles_us + 1.5f + 2.0f * short_k + 0.21f * both + 0.7f * beyond(both, 85) + (splits > 1 ? 3.9f + 1.5f * partials : 0.0f) <
+        return tiles_us + 1.5f + 2.0f * short_k + 0.21f * both + 0.7f * beyond(both, 85) + 1.5f * crowded + (splits > 1 ? 3.9f + 1.5f * partials : 0.0f) <
                packed_cost(M, N, K, g, 1.21f, 4.5f, 1.45f);
     }
     if (expand) {
         if (g.splits > 1) return false;  // (the pass and two sums of partials against one)
         const float packed = packed_cost(M, N, K, g, 1.0f, 0.0f, 0.0f);
-        return tiles_us + 6.0f + 1.2f * short_k + 0.32f * a + 0.8f * beyond(a, 55) + 1.5f * crowded + (splits > 1 ? 1.1f + 1.75f * partials : 0.0f) <
-               0.945f * packed + 0.08f * beyond(packed, 90);
+        return tiles_us + 5.5f + 0.31f * a + 1.4f * exposed * beyond(a, 48) + 2.0f * crowded + (splits > 1 ? 1.75f * partials : 0.0f) <
+               0.94f * packed + 0.08f * beyond(packed, 90);
     }
-    return tiles_us + 2.7f + 2.0f * short_k + 0.05f * a + 0.55f * beyond(a, 21) + 5.0f * crowded + (splits > 1 ? 2.6f + 1.9f * partials : 0.0f) <
-           packed_cost(M, N, K, g, 1.0f, 6.0f, 1.6f);
+    return tiles_us + 2.7f + 1.5f * short_k + 0.05f * a + 0.75f * exposed * beyond(a, 21) + 4.0f * crowded + (splits > 1 ? 2.6f + 1.9f * partials : 0.0f) <
+           packed_cost(M, N, K, g, 1.0f, 5.6f, 1.8f);
 }
 
 // 65 ... 128 rows of a layer: the streaming form, in as many splits as leave a wavefront two chunks, against the weight-streaming kernel
