@@ -746,8 +746,10 @@ __global__ __launch_bounds__(64 * skinny_waves(WN), (WN == 2 && MT == 2) ? 2 : 1
 // fp16(value * scale) in the order the matrix instructions read them.  A kernel of its own in front cost a launch, its
 // latency and, at 16 rows, 9 us in which 64 workgroups scanned the tensor while the weight could have been on its way: here
 // it is in flight behind x.  What each workgroup quantizes again is what bounds it, so K is split
-// where that is more than kFusedElements (plan_decode).  Layers, us a call / in a graph: 1 x 4096 -> 4096 14.4 / 12.6 -> 12.1 / 11.0,
-// 16 x 4096 -> 4096 17.6 / 15.3 -> 14.9 / 16.4, 1 x 14336 -> 4096 19.2 / 17.7 -> 13.1 / 13.5.
+// where that is more than kFusedElements (plan_decode).  Layers in two launches and here, us a call / in a graph (one box): 1 x 4096 -> 4096
+// 14.8 / 12.2 and 12.4 / 11.0, 16 x 4096 -> 4096 15.3 / 14.7 and 15.1 / 14.5 (17.5 / 15.6 in two launches before the scan of the
+// quantize kernel kept its loads in flight), 1 x 14336 -> 4096 16.7 / 17.2 and 13.0 / 14.3.  357 shapes: 15 % less a call, 9 % in a
+// graph, where launches are cheap and the least work per workgroup loses (4 x 1024 -> 8192 10.0 and 11.0).
 template <int NB>
 struct DecodeRegs {
     uint4 b[NB][2];   // 64 codes of NB rows of B
@@ -1239,7 +1241,8 @@ struct HalfPlan {
 };
 
 // Time of `tiles` output tiles (us at K = 4096, without what a launch takes at any K): 256 workgroups of the 256 x 256 tile
-// run at a time, 512 of the others.  Measured with the fragments given, 128 ... 8192 rows, N = 1024 ... 14336, K = 1024 ... 14336.
+// run at a time, 512 of the others (of the 128 x 128 tile, with 160 registers and 51 KB of LDS, up to 768: the table covers 512 and
+// takes what is beyond for a second generation).  Measured with the fragments given, 128 ... 8192 rows, N = 1024 ... 14336, K = 1024 ... 14336.
 static float half_cost(int tile, int64_t tiles, float k) {
     static const float big[8] = {65, 66, 67, 70, 71.5f, 75.5f, 79.5f, 86}, wide[8] = {42, 43.5f, 46, 50, 77, 79, 83, 89},
                        small[8] = {28.5f, 29, 30, 32, 43, 45.5f, 48, 52};
@@ -1559,10 +1562,11 @@ extern "C" int fos_gemm_linear_rows(int dtype, const uint8_t *A, const uint8_t *
 }
 
 // A layer's call in one launch (splits == 1), or with K split: at most 16 rows, K in whole steps, an input that
-// every workgroup can scan, and quantize its share of.  One workgroup per compute unit: the quantization is done by
-// each of them, so there are as few as fill the chip, of 16, 32 or 64 rows of B.  Beyond 8192 columns a workgroup's share of B
-// takes longer than a launch saves (1 x 4096 -> 14336: 15.0 / 17 us a call / in a graph, two launches 15.3 / 14.4), and beyond
-// 65536 elements the quantization does (8 x 14336 -> 4096 20.5 / 22.5 and 20.3 / 20.5, 4 x 14336 17.5 / 19.4 and 25.0 / 21.1).
+// every workgroup can scan, and quantize its share of.  The quantization is done by each workgroup, so there are as few as
+// fill the chip, of 16, 32 or 64 rows of B.  Beyond 8192 columns they no longer run all at once: the kernel takes 176 registers at 32 rows
+// of B and 236 at 64, which leaves a compute unit one workgroup, and N = 14336 has 448 of 32 rows (1 x 4096 -> 14336 15.0 / 17 us a
+// call / in a graph, two launches 14.7 / 14.4).  Beyond 65536 elements the quantization takes longer than a launch saves (8 x 14336 -> 4096
+// 20.5 / 22.5 and 20.3 / 20.5, 4 x 14336 17.5 / 19.4 and 25.0 / 21.1).
 struct DecodePlan {
     int splits = 0, steps = 0, nb = 0;  // (splits 0: not taken)
 };
