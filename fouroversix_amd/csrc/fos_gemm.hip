@@ -1279,8 +1279,8 @@ static bool half_pays(int64_t M, int64_t N, int64_t K, bool if4, bool expand, fl
     const float crowded = splits > 1 && tile == kHalfSmall && workgroups > 256 && workgroups <= 384 ? 1.0f : 0.0f;
     const float short_k = K <= 2048 && g.splits == 1 ? 1.0f : 0.0f;
     if (if4) {
-        const float both = a + 1e-6f * N * K;
-        return tiles_us + 1.5f + 2.0f * short_k + 0.21f * both + 0.7f * beyond(both, 85) + 1.5f * crowded + (splits > 1 ? 3.9f + 1.5f * partials : 0.0f) <
+        const float both = a + 1e-6f * N * K, hidden = tiles_us > 142 ? 0.6f * tiles_us : 85;  // (elements behind the multiplication)
+        return tiles_us + 1.5f + 2.0f * short_k + 0.21f * both + 0.7f * beyond(both, hidden) + 1.2f * crowded + (splits > 1 ? 3.9f + 1.5f * partials : 0.0f) <
                packed_cost(M, N, K, g, 1.21f, 4.5f, 1.45f);
     }
     if (expand) {
