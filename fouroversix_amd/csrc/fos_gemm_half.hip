@@ -370,7 +370,8 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N, OCC) void gemm_half_kernel(c
 // repeat (gemm_nvfp4_skinny_kernel); this one by what a compute unit reads of A out of L2, about 30 bytes a cycle.
 // (Eight wavefronts with A a step ahead: 24.5 us at 128 x 4096 x 14336 in four splits, 23.5 here.)
 // The accumulators are summed over the wavefronts in two halves through LDS, in fixed order.
-template <int OUT>
+// HALF_CHUNK: K % 128 = 64, whose last chunk exists by half (the choice of lane offsets in the loop cost 1 % of the layer of 128 x 14336 -> 4096).
+template <int OUT, bool HALF_CHUNK>
 __global__ __launch_bounds__(256, 1) void gemm_half_stream_kernel(const GemmParams p) {
     constexpr bool OUT_BF16 = OUT == kOutBF16;
     constexpr int WM = 8, WN = 4, kWaves = 4, HALF = WM * WN / 2;  // HALF: groups of four accumulators a lane hands over at a time
@@ -394,7 +395,7 @@ __global__ __launch_bounds__(256, 1) void gemm_half_stream_kernel(const GemmPara
         fa[w][i] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(va + i * 1024), (int)at, 0));
     };
     auto load_b = [&](int chunk, int set) {
-        const bool half = is_half(chunk, kbytes);
+        const bool half = HALF_CHUNK && is_half(chunk, kbytes);
 #pragma unroll
         for (int j = 0; j < WN; ++j)
             codes[set][j] = __builtin_amdgcn_raw_buffer_load_b128(rb, (int)stream_codes_lane(lane, j, kbytes, half), chunk * 64, 0);
@@ -486,9 +487,11 @@ __global__ __launch_bounds__(256, 1) void gemm_half_stream_kernel(const GemmPara
     }
 }
 
+template <bool HALF_CHUNK>
 static int launch_stream(GemmParams &p, int out_type, hipStream_t s) {
     constexpr int lds_bytes = 64 * 1024;  // half the accumulators of four wavefronts
-    auto kernel = p.splits > 1 ? gemm_half_stream_kernel<kOutPartial> : out_type == FOS_T_BF16 ? gemm_half_stream_kernel<kOutBF16> : gemm_half_stream_kernel<kOutF16>;
+    auto kernel = p.splits > 1 ? gemm_half_stream_kernel<kOutPartial, HALF_CHUNK>
+                  : out_type == FOS_T_BF16 ? gemm_half_stream_kernel<kOutBF16, HALF_CHUNK> : gemm_half_stream_kernel<kOutF16, HALF_CHUNK>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)(p.N / 64), (unsigned)p.splits), dim3(256), lds_bytes, s, p);
     return hipGetLastError() == hipSuccess ? FOS_OK : FOS_E_LAUNCH;
 }
@@ -513,7 +516,7 @@ int launch_gemm_half(GemmParams &p, int tile, bool if4, int out_type, hipStream_
         if (tile == kHalfWide) return launch_tiles<1, 4, 8, 12, 2, true>(p, out_type, s);
         return launch_tiles<2, 2, 4, 4, 2, true>(p, out_type, s);
     }
-    if (tile == kHalfStream) return launch_stream(p, out_type, s);
+    if (tile == kHalfStream) return p.K % 128 ? launch_stream<true>(p, out_type, s) : launch_stream<false>(p, out_type, s);
     if (tile == kHalf256) return launch_tiles<2, 4, 8, 12, 2, false>(p, out_type, s);
     if (tile == kHalfWide) return launch_tiles<1, 4, 8, 12, 2, false>(p, out_type, s);
     return launch_tiles<2, 2, 4, 4, 2, false>(p, out_type, s);

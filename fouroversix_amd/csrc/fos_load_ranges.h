@@ -68,8 +68,8 @@ constexpr uint32_t mx_codes_lane(int first_row, int lane, bool odd, uint32_t kby
     return (uint32_t)(first_row + (lane >> 3)) * kbytes + mx_unit(lane, odd);
 }
 constexpr uint32_t mx_whole_or(bool half, int lane, bool odd, uint32_t offset) { return half && mx_unit(lane, odd) >= 64 ? kNoRead : offset; }
-constexpr uint32_t mx_codes_scalar(int t, int step, uint32_t kbytes) { return (uint32_t)step * 128 + (uint32_t)t * 8 * kbytes; }
+constexpr int mx_codes_scalar(int t, int step, int kbytes) { return step * 128 + t * 8 * kbytes; }
 constexpr uint32_t mx_scales_lane(int lane) { return (uint32_t)lane * 16; }
-constexpr uint32_t mx_scales_scalar(int step) { return (uint32_t)step * 1024; }
+constexpr int mx_scales_scalar(int step) { return step * 1024; }
 
 }  // namespace fos

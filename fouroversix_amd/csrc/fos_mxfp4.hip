@@ -635,8 +635,9 @@ FOS_DEVICE mx_v4i mx_raw_rsrc(const void *base, uint32_t bytes) {
 // s_waitcnt vmcnt(n) alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14, the other counters at their maxima)
 #define MX_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
 
-// BM, BN = 128 or 256: eight wavefronts, two rows of four, each BM / 2 x BN / 4.
-template <int BM, int BN, int STAGES, bool OUT_BF16>
+// BM, BN = 128 or 256: eight wavefronts, two rows of four, each BM / 2 x BN / 4.  HALF_STEP: K % 256 = 128, whose last step is filled by half
+// (the choice of lane offsets in every step cost 0.5 % of the layer of 2048 x 14336 -> 4096, a clamped first byte 1 to 2 %).
+template <int BM, int BN, int STAGES, bool OUT_BF16, bool HALF_STEP>
 __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams p) {
     constexpr int WAVES_N = 4, WM = BM / 64, WN = BN / 128;
     constexpr int kRow = 128;  // bytes of a row in a stage
@@ -681,7 +682,7 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
     const uint32_t sf_to = (uint32_t)(kOperandBytes + sf_tile * 1024);
     const uint32_t lds_base = (uint32_t)(uintptr_t)(MxLdsPtr)mx_lds;
     auto issue = [&](int ks, int stage) {
-        const bool half = mx_is_half(ks, row_bytes);
+        const bool half = HALF_STEP && mx_is_half(ks, row_bytes);
         const uint32_t a_off[2] = {mx_whole_or(half, lane, false, lda_off), mx_whole_or(half, lane, true, lda_odd)};
         const uint32_t b_off[2] = {mx_whole_or(half, lane, false, ldb_off), mx_whole_or(half, lane, true, ldb_odd)};
         const uint32_t base = lds_base + (uint32_t)(stage * kStageBytes);
@@ -694,13 +695,13 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
         for (int t = 0; t < PA; ++t)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                          :
-                         : "s"(run_a + t * 1024), "v"(a_off[t & 1]), "s"(ra), "s"(mx_codes_scalar(t, ks, row_bytes))
+                         : "s"(run_a + t * 1024), "v"(a_off[t & 1]), "s"(ra), "s"(mx_codes_scalar(t, ks, (int)row_bytes))
                          : "memory");
 #pragma unroll
         for (int t = 0; t < PB; ++t)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                          :
-                         : "s"(run_b + t * 1024), "v"(b_off[t & 1]), "s"(rb), "s"(mx_codes_scalar(t, ks, row_bytes))
+                         : "s"(run_b + t * 1024), "v"(b_off[t & 1]), "s"(rb), "s"(mx_codes_scalar(t, ks, (int)row_bytes))
                          : "memory");
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :
@@ -794,8 +795,11 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_dma_kernel(const MxGemmParams 
     };
     const int full = (int)(chunks >> 1);
     for (int ks = 0; ks < full; ++ks) kstep(ks, std::integral_constant<int, 2>{});
-    if (full < ksteps) kstep(full, std::integral_constant<int, 1>{});
-    // loads still in flight write LDS: drain them before the stages are used again
+    if constexpr (HALF_STEP) kstep(full, std::integral_constant<int, 1>{});
+    // loads still in flight write LDS: drain them before the stages are used again.  (The empty statement keeps the last step's
+    // fragment reads here: without it the compiler moved those of a half step, which stands in no loop, behind the barrier and
+    // into the branches of the epilogue, whose writes of LDS they then met)
+    asm volatile("" ::: "memory");
     MX_WAIT_VMCNT(0);
     __syncthreads();  // ... those of every wavefront, and all fragment reads are done
 
@@ -826,7 +830,9 @@ static int launch_gemm_mxfp4_dma(MxGemmParams &p, int out_type, hipStream_t s) {
     constexpr size_t lds_bytes = (size_t)STAGES * dma_stage_bytes(BM, BN);
     p.tiles_m = (int)((p.M + BM - 1) / BM);
     p.tiles_n = (int)((p.N + BN - 1) / BN);
-    auto kernel = out_type == FOS_T_BF16 ? gemm_mxfp4_dma_kernel<BM, BN, STAGES, true> : gemm_mxfp4_dma_kernel<BM, BN, STAGES, false>;
+    const bool bf16 = out_type == FOS_T_BF16, half = p.K % 256 != 0;
+    auto kernel = half ? (bf16 ? gemm_mxfp4_dma_kernel<BM, BN, STAGES, true, true> : gemm_mxfp4_dma_kernel<BM, BN, STAGES, false, true>)
+                       : (bf16 ? gemm_mxfp4_dma_kernel<BM, BN, STAGES, true, false> : gemm_mxfp4_dma_kernel<BM, BN, STAGES, false, false>);
     if (hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
         return FOS_E_LAUNCH;
     hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(512), lds_bytes, s, p);
