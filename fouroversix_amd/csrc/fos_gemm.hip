@@ -1335,13 +1335,15 @@ static HalfPlan plan_half(int64_t M, int64_t N, int64_t K, bool if4, bool expand
     } else {
         float best = 3e38f, tiles_us = 0.0f;
         int64_t workgroups = 0;
+        const unsigned n = (unsigned)chunks;
+        const unsigned shares[17] = {0, n, (n + 1) / 2, (n + 2) / 3, (n + 3) / 4, 0, 0, 0, (n + 7) / 8, 0, 0, 0, 0, 0, 0, 0, (n + 15) / 16};  // chunks a split
         for (int tile = kHalf256; tile <= kHalfSmall; ++tile) {
             const int64_t tiles = tile == kHalf256 ? m256 * n256 : tile == kHalfWide ? m128 * n256 : m128 * n128;
             for (int s = 1; s <= 16; s = s < 4 ? s + 1 : s * 2) {
                 if (s > 1 && (chunks < 2 * s || tiles > 512)) break;
                 if (forced_splits && s != forced_splits) continue;
                 // (a split's partials are written and read again by a kernel of their own)
-                const float us = half_cost(tile, tiles * s, (float)((chunks + s - 1) / s) / 32), cost = us + (s > 1 ? 5.5f + 0.25e-6f * 4 * s * M * N : 0.0f);
+                const float us = half_cost(tile, tiles * s, (float)shares[s] / 32), cost = us + (s > 1 ? 5.5f + 0.25e-6f * 4 * s * M * N : 0.0f);
                 if (cost < best) best = cost, tiles_us = us, h.tile = tile, splits = s, workgroups = tiles * s;
             }
         }
@@ -1621,15 +1623,14 @@ int fos::gemm_decode_linear(const void *x, int64_t cols, int rule, const float *
     return launch_decode_layer<FOS_RULE_ABS_MAX>(p, in, d.nb, out_type, s);
 }
 
-size_t fos::linear_scratch_bytes(int64_t M, int64_t N, int64_t K) {
+fos::LinearSizes fos::linear_sizes(int64_t M, int64_t N, int64_t K) {
     // (an input the quantizer does not write fragments of may take the codes' plan)
     const HalfPlan h = plan_half(M, N, K, false, false);
     const int splits = plan_decode(M, N, K).splits;
-    const size_t other = fos_gemm_workspace_bytes(M, N, K), partials = splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
-    const size_t most = partials > other ? partials : other;
-    return h.tile && h.bytes > most ? h.bytes : most;
+    const size_t least = fos_gemm_workspace_bytes(M, N, K), partials = splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+    const size_t most = partials > least ? partials : least;
+    return {least, h.tile && h.bytes > most ? h.bytes : most, h.tile != 0};
 }
-bool fos::linear_reads_fragments(int64_t M, int64_t N, int64_t K) { return plan_half(M, N, K, false, false).tile != 0; }
 int fos::gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
                      double denominator, int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
                      float *d_amax, bool as_given, void *scratch, size_t scratch_bytes, fos_stream_t stream) {

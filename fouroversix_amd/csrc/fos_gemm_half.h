@@ -33,12 +33,16 @@ int launch_gemm_half(GemmParams &p, int tile, bool if4, int out_type, hipStream_
 // The argument checks of an NVFP4 fos_gemm_linear_rows, nothing launched: for a caller that launches something ahead of it.
 int check_gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
                       double denominator, int64_t M, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias, float *d_amax);
-// The product of a layer's call.  Its plan is made for fragments that the quantize kernel writes: linear_reads_fragments says
-// whether the shape takes them, at the beginning of the scratch; A null: they are there, otherwise codes and scales, for the
+// The product of a layer's call.  Its plan is made for fragments that the quantize kernel writes: linear_sizes says
+// whether the shape takes them, at the beginning of the scratch, and how much of that there should be (`best`) or can be (`least`: from
+// codes).  A null: they are there, otherwise codes and scales, for the
 // same plan (`as_given`: an input that the streaming quantize kernels would read at another address) or for the one of
 // products from codes.  Arguments checked by check_gemm_linear.
-size_t linear_scratch_bytes(int64_t M, int64_t N, int64_t K);
-bool linear_reads_fragments(int64_t M, int64_t N, int64_t K);
+struct LinearSizes {
+    size_t least, best;
+    bool fragments;
+};
+LinearSizes linear_sizes(int64_t M, int64_t N, int64_t K);
 int gemm_linear(const uint8_t *A, const uint8_t *B, const uint8_t *sfA, const uint8_t *sfB, const float *amax_a, const float *amax_b,
                 double denominator, int64_t M, int64_t rows, int64_t N, int64_t K, void *D, int out_type, int64_t ldd, const void *bias,
                 float *d_amax, bool as_given, void *scratch, size_t scratch_bytes, fos_stream_t stream);

@@ -546,7 +546,7 @@ extern "C" int fos_quantize(const void *x, int x_type, int64_t rows, int64_t col
 namespace {
 struct LinearScratch {
     size_t codes = 0, sf, amax, partials, gemm, least, total;  // (least: without room for the operand as fragments)
-    LinearScratch(int64_t rows, int64_t cols, int64_t N, bool direct = false) {
+    LinearScratch(int64_t rows, int64_t cols, const fos::LinearSizes &product, bool direct) {
         auto up = [](size_t v) { return (v + 255) / 256 * 256; };
         const size_t elems = direct ? 0 : (size_t)fos_padded_rows(rows) * (size_t)fos_padded_cols(cols);
         sf = up(elems / 2);
@@ -555,9 +555,10 @@ struct LinearScratch {
         gemm = partials + up(fos_quantize_workspace_bytes(rows, cols));
         // (fragments from a 64 KiB boundary: 8.3 KiB into the block the layer of 128 x 14336 -> 4096 took 33.1 us, so 32.9)
         if (direct) gemm = (gemm + 65535) / 65536 * 65536;
-        least = gemm + fos_gemm_workspace_bytes(gemm_rows(rows, cols), N, fos_padded_cols(cols));
-        total = gemm + fos::linear_scratch_bytes(gemm_rows(rows, cols), N, fos_padded_cols(cols));
+        least = gemm + product.least;
+        total = gemm + product.best;
     }
+    static fos::LinearSizes product(int64_t rows, int64_t cols, int64_t N) { return fos::linear_sizes(gemm_rows(rows, cols), N, fos_padded_cols(cols)); }
     // rows the product is made for: a small batch's own where the weight-streaming kernels take it
     static int64_t gemm_rows(int64_t rows, int64_t cols) {
         return rows < 128 && fos_padded_cols(cols) % 256 == 0 ? rows : fos_padded_rows(rows);
@@ -567,22 +568,23 @@ struct LinearScratch {
 
 extern "C" size_t fos_linear_nvfp4_scratch_bytes(int64_t rows, int64_t cols, int64_t N) {
     if (rows <= 0 || cols <= 0 || N <= 0) return 0;
-    return LinearScratch(rows, cols, N).total;
+    return LinearScratch(rows, cols, LinearScratch::product(rows, cols, N), false).total;
 }
 
 // What a streaming quantize kernel reads, and the product wants converted, goes straight into the product's scratch.
-static bool writes_fragments(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int64_t N) {
-    return x_type != FOS_T_F32 && streamable(x, cols, ld) && fos::linear_reads_fragments(LinearScratch::gemm_rows(rows, cols), N, fos_padded_cols(cols));
+static bool writes_fragments(const void *x, int x_type, int64_t cols, int64_t ld, const fos::LinearSizes &product) {
+    return product.fragments && x_type != FOS_T_F32 && streamable(x, cols, ld);
 }
 
 extern "C" size_t fos_linear_nvfp4_scratch_for(const void *x, int x_type, int64_t rows, int64_t cols, int64_t ld, int64_t N, size_t *least) {
-    const bool sizes = rows > 0 && cols > 0 && N > 0;
-    const LinearScratch at = sizes ? LinearScratch(rows, cols, N) : LinearScratch(1, 1, 1);
+    if (least) *least = 0;
+    if (rows <= 0 || cols <= 0 || N <= 0) return 0;
+    const fos::LinearSizes product = LinearScratch::product(rows, cols, N);
+    const LinearScratch at(rows, cols, product, false);
+    const size_t best = writes_fragments(x, x_type, cols, ld, product) ? LinearScratch(rows, cols, product, true).total : at.total;
     const size_t fewest = at.least < at.total ? at.least : at.total;
-    size_t best = at.total;
-    if (sizes && writes_fragments(x, x_type, rows, cols, ld, N)) best = LinearScratch(rows, cols, N, true).total;
-    if (least) *least = !sizes ? 0 : fewest < best ? fewest : best;
-    return sizes ? best : 0;
+    if (least) *least = fewest < best ? fewest : best;
+    return best;
 }
 
 extern "C" int64_t fos_linear_nvfp4_rows(int64_t rows, int64_t cols) {
@@ -606,9 +608,13 @@ extern "C" int fos_linear_nvfp4_into_zero(const void *x, int x_type, int64_t row
     if (!scratch) return FOS_E_NULL_POINTER;
     if (rows <= 0 || cols <= 0 || N <= 0) return FOS_E_BAD_SHAPE;
     if (((uintptr_t)scratch & 255) || ((uintptr_t)d_amax & 3)) return FOS_E_BAD_ALIGNMENT;
-    const LinearScratch lean(rows, cols, N, true);
-    const bool direct = scratch_bytes >= lean.total && writes_fragments(x, x_type, rows, cols, ld, N);
-    const LinearScratch at = direct ? lean : LinearScratch(rows, cols, N);
+    const fos::LinearSizes product = LinearScratch::product(rows, cols, N);
+    bool direct = writes_fragments(x, x_type, cols, ld, product);
+    LinearScratch at(rows, cols, product, direct);
+    if (direct && scratch_bytes < at.total) {
+        direct = false;
+        at = LinearScratch(rows, cols, product, false);
+    }
     if (!direct && scratch_bytes < (at.least < at.total ? at.least : at.total)) return FOS_E_WORKSPACE;
     uint8_t *base = static_cast<uint8_t *>(scratch);
     float *amax = x_amax ? const_cast<float *>(x_amax) : reinterpret_cast<float *>(base + at.amax);
